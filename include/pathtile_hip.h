@@ -276,6 +276,52 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
                   int L, int K, int GZ, void* stream);
 
 /*
+ * The S4ConvD block around the convolution (kernels/warp_tiled_ampere.py:
+ * 1122-1190 in the reference), FP32, in fused passes. For x [B, L, H], the
+ * diagonal state-space parameters log_dt [H], c_re, c_im, log_a_re, a_im
+ * [H, states], skip [H], the projection w [2H, H] and bias [2H]:
+ *   taps[h][t] = 2 Re sum_n C_eff[h,n] exp(dt A t) (+ skip[h] at t = L / 2)
+ *   u = conv(x transposed to [B, H, L], taps)              (_mix)
+ *   y = GLU(w gelu(v) + bias) + x, v = dropout(u) or u     (_tail)
+ * and the gradients of y for gy [B, L, H] (_bwd). Served: H a multiple of 32
+ * up to 256, 1 <= L <= 48, B >= 1, B H L < 2^31 (PT_ERR_SHAPE otherwise);
+ * x, xt, u, v, y, gy, gx, prep, bias and workspace 16-byte aligned
+ * (PT_ERR_ALIGN). The projection runs on the BF16 matrix cores with both
+ * operands split three ways (FP32 accuracy; a sum that is not finite is
+ * recomputed by the FP32 chain).
+ *
+ * prep holds the taps and the split projection between the calls of one
+ * block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
+ * also lays out what _bwd needs. xt and u are [B, H, L]; _bwd takes xt, the
+ * tail's input v, and dropout's byte mask and scale (mask NULL: none). Its
+ * outputs gx, {dw, dbias} and the six parameter gradients (all or none, by
+ * d_skip) are each skipped where NULL. waves_per_block, algo,
+ * dx_waves_per_block and threads_per_block are the convolution's
+ * (pt_dwconv1d_fwd_f32_algo, pt_dwconv1d_dk_det_f32).
+ */
+int pt_s4_block_prep_values(int H, int L, size_t* floats);
+int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re,
+                        const float* c_im, const float* log_a_re, const float* a_im,
+                        const float* skip, const float* w, float* prep, float* xt,
+                        float* u, int B, int H, int L, int states, int backward,
+                        int waves_per_block, int algo, void* stream);
+int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep,
+                         const float* w, const float* bias, float* y, int B, int H,
+                         int L, void* stream);
+int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block,
+                                    size_t* bytes);
+int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v,
+                        const unsigned char* mask, float scale, const float* prep,
+                        const float* w, const float* bias, const float* log_dt,
+                        const float* c_re, const float* c_im, const float* log_a_re,
+                        const float* a_im, float* gx, float* d_log_dt, float* d_c_re,
+                        float* d_c_im, float* d_log_a_re, float* d_a_im,
+                        float* d_skip, float* dw, float* dbias, void* workspace,
+                        size_t workspace_bytes, int B, int H, int L, int states,
+                        int dx_waves_per_block, int algo, int threads_per_block,
+                        void* stream);
+
+/*
  * Compiled resources of the kernel that serves (L, K) for `kernel_id`
  * (PT_KERNEL_*), as hipFuncGetAttributes reports them on the current device:
  * registers per lane, static LDS bytes, scratch (private) bytes per lane and

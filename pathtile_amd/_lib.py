@@ -77,6 +77,13 @@ SIGNATURES = {
     "pt_dwconv1d_dk_long_f32": (
         _i, [_vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _vp]
     ),
+    "pt_s4_block_prep_values": (_i, [_i, _i, _szp]),
+    "pt_s4_block_mix_f32": (_i, [_vp] * 11 + [_i] * 7 + [_vp]),
+    "pt_s4_block_tail_f32": (_i, [_vp] * 6 + [_i] * 3 + [_vp]),
+    "pt_s4_block_bwd_workspace_bytes": (_i, [_i, _i, _i, _i, _szp]),
+    "pt_s4_block_bwd_f32": (
+        _i, [_vp] * 4 + [ctypes.c_float] + [_vp] * 18 + [ctypes.c_size_t] + [_i] * 7 + [_vp]
+    ),
     "pt_kernel_attributes": (_i, [_i, _i, _i, _ip, _ip, _ip, _ip]),
     "pt_dynamic_lds_bytes": (_i, [_i, _i, _i, _i, _ip]),
 }

@@ -41,6 +41,7 @@ SOURCES = [
     "inst_long_vec.hip",
     "inst_long_s3.hip",
     "inst_long_s3_vec.hip",
+    "s4_block.hip",
 ]
 INCLUDE = ROOT / "include"
 BUILD_DIR = PKG / "_build"

@@ -13,6 +13,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "dwconv1d_host.hpp"
 #include "dwconv1d_kernels.hpp"
 #include "dwconv1d_tables.hpp"
 #include "pathtile_hip.h"
@@ -103,7 +104,7 @@ static int device_attr(int fallback) {
   return n;
 }
 
-static int num_cus() { return device_attr<hipDeviceAttributeMultiprocessorCount>(256); }
+int num_cus() { return device_attr<hipDeviceAttributeMultiprocessorCount>(256); }
 
 struct OccEntry {
   const void* fn;
@@ -116,7 +117,7 @@ static OccEntry g_occ[512];
 static int g_occ_n = 0;
 
 // Resident workgroups per CU for (kernel, block size, dynamic LDS).
-static int blocks_per_cu(const void* fn, int block, size_t lds) {
+int blocks_per_cu(const void* fn, int block, size_t lds) {
   {
     std::lock_guard<std::mutex> lk(g_occ_mu);
     for (int i = 0; i < g_occ_n; ++i)
@@ -398,7 +399,7 @@ static bool valid_dk_threads(int t) {
   return t >= kWave && t <= kMaxDkThreads && (t % kWave) == 0;
 }
 
-static int launch(const void* fn, uint32_t grid, uint32_t block, size_t lds,
+int launch(const void* fn, uint32_t grid, uint32_t block, size_t lds,
                   void* stream, void** args) {
   hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(block), args, lds,
                                  (hipStream_t)stream);

@@ -1,0 +1,248 @@
+// s4_block.hip — the S4ConvD block's entry points: argument checks, workspace
+// layout and the launches of s4_kernels.hpp around the convolution's own.
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include "dwconv1d_host.hpp"
+#include "pathtile_hip.h"
+#include "s4_kernels.hpp"
+
+namespace pt {
+
+using TailFwdFn = void (*)(const float*, const float*, const __bf16*, const float*, const float*,
+                           float*, uint32_t, uint32_t, uint32_t);
+using TailBwdFn = void (*)(const float*, const float*, const uint8_t*, float, const __bf16*,
+                           const float*, const float*, float*, float*, uint32_t, uint32_t, uint32_t,
+                           uint32_t);
+using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t, uint32_t,
+                      uint32_t);
+
+struct TailKernels {
+  TailFwdFn fwd;
+  TailBwdFn bwd;
+  DwFn dw[2];  // [16-byte loads]
+  int nw, bt, dw_nw, dw_split;
+  size_t dw_lds;
+};
+
+template <int CT>
+constexpr TailKernels tail_kernels() {
+  return {&s4_tail_fwd_kernel<CT>, &s4_tail_bwd_kernel<CT>,
+          {&s4_dw_kernel<CT, false>, &s4_dw_kernel<CT, true>},
+          TailGeo<CT>::NW, TailGeo<CT>::BT, DwGeo<CT>::NW, DwGeo<CT>::SPLIT, DwGeo<CT>::lds};
+}
+
+// [H / 32 - 1]
+static const TailKernels kTail[8] = {tail_kernels<2>(),  tail_kernels<4>(),  tail_kernels<6>(),
+                                     tail_kernels<8>(),  tail_kernels<10>(), tail_kernels<12>(),
+                                     tail_kernels<14>(), tail_kernels<16>()};
+
+static int check_block(int B, int H, int L, int states) {
+  if (B < 1 || H < 32 || H > kS4MaxH || H % 32 != 0 || L < 1 || L > kMaxL || states < 1)
+    return PT_ERR_SHAPE;
+  if ((long long)B * H * L >= (1LL << 31) || (long long)H * states >= (1LL << 28))
+    return PT_ERR_SHAPE;
+  return PT_OK;
+}
+
+static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+static size_t round_up(size_t n, size_t q) { return (n + q - 1) / q * q; }
+
+// Token ranges of the weight gradient: one workgroup per CU (its accumulators
+// and fragments take half of the registers), at least four 32-token steps
+// each. A function of the shape alone, so that the workspace is too.
+static uint32_t dw_steps_per_range(uint32_t nsteps, int split) {
+  const uint32_t ranges = 256u / (uint32_t)split;
+  const uint32_t per = (nsteps + ranges - 1) / ranges;
+  return per < 4 ? 4 : per;
+}
+
+// Workspace of the backward, in floats: dP [2H][np] (later dX before its
+// transpose), du [B,H,L], the weight gradient's partials, dk [H][L], and the
+// convolution's own partials.
+struct BwdLayout {
+  size_t np, du, part, dk, conv, conv_bytes, total;
+  uint32_t nsteps, per, ranges;
+};
+
+static int bwd_layout(int B, int H, int L, int threads, BwdLayout* o) {
+  const TailKernels& k = kTail[H / 32 - 1];
+  const size_t ntok = (size_t)B * L;
+  o->np = round_up(ntok, 64);
+  o->nsteps = (uint32_t)((ntok + kDwTok - 1) / kDwTok);
+  o->per = dw_steps_per_range(o->nsteps, k.dw_split);
+  o->ranges = (o->nsteps + o->per - 1) / o->per;
+  o->du = (size_t)2 * H * o->np;
+  o->part = o->du + ntok * H;
+  o->dk = o->part + round_up((size_t)o->ranges * (2 * H * H + 2 * H), 64);
+  o->conv = o->dk + round_up((size_t)H * L, 64);
+  const int st = pt_dwconv1d_dk_det_workspace_bytes(B, H, L, L, threads, &o->conv_bytes);
+  if (st != PT_OK) return st;
+  o->total = o->conv * sizeof(float) + o->conv_bytes;
+  return PT_OK;
+}
+
+static uint32_t resident_grid(const void* fn, int block, size_t lds, uint32_t work) {
+  const uint32_t n = (uint32_t)(blocks_per_cu(fn, block, lds) * num_cus());
+  return n < work ? n : work;
+}
+
+static int transpose_launch(const float* d, const float* add, float* out, int B, int H, int L,
+                            void* stream) {
+  const size_t lds = (size_t)L * (H + 1) * sizeof(float);
+  const bool vec = L % 4 == 0 && aligned16(d) && aligned16(out);
+  if (add) {
+    const void* fn = vec ? (const void*)&s4_transpose_add_kernel<true>
+                         : (const void*)&s4_transpose_add_kernel<false>;
+    void* args[] = {&d, &add, &out, &B, &H, &L};
+    return launch(fn, resident_grid(fn, kTransThreads, lds, (uint32_t)B), kTransThreads, lds,
+                  stream, args);
+  }
+  const void* fn =
+      vec ? (const void*)&s4_transpose_kernel<true> : (const void*)&s4_transpose_kernel<false>;
+  void* args[] = {&d, &out, &B, &H, &L};
+  return launch(fn, resident_grid(fn, kTransThreads, lds, (uint32_t)B), kTransThreads, lds, stream,
+                args);
+}
+
+}  // namespace pt
+
+extern "C" {
+
+int pt_s4_block_prep_values(int H, int L, size_t* floats) {
+  if (!floats) return PT_ERR_NULL;
+  const int st = pt::check_block(1, H, L, 1);
+  if (st != PT_OK) return st;
+  *floats = pt::round_up((size_t)H * L, 64) + pt::wfrag_values(H);
+  return PT_OK;
+}
+
+int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, const float* c_im,
+                        const float* log_a_re, const float* a_im, const float* skip,
+                        const float* w, float* prep, float* xt, float* u, int B, int H, int L,
+                        int states, int backward, int waves_per_block, int algo, void* stream) {
+  int st = pt::check_block(B, H, L, states);
+  if (st != PT_OK) return st;
+  if (!x || !log_dt || !c_re || !c_im || !log_a_re || !a_im || !skip || !w || !prep || !xt || !u)
+    return PT_ERR_NULL;
+  if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(xt) || !pt::aligned16(u))
+    return PT_ERR_ALIGN;
+  float* taps = prep;
+  __bf16* wf = reinterpret_cast<__bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  {
+    const int frags = 2 * H * H / 8 * (backward ? 2 : 1);
+    const uint32_t grid =
+        (uint32_t)(H + (frags + pt::kPrepThreads - 1) / pt::kPrepThreads);
+    void* args[] = {&log_dt, &c_re, &c_im, &log_a_re, &a_im, &skip, &w, &taps, &wf, &H, &L,
+                    &states, &backward};
+    st = pt::launch((const void*)&pt::s4_prep_kernel, grid, pt::kPrepThreads, 0, stream, args);
+    if (st != PT_OK) return st;
+  }
+  st = pt::transpose_launch(x, nullptr, xt, B, H, L, stream);
+  if (st != PT_OK) return st;
+  return pt_dwconv1d_fwd_f32_algo(xt, taps, u, B, H, L, L, waves_per_block, algo, stream);
+}
+
+int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
+                         const float* bias, float* y, int B, int H, int L, void* stream) {
+  const int st = pt::check_block(B, H, L, 1);
+  if (st != PT_OK) return st;
+  if (!v || !x || !prep || !w || !bias || !y) return PT_ERR_NULL;
+  if (!pt::aligned16(v) || !pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(bias) ||
+      !pt::aligned16(y))
+    return PT_ERR_ALIGN;
+  const pt::TailKernels& k = pt::kTail[H / 32 - 1];
+  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L;
+  uint32_t ntiles = (ntok + pt::kTailTok - 1) / pt::kTailTok;
+  const size_t lds = pt::tail_fwd_lds(H);
+  const int block = k.nw * pt::kWave;
+  void* args[] = {&v, &x, &wf, &w, &bias, &y, &ntok, &uL, &ntiles};
+  return pt::launch((const void*)k.fwd,
+                    pt::resident_grid((const void*)k.fwd, block, lds, ntiles), (uint32_t)block,
+                    lds, stream, args);
+}
+
+int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block, size_t* bytes) {
+  if (!bytes) return PT_ERR_NULL;
+  int st = pt::check_block(B, H, L, 1);
+  if (st != PT_OK) return st;
+  pt::BwdLayout o;
+  st = pt::bwd_layout(B, H, L, threads_per_block, &o);
+  if (st == PT_OK) *bytes = o.total;
+  return st;
+}
+
+int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const unsigned char* mask,
+                        float scale, const float* prep, const float* w, const float* bias,
+                        const float* log_dt, const float* c_re, const float* c_im,
+                        const float* log_a_re, const float* a_im, float* gx, float* d_log_dt,
+                        float* d_c_re, float* d_c_im, float* d_log_a_re, float* d_a_im,
+                        float* d_skip, float* dw, float* dbias, void* workspace,
+                        size_t workspace_bytes, int B, int H, int L, int states,
+                        int dx_waves_per_block, int algo, int threads_per_block, void* stream) {
+  int st = pt::check_block(B, H, L, states);
+  if (st != PT_OK) return st;
+  if (!gy || !xt || !v || !prep || !w || !bias) return PT_ERR_NULL;
+  const bool taps_grad = d_skip != nullptr;
+  if (taps_grad && (!log_dt || !c_re || !c_im || !log_a_re || !a_im || !d_log_dt || !d_c_re ||
+                    !d_c_im || !d_log_a_re || !d_a_im))
+    return PT_ERR_NULL;
+  if ((dw == nullptr) != (dbias == nullptr)) return PT_ERR_NULL;
+  if (!pt::aligned16(gy) || !pt::aligned16(xt) || !pt::aligned16(v) || !pt::aligned16(prep) ||
+      !pt::aligned16(bias) || !pt::aligned16(workspace) || (gx && !pt::aligned16(gx)))
+    return PT_ERR_ALIGN;
+  pt::BwdLayout o;
+  st = pt::bwd_layout(B, H, L, threads_per_block, &o);
+  if (st != PT_OK) return st;
+  if (!workspace || workspace_bytes < o.total) return PT_ERR_WORKSPACE;
+  const pt::TailKernels& k = pt::kTail[H / 32 - 1];
+  float* const ws = static_cast<float*>(workspace);
+  float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk, *dxt = ws;
+  const float* taps = prep;
+  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, np = (uint32_t)o.np;
+  {
+    uint32_t ntiles = (ntok + k.bt - 1) / k.bt;
+    const size_t lds = pt::tail_bwd_lds(H);
+    const int block = k.nw * pt::kWave;
+    void* args[] = {&gy, &v, &mask, &scale, &wf, &w, &bias, &du, &dp, &ntok, &uL, &ntiles, &np};
+    st = pt::launch((const void*)k.bwd, pt::resident_grid((const void*)k.bwd, block, lds, ntiles),
+                    (uint32_t)block, lds, stream, args);
+    if (st != PT_OK) return st;
+  }
+  if (dw) {
+    const void* fn = (const void*)k.dw[L % 4 == 0];
+    const float* cdp = dp;
+    void* args[] = {&cdp, &v, &part, &ntok, &uL, &o.nsteps, &o.per, &np};
+    st = pt::launch(fn, o.ranges * (uint32_t)k.dw_split, (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds,
+                    stream, args);
+    if (st != PT_OK) return st;
+    int nw = 2 * H * H, nb = 2 * H, nr = (int)o.ranges;
+    const float* cpart = part;
+    void* rargs[] = {&cpart, &dw, &dbias, &nw, &nb, &nr};
+    st = pt::launch((const void*)&pt::s4_dw_reduce_kernel, (uint32_t)((nw + nb + 15) / 16), 256, 0,
+                    stream, rargs);
+    if (st != PT_OK) return st;
+  }
+  if (gx) {  // dX before its transpose takes dP's place, which is read by now
+    st = pt_dwconv1d_dx_f32_algo(du, taps, dxt, B, H, L, L, dx_waves_per_block, algo, stream);
+    if (st != PT_OK) return st;
+    st = pt::transpose_launch(dxt, gy, gx, B, H, L, stream);
+    if (st != PT_OK) return st;
+  }
+  if (!taps_grad) return PT_OK;
+  st = pt_dwconv1d_dk_det_f32(du, xt, dk, ws + o.conv, o.conv_bytes, B, H, L, L, threads_per_block,
+                              stream);
+  if (st != PT_OK) return st;
+  const float* cdk = dk;
+  void* targs[] = {&cdk, &log_dt, &c_re, &c_im, &log_a_re, &a_im, &d_log_dt, &d_c_re, &d_c_im,
+                   &d_log_a_re, &d_a_im, &d_skip, &L, &states};
+  return pt::launch((const void*)&pt::s4_taps_grad_kernel, (uint32_t)H, pt::kPrepThreads, 0, stream,
+                    targs);
+}
+
+}  // extern "C"

@@ -26,13 +26,17 @@ reference's composition (``reference_depthwise_conv`` + a separate skip add).
 
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Any
 
 import torch
 from torch import nn
 
-from .runtime import MAX_L, get_runtime, reference_depthwise_conv
+from . import _lib
+from .runtime import (
+    KERNEL_EVENTS, MAX_L, _ptr, _stream_handle, get_runtime, reference_depthwise_conv,
+)
 
 
 def _backend() -> str:
@@ -89,6 +93,20 @@ def depthwise_conv_skip_ampere(x: torch.Tensor, k: torch.Tensor, skip: torch.Ten
     return DepthConvSkipAmpere.apply(x, k, skip)
 
 
+def _taps(log_dt, C_re, C_im, log_A_re, A_im, taps: int,
+          device: torch.device | None = None) -> torch.Tensor:
+    dt = log_dt.exp()
+    A = torch.complex(-log_A_re.exp(), A_im)
+    C = torch.complex(C_re, C_im)
+    dtA = A * dt[:, None]
+    C_eff = C * (dtA.exp() - 1.0) / A
+    t = torch.arange(taps, device=log_dt.device if device is None else device,
+                     dtype=torch.float32)
+    powers = torch.exp(dtA[:, :, None] * t)  # [H, N/2, taps]
+    # elementwise product and sum over n (no batched matmul)
+    return (2.0 * (C_eff[:, :, None] * powers).sum(dim=1).real).contiguous()
+
+
 class S4ConvKernel(nn.Module):
     """Diagonal SSM convolution kernel (:1122-1169). For channel h and tap t:
     ``k[h, t] = 2 Re( sum_n C_eff[h, n] * exp(dt[h] A[h, n] t) )`` with
@@ -108,15 +126,7 @@ class S4ConvKernel(nn.Module):
         self.A_im = nn.Parameter(torch.ones(hidden_dim, half))
 
     def build_kernel(self, taps: int, device: torch.device) -> torch.Tensor:
-        dt = self.log_dt.exp()
-        A = torch.complex(-self.log_A_re.exp(), self.A_im)
-        C = torch.complex(self.C_re, self.C_im)
-        dtA = A * dt[:, None]
-        C_eff = C * (dtA.exp() - 1.0) / A
-        t = torch.arange(taps, device=device, dtype=torch.float32)
-        powers = torch.exp(dtA[:, :, None] * t)  # [H, N/2, taps]
-        # elementwise product and sum over n (no batched matmul)
-        return (2.0 * (C_eff[:, :, None] * powers).sum(dim=1).real).contiguous()
+        return _taps(self.log_dt, self.C_re, self.C_im, self.log_A_re, self.A_im, taps, device)
 
     def forward(self, x: torch.Tensor, skip: torch.Tensor | None = None) -> torch.Tensor:
         """``conv(x, k)`` with ``k = build_kernel(L)``; with ``skip`` the block's
@@ -140,6 +150,145 @@ class S4ConvKernel(nn.Module):
         raise RuntimeError(f"Unknown training backend: {backend}")
 
 
+# ---------------------------------------------------------------------------
+# The whole block in fused HIP passes (pt_s4_block_*)
+# ---------------------------------------------------------------------------
+FUSED_MAX_H = 256  # H a multiple of 32 up to here
+
+
+def _size_query(fn: str, *args: int) -> int:
+    out = ctypes.c_size_t(0)
+    _lib.check(getattr(_lib.load(), fn)(*args, ctypes.byref(out)), fn)
+    return int(out.value)
+
+
+def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight,
+               backward: bool):
+    """Taps, split projection, transposed input and the convolution's output:
+    (prep, xt, u), xt and u [B, H, L]."""
+    runtime = get_runtime()
+    runtime._check_open()
+    B, L, H = x.shape
+    prep = torch.empty(_size_query("pt_s4_block_prep_values", H, L), device=x.device)
+    xt, u = torch.empty((2, B, H, L), device=x.device).unbind(0)
+    with torch.cuda.device(x.device):
+        st = runtime._lib.pt_s4_block_mix_f32(
+            _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
+            _ptr(skip), _ptr(weight), _ptr(prep), _ptr(xt), _ptr(u), B, H, L, c_re.shape[1],
+            int(backward), runtime.waves_per_block, runtime._rows_algo_id,
+            _stream_handle(x.device))
+    _lib.check(st, "pt_s4_block_mix_f32")
+    return prep, xt, u
+
+
+def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias) -> torch.Tensor:
+    runtime = get_runtime()
+    B, L, H = x.shape
+    y = torch.empty_like(x)
+    with torch.cuda.device(x.device):
+        st = runtime._lib.pt_s4_block_tail_f32(
+            _ptr(v), _ptr(x), _ptr(prep), _ptr(weight), _ptr(bias), _ptr(y), B, H, L,
+            _stream_handle(x.device))
+    _lib.check(st, "pt_s4_block_tail_f32")
+    return y
+
+
+class S4BlockFused(torch.autograd.Function):
+    """``S4ConvBlock.forward`` as one function of the input and the block's
+    parameters: transposes, taps, convolution with the skip term, dropout,
+    GELU, projection, GLU and residual. Dropout's mask is PyTorch's own draw
+    for a tensor of the convolution's shape, as the separate module draws it."""
+
+    @staticmethod
+    def forward(ctx: Any, x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, p: float):
+        prep, xt, v = _fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, True)
+        mask = None
+        if p > 0.0:
+            v, mask = torch.native_dropout(v, p, True)
+        y = _fused_tail(v, x, prep, weight, bias)
+        ctx.save_for_backward(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
+                              prep, xt, v, mask)
+        ctx.scale = 1.0 / (1.0 - p)
+        return y
+
+    @staticmethod
+    def backward(ctx: Any, gy: torch.Tensor):
+        (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
+         prep, xt, v, mask) = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():  # create_graph: differentiate the composition
+            return _composed_grads(ctx, gy, mask)
+        runtime = get_runtime()
+        runtime._check_open()
+        B, L, H = x.shape
+        gy = gy.contiguous()
+        if gy.data_ptr() % 16:
+            gy = gy.clone()
+        gx = torch.empty_like(x) if need[0] else None
+        taps = any(need[1:7])
+        gp = [torch.empty_like(t) for t in (log_dt, c_re, c_im, log_a_re, a_im, skip)] \
+            if taps else [None] * 6
+        proj = need[7] or need[8]
+        gw, gb = (torch.empty_like(weight), torch.empty_like(bias)) if proj else (None, None)
+        nbytes = _size_query("pt_s4_block_bwd_workspace_bytes", B, H, L, runtime.bwdk_block)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+
+        def opt(t):
+            return None if t is None else _ptr(t)
+
+        with torch.cuda.device(x.device):
+            st = runtime._lib.pt_s4_block_bwd_f32(
+                _ptr(gy), _ptr(xt), _ptr(v), opt(mask), ctx.scale, _ptr(prep), _ptr(weight),
+                _ptr(bias), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
+                opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
+                c_re.shape[1], runtime.dx_waves_per_block, runtime._rows_algo_id,
+                runtime.bwdk_block, _stream_handle(x.device))
+        _lib.check(st, "pt_s4_block_bwd_f32")
+        grads = [gx, gp[5], *gp[:5], gw, gb]
+        return (*(g if n else None for g, n in zip(grads, need)), None)
+
+
+def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
+    """The block's gradients through differentiable operations on the saved
+    inputs, for a backward that is itself differentiated (the convolution's
+    own backward stays first order, as its autograd function is)."""
+    inputs = ctx.saved_tensors[:9]
+    x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
+    k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
+    v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)
+    if mask is not None:
+        v = v * mask * ctx.scale
+    z = nn.functional.conv1d(nn.functional.gelu(v), weight, bias)
+    y = nn.functional.glu(z, dim=1).transpose(1, 2) + x
+    need = ctx.needs_input_grad[:9]
+    got = iter(torch.autograd.grad(y, [t for t, n in zip(inputs, need) if n], gy,
+                                   create_graph=True))
+    return (*(next(got) if n else None for n in need), None)
+
+
+def _no_hooks(m: nn.Module) -> bool:
+    return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or "forward" in m.__dict__)
+
+
+def _tracing() -> bool:
+    """True where something watches or rewrites the block's single operations:
+    compilers and tracers, functorch transforms, forward-mode AD, dispatch and
+    function modes (but the default-device one), autocast, module hooks."""
+    if torch._C._len_torch_function_stack():
+        from torch.overrides import _get_current_function_mode_stack
+        from torch.utils._device import DeviceContext
+
+        if any(type(m) is not DeviceContext for m in _get_current_function_mode_stack()):
+            return True
+    return bool(torch._C._len_torch_dispatch_stack()
+                or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.is_autocast_enabled("cuda")
+                or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or nn.modules.module._has_any_global_hook())
+
+
 class S4ConvBlock(nn.Module):
     """Depthwise S4 convolution + skip, GELU, dropout, GLU projection and a
     residual connection (:1172-1190); input and output are ``[B, L, H]``."""
@@ -155,7 +304,55 @@ class S4ConvBlock(nn.Module):
             nn.GLU(dim=1),
         )
 
+    def _fused_inputs(self, x: torch.Tensor):
+        """The parameters in S4BlockFused's order, or None where the block
+        runs as separate operations: another backend, layout, type or device,
+        a shape the fused passes do not serve, modules that were replaced,
+        subclassed or hooked, kernel timing through KERNEL_EVENTS (its phases
+        are the separate launches), or tracing of any kind."""
+        kl, act, drop, out = self.kernel_layer, self.activation, self.dropout, self.output_linear
+        if not (type(x) is torch.Tensor and x.dim() == 3 and x.is_cuda
+                and type(kl) is S4ConvKernel and type(act) is nn.GELU
+                and "build_kernel" not in kl.__dict__ and act.approximate == "none"
+                and type(drop) is nn.Dropout and not drop.inplace and 0.0 <= drop.p < 1.0
+                and type(out) is nn.Sequential and len(out) == 2
+                and type(out[0]) is nn.Conv1d and type(out[1]) is nn.GLU and out[1].dim == 1):
+            return None
+        B, L, H = x.shape
+        conv = out[0]
+        params = (self.skip, kl.log_dt, kl.C_re, kl.C_im, kl.log_A_re, kl.A_im, conv.weight,
+                  conv.bias)
+        half = kl.C_re.shape[-1]
+        shapes = ((H,), (H,), (H, half), (H, half), (H, half), (H, half), (2 * H, H, 1), (2 * H,))
+        if not (x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
+                and 1 <= L <= MAX_L and 32 <= H <= FUSED_MAX_H and H % 32 == 0 and kl.H == H
+                and half >= 1 and B >= 1 and x.numel() < 2**31
+                and conv.groups == 1 and conv.stride == (1,) and conv.padding == (0,)
+                and conv.bias is not None and _backend() == "warp"
+                and not KERNEL_EVENTS.enabled):
+            return None
+        for t, shape in zip(params, shapes):
+            if not (type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32
+                    and t.device == x.device and t.shape == shape and t.is_contiguous()):
+                return None
+        if conv.bias.data_ptr() % 16 or _tracing():
+            return None
+        if not all(_no_hooks(m) for m in (kl, act, drop, out, conv, out[1])):
+            return None
+        return params
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        params = self._fused_inputs(x)
+        if params is not None:
+            p = float(self.dropout.p) if self.dropout.training else 0.0
+            if torch.is_grad_enabled() and (x.requires_grad
+                                            or any(t.requires_grad for t in params)):
+                return S4BlockFused.apply(x, *params, p)
+            skip, *kernel, weight, bias = params
+            prep, _, v = _fused_mix(x, skip, *kernel, weight, False)
+            if p > 0.0:
+                v = torch.native_dropout(v, p, True)[0]
+            return _fused_tail(v, x, prep, weight, bias)
         x_hl = x.transpose(1, 2).contiguous()
         y = self.kernel_layer(x_hl, self.skip)
         y = self.output_linear(self.activation(self.dropout(y)))

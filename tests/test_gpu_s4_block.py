@@ -1,0 +1,230 @@
+"""The S4ConvD block's fused HIP passes (pt_s4_block_*) on the GPU (marked
+``gpu``): output and every gradient against the same block in FP64 on the CPU
+(the "pytorch" composition), over the channel counts, row lengths, state
+counts and batch sizes where tiles end; and that every condition for running
+the separate operations instead still gives the block's result.
+
+Bar: 2e-6 of the tensor's 2-norm for outputs and input gradients (sums of up
+to 512 products in FP32: sqrt(512) 2^-24 = 1.3e-6 for one rounding each at
+random), 2e-5 for the parameters' (sums over all columns, and the taps'
+gradients lose up to 1 / |dt A| through FP32 inputs of the chain)."""
+
+from __future__ import annotations
+
+import copy
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ACT_TOL = 2e-6
+PAR_TOL = 2e-5
+
+
+@pytest.fixture(scope="module", autouse=True)
+def rt():
+    from pathtile_amd import runtime
+
+    runtime.install_runtime(runtime.HipWarpRuntime())
+
+
+def _rel(a, b):
+    a, b = a.detach().double().cpu(), b.detach().double().cpu()
+    return float((a - b).norm() / b.norm().clamp_min(1e-30))
+
+
+def _make(B, H, L, state, p=0.0, seed=0):
+    from pathtile_amd import s4convd
+
+    torch.manual_seed(1000 + seed + B + H + L)
+    block = s4convd.S4ConvBlock(H, state, p)
+    x, gy = torch.randn(B, L, H), torch.randn(B, L, H)
+    return block, x, gy
+
+
+def _grads(block, x, gy):
+    x = x.clone().requires_grad_(True)
+    y = block(x)
+    return [y, *torch.autograd.grad(y, (x, *block.parameters()), gy.to(y.dtype))]
+
+
+def _fp64(block, x, gy):
+    from pathtile_amd.kernels import warp_tiled_ampere as wta
+
+    old, wta.TRAIN_CONV_BACKEND = wta.TRAIN_CONV_BACKEND, "pytorch"
+    try:
+        b = copy.deepcopy(block).cpu().double()
+        # build_kernel's tap index is FP32; whole numbers, so exact in FP64 too
+        return _grads(b, x.cpu().double(), gy.cpu().double())
+    finally:
+        wta.TRAIN_CONV_BACKEND = old
+
+
+def _check(got, ref, names):
+    for i, (a, b, n) in enumerate(zip(got, ref, names)):
+        assert a.shape == b.shape, n
+        assert _rel(a, b) < (ACT_TOL if i < 2 else PAR_TOL), (n, _rel(a, b))
+
+
+@pytest.mark.parametrize("B,H,L,state", [
+    (3, 32, 48, 64), (1, 32, 1, 2), (5, 64, 17, 16), (2, 64, 48, 70), (7, 96, 33, 32),
+    (4, 128, 48, 64), (11, 128, 23, 64), (1, 128, 5, 6), (40, 128, 48, 64), (3, 160, 20, 16),
+    (5, 192, 47, 32), (2, 224, 12, 8), (3, 256, 48, 64), (9, 256, 31, 18)])
+def test_fused_block_against_fp64(B, H, L, state):
+    print(f"[case] fused block B={B} H={H} L={L} state={state}", flush=True)
+    block, x, gy = _make(B, H, L, state)
+    names = ["y", "gx", *(n for n, _ in block.named_parameters())]
+    ref = _fp64(block, x, gy)
+    block.cuda()
+    assert block._fused_inputs(x.cuda()) is not None
+    got = _grads(block, x.cuda(), gy.cuda())
+    _check(got, ref, names)
+    again = _grads(block, x.cuda(), gy.cuda())
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    with torch.no_grad():
+        assert torch.equal(block(x.cuda()), got[0])
+
+
+def test_fused_block_many_tiles_per_workgroup():
+    """More tiles than resident workgroups, and several 32-token steps per
+    range of the weight gradient, against the separate operations."""
+    block, x, gy = _make(3000, 64, 37, 16)
+    block.cuda()
+    got = _grads(block, x.cuda(), gy.cuda())
+    block.activation.register_forward_hook(lambda *a: None)  # runs the separate operations
+    assert block._fused_inputs(x.cuda()) is None
+    with torch.backends.cudnn.flags(enabled=False):
+        ref = _grads(block, x.cuda(), gy.cuda())
+    names = ["y", "gx", *(n for n, _ in block.named_parameters())]
+    _check(got, ref, names)
+
+
+def test_fused_block_dropout_draws_the_modules_mask():
+    """Training with dropout: the mask of the separate module under the same
+    seed, in the output and the gradients."""
+    block, x, gy = _make(33, 96, 29, 16, p=0.3)
+    block.cuda().train()
+    torch.manual_seed(5)
+    got = _grads(block, x.cuda(), gy.cuda())
+    after = torch.cuda.get_rng_state()
+    block.activation.register_forward_hook(lambda *a: None)
+    torch.manual_seed(5)
+    with torch.backends.cudnn.flags(enabled=False):
+        ref = _grads(block, x.cuda(), gy.cuda())
+    assert torch.equal(after, torch.cuda.get_rng_state())
+    _check(got, ref, ["y", "gx", *(n for n, _ in block.named_parameters())])
+
+
+def test_fused_block_partial_gradients():
+    """Only what needs a gradient gets one, and it is the same."""
+    block, x, gy = _make(6, 64, 48, 16)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+    full = dict(zip(["x", *(n for n, _ in block.named_parameters())], _grads(block, x, gy)[1:]))
+    for keep in (["x"], ["output_linear.0.weight"], ["kernel_layer.C_re"], ["skip"]):
+        for n, q in block.named_parameters():
+            q.requires_grad_(n in keep)
+            q.grad = None
+        xi = x.clone().requires_grad_("x" in keep)
+        block(xi).backward(gy)
+        have = {n: q.grad for n, q in block.named_parameters() if q.grad is not None}
+        if xi.grad is not None:
+            have["x"] = xi.grad
+        assert set(have) == set(keep)
+        assert all(torch.equal(have[n], full[n]) for n in keep)
+
+
+def test_fused_block_second_order_through_the_projection():
+    """create_graph works as it does for the separate operations."""
+    block, x, gy = _make(3, 32, 20, 8)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+
+    def second(b):
+        y = b(x)
+        w = b.output_linear[0].weight
+        (g,) = torch.autograd.grad(y, w, gy, create_graph=True)
+        return g, torch.autograd.grad(g.square().sum(), w)[0]
+
+    with torch.backends.cudnn.flags(enabled=False):
+        got = second(block)
+        block.activation.register_forward_hook(lambda *a: None)
+        ref = second(block)
+    assert _rel(got[0], ref[0]) < PAR_TOL and _rel(got[1], ref[1]) < PAR_TOL
+
+
+def test_fused_block_non_finite_values_stay_in_their_windows():
+    """An Inf or NaN input reaches the tokens that the separate operations
+    give it to, with the same kind of value, and no others."""
+    block, x, gy = _make(4, 64, 24, 16)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+    x[1, 5, 3] = float("inf")
+    x[2, 20, 7] = float("nan")
+    gy[3, 2, 9] = float("inf")
+    got = _grads(block, x, gy)
+    block.activation.register_forward_hook(lambda *a: None)
+    with torch.backends.cudnn.flags(enabled=False):
+        ref = _grads(block, x, gy)
+    for a, b in zip(got[:2], ref[:2]):
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+        fine = torch.isfinite(b)
+        assert _rel(a[fine], b[fine]) < 1e-5
+    for a, b in zip(got[2:], ref[2:]):
+        assert bool((torch.isfinite(a) == torch.isfinite(b)).all())
+
+
+@pytest.mark.parametrize("how", ["hook", "collector", "strided", "autocast", "channels", "gelu"])
+def test_separate_operations_still_serve(how):
+    """Each condition that rules the fused passes out runs the separate
+    operations, with the block's result."""
+    from pathtile_amd.runtime import KERNEL_EVENTS
+
+    H = 40 if how == "channels" else 64
+    block, x, gy = _make(5, H, 16, 8)
+    if how == "gelu":
+        block.activation = torch.nn.GELU(approximate="tanh")
+    ref = _fp64(block, x, gy)
+    block.cuda()
+    x = x.cuda()
+    seen = []
+    with torch.backends.cudnn.flags(enabled=False), \
+            torch.autocast("cuda", torch.bfloat16, enabled=how == "autocast"):
+        if how == "hook":
+            block.output_linear[1].register_forward_hook(lambda m, i, o: seen.append(o.shape))
+        if how == "strided":
+            x = x.transpose(0, 1).contiguous().transpose(0, 1)
+        KERNEL_EVENTS.enabled = how == "collector"
+        try:
+            assert block._fused_inputs(x) is None
+            y = block(x)
+        finally:
+            phases = [r["phase"] for r in KERNEL_EVENTS.rows()]
+            KERNEL_EVENTS.enabled = False
+            KERNEL_EVENTS.clear()
+    assert (how != "hook") or seen
+    assert (how != "collector") or phases == ["fwd"]
+    assert _rel(y, ref[0]) < (5e-2 if how == "autocast" else 1e-5)
+
+
+def test_fused_block_on_a_side_stream_under_graph_capture():
+    """The block's forward and backward in a captured graph, replayed with
+    new inputs and eager work between the replays."""
+    block, x, gy = _make(20, 64, 48, 16)
+    block.cuda()
+    xs, gys = x.cuda(), gy.cuda()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        _grads(block, xs, gys)  # first calls look up device attributes
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = _grads(block, xs, gys)
+    for k in range(3):
+        xs.copy_(x.cuda() + k)
+        graph.replay()
+        torch.cuda.synchronize()
+        ref = _grads(block, xs, gys)
+        assert all(torch.equal(a, b) for a, b in zip(out, ref)), k
