@@ -1,5 +1,5 @@
 // s4_block.hip — the S4ConvD block's entry points: argument checks, workspace
-// layout and the launches of s4_kernels.hpp around the convolution's own.
+// layout and the launches of the s4 kernels around the convolution's own.
 
 #include <hip/hip_runtime.h>
 #include <stddef.h>
@@ -7,37 +7,24 @@
 
 #include "dwconv1d_host.hpp"
 #include "pathtile_hip.h"
-#include "s4_kernels.hpp"
+#include "s4_small.hpp"
+#include "s4_tables.hpp"
 
 namespace pt {
 
-using TailFwdFn = void (*)(const float*, const float*, const __bf16*, const float*, const float*,
-                           float*, uint32_t, uint32_t, uint32_t);
-using TailBwdFn = void (*)(const float*, const float*, const uint8_t*, float, const __bf16*,
-                           const float*, const float*, float*, float*, uint32_t, uint32_t, uint32_t,
-                           uint32_t);
-using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t, uint32_t,
-                      uint32_t);
-
-struct TailKernels {
-  TailFwdFn fwd;
-  TailBwdFn bwd;
-  DwFn dw[2];  // [16-byte loads]
-  int nw, bt, dw_nw, dw_split;
+struct TailGeometry {
+  int nw, tok, dw_nw, dw_split;
   size_t dw_lds;
 };
 
 template <int CT>
-constexpr TailKernels tail_kernels() {
-  return {&s4_tail_fwd_kernel<CT>, &s4_tail_bwd_kernel<CT>,
-          {&s4_dw_kernel<CT, false>, &s4_dw_kernel<CT, true>},
-          TailGeo<CT>::NW, TailGeo<CT>::BT, DwGeo<CT>::NW, DwGeo<CT>::SPLIT, DwGeo<CT>::lds};
+constexpr TailGeometry tail_geometry() {
+  return {TailGeo<CT>::NW, TailGeo<CT>::TOK, DwGeo<CT>::NW, DwGeo<CT>::SPLIT, DwGeo<CT>::lds};
 }
 
-// [H / 32 - 1]
-static const TailKernels kTail[8] = {tail_kernels<2>(),  tail_kernels<4>(),  tail_kernels<6>(),
-                                     tail_kernels<8>(),  tail_kernels<10>(), tail_kernels<12>(),
-                                     tail_kernels<14>(), tail_kernels<16>()};
+static constexpr TailGeometry kTail[kNumS4H] = {
+    tail_geometry<2>(),  tail_geometry<4>(),  tail_geometry<6>(),  tail_geometry<8>(),
+    tail_geometry<10>(), tail_geometry<12>(), tail_geometry<14>(), tail_geometry<16>()};
 
 static int check_block(int B, int H, int L, int states) {
   if (B < 1 || H < 32 || H > kS4MaxH || H % 32 != 0 || L < 1 || L > kMaxL || states < 1)
@@ -48,6 +35,9 @@ static int check_block(int B, int H, int L, int states) {
 }
 
 static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// token_base's multiplier for n / L.
+static uint32_t token_magic(int L) { return L == 1 ? 0u : (uint32_t)((1ULL << 32) / (unsigned)L) + 1u; }
 
 static size_t round_up(size_t n, size_t q) { return (n + q - 1) / q * q; }
 
@@ -69,7 +59,7 @@ struct BwdLayout {
 };
 
 static int bwd_layout(int B, int H, int L, int threads, BwdLayout* o) {
-  const TailKernels& k = kTail[H / 32 - 1];
+  const TailGeometry& k = kTail[H / 32 - 1];
   const size_t ntok = (size_t)B * L;
   o->np = round_up(ntok, 64);
   o->nsteps = (uint32_t)((ntok + kDwTok - 1) / kDwTok);
@@ -154,16 +144,16 @@ int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, cons
   if (!pt::aligned16(v) || !pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(bias) ||
       !pt::aligned16(y))
     return PT_ERR_ALIGN;
-  const pt::TailKernels& k = pt::kTail[H / 32 - 1];
+  const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
-  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L;
-  uint32_t ntiles = (ntok + pt::kTailTok - 1) / pt::kTailTok;
+  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, magic = pt::token_magic(L);
+  uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
   const size_t lds = pt::tail_fwd_lds(H);
   const int block = k.nw * pt::kWave;
-  void* args[] = {&v, &x, &wf, &w, &bias, &y, &ntok, &uL, &ntiles};
-  return pt::launch((const void*)k.fwd,
-                    pt::resident_grid((const void*)k.fwd, block, lds, ntiles), (uint32_t)block,
-                    lds, stream, args);
+  void* args[] = {&v, &x, &wf, &w, &bias, &y, &ntok, &uL, &magic, &ntiles};
+  const void* fn = (const void*)pt::kTailFwd[H / 32 - 1];
+  return pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
+                    args);
 }
 
 int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block, size_t* bytes) {
@@ -199,25 +189,27 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
   st = pt::bwd_layout(B, H, L, threads_per_block, &o);
   if (st != PT_OK) return st;
   if (!workspace || workspace_bytes < o.total) return PT_ERR_WORKSPACE;
-  const pt::TailKernels& k = pt::kTail[H / 32 - 1];
+  const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   float* const ws = static_cast<float*>(workspace);
   float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk, *dxt = ws;
   const float* taps = prep;
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
   uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, np = (uint32_t)o.np;
+  uint32_t magic = pt::token_magic(L);
   {
-    uint32_t ntiles = (ntok + k.bt - 1) / k.bt;
+    uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
     const size_t lds = pt::tail_bwd_lds(H);
     const int block = k.nw * pt::kWave;
-    void* args[] = {&gy, &v, &mask, &scale, &wf, &w, &bias, &du, &dp, &ntok, &uL, &ntiles, &np};
-    st = pt::launch((const void*)k.bwd, pt::resident_grid((const void*)k.bwd, block, lds, ntiles),
-                    (uint32_t)block, lds, stream, args);
+    void* args[] = {&gy, &v, &mask, &scale, &wf, &w, &bias, &du, &dp, &ntok, &uL, &magic, &ntiles, &np};
+    const void* fn = (const void*)pt::kTailBwd[H / 32 - 1];
+    st = pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
+                    args);
     if (st != PT_OK) return st;
   }
   if (dw) {
-    const void* fn = (const void*)k.dw[L % 4 == 0];
+    const void* fn = (const void*)pt::kDw[H / 32 - 1][L % 4 == 0];
     const float* cdp = dp;
-    void* args[] = {&cdp, &v, &part, &ntok, &uL, &o.nsteps, &o.per, &np};
+    void* args[] = {&cdp, &v, &part, &ntok, &uL, &magic, &o.nsteps, &o.per, &np};
     st = pt::launch(fn, o.ranges * (uint32_t)k.dw_split, (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds,
                     stream, args);
     if (st != PT_OK) return st;

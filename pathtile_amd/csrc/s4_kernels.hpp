@@ -7,10 +7,10 @@
 //   u [b,h,t]  = conv(x^T, taps),  v = dropout(u),  g = gelu(v)
 //   P [b,c,t]  = sum_h W[c][h] g[b,h,t] + bias[c],  c < 2 H
 //   y [b,t,c]  = P[c] sigmoid(P[H + c]) + x[b,t,c],  c < H
-// The convolution runs on the kernels of dwconv1d_kernels.hpp. Here are the
-// taps and their gradient, the [B,L,H] <-> [B,H,L] transposes, and the tail
-// (GELU, projection, GLU, residual) with its backward, each one pass over
-// its tensors. The tail treats the B L columns as one list of tokens
+// The convolution runs on the kernels of dwconv1d_kernels.hpp, the taps, their
+// gradient and the [B,L,H] <-> [B,H,L] transposes on those of s4_small.hpp.
+// Here is the tail (GELU, projection, GLU, residual) with its backward, each
+// one pass over its tensors. The tail treats the B L columns as one list of tokens
 // (token = b L + t), so its tiles do not depend on L.
 //
 // The projection runs on the BF16 matrix cores with both operands split into
@@ -24,7 +24,6 @@
 
 namespace pt {
 
-constexpr int kTailTok = 64;     // tokens per tile of the tail's forward
 constexpr int kS4MaxH = 256;     // largest H of the fused block (H % 32 == 0)
 constexpr int kDwTok = 32;       // tokens per step of the weight gradient
 
@@ -44,35 +43,66 @@ struct TailGeo {
   static constexpr int GS = H + 8;       // BF16 values per token row of a g part
   static constexpr int PS = 2 * H + 8;   // the same for a dP part
   static constexpr int OS = H + 4;       // floats per token row of the output stage
-  // tokens per backward tile: the dP parts of 64 tokens fit the LDS up to H = 128
-  static constexpr int BT = CT <= 8 ? 64 : 32;
+  // tokens per tile: the LDS holds the stages of 64 tokens up to H = 128
+  static constexpr int TOK = CT <= 8 ? 64 : 32;
 };
 
-__host__ __device__ constexpr size_t tail_fwd_lds(int H) {
-  const size_t g = (size_t)3 * kTailTok * (H + 8) * 2;
-  const size_t o = (size_t)kTailTok * (H + 4) * 4;
-  return g > o ? g : o;
+__host__ __device__ constexpr int tail_tok(int H) { return H <= 128 ? 64 : 32; }
+__host__ __device__ constexpr size_t tail_fwd_lds(int H) {  // two g stages, the output stage
+  return (size_t)tail_tok(H) * (2 * 3 * (H + 8) * 2 + (H + 4) * 4);
 }
-__host__ __device__ constexpr size_t tail_bwd_lds(int H) {
-  const size_t bt = H <= 128 ? 64 : 32;
-  return (size_t)3 * bt * (2 * H + 8) * 2;  // dP parts, over the g parts
+__host__ __device__ constexpr size_t tail_bwd_lds(int H) {  // g parts, dP parts
+  return (size_t)tail_tok(H) * 3 * ((H + 8) + (2 * H + 8)) * 2;
 }
 
 // Values of the split weights in the workspace: W as A operands of the
 // forward product, then W^T as A operands of the backward one.
 __host__ __device__ constexpr size_t wfrag_values(int H) { return (size_t)3 * 2 * H * H; }
 
-__device__ __forceinline__ float gelu_f(float x) {
-  return x * 0.5f * (1.0f + erff(x * 0.70710678118654752f));
+// The normal distribution function without branches: for a = |x|,
+// Q(a) = 1 - cdf(a) = exp(-a^2 / 2) R(a) with R(a) = erfcx(a / sqrt 2) / 2 as
+// an 8-term polynomial in t = 1 / (1 + 9/32 a), fitted (weighted minimax, the
+// coefficients rounded to FP32 one after the other) to 4e-10 of gelu; 20
+// instructions where erff takes about 75 on both of its branches. The
+// exponential also gives the density. a is cut at 20, where Q underflows, so
+// that infinities keep the formula's values (gelu(-inf) = NaN).
+struct NormalCdf {
+  float cdf, e;  // e = exp(-x^2 / 2)
+};
+__device__ __forceinline__ NormalCdf normal_cdf(float x) {
+  const float a = fminf(fabsf(x), 20.0f);
+  const float d = fmaf(0.28125f, a, 1.0f);
+  float t = __builtin_amdgcn_rcpf(d);
+  t = fmaf(t, fmaf(-d, t, 1.0f), t);
+  const float s = a * a;
+  const float e = __builtin_amdgcn_exp2f(-fmaf(s, 0.72134751081466675f, s * 9.6298152e-09f));
+  float r = 0.0391756147146225f;
+  r = fmaf(r, t, -0.20986095070838928f);
+  r = fmaf(r, t, 0.37282636761665344f);
+  r = fmaf(r, t, -0.21809245645999908f);
+  r = fmaf(r, t, 0.22155848145484924f);
+  r = fmaf(r, t, 0.06441713869571686f);
+  r = fmaf(r, t, 0.11812617629766464f);
+  r = fmaf(r, t, 0.11184962838888168f);
+  const float q = r * t * e;
+  return {x < 0.0f ? q : 1.0f - q, e};
 }
+
+__device__ __forceinline__ float gelu_f(float x) { return x * normal_cdf(x).cdf; }
 
 __device__ __forceinline__ float gelu_grad_f(float x) {
-  const float cdf = 0.5f * (1.0f + erff(x * 0.70710678118654752f));
-  const float pdf = expf(-0.5f * x * x) * 0.39894228040143268f;
-  return cdf + x * pdf;
+  const NormalCdf n = normal_cdf(x);
+  return fmaf(x, n.e * 0.39894228040143268f, n.cdf);
 }
 
-__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+// 1 / (1 + exp(-x)), NaN kept; past 87 the result is 1 or below FP32's range.
+__device__ __forceinline__ float sigmoid_f(float x) {
+  const float c = x > 87.0f ? 87.0f : x < -87.0f ? -87.0f : x;
+  const float d =
+      1.0f + __builtin_amdgcn_exp2f(-fmaf(c, 1.44269502162933349609375f, c * 1.92596303e-08f));
+  const float t = __builtin_amdgcn_rcpf(d);
+  return fmaf(t, fmaf(-d, t, 1.0f), t);
+}
 
 __device__ __forceinline__ bool finite4(float a, float b, float c, float d) {
   return fabsf(a) + fabsf(b) + fabsf(c) + fabsf(d) < INFINITY;
@@ -80,16 +110,6 @@ __device__ __forceinline__ bool finite4(float a, float b, float c, float d) {
 
 __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// The six part products of one 16x16 tile, small ones first.
-__device__ __forceinline__ f32x4 mfma_split6(const bf16x8 (&a)[3], const bf16x8 (&b)[3], f32x4 c) {
-  c = mfma_bf16(a[2], b[0], c);
-  c = mfma_bf16(a[0], b[2], c);
-  c = mfma_bf16(a[1], b[1], c);
-  c = mfma_bf16(a[1], b[0], c);
-  c = mfma_bf16(a[0], b[1], c);
-  return mfma_bf16(a[0], b[0], c);
 }
 
 // The matrix instruction's internal sum rounds towards minus infinity
@@ -108,333 +128,89 @@ __device__ __forceinline__ void negate(f32x4 (&acc)[N]) {
 }
 
 // ---------------------------------------------------------------------------
-// Preparation: taps and split weights, one launch per block and pass.
-// Blocks 0 .. H - 1 compute the taps of one channel; the others split W
-// [2 H][H] into A-operand fragments of 64 lanes x 8 values (lane l holds row
-// l % 16, contraction values 8 (l / 16) .. + 7), three parts each:
-//   wf[((ct * 2 + half) * KS + ks) * 3 + part][lane][8]   rows of W
-//   wt[(ct * 2 KS + ks) * 3 + part][lane][8]              rows of W^T
-// so that a wave's fragment is one contiguous 1 KiB read.
-// The taps are the reference's formula in FP32 with exp(dt A) - 1 from
-// expm1 and sin^2 (no cancellation at small dt A).
-// ---------------------------------------------------------------------------
-struct Cf { float re, im; };
-__device__ __forceinline__ Cf cmul(Cf a, Cf b) {
-  return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-}
-__device__ __forceinline__ Cf cdiv(Cf a, Cf b) {
-  const float d = 1.0f / (b.re * b.re + b.im * b.im);
-  return {(a.re * b.re + a.im * b.im) * d, (a.im * b.re - a.re * b.im) * d};
-}
-__device__ __forceinline__ Cf cexpm1(Cf a) {
-  float s, c;
-  sincosf(a.im, &s, &c);
-  const float h = sinf(0.5f * a.im);
-  return {expm1f(a.re) * c - 2.0f * h * h, expf(a.re) * s};
-}
-__device__ __forceinline__ Cf cexp_at(Cf a, float t) {
-  float s, c;
-  sincosf(a.im * t, &s, &c);
-  const float e = expf(a.re * t);
-  return {e * c, e * s};
-}
-
-constexpr int kPrepThreads = 256;
-constexpr int kPrepStates = 32;  // states per LDS pass
-
-__global__ __launch_bounds__(kPrepThreads) void s4_prep_kernel(
-    const float* __restrict__ log_dt, const float* __restrict__ c_re,
-    const float* __restrict__ c_im, const float* __restrict__ log_a_re,
-    const float* __restrict__ a_im, const float* __restrict__ skip,
-    const float* __restrict__ w, float* __restrict__ taps, __bf16* __restrict__ wf,
-    int H, int L, int N2, int transposed) {
-  const int tid = threadIdx.x;
-  if ((int)blockIdx.x < H) {
-    const int h = blockIdx.x;
-    __shared__ float ce[2][kPrepStates], da[2][kPrepStates];
-    __shared__ float part[kMaxL][kPrepStates + 1];
-    const float dt = expf(log_dt[h]);
-    float acc = 0.0f;  // thread t < L: taps[h][t]
-    for (int n0 = 0; n0 < N2; n0 += kPrepStates) {
-      const int nn = N2 - n0 < kPrepStates ? N2 - n0 : kPrepStates;
-      if (tid < nn) {
-        const int i = h * N2 + n0 + tid;
-        const Cf A = {-expf(log_a_re[i]), a_im[i]};
-        const Cf dA = {A.re * dt, A.im * dt};
-        const Cf e = cdiv(cmul(Cf{c_re[i], c_im[i]}, cexpm1(dA)), A);
-        ce[0][tid] = e.re;
-        ce[1][tid] = e.im;
-        da[0][tid] = dA.re;
-        da[1][tid] = dA.im;
-      }
-      __syncthreads();
-      for (int q = tid; q < nn * L; q += kPrepThreads) {
-        const int t = q / nn, n = q - t * nn;
-        const Cf z = cexp_at(Cf{da[0][n], da[1][n]}, (float)t);
-        part[t][n] = ce[0][n] * z.re - ce[1][n] * z.im;
-      }
-      __syncthreads();
-      if (tid < L)
-        for (int n = 0; n < nn; ++n) acc += part[tid][n];
-      __syncthreads();
-    }
-    if (tid < L) taps[h * L + tid] = 2.0f * acc + (tid == L / 2 ? skip[h] : 0.0f);
-    return;
-  }
-  // one fragment lane (8 values) per thread
-  const int KS = H / 32, nf = 2 * H * H / 8;
-  int q = ((int)blockIdx.x - H) * kPrepThreads + tid;
-  const bool back = q >= nf;
-  if (back) q -= nf;
-  if (q >= nf || (back && !transposed)) return;
-  const int lane = q & 63, f = q >> 6;
-  const int row = lane & 15, k0 = 8 * (lane >> 4);
-  float v[8];
-  __bf16* dst;
-  const int ks = f % (back ? 2 * KS : KS);
-  if (!back) {
-    const int tile = f / KS;  // tile = ct * 2 + half
-    const float* src = w + (size_t)((tile & 1) * H + 16 * (tile >> 1) + row) * H + 32 * ks + k0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = src[i];
-    dst = wf + (size_t)f * 3 * 512;
-  } else {
-    const int ct = f / (2 * KS);
-    const float* src = w + (size_t)(32 * ks + k0) * H + 16 * ct + row;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = src[(size_t)i * H];
-    dst = wf + wfrag_values(H) + (size_t)f * 3 * 512;
-  }
-  if (step_negated(ks)) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = -v[i];
-  }
-  bf16x8 hi, mid, lo;
-  split3_bf16x8(v, hi, mid, lo);
-  *reinterpret_cast<bf16x8*>(dst + 0 * 512 + lane * 8) = hi;
-  *reinterpret_cast<bf16x8*>(dst + 1 * 512 + lane * 8) = mid;
-  *reinterpret_cast<bf16x8*>(dst + 2 * 512 + lane * 8) = lo;
-}
-
-// ---------------------------------------------------------------------------
-// Gradient of the taps with respect to the kernel's parameters, from
-// dk [H][L]: with z = exp(dt A), E = z - 1, S0 = sum_t dk[t] z^t,
-// S1 = sum_t t dk[t] z^t per state,
-//   dL = 2 Re sum_n ( S0 E / A dC + R dA + (S0 C z + C_eff A S1) ddt ),
-//   R  = S0 C / A^2 (z dt A - E) + dt C_eff S1,
-// one workgroup per channel. z dt A - E cancels to second order in dt A, so
-// that factor and E are computed in FP64 (a handful of operations per state).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kPrepThreads) void s4_taps_grad_kernel(
-    const float* __restrict__ dk, const float* __restrict__ log_dt,
-    const float* __restrict__ c_re, const float* __restrict__ c_im,
-    const float* __restrict__ log_a_re, const float* __restrict__ a_im,
-    float* __restrict__ d_log_dt, float* __restrict__ d_c_re, float* __restrict__ d_c_im,
-    float* __restrict__ d_log_a_re, float* __restrict__ d_a_im, float* __restrict__ d_skip,
-    int L, int N2) {
-  constexpr int kChunks = 8;  // threads per state
-  __shared__ float sdk[kMaxL];
-  __shared__ float s0r[kPrepStates][kChunks], s0i[kPrepStates][kChunks];
-  __shared__ float s1r[kPrepStates][kChunks], s1i[kPrepStates][kChunks];
-  __shared__ float ddt[kPrepStates];
-  const int h = blockIdx.x, tid = threadIdx.x;
-  if (tid < L) sdk[tid] = dk[h * L + tid];
-  __syncthreads();
-  const float dt = expf(log_dt[h]);
-  float ddt_sum = 0.0f;  // thread 0
-  for (int n0 = 0; n0 < N2; n0 += kPrepStates) {
-    const int nn = N2 - n0 < kPrepStates ? N2 - n0 : kPrepStates;
-    const int n = tid / kChunks, q = tid % kChunks;
-    if (n < nn) {
-      const int i = h * N2 + n0 + n;
-      const Cf dA = {-expf(log_a_re[i]) * dt, a_im[i] * dt};
-      Cf s0 = {0.f, 0.f}, s1 = {0.f, 0.f};
-      for (int t = q; t < L; t += kChunks) {
-        const Cf z = cexp_at(dA, (float)t);
-        const float d = sdk[t], td = d * (float)t;
-        s0.re += d * z.re;
-        s0.im += d * z.im;
-        s1.re += td * z.re;
-        s1.im += td * z.im;
-      }
-      s0r[n][q] = s0.re;
-      s0i[n][q] = s0.im;
-      s1r[n][q] = s1.re;
-      s1i[n][q] = s1.im;
-    }
-    __syncthreads();
-    if (tid < nn) {
-      const int i = h * N2 + n0 + tid;
-      double S0r = 0, S0i = 0, S1r = 0, S1i = 0;
-      for (int k = 0; k < kChunks; ++k) {
-        S0r += s0r[tid][k];
-        S0i += s0i[tid][k];
-        S1r += s1r[tid][k];
-        S1i += s1i[tid][k];
-      }
-      const double ar = -(double)expf(log_a_re[i]), ai = a_im[i], d = dt;
-      const double cr = c_re[i], ci = c_im[i];
-      const double xr = ar * d, xi = ai * d;
-      double sn, cs;
-      sincos(xi, &sn, &cs);
-      const double ex = exp(xr), zr = ex * cs, zi = ex * sn;
-      const double hs = sin(0.5 * xi);
-      const double Er = expm1(xr) * cs - 2.0 * hs * hs, Ei = zi;
-      const double inv = 1.0 / (ar * ar + ai * ai);
-      // E / A
-      const double er = (Er * ar + Ei * ai) * inv, ei = (Ei * ar - Er * ai) * inv;
-      // dC: S0 E / A
-      const double gr = S0r * er - S0i * ei, gi = S0r * ei + S0i * er;
-      // C_eff = C E / A
-      const double fr = cr * er - ci * ei, fi = cr * ei + ci * er;
-      // C_eff S1
-      const double pr = fr * S1r - fi * S1i, pi = fr * S1i + fi * S1r;
-      // S0 C
-      const double qr = S0r * cr - S0i * ci, qi = S0r * ci + S0i * cr;
-      // (z dt A - E) / A^2
-      const double mr = zr * xr - zi * xi - Er, mi = zr * xi + zi * xr - Ei;
-      const double a1r = (mr * ar + mi * ai) * inv, a1i = (mi * ar - mr * ai) * inv;
-      const double a2r = (a1r * ar + a1i * ai) * inv, a2i = (a1i * ar - a1r * ai) * inv;
-      const double Rr = qr * a2r - qi * a2i + d * pr, Ri = qr * a2i + qi * a2r + d * pi;
-      // ddt: S0 C z + C_eff S1 A
-      const double Dr = qr * zr - qi * zi + pr * ar - pi * ai;
-      d_c_re[i] = (float)(2.0 * gr);
-      d_c_im[i] = (float)(-2.0 * gi);
-      d_log_a_re[i] = (float)(2.0 * Rr * ar);
-      d_a_im[i] = (float)(-2.0 * Ri);
-      ddt[tid] = (float)(2.0 * Dr * d);
-    }
-    __syncthreads();
-    if (tid == 0)
-      for (int k = 0; k < nn; ++k) ddt_sum += ddt[k];
-    __syncthreads();
-  }
-  if (tid == 0) {
-    d_log_dt[h] = ddt_sum;
-    d_skip[h] = sdk[L / 2];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Transposes of whole samples, [L][H] <-> [H][L]; both sides move 16-byte
-// pieces (dwords where L % 4 != 0) through one LDS tile per workgroup with an
-// odd row stride. ADD: the [L][H] result also gets `add` (the residual
-// gradient). Bound by HBM: one read and one write of the tensor.
-// ---------------------------------------------------------------------------
-constexpr int kTransThreads = 256;
-
-template <bool VEC>
-__global__ __launch_bounds__(kTransThreads) void s4_transpose_kernel(
-    const float* __restrict__ x, float* __restrict__ out, int B, int H, int L) {
-  extern __shared__ float tile[];  // [L][S]
-  const int S = H + 1, n4 = L * H / 4, h4 = H / 4;
-  for (int b = blockIdx.x; b < B; b += gridDim.x) {
-    const float* src = x + (size_t)b * L * H;
-    float* dst = out + (size_t)b * L * H;
-    for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-      const float4 v = reinterpret_cast<const float4*>(src)[i];
-      const int t = i / h4, c = 4 * (i - t * h4);
-      float* p = tile + t * S + c;
-      p[0] = v.x;
-      p[1] = v.y;
-      p[2] = v.z;
-      p[3] = v.w;
-    }
-    __syncthreads();
-    if constexpr (VEC) {
-      const int l4 = L / 4;
-      for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-        const int c = i / l4, t = 4 * (i - c * l4);
-        const float* p = tile + t * S + c;
-        reinterpret_cast<float4*>(dst)[i] = float4{p[0], p[S], p[2 * S], p[3 * S]};
-      }
-    } else {
-      for (int i = threadIdx.x; i < L * H; i += kTransThreads) {
-        const int c = i / L, t = i - c * L;
-        dst[i] = tile[t * S + c];
-      }
-    }
-    __syncthreads();
-  }
-}
-
-template <bool VEC>
-__global__ __launch_bounds__(kTransThreads) void s4_transpose_add_kernel(
-    const float* __restrict__ d, const float* __restrict__ add, float* __restrict__ out, int B,
-    int H, int L) {
-  extern __shared__ float tile[];
-  const int S = H + 1, n4 = L * H / 4, h4 = H / 4;
-  for (int b = blockIdx.x; b < B; b += gridDim.x) {
-    const float* src = d + (size_t)b * L * H;
-    if constexpr (VEC) {
-      const int l4 = L / 4;
-      for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-        const float4 v = reinterpret_cast<const float4*>(src)[i];
-        const int c = i / l4, t = 4 * (i - c * l4);
-        float* p = tile + t * S + c;
-        p[0] = v.x;
-        p[S] = v.y;
-        p[2 * S] = v.z;
-        p[3 * S] = v.w;
-      }
-    } else {
-      for (int i = threadIdx.x; i < L * H; i += kTransThreads) {
-        const int c = i / L, t = i - c * L;
-        tile[t * S + c] = src[i];
-      }
-    }
-    __syncthreads();
-    const float4* a4 = reinterpret_cast<const float4*>(add + (size_t)b * L * H);
-    float4* o4 = reinterpret_cast<float4*>(out + (size_t)b * L * H);
-    for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-      const int t = i / h4, c = 4 * (i - t * h4);
-      const float* p = tile + t * S + c;
-      const float4 a = a4[i];
-      o4[i] = float4{p[0] + a.x, p[1] + a.y, p[2] + a.z, p[3] + a.w};
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Tail, shared pieces
 // ---------------------------------------------------------------------------
-// Element offset of (token n, channel 0) in a [B, H, L] tensor.
-__device__ __forceinline__ uint32_t token_base(uint32_t n, uint32_t H, uint32_t L) {
-  const uint32_t b = n / L;
-  return b * H * L + (n - b * L);
+// Element offset of (token n, channel 0) in a [B, H, L] tensor. magic =
+// floor(2^32 / L) + 1 (0 at L = 1): umulhi(n, magic) = n / L for every
+// n < 2^32 / L, and there are at most 2^31 / 32 tokens.
+__device__ __forceinline__ uint32_t token_sample(uint32_t n, uint32_t magic) {
+  return magic ? __umulhi(n, magic) : n;
+}
+__device__ __forceinline__ uint32_t token_base(uint32_t n, uint32_t H, uint32_t L, uint32_t magic) {
+  const uint32_t b = token_sample(n, magic);
+  return b * (H * L) + (n - b * L);
 }
 
-// gelu(v) of TOK tokens from token n0 on, split into the three parts of the
-// LDS stage [part][token][GS]: a lane takes one token and eight channels, so
-// a wave's loads run along the tokens of one channel.
-template <int CT, int TOK>
-__device__ __forceinline__ void stage_gelu(__bf16* sg, const float* __restrict__ v, uint32_t n0,
-                                           uint32_t ntok, uint32_t L) {
-  using G = TailGeo<CT>;
-  constexpr int kUnits = TOK * (G::H / 8);
-  for (int u = threadIdx.x; u < kUnits; u += G::NW * kWave) {
-    const int tk = u % TOK, c = 8 * (u / TOK);
-    float g[8];
-    const uint32_t n = n0 + tk;
-    if (n < ntok) {
-      const float* src = v + token_base(n, G::H, L) + (size_t)c * L;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) g[i] = src[i * L];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) g[i] = gelu_f(g[i]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) g[i] = 0.0f;
-    }
-    bf16x8 hi, mid, lo;
-    split3_bf16x8(g, hi, mid, lo);
-    __bf16* d = sg + tk * G::GS + c;
-    *reinterpret_cast<bf16x8*>(d) = hi;
-    *reinterpret_cast<bf16x8*>(d + TOK * G::GS) = mid;
-    *reinterpret_cast<bf16x8*>(d + 2 * TOK * G::GS) = lo;
-  }
+// A [B, H, L] tensor (elements of `size` bytes) from the sample of token n0
+// on, as a buffer that ends with the tensor: loads of later tokens read 0 and
+// stores to them are dropped, without a branch. Byte offsets within a tile
+// stay far below 2 GiB (64 tokens touch at most 65 samples at L = 1).
+struct Slab {
+  __amdgpu_buffer_rsrc_t r;
+  uint32_t first;  // element offset of the slab
+};
+template <int SIZE = 4>
+__device__ __forceinline__ Slab make_slab(const void* t, uint32_t n0, uint32_t ntok, uint32_t H,
+                                          uint32_t L, uint32_t magic) {
+  const uint32_t first = token_sample(n0, magic) * (H * L), all = ntok * H;
+  const uint64_t left = first < all ? (uint64_t)(all - first) * SIZE : 0;
+  const uint32_t bytes = left < (uint64_t)kNumRecords ? (uint32_t)left : (uint32_t)kNumRecords;
+  return {__builtin_amdgcn_make_buffer_rsrc(
+              const_cast<char*>(static_cast<const char*>(t)) + (size_t)first * SIZE, 0, (int)bytes,
+              kRsrcWord3),
+          first};
 }
+// Rows n0 .. of a [tokens, H] tensor.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_token_rows(const float* t, uint32_t n0,
+                                                                  uint32_t ntok, uint32_t H) {
+  const uint64_t left = n0 < ntok ? (uint64_t)(ntok - n0) * H * 4 : 0;
+  const uint32_t bytes = left < (uint64_t)kNumRecords ? (uint32_t)left : (uint32_t)kNumRecords;
+  return make_rsrc_n(t + (size_t)n0 * H, bytes);
+}
+
+// gelu(v) of TOK tokens, split into the three parts of the LDS stage
+// [part][token][GS]: a lane takes one token and eight channels, so a wave's
+// loads run along the tokens of one channel. store<I, N> does the I-th of N
+// slices of the work.
+template <int CT, int TOK>
+struct GeluStage {
+  using G = TailGeo<CT>;
+  static constexpr int TH = G::NW * kWave, kUnits = TOK * (G::H / 8);
+  static constexpr int U = (kUnits + TH - 1) / TH;
+  float x[U][8];
+
+  __device__ __forceinline__ void load(const float* __restrict__ v, uint32_t n0, uint32_t ntok,
+                                       uint32_t L, uint32_t magic) {
+    const Slab s = make_slab(v, n0, ntok, G::H, L, magic);
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const int u = threadIdx.x + i * TH;
+      const uint32_t at = token_base(n0 + u % TOK, G::H, L, magic) - s.first + 8 * (u / TOK) * L;
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        x[i][k] = buf_load1(s.r, kUnits % TH == 0 || u < kUnits ? 4 * (at + k * L) : kOob, 0);
+    }
+  }
+
+  template <int I, int N>
+  __device__ __forceinline__ void store(__bf16* sg) {
+#pragma unroll
+    for (int e = 8 * U * I / N; e < 8 * U * (I + 1) / N; ++e) {
+      const int i = e / 8;
+      x[i][e % 8] = gelu_f(x[i][e % 8]);  // 0 past the last token
+      if (e % 8 == 7) {
+        const int u = threadIdx.x + i * TH;
+        bf16x8 hi, mid, lo;
+        split3_bf16x8(x[i], hi, mid, lo);
+        // units past the end write to a row padding that nothing reads
+        __bf16* d = sg + (u % TOK) * G::GS + (kUnits % TH == 0 || u < kUnits ? 8 * (u / TOK) : G::H);
+        *reinterpret_cast<bf16x8*>(d) = hi;
+        *reinterpret_cast<bf16x8*>(d + TOK * G::GS) = mid;
+        *reinterpret_cast<bf16x8*>(d + 2 * TOK * G::GS) = lo;
+      }
+    }
+  }
+};
 
 // Weight fragments of N row tiles `steps` contraction steps apart.
 template <int N>
@@ -447,49 +223,79 @@ __device__ __forceinline__ void load_frags(bf16x8 (&a)[N][3], const __bf16* __re
       a[m][p] = *reinterpret_cast<const bf16x8*>(w + ((size_t)m * steps * 3 + p) * 512);
 }
 
-// P tiles of this wave: acc[m][half][nt] = W rows (16 (ct0 + m) .. of half)
-// times the staged tokens 16 (nt0 + nt) .. .
-template <int CT, int TOK, int NT>
-__device__ __forceinline__ void project(f32x4 (&acc)[TailGeo<CT>::MT][2][NT], const __bf16* sg,
-                                        const __bf16* __restrict__ wf, int ct0, int nt0, int lane) {
-  using G = TailGeo<CT>;
+// Weight fragments of M row tiles and KS contraction steps, streamed from the
+// L2 (the next step's load while a step multiplies) or kept in registers.
+template <int M, int KS>
+struct StreamedFrags {
+  const __bf16* w0;
+  const __bf16* w;
+  bf16x8 a[2][M][3];
+  __device__ __forceinline__ explicit StreamedFrags(const __bf16* p) : w0(p), w(p) {}
+  __device__ __forceinline__ void begin() {
+    // Opaque to the compiler, which would otherwise keep every fragment in
+    // registers over the tile loop and spill.
+    uint32_t zero = 0;
+    asm volatile("" : "+s"(zero));
+    w = w0 + zero;
+    load_frags<M>(a[0], w, KS);
+  }
+  template <int ks>
+  __device__ __forceinline__ void ahead() {
+    if constexpr (ks + 1 < KS) load_frags<M>(a[(ks + 1) & 1], w + (ks + 1) * 3 * 512, KS);
+  }
+  template <int ks>
+  __device__ __forceinline__ bf16x8 frag(int m, int p) const { return a[ks & 1][m][p]; }
+};
+template <int M, int KS>
+struct ResidentFrags {
+  bf16x8 a[KS][M][3];
+  __device__ __forceinline__ explicit ResidentFrags(const __bf16* p) {
 #pragma unroll
-  for (int m = 0; m < G::MT; ++m)
+    for (int ks = 0; ks < KS; ++ks) load_frags<M>(a[ks], p + ks * 3 * 512, KS);
+  }
+  __device__ __forceinline__ void begin() {}
+  template <int ks>
+  __device__ __forceinline__ void ahead() {}
+  template <int ks>
+  __device__ __forceinline__ bf16x8 frag(int m, int p) const { return a[ks][m][p]; }
+};
+
+// acc[m][nt] = M row tiles of the weights (fragments from w0, KS steps) times
+// NT token tiles of the stage from b0 on (row stride RS, parts TOK * RS
+// apart). The next step's fragments load while a step multiplies, and
+// shadow(step) adds vector work that runs beside the step's products.
+template <int M, int NT, int KS, int RS, int TOK, typename W, typename F>
+__device__ __forceinline__ void multiply(f32x4 (&acc)[M][NT], W& w, const __bf16* b0, F&& shadow) {
 #pragma unroll
-    for (int hf = 0; hf < 2; ++hf)
+  for (int m = 0; m < M; ++m)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) acc[m][hf][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const __bf16* const b0 = sg + (16 * nt0 + (lane & 15)) * G::GS + 8 * (lane >> 4);
-  const __bf16* const a0 = wf + (size_t)ct0 * 2 * G::KS * 3 * 512 + lane * 8;
-  bf16x8 a[G::MT][2][3];
-  load_frags<G::MT * 2>(reinterpret_cast<bf16x8(&)[G::MT * 2][3]>(a), a0, G::KS);
-#pragma unroll 1
-  for (int ks = 0; ks < G::KS; ++ks) {
-    // the next step's weight fragments are on their way during this step
-    bf16x8 an[G::MT][2][3];
-    load_frags<G::MT * 2>(reinterpret_cast<bf16x8(&)[G::MT * 2][3]>(an),
-                          a0 + (ks + 1 < G::KS ? ks + 1 : 0) * 3 * 512, G::KS);
-    if (ks > 0 && step_negated(ks) != step_negated(ks - 1))
-      negate(reinterpret_cast<f32x4(&)[G::MT * 2 * NT]>(acc));
+    for (int nt = 0; nt < NT; ++nt) acc[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  static_for<0, KS>([&](auto step) {
+    constexpr int ks = decltype(step)::value;
+    w.template ahead<ks>();
+    if constexpr (ks > 0 && step_negated(ks) != step_negated(ks - 1))
+      negate(reinterpret_cast<f32x4(&)[M * NT]>(acc));
+    bf16x8 b[NT][3];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      bf16x8 b[3];
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int p = 0; p < 3; ++p)
-        b[p] = *reinterpret_cast<const bf16x8*>(b0 + (p * TOK + 16 * nt) * G::GS + 32 * ks);
+        b[nt][p] = *reinterpret_cast<const bf16x8*>(b0 + (p * TOK + 16 * nt) * RS + 32 * ks);
+    // after the reads in program order: its LDS writes cannot pass them
+    shadow(step);
+    // one product of every tile after the other: an accumulator's next
+    // product waits for its last
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};  // small ones first
 #pragma unroll
-      for (int m = 0; m < G::MT; ++m)
+    for (int q = 0; q < 6; ++q)
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf) acc[m][hf][nt] = mfma_split6(a[m][hf], b, acc[m][hf][nt]);
-    }
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int m = 0; m < G::MT; ++m)
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) a[m][hf][p] = an[m][hf][p];
-  }
-  if (step_negated(G::KS - 1)) negate(reinterpret_cast<f32x4(&)[G::MT * 2 * NT]>(acc));
+        for (int m = 0; m < M; ++m)
+          acc[m][nt] = mfma_bf16(w.template frag<ks>(m, pa[q]), b[nt][pb[q]], acc[m][nt]);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  if constexpr (step_negated(KS - 1)) negate(reinterpret_cast<f32x4(&)[M * NT]>(acc));
 }
 
 // One pre-activation of one token by the FP32 chain, for values that the
@@ -502,64 +308,86 @@ __device__ __forceinline__ float project_one(const float* __restrict__ v, const 
   return s;
 }
 
+__device__ __forceinline__ void set_elem(f32x4& a, int r, float v) {
+  a[0] = r == 0 ? v : a[0];
+  a[1] = r == 1 ? v : a[1];
+  a[2] = r == 2 ? v : a[2];
+  a[3] = r == 3 ? v : a[3];
+}
+
 // Recomputes a lane's four value and gate sums where one is not finite.
 __device__ __forceinline__ void project_fix(f32x4& a, f32x4& b, const float* __restrict__ v,
-                                            const float* __restrict__ w, uint32_t n, int c, int H,
-                                            uint32_t L) {
-  const uint32_t base = token_base(n, H, L);
+                                            const float* __restrict__ w, uint32_t base, int c,
+                                            int H, uint32_t L) {
 #pragma unroll 1
   for (int r = 0; r < 4; ++r) {
-    const float pa = project_one(v, w, base, c + r, H, L);
-    const float pb = project_one(v, w, base, H + c + r, H, L);
-    a[0] = r == 0 ? pa : a[0];
-    a[1] = r == 1 ? pa : a[1];
-    a[2] = r == 2 ? pa : a[2];
-    a[3] = r == 3 ? pa : a[3];
-    b[0] = r == 0 ? pb : b[0];
-    b[1] = r == 1 ? pb : b[1];
-    b[2] = r == 2 ? pb : b[2];
-    b[3] = r == 3 ? pb : b[3];
+    set_elem(a, r, project_one(v, w, base, c + r, H, L));
+    set_elem(b, r, project_one(v, w, base, H + c + r, H, L));
   }
 }
 
 // ---------------------------------------------------------------------------
 // Tail forward: y = GLU(W gelu(v) + bias) + x, v [B,H,L], x and y [B,L,H].
-// A persistent workgroup takes tiles of 64 tokens: gelu and split into LDS,
-// the projection (the weight fragments stream from the L2, the token parts
-// from LDS), GLU into an FP32 stage over the same LDS, then flat 16-byte rows
-// with the residual. Two workgroups per CU at H <= 128, so that one's gelu
-// (VALU) runs beside the other's matrix work.
+// A persistent workgroup, one per CU, walks tiles of 64 tokens (32 above
+// H = 128, what the LDS holds). gelu is as much vector work as the products
+// are matrix work, and both kinds from one wave overlap where they are
+// interleaved in one stretch of code (two workgroups that share a CU fall
+// into step instead and add the two up: 452 us at B16384 L48 H128, 388
+// here, 3.1 TB/s with the matrix cores 42% busy), so tile t + 1's gelu and split
+// run in the shadow of tile t's products, into the other of two stages. The
+// weight fragments stay in registers up to H = 128 (streamed from the L2 they
+// cost 511 us) and stream above. GLU results pass through an FP32 stage
+// to flat 16-byte rows with the residual.
 // ---------------------------------------------------------------------------
 template <int CT>
-__global__ __launch_bounds__(TailGeo<CT>::NW* kWave, CT <= 8 ? 4 : 2) void s4_tail_fwd_kernel(
+__global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
     const float* __restrict__ v, const float* __restrict__ x, const __bf16* __restrict__ wf,
     const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y,
-    uint32_t ntok, uint32_t L, uint32_t ntiles) {
+    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t ntiles) {
   using G = TailGeo<CT>;
-  constexpr int NT = kTailTok / 16 / G::WPT;
+  constexpr int TOK = G::TOK, NT = TOK / 16 / G::WPT, SZ = 3 * TOK * G::GS, TH = G::NW * kWave;
+  constexpr int R4 = TOK * G::H / 4 / TH;  // 16-byte pieces of a tile's rows per thread
+  static_assert(TOK * G::H / 4 % TH == 0 && NT >= 1, "whole pieces and token tiles");
   extern __shared__ __align__(16) char smem[];
   __bf16* const sg = reinterpret_cast<__bf16*>(smem);
-  float* const so = reinterpret_cast<float*>(smem);
+  float* const so = reinterpret_cast<float*>(smem + (size_t)2 * SZ * 2);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct0 = (wave % G::WPC) * G::MT, nt0 = (wave / G::WPC) * NT;
-  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const uint32_t n0 = tile * kTailTok;
-    stage_gelu<CT, kTailTok>(sg, v, n0, ntok, L);
-    __syncthreads();
-    f32x4 acc[G::MT][2][NT];
-    project<CT, kTailTok, NT>(acc, sg, wf, ct0, nt0, lane);
-    __syncthreads();  // the stage is read; the output stage takes its place
+  const int tk0 = 16 * nt0 + (lane & 15);     // this lane's token of tile nt: tk0 + 16 nt
+  const int c0 = 16 * ct0 + 4 * (lane >> 4);  // this lane's channels: c0 + 16 m + r
+  const __bf16* const w0 = wf + (size_t)ct0 * 2 * G::KS * 3 * 512 + lane * 8;
+  std::conditional_t<CT <= 8, ResidentFrags<2 * G::MT, G::KS>, StreamedFrags<2 * G::MT, G::KS>>
+      frags(w0);
+  GeluStage<CT, TOK> stage;
+  stage.load(v, blockIdx.x * TOK, ntok, L, magic);
+  stage.template store<0, 1>(sg);
+  stage.load(v, (blockIdx.x + gridDim.x) * TOK, ntok, L, magic);
+  uint32_t cur = 0;
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, cur ^= 1) {
+    const uint32_t n0 = tile * TOK;
+    __syncthreads();  // stage `cur` is written, the output stage read
+    const __amdgpu_buffer_rsrc_t xr = make_token_rows(x, n0, ntok, G::H);
+    float4 res[R4];
+#pragma unroll
+    for (int i = 0; i < R4; ++i) res[i] = buf_load4(xr, 16 * (threadIdx.x + i * TH), 0);
+    f32x4 acc[2 * G::MT][NT];
+    frags.begin();
+    multiply<2 * G::MT, NT, G::KS, G::GS, TOK>(
+        acc, frags, sg + cur * SZ + tk0 * G::GS + 8 * (lane >> 4), [&](auto ks) {
+          stage.template store<decltype(ks)::value, G::KS>(sg + (cur ^ 1) * SZ);
+        });
+    stage.load(v, (tile + 2 * gridDim.x) * TOK, ntok, L, magic);
 #pragma unroll
     for (int m = 0; m < G::MT; ++m) {
-      const int c = 16 * (ct0 + m) + 4 * (lane >> 4);
+      const int c = c0 + 16 * m;
       const float4 ba = *reinterpret_cast<const float4*>(bias + c);
       const float4 bb = *reinterpret_cast<const float4*>(bias + G::H + c);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const int tk = 16 * (nt0 + nt) + (lane & 15);
-        f32x4 a = acc[m][0][nt], b = acc[m][1][nt];
+        const int tk = tk0 + 16 * nt;
+        f32x4 a = acc[2 * m][nt], b = acc[2 * m + 1][nt];
         if (__builtin_expect(!(finite4(a[0], a[1], a[2], a[3]) && finite4(b[0], b[1], b[2], b[3])), 0)) {
-          if (n0 + tk < ntok) project_fix(a, b, v, w, n0 + tk, c, G::H, L);
+          if (n0 + tk < ntok) project_fix(a, b, v, w, token_base(n0 + tk, G::H, L, magic), c, G::H, L);
         }
         float4 o;
         o.x = (a[0] + ba.x) * sigmoid_f(b[0] + bb.x);
@@ -570,16 +398,13 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, CT <= 8 ? 4 : 2) void s4_ta
       }
     }
     __syncthreads();
-    const float4* const x4 = reinterpret_cast<const float4*>(x + (size_t)n0 * G::H);
-    float4* const y4 = reinterpret_cast<float4*>(y + (size_t)n0 * G::H);
-    const uint32_t left = ntok - n0 < kTailTok ? ntok - n0 : kTailTok;
-    for (uint32_t i = threadIdx.x; i < left * (G::H / 4); i += G::NW * kWave) {
-      const uint32_t tk = i / (G::H / 4), c = 4 * (i % (G::H / 4));
+    const __amdgpu_buffer_rsrc_t yr = make_token_rows(y, n0, ntok, G::H);
+#pragma unroll
+    for (int i = 0; i < R4; ++i) {
+      const int q = threadIdx.x + i * TH, tk = q / (G::H / 4), c = 4 * (q % (G::H / 4));
       const float4 o = *reinterpret_cast<const float4*>(so + tk * G::OS + c);
-      const float4 r = x4[i];
-      y4[i] = float4{o.x + r.x, o.y + r.y, o.z + r.z, o.w + r.w};
+      buf_store4(float4{o.x + res[i].x, o.y + res[i].y, o.z + res[i].z, o.w + res[i].w}, yr, 16 * q);
     }
-    __syncthreads();
   }
 }
 
@@ -587,50 +412,128 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, CT <= 8 ? 4 : 2) void s4_ta
 // Tail backward with respect to its input: from gy [B,L,H], du = dL/du
 // [B,H,L] (through GLU, projection, gelu and the dropout mask) and
 // dP [2 H][np] (token-contiguous rows, zero past the last token) for the
-// weight gradient. The pre-activations are recomputed. The dP parts
-// [part][token][PS] are the B operands of W^T dP and lie over the g parts.
+// weight gradient. The pre-activations are recomputed. Per tile t: the
+// projection with tile t - 1's gelu gradient in its shadow, the GLU gradient
+// into the dP parts [part][token][PS], then W^T dP with tile t + 1's gelu in
+// its shadow; two barriers. B16384 L48 H128: 1421 us with the vector work in
+// phases of its own and erff, 1008 us now; what bounds it is the sum of matrix
+// (13 k cycles a tile) and vector work (16 k), which overlap in part.
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
     const float* __restrict__ gy, const float* __restrict__ v, const uint8_t* __restrict__ mask,
     float scale, const __bf16* __restrict__ wf, const float* __restrict__ w,
     const float* __restrict__ bias, float* __restrict__ du, float* __restrict__ dp, uint32_t ntok,
-    uint32_t L, uint32_t ntiles, uint32_t np) {
+    uint32_t L, uint32_t magic, uint32_t ntiles, uint32_t np) {
   using G = TailGeo<CT>;
-  constexpr int TOK = G::BT;
-  constexpr int WPT = G::WPT < TOK / 16 ? G::WPT : TOK / 16;
-  static_assert(WPT == G::WPT, "every wave has tokens");
-  constexpr int NT = TOK / 16 / G::WPT;
+  constexpr int TOK = G::TOK, NT = TOK / 16 / G::WPT;
+  typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
   extern __shared__ __align__(16) char smem[];
   __bf16* const sg = reinterpret_cast<__bf16*>(smem);
-  __bf16* const sp = sg;
+  __bf16* const sp = sg + 3 * TOK * G::GS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct0 = (wave % G::WPC) * G::MT, nt0 = (wave / G::WPC) * NT;
-  const __bf16* const wt = wf + wfrag_values(G::H);
-  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const uint32_t n0 = tile * TOK;
-    stage_gelu<CT, TOK>(sg, v, n0, ntok, L);
-    __syncthreads();
-    f32x4 acc[G::MT][2][NT];
-    project<CT, TOK, NT>(acc, sg, wf, ct0, nt0, lane);
-    __syncthreads();  // the g parts are read; the dP parts take their place
+  const int tk0 = 16 * nt0 + (lane & 15);
+  const int c0 = 16 * ct0 + 4 * (lane >> 4);
+  const __bf16* const w0 = wf + (size_t)ct0 * 2 * G::KS * 3 * 512 + lane * 8;
+  const __bf16* const wt0 = w0 + wfrag_values(G::H);
+  StreamedFrags<2 * G::MT, G::KS> frags(w0);
+  StreamedFrags<G::MT, 2 * G::KS> tfrags(wt0);
+  const bool masked = mask != nullptr;
+  const float keep = masked ? scale : 1.0f;
+  GeluStage<CT, TOK> stage;
+  stage.load(v, blockIdx.x * TOK, ntok, L, magic);
+  stage.template store<0, 1>(sg);
+  float4 g4[G::MT][NT];
+  auto load_gy = [&](uint32_t n0) {
+    const __amdgpu_buffer_rsrc_t gr = make_token_rows(gy, n0, ntok, G::H);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int m = 0; m < G::MT; ++m)
+        g4[m][nt] = buf_load4(gr, 4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m), 0);
+  };
+  load_gy(blockIdx.x * TOK);
+  frags.begin();
+  // the tile before: its W^T dP, inputs and mask, and where du goes (nowhere yet)
+  f32x4 dg[G::MT][NT];
+  float vv[G::MT][NT][4];
+  uint32_t mk[G::MT][NT][4], at[NT];
+  Slab out = make_slab(du, ntok, ntok, G::H, L, magic);
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    at[nt] = 0;
 #pragma unroll
     for (int m = 0; m < G::MT; ++m) {
-      const int c = 16 * (ct0 + m) + 4 * (lane >> 4);
+      dg[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        vv[m][nt][r] = 0.0f;
+        mk[m][nt][r] = 0;
+      }
+    }
+  }
+  constexpr int E = G::MT * NT;  // groups of four du values per lane and tile
+  auto finish = [&](auto slice, auto slices) {  // du of the tile before
+    constexpr int I = decltype(slice)::value, N = decltype(slices)::value;
+#pragma unroll
+    for (int e = E * I / N; e < E * (I + 1) / N; ++e) {
+      const int m = e % G::MT, nt = e / G::MT;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float o = dg[m][nt][r] * gelu_grad_f(vv[m][nt][r]);
+        o = o * (masked ? (float)mk[m][nt][r] : 1.0f) * keep;
+        buf_store1(o, out.r, 4 * (at[nt] + (uint32_t)(16 * m + r) * L));
+      }
+    }
+  };
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    const uint32_t n0 = tile * TOK;
+    __syncthreads();  // tile t's g parts are written, tile t - 1's dP parts read
+    f32x4 acc[2 * G::MT][NT];
+    multiply<2 * G::MT, NT, G::KS, G::GS, TOK>(
+        acc, frags, sg + tk0 * G::GS + 8 * (lane >> 4),
+        [&](auto ks) { finish(ks, std::integral_constant<int, G::KS>{}); });
+    // Loads return in order, so the ones from HBM are issued where the next
+    // wait for a weight fragment is far off: behind the projection, with the
+    // GLU gradient and the next product's first step in between.
+    tfrags.begin();
+    out = make_slab(du, n0, ntok, G::H, L, magic);
+    stage.load(v, (tile + gridDim.x) * TOK, ntok, L, magic);
+    {
+      const Slab in = make_slab(v, n0, ntok, G::H, L, magic);
+      const __amdgpu_buffer_rsrc_t mr =
+          make_slab<1>(mask, masked ? n0 : ntok, ntok, G::H, L, magic).r;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        at[nt] = token_base(n0 + tk0 + 16 * nt, G::H, L, magic) - in.first + (uint32_t)c0 * L;
+#pragma unroll
+        for (int m = 0; m < G::MT; ++m)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const uint32_t o = at[nt] + (uint32_t)(16 * m + r) * L;
+            vv[m][nt][r] = buf_load1(in.r, 4 * o, 0);
+            mk[m][nt][r] = __builtin_amdgcn_raw_buffer_load_b8(mr, o, 0, 0);
+          }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < G::MT; ++m) {
+      const int c = c0 + 16 * m;
       const float4 ba = *reinterpret_cast<const float4*>(bias + c);
       const float4 bb = *reinterpret_cast<const float4*>(bias + G::H + c);
       const float vba[4] = {ba.x, ba.y, ba.z, ba.w}, vbb[4] = {bb.x, bb.y, bb.z, bb.w};
+      float* const da_row = dp + (size_t)c * np + n0 + tk0;
+      float* const db_row = da_row + (size_t)G::H * np;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const int tk = 16 * (nt0 + nt) + (lane & 15);
+        const int tk = tk0 + 16 * nt;
         const bool in = n0 + tk < ntok;
-        f32x4 a = acc[m][0][nt], b = acc[m][1][nt];
-        float4 g4 = {0.f, 0.f, 0.f, 0.f};
-        if (in) g4 = *reinterpret_cast<const float4*>(gy + (size_t)(n0 + tk) * G::H + c);
+        f32x4 a = acc[2 * m][nt], b = acc[2 * m + 1][nt];
         if (__builtin_expect(!(finite4(a[0], a[1], a[2], a[3]) && finite4(b[0], b[1], b[2], b[3])), 0)) {
-          if (in) project_fix(a, b, v, w, n0 + tk, c, G::H, L);
+          if (in) project_fix(a, b, v, w, token_base(n0 + tk, G::H, L, magic), c, G::H, L);
         }
-        const float g[4] = {g4.x, g4.y, g4.z, g4.w};
+        const float g[4] = {g4[m][nt].x, g4[m][nt].y, g4[m][nt].z, g4[m][nt].w};
         float pa[8];  // four value and four gate gradients
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -639,15 +542,16 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
           const float db = (1.0f - s) * s * g[r] * (a[r] + vba[r]);
           pa[r] = in ? da : 0.0f;
           pa[4 + r] = in ? db : 0.0f;
-          dp[(size_t)(c + r) * np + n0 + tk] = pa[r];
-          dp[(size_t)(G::H + c + r) * np + n0 + tk] = pa[4 + r];
         }
-        bf16x8 hi, mid, lo;
-        split3_bf16x8(pa, hi, mid, lo);
-        const bf16x8 parts[3] = {hi, mid, lo};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          da_row[(size_t)r * np + 16 * nt] = pa[r];
+          db_row[(size_t)r * np + 16 * nt] = pa[4 + r];
+        }
+        bf16x8 parts[3];
+        split3_bf16x8(pa, parts[0], parts[1], parts[2]);
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
-          typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
           __bf16* d = sp + (p * TOK + tk) * G::PS + c;
           *reinterpret_cast<bf16x4v*>(d) =
               bf16x4v{parts[p][0], parts[p][1], parts[p][2], parts[p][3]};
@@ -657,72 +561,34 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
       }
     }
     __threadfence_block();
-    __syncthreads();
-    // dg = W^T dP
-    f32x4 dg[G::MT][NT];
+    __syncthreads();  // the dP parts are written, the g parts read
+    load_gy((tile + gridDim.x) * TOK);
+    multiply<G::MT, NT, 2 * G::KS, G::PS, TOK>(
+        dg, tfrags, sp + tk0 * G::PS + 8 * (lane >> 4),
+        [&](auto ks) { stage.template store<decltype(ks)::value, 2 * G::KS>(sg); });
+    frags.begin();
 #pragma unroll
-    for (int m = 0; m < G::MT; ++m)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) dg[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const __bf16* const b0 = sp + (16 * nt0 + (lane & 15)) * G::PS + 8 * (lane >> 4);
-    const __bf16* const a0 = wt + (size_t)ct0 * 2 * G::KS * 3 * 512 + lane * 8;
-    bf16x8 a[G::MT][3];
-    load_frags<G::MT>(a, a0, 2 * G::KS);
-#pragma unroll 1
-    for (int ks = 0; ks < 2 * G::KS; ++ks) {
-      bf16x8 an[G::MT][3];
-      load_frags<G::MT>(an, a0 + (ks + 1 < 2 * G::KS ? ks + 1 : 0) * 3 * 512, 2 * G::KS);
-      if (ks > 0 && step_negated(ks) != step_negated(ks - 1))
-        negate(reinterpret_cast<f32x4(&)[G::MT * NT]>(dg));
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        bf16x8 b[3];
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          b[p] = *reinterpret_cast<const bf16x8*>(b0 + (p * TOK + 16 * nt) * G::PS + 32 * ks);
-#pragma unroll
-        for (int m = 0; m < G::MT; ++m) dg[m][nt] = mfma_split6(a[m], b, dg[m][nt]);
-      }
-#pragma unroll
-      for (int m = 0; m < G::MT; ++m)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) a[m][p] = an[m][p];
-    }
-    if (step_negated(2 * G::KS - 1)) negate(reinterpret_cast<f32x4(&)[G::MT * NT]>(dg));
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const uint32_t tk = 16 * (nt0 + nt) + (lane & 15), n = n0 + tk;
-      if (n < ntok) {
-        const uint32_t base = token_base(n, G::H, L);
-#pragma unroll
-        for (int m = 0; m < G::MT; ++m) {
-          const int c = 16 * (ct0 + m) + 4 * (lane >> 4);
-          f32x4 d = dg[m][nt];
-          if (__builtin_expect(!finite4(d[0], d[1], d[2], d[3]), 0)) {
+      for (int m = 0; m < G::MT; ++m) {
+        const uint32_t n = n0 + tk0 + 16 * nt;
+        f32x4& d = dg[m][nt];
+        if (__builtin_expect(!finite4(d[0], d[1], d[2], d[3]), 0)) {
+          if (n < ntok) {
 #pragma unroll 1
             for (int r = 0; r < 4; ++r) {
+              const int c = c0 + 16 * m + r;
               float s = 0.0f;
 #pragma unroll 1
               for (int o = 0; o < 2 * G::H; ++o)
-                s = fmaf(w[(size_t)o * G::H + c + r], dp[(size_t)o * np + n], s);
-              d[0] = r == 0 ? s : d[0];
-              d[1] = r == 1 ? s : d[1];
-              d[2] = r == 2 ? s : d[2];
-              d[3] = r == 3 ? s : d[3];
+                s = fmaf(w[(size_t)o * G::H + c], dp[(size_t)o * np + n], s);
+              set_elem(d, r, s);
             }
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t at = base + (uint32_t)(c + r) * L;
-            float o = d[r] * gelu_grad_f(v[at]);
-            if (mask) o = o * (float)mask[at] * scale;
-            du[at] = o;
           }
         }
       }
-    }
-    __syncthreads();
   }
+  finish(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -732,7 +598,9 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
 // rows of dP, read straight from memory in the A layout (each row's 32 tokens
 // are one 128-byte line) and split in registers; g is computed, split and
 // shared through LDS [part][channel][40]. Partials [range][2 H H + 2 H] go to
-// the workspace for a fixed-order reduction.
+// the workspace for a fixed-order reduction. Step s + 1's gelu and splits run
+// in the shadow of step s's products: 381 us at B16384 L48 H128, 430 with them
+// ahead of the products.
 // ---------------------------------------------------------------------------
 template <int CT>
 struct DwGeo {
@@ -748,7 +616,7 @@ struct DwGeo {
 template <int CT, bool VEC>
 __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     const float* __restrict__ dp, const float* __restrict__ v, float* __restrict__ part,
-    uint32_t ntok, uint32_t L, uint32_t nsteps, uint32_t steps_per, uint32_t np) {
+    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t nsteps, uint32_t steps_per, uint32_t np) {
   using D = DwGeo<CT>;
   constexpr int H = 16 * CT, NC = 16 * D::NB, TH = D::NW * kWave;
   constexpr int kUnits = NC * (kDwTok / 8);  // (channel, eight tokens)
@@ -773,30 +641,27 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
   float vr[U][8];
   float ar[D::MT][8];
   auto load_v = [&](uint32_t s) {
+    const Slab in = make_slab(v, s * kDwTok, ntok, H, L, magic);
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const int u = threadIdx.x + i * TH;
-      const int c = u >> 2, q = u & 3;
-      const uint32_t n = s * kDwTok + 8 * q;
-      const bool on = u < kUnits;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vr[i][e] = 0.0f;
+      const uint32_t n = s * kDwTok + 8 * (u & 3);
+      const uint32_t c = (uint32_t)(nb * NC + (u >> 2)) * L - in.first;
+      const bool on = kUnits % TH == 0 || u < kUnits;
       if constexpr (VEC) {  // L % 4 == 0: four tokens from a multiple of four lie in one row
 #pragma unroll
         for (int e = 0; e < 8; e += 4) {
-          if (on && n + e < ntok) {
-            const float4 f = *reinterpret_cast<const float4*>(
-                v + token_base(n + e, H, L) + (size_t)(nb * NC + c) * L);
-            vr[i][e] = f.x;
-            vr[i][e + 1] = f.y;
-            vr[i][e + 2] = f.z;
-            vr[i][e + 3] = f.w;
-          }
+          const float4 f =
+              buf_load4(in.r, on ? 4 * (token_base(n + e, H, L, magic) + c) : kOob, 0);
+          vr[i][e] = f.x;
+          vr[i][e + 1] = f.y;
+          vr[i][e + 2] = f.z;
+          vr[i][e + 3] = f.w;
         }
       } else {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          if (on && n + e < ntok) vr[i][e] = v[token_base(n + e, H, L) + (size_t)(nb * NC + c) * L];
+          vr[i][e] = buf_load1(in.r, on ? 4 * (token_base(n + e, H, L, magic) + c) : kOob, 0);
       }
     }
   };
@@ -816,49 +681,84 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
       ar[m][7] = f1.w;
     }
   };
-  if (s0 < s1) {
-    load_v(s0);
-    load_a(s0);
-  }
-  for (uint32_t s = s0; s < s1; ++s) {
-    __bf16* const st = sg + ((s - s0) & 1) * SZ;
+  // gelu and split of the values held in vr into a stage
+  auto store_v = [&](__bf16* st) {
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const int u = threadIdx.x + i * TH;
-      if (u < kUnits) {
-        float g[8];
+      float g[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) g[e] = gelu_f(vr[i][e]);  // gelu(0) = 0 past the end
-        bf16x8 hi, mid, lo;
-        split3_bf16x8(g, hi, mid, lo);
+      for (int e = 0; e < 8; ++e) g[e] = gelu_f(vr[i][e]);  // gelu(0) = 0 past the end
+      bf16x8 hi, mid, lo;
+      split3_bf16x8(g, hi, mid, lo);
+      if (kUnits % TH == 0 || u < kUnits) {
         __bf16* d = st + (u >> 2) * D::CS + 8 * (u & 3);
         *reinterpret_cast<bf16x8*>(d) = hi;
         *reinterpret_cast<bf16x8*>(d + NC * D::CS) = mid;
         *reinterpret_cast<bf16x8*>(d + 2 * NC * D::CS) = lo;
       }
     }
-    bf16x8 a[D::MT][3];
+  };
+  bf16x8 a[D::MT][3], an[D::MT][3];
+  auto split_a = [&](bf16x8 (&o)[D::MT][3]) {
 #pragma unroll
     for (int m = 0; m < D::MT; ++m) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) rows[m] += ar[m][e];
-      split3_bf16x8(ar[m], a[m][0], a[m][1], a[m][2]);
+      split3_bf16x8(ar[m], o[m][0], o[m][1], o[m][2]);
     }
-    if (s + 1 < s1) {
-      load_v(s + 1);
-      load_a(s + 1);
+  };
+  if (s0 < s1) {
+    load_v(s0);
+    load_a(s0);
+    store_v(sg);
+    split_a(a);
+    if (s0 + 1 < s1) {
+      load_v(s0 + 1);
+      load_a(s0 + 1);
     }
-    __syncthreads();  // one per step: the stages alternate
+  }
+  auto products = [&](const __bf16* st) {
     const __bf16* const b0 = st + (lane & 15) * D::CS + 8 * (lane >> 4);
+    constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};  // small ones first
+    constexpr int NG = D::NB % 4 == 0 ? 4 : D::NB % 3 == 0 ? 3 : D::NB % 5 == 0 ? 5 : D::NB;
 #pragma unroll
-    for (int n = 0; n < D::NB; ++n) {
-      bf16x8 b[3];
+    for (int n0 = 0; n0 < D::NB; n0 += NG) {
+      bf16x8 b[NG][3];
 #pragma unroll
-      for (int p = 0; p < 3; ++p)
-        b[p] = *reinterpret_cast<const bf16x8*>(b0 + (p * NC + 16 * n) * D::CS);
+      for (int n = 0; n < NG; ++n)
 #pragma unroll
-      for (int m = 0; m < D::MT; ++m) acc[m][n] = mfma_split6(a[m], b, acc[m][n]);
+        for (int p = 0; p < 3; ++p)
+          b[n][p] = *reinterpret_cast<const bf16x8*>(b0 + (p * NC + 16 * (n0 + n)) * D::CS);
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int n = 0; n < NG; ++n)
+#pragma unroll
+          for (int m = 0; m < D::MT; ++m)
+            acc[m][n0 + n] = mfma_bf16(a[m][pa[q]], b[n][pb[q]], acc[m][n0 + n]);
     }
+  };
+  uint32_t s = s0;
+  for (; s + 1 < s1; ++s) {
+    __syncthreads();  // one per step: the stages alternate
+    // step s's products, and in their shadow step s + 1's gelu and splits
+    // (after them in program order: LDS writes cannot pass the products' reads)
+    products(sg + ((s - s0) & 1) * SZ);
+    store_v(sg + ((s + 1 - s0) & 1) * SZ);
+    split_a(an);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t ahead = s + 2 < s1 ? s + 2 : s1 - 1;
+    load_v(ahead);
+    load_a(ahead);
+#pragma unroll
+    for (int m = 0; m < D::MT; ++m)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) a[m][p] = an[m][p];
+  }
+  if (s < s1) {
+    __syncthreads();
+    products(sg + ((s - s0) & 1) * SZ);
   }
   float* const dst = part + (size_t)range * (2 * H * H + 2 * H);
 #pragma unroll
@@ -876,7 +776,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
           const uint32_t e1 = s1 * kDwTok < ntok ? s1 * kDwTok : ntok;
 #pragma unroll 1
           for (uint32_t k = s0 * kDwTok; k < e1; ++k)
-            s = fmaf(dp[(size_t)c * np + k], gelu_f(v[token_base(k, H, L) + (uint32_t)h * L]), s);
+            s = fmaf(dp[(size_t)c * np + k], gelu_f(v[token_base(k, H, L, magic) + (uint32_t)h * L]), s);
         }
         dst[(size_t)c * H + h] = s;
       }
@@ -885,29 +785,6 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     t += __shfl_xor(t, 16);
     t += __shfl_xor(t, 32);
     if (nb == 0 && lane < 16) dst[(size_t)2 * H * H + r0 + lane] = t;
-  }
-}
-
-// Sums the ranges in a fixed order: 16 threads per element take every 16th
-// range, then a tree over them.
-__global__ __launch_bounds__(256) void s4_dw_reduce_kernel(const float* __restrict__ part,
-                                                           float* __restrict__ dw,
-                                                           float* __restrict__ dbias, int nw, int nb,
-                                                           int nranges) {
-  __shared__ float s[16][17];
-  const int e = threadIdx.x & 15, q = threadIdx.x >> 4;
-  const int i = blockIdx.x * 16 + e, n = nw + nb;
-  float acc = 0.0f;
-  if (i < n)
-    for (int r = q; r < nranges; r += 16) acc += part[(size_t)r * n + i];
-  s[q][e] = acc;
-  __syncthreads();
-  if (q == 0 && i < n) {
-    float t = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) t += s[k][e];
-    if (i < nw) dw[i] = t;
-    else dbias[i - nw] = t;
   }
 }
 
