@@ -295,12 +295,24 @@ def summarize_kernel_times(raw):
 # =============================================================================
 # Runtime
 # =============================================================================
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
-def _stream_handle(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _call(fn: Callable[..., int], device: torch.device, *args: Any) -> None:
+    """``fn(*args, stream)`` of the native library on torch's current stream
+    of `device`, with that device current; raises for a negative status. The
+    device context and torch's stream object cost 3 us a call, so the context
+    is entered only from another device and the stream is taken as its raw
+    handle (launch_fwd of 64 x 16 rows: 9.8 -> 6.3 us on the host)."""
+    index = device.index
+    if torch._C._cuda_getDevice() == index:
+        status = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    else:
+        with torch.cuda.device(device):
+            status = fn(*args, torch._C._cuda_getCurrentRawStream(index))
+    if status != _lib.PT_OK:
+        _lib.check(status, fn.__name__)
 
 
 # FWD/dX kernel choice of HipWarpRuntime(rows_algo=...): the C ABI's
@@ -464,11 +476,8 @@ class HipWarpRuntime:
         self._require_contiguous(x, k, y)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_fwd_f32_algo(
-                    _ptr(x), _ptr(k), _ptr(y), B, H, L, K,
-                    self.waves_per_block, self._rows_algo_id, _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_fwd_f32_algo")
+            _call(self._lib.pt_dwconv1d_fwd_f32_algo, x.device,
+                  _ptr(x), _ptr(k), _ptr(y), B, H, L, K, self.waves_per_block, self._rows_algo_id)
 
         (collector or KERNEL_EVENTS).launch("fwd", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -486,11 +495,9 @@ class HipWarpRuntime:
         self._require_contiguous(gy, k, gx)
 
         def launch() -> None:
-            with torch.cuda.device(gy.device):
-                st = self._lib.pt_dwconv1d_dx_f32_algo(
-                    _ptr(gy), _ptr(k), _ptr(gx), B, H, L, K,
-                    self.dx_waves_per_block, self._rows_algo_id, _stream_handle(gy.device))
-            _lib.check(st, "pt_dwconv1d_dx_f32_algo")
+            _call(self._lib.pt_dwconv1d_dx_f32_algo, gy.device,
+                  _ptr(gy), _ptr(k), _ptr(gx), B, H, L, K, self.dx_waves_per_block,
+                  self._rows_algo_id)
 
         (collector or KERNEL_EVENTS).launch("bwd_input", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -529,11 +536,8 @@ class HipWarpRuntime:
         B, H, L = self._check_bwd_weight(gy, x, gk, K)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_dk_atomic_f32(
-                    _ptr(gy), _ptr(x), _ptr(gk), B, H, L, K, self.bwdk_block,
-                    1 if zero_first else 0, _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_dk_atomic_f32")
+            _call(self._lib.pt_dwconv1d_dk_atomic_f32, x.device,
+                  _ptr(gy), _ptr(x), _ptr(gk), B, H, L, K, self.bwdk_block, 1 if zero_first else 0)
 
         phase = "bwd_weight_zero" if zero_first else "bwd_weight"
         (collector or KERNEL_EVENTS).launch(phase, launch, {"B": B, "H": H, "L": L, "K": K})
@@ -558,12 +562,12 @@ class HipWarpRuntime:
         kept, the least recently used dropped first, so callers that make
         short-lived streams do not pile up workspaces; an entry holds its
         stream, so no live entry's handle can be recycled by a new stream."""
-        stream = torch.cuda.current_stream(device)
-        key = (device.index if device.index is not None else torch.cuda.current_device(),
-               int(stream.cuda_stream))
+        index = device.index if device.index is not None else torch.cuda.current_device()
+        key = (index, torch._C._cuda_getCurrentRawStream(index))
         with self._ws_lock:
             entry = self._workspaces.get(key)
             if entry is None or entry[1].numel() < nbytes:
+                stream = torch.cuda.current_stream(device)
                 with torch.cuda.stream(stream):
                     ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
                 self._workspaces[key] = (stream, ws)
@@ -593,11 +597,8 @@ class HipWarpRuntime:
         ws = self._get_workspace(nbytes, x.device)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_dk_det_f32(
-                    _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(),
-                    B, H, L, K, self.bwdk_block, _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_dk_det_f32")
+            _call(self._lib.pt_dwconv1d_dk_det_f32, x.device,
+                  _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K, self.bwdk_block)
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_det", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -631,10 +632,7 @@ class HipWarpRuntime:
         self._require_contiguous(x, k, y)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_fwd_bf16(_ptr(x), _ptr(k), _ptr(y), B, H, L, K,
-                                                    _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_fwd_bf16")
+            _call(self._lib.pt_dwconv1d_fwd_bf16, x.device, _ptr(x), _ptr(k), _ptr(y), B, H, L, K)
 
         (collector or KERNEL_EVENTS).launch("fwd_bf16", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -647,10 +645,7 @@ class HipWarpRuntime:
         self._require_contiguous(gy, k, gx)
 
         def launch() -> None:
-            with torch.cuda.device(gy.device):
-                st = self._lib.pt_dwconv1d_dx_bf16(_ptr(gy), _ptr(k), _ptr(gx), B, H, L, K,
-                                                   _stream_handle(gy.device))
-            _lib.check(st, "pt_dwconv1d_dx_bf16")
+            _call(self._lib.pt_dwconv1d_dx_bf16, gy.device, _ptr(gy), _ptr(k), _ptr(gx), B, H, L, K)
 
         (collector or KERNEL_EVENTS).launch("bwd_input_bf16", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -678,11 +673,8 @@ class HipWarpRuntime:
         B, H, L = self._check_bf16_dk(gy, x, gk, K)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_dk_atomic_bf16(
-                    _ptr(gy), _ptr(x), _ptr(gk), B, H, L, K, self.bwdk_block,
-                    1 if zero_first else 0, _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_dk_atomic_bf16")
+            _call(self._lib.pt_dwconv1d_dk_atomic_bf16, x.device,
+                  _ptr(gy), _ptr(x), _ptr(gk), B, H, L, K, self.bwdk_block, 1 if zero_first else 0)
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_bf16", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -700,11 +692,8 @@ class HipWarpRuntime:
         ws = self._get_workspace(int(out.value), x.device)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_dk_det_bf16(
-                    _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(),
-                    B, H, L, K, self.bwdk_block, _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_dk_det_bf16")
+            _call(self._lib.pt_dwconv1d_dk_det_bf16, x.device,
+                  _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K, self.bwdk_block)
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_det_bf16", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -733,10 +722,8 @@ class HipWarpRuntime:
             dw.zero_()
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.flash_dk_fp32(_ptr(x), _ptr(gy), _ptr(dw), B, H, L, K, int(gz),
-                                             _stream_handle(x.device))
-            _lib.check(st, "flash_dk_fp32")
+            _call(self._lib.flash_dk_fp32, x.device,
+                  _ptr(x), _ptr(gy), _ptr(dw), B, H, L, K, int(gz))
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_cl", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -768,10 +755,8 @@ class HipWarpRuntime:
         self._require_contiguous(x, k, y)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_fwd_long_f32(_ptr(x), _ptr(k), _ptr(y), B, H, L, K,
-                                                        _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_fwd_long_f32")
+            _call(self._lib.pt_dwconv1d_fwd_long_f32, x.device,
+                  _ptr(x), _ptr(k), _ptr(y), B, H, L, K)
 
         (collector or KERNEL_EVENTS).launch("fwd_long", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -786,10 +771,8 @@ class HipWarpRuntime:
         self._require_contiguous(gy, k, gx)
 
         def launch() -> None:
-            with torch.cuda.device(gy.device):
-                st = self._lib.pt_dwconv1d_dx_long_f32(_ptr(gy), _ptr(k), _ptr(gx), B, H, L, K,
-                                                       _stream_handle(gy.device))
-            _lib.check(st, "pt_dwconv1d_dx_long_f32")
+            _call(self._lib.pt_dwconv1d_dx_long_f32, gy.device,
+                  _ptr(gy), _ptr(k), _ptr(gx), B, H, L, K)
 
         (collector or KERNEL_EVENTS).launch("bwd_input_long", launch, {"B": B, "H": H, "L": L, "K": K})
 
@@ -817,11 +800,8 @@ class HipWarpRuntime:
         ws = self._get_workspace(int(out.value), x.device)
 
         def launch() -> None:
-            with torch.cuda.device(x.device):
-                st = self._lib.pt_dwconv1d_dk_long_f32(
-                    _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K,
-                    _stream_handle(x.device))
-            _lib.check(st, "pt_dwconv1d_dk_long_f32")
+            _call(self._lib.pt_dwconv1d_dk_long_f32, x.device,
+                  _ptr(gy), _ptr(x), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K)
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_long", launch, {"B": B, "H": H, "L": L, "K": K})
 

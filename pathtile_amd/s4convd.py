@@ -35,7 +35,7 @@ from torch import nn
 
 from . import _lib
 from .runtime import (
-    KERNEL_EVENTS, MAX_L, _ptr, _stream_handle, get_runtime, reference_depthwise_conv,
+    KERNEL_EVENTS, MAX_L, _call, _ptr, get_runtime, reference_depthwise_conv,
 )
 
 
@@ -171,13 +171,10 @@ def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight
     B, L, H = x.shape
     prep = torch.empty(_size_query("pt_s4_block_prep_values", H, L), device=x.device)
     xt, u = torch.empty((2, B, H, L), device=x.device).unbind(0)
-    with torch.cuda.device(x.device):
-        st = runtime._lib.pt_s4_block_mix_f32(
-            _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
-            _ptr(skip), _ptr(weight), _ptr(prep), _ptr(xt), _ptr(u), B, H, L, c_re.shape[1],
-            int(backward), runtime.waves_per_block, runtime._rows_algo_id,
-            _stream_handle(x.device))
-    _lib.check(st, "pt_s4_block_mix_f32")
+    _call(runtime._lib.pt_s4_block_mix_f32, x.device,
+          _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
+          _ptr(skip), _ptr(weight), _ptr(prep), _ptr(xt), _ptr(u), B, H, L, c_re.shape[1],
+          int(backward), runtime.waves_per_block, runtime._rows_algo_id)
     return prep, xt, u
 
 
@@ -185,11 +182,8 @@ def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias) -> torch.T
     runtime = get_runtime()
     B, L, H = x.shape
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
-        st = runtime._lib.pt_s4_block_tail_f32(
-            _ptr(v), _ptr(x), _ptr(prep), _ptr(weight), _ptr(bias), _ptr(y), B, H, L,
-            _stream_handle(x.device))
-    _lib.check(st, "pt_s4_block_tail_f32")
+    _call(runtime._lib.pt_s4_block_tail_f32, x.device,
+          _ptr(v), _ptr(x), _ptr(prep), _ptr(weight), _ptr(bias), _ptr(y), B, H, L)
     return y
 
 
@@ -236,14 +230,12 @@ class S4BlockFused(torch.autograd.Function):
         def opt(t):
             return None if t is None else _ptr(t)
 
-        with torch.cuda.device(x.device):
-            st = runtime._lib.pt_s4_block_bwd_f32(
-                _ptr(gy), _ptr(xt), _ptr(v), opt(mask), ctx.scale, _ptr(prep), _ptr(weight),
-                _ptr(bias), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
-                opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
-                c_re.shape[1], runtime.dx_waves_per_block, runtime._rows_algo_id,
-                runtime.bwdk_block, _stream_handle(x.device))
-        _lib.check(st, "pt_s4_block_bwd_f32")
+        _call(runtime._lib.pt_s4_block_bwd_f32, x.device,
+              _ptr(gy), _ptr(xt), _ptr(v), opt(mask), ctx.scale, _ptr(prep), _ptr(weight),
+              _ptr(bias), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
+              opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
+              c_re.shape[1], runtime.dx_waves_per_block, runtime._rows_algo_id,
+              runtime.bwdk_block)
         grads = [gx, gp[5], *gp[:5], gw, gb]
         return (*(g if n else None for g, n in zip(grads, need)), None)
 
