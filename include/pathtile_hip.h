@@ -322,6 +322,29 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v,
                         void* stream);
 
 /*
+ * The ends of the S4ConvD model (kernels/warp_tiled_ampere.py:1193-1215 in
+ * the reference), FP32, H a multiple of 4 up to 1024. Encoder: y [B, L, H] =
+ * x [B, L, inputs] w^T + bias, w [H, inputs], inputs <= 8. Head: out [B,
+ * outputs] = x[:, L-1, :] w^T + bias, w [outputs, H], outputs <= 4: the
+ * decoder at the one column that the model returns. The *_grad calls give the
+ * gradients of w and bias by a fixed-order reduction, and the head's gx [B,
+ * L, H] (NULL: skipped), zero before the last column. bias, y, gy of the
+ * encoder and x, gx of the head are 16-byte aligned.
+ */
+int pt_s4_encode_f32(const float* x, const float* w, const float* bias, float* y, int B,
+                     int L, int inputs, int H, void* stream);
+int pt_s4_encode_grad_workspace_bytes(int B, int L, int inputs, int H, size_t* bytes);
+int pt_s4_encode_grad_f32(const float* x, const float* gy, float* dw, float* dbias,
+                          void* workspace, size_t workspace_bytes, int B, int L,
+                          int inputs, int H, void* stream);
+int pt_s4_head_f32(const float* x, const float* w, const float* bias, float* out, int B,
+                   int H, int L, int outputs, void* stream);
+int pt_s4_head_grad_workspace_bytes(int B, int H, int L, int outputs, size_t* bytes);
+int pt_s4_head_grad_f32(const float* x, const float* gy, const float* w, float* gx,
+                        float* dw, float* dbias, void* workspace, size_t workspace_bytes,
+                        int B, int H, int L, int outputs, void* stream);
+
+/*
  * Compiled resources of the kernel that serves (L, K) for `kernel_id`
  * (PT_KERNEL_*), as hipFuncGetAttributes reports them on the current device:
  * registers per lane, static LDS bytes, scratch (private) bytes per lane and

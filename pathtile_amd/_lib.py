@@ -84,6 +84,12 @@ SIGNATURES = {
     "pt_s4_block_bwd_f32": (
         _i, [_vp] * 4 + [ctypes.c_float] + [_vp] * 18 + [ctypes.c_size_t] + [_i] * 7 + [_vp]
     ),
+    "pt_s4_encode_f32": (_i, [_vp] * 4 + [_i] * 4 + [_vp]),
+    "pt_s4_encode_grad_workspace_bytes": (_i, [_i] * 4 + [_szp]),
+    "pt_s4_encode_grad_f32": (_i, [_vp] * 5 + [ctypes.c_size_t] + [_i] * 4 + [_vp]),
+    "pt_s4_head_f32": (_i, [_vp] * 4 + [_i] * 4 + [_vp]),
+    "pt_s4_head_grad_workspace_bytes": (_i, [_i] * 4 + [_szp]),
+    "pt_s4_head_grad_f32": (_i, [_vp] * 7 + [ctypes.c_size_t] + [_i] * 4 + [_vp]),
     "pt_kernel_attributes": (_i, [_i, _i, _i, _ip, _ip, _ip, _ip]),
     "pt_dynamic_lds_bytes": (_i, [_i, _i, _i, _i, _ip]),
 }

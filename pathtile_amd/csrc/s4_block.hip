@@ -98,6 +98,39 @@ static int transpose_launch(const float* d, const float* add, float* out, int B,
                 args);
 }
 
+// --- the model's ends ---------------------------------------------------------
+constexpr int kEndRanges = 1024;  // partials of the ends' weight gradients
+
+static int check_ends(int B, int H, int L, int n, int most) {
+  if (B < 1 || L < 1 || H < 4 || H > 4 * kEndThreads || H % 4 != 0 || n < 1 || n > most)
+    return PT_ERR_SHAPE;
+  if ((long long)B * H * L >= (1LL << 31)) return PT_ERR_SHAPE;
+  return PT_OK;
+}
+
+static uint32_t encode_grid(uint32_t ntok, int H) {
+  const uint32_t per = (uint32_t)(kEndThreads / (H / 4));
+  const uint32_t n = (ntok + per - 1) / per;
+  return n < (uint32_t)kEndRanges ? n : (uint32_t)kEndRanges;
+}
+
+template <int NI>
+static const void* encode_fn(int ni, bool grad) {
+  if constexpr (NI <= kEncMaxIn) {
+    if (ni == NI)
+      return grad ? (const void*)&s4_encode_grad_kernel<NI> : (const void*)&s4_encode_kernel<NI>;
+    return encode_fn<NI + 1>(ni, grad);
+  }
+  return nullptr;
+}
+
+static int reduce_launch(const float* part, float* dw, float* db, int nw, int nb, int nr,
+                         void* stream) {
+  void* args[] = {&part, &dw, &db, &nw, &nb, &nr};
+  return launch((const void*)&s4_dw_reduce_kernel, (uint32_t)((nw + nb + 15) / 16), 256, 0, stream,
+                args);
+}
+
 }  // namespace pt
 
 extern "C" {
@@ -213,11 +246,7 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
     st = pt::launch(fn, o.ranges * (uint32_t)k.dw_split, (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds,
                     stream, args);
     if (st != PT_OK) return st;
-    int nw = 2 * H * H, nb = 2 * H, nr = (int)o.ranges;
-    const float* cpart = part;
-    void* rargs[] = {&cpart, &dw, &dbias, &nw, &nb, &nr};
-    st = pt::launch((const void*)&pt::s4_dw_reduce_kernel, (uint32_t)((nw + nb + 15) / 16), 256, 0,
-                    stream, rargs);
+    st = pt::reduce_launch(part, dw, dbias, 2 * H * H, 2 * H, (int)o.ranges, stream);
     if (st != PT_OK) return st;
   }
   if (gx) {  // dX before its transpose takes dP's place, which is read by now
@@ -235,6 +264,84 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
                    &d_log_a_re, &d_a_im, &d_skip, &L, &states};
   return pt::launch((const void*)&pt::s4_taps_grad_kernel, (uint32_t)H, pt::kPrepThreads, 0, stream,
                     targs);
+}
+
+int pt_s4_encode_f32(const float* x, const float* w, const float* bias, float* y, int B, int L,
+                     int inputs, int H, void* stream) {
+  const int st = pt::check_ends(B, H, L, inputs, pt::kEncMaxIn);
+  if (st != PT_OK) return st;
+  if (!x || !w || !bias || !y) return PT_ERR_NULL;
+  if (!pt::aligned16(bias) || !pt::aligned16(y)) return PT_ERR_ALIGN;
+  uint32_t ntok = (uint32_t)B * (uint32_t)L;
+  const uint32_t per = (uint32_t)(pt::kEndThreads / (H / 4));
+  const void* fn = pt::encode_fn<1>(inputs, false);
+  void* args[] = {&x, &w, &bias, &y, &ntok, &H};
+  return pt::launch(fn, pt::resident_grid(fn, pt::kEndThreads, 0, (ntok + per - 1) / per),
+                    per * (uint32_t)(H / 4), 0, stream, args);
+}
+
+int pt_s4_encode_grad_workspace_bytes(int B, int L, int inputs, int H, size_t* bytes) {
+  if (!bytes) return PT_ERR_NULL;
+  const int st = pt::check_ends(B, H, L, inputs, pt::kEncMaxIn);
+  if (st == PT_OK)
+    *bytes = (size_t)pt::encode_grid((uint32_t)B * (uint32_t)L, H) * (H * inputs + H) * 4;
+  return st;
+}
+
+int pt_s4_encode_grad_f32(const float* x, const float* gy, float* dw, float* dbias,
+                          void* workspace, size_t workspace_bytes, int B, int L, int inputs, int H,
+                          void* stream) {
+  size_t need = 0;
+  int st = pt_s4_encode_grad_workspace_bytes(B, L, inputs, H, &need);
+  if (st != PT_OK) return st;
+  if (!x || !gy || !dw || !dbias) return PT_ERR_NULL;
+  if (!pt::aligned16(gy)) return PT_ERR_ALIGN;
+  if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
+  uint32_t ntok = (uint32_t)B * (uint32_t)L;
+  const uint32_t grid = pt::encode_grid(ntok, H), per = (uint32_t)(pt::kEndThreads / (H / 4));
+  float* part = static_cast<float*>(workspace);
+  void* args[] = {&x, &gy, &part, &ntok, &H};
+  st = pt::launch(pt::encode_fn<1>(inputs, true), grid, per * (uint32_t)(H / 4), 0, stream, args);
+  if (st != PT_OK) return st;
+  return pt::reduce_launch(part, dw, dbias, H * inputs, H, (int)grid, stream);
+}
+
+int pt_s4_head_f32(const float* x, const float* w, const float* bias, float* out, int B, int H,
+                   int L, int outputs, void* stream) {
+  const int st = pt::check_ends(B, H, L, outputs, pt::kHeadMaxOut);
+  if (st != PT_OK) return st;
+  if (!x || !w || !bias || !out) return PT_ERR_NULL;
+  void* args[] = {&x, &w, &bias, &out, &B, &H, &L, &outputs};
+  const uint32_t per = pt::kEndThreads / pt::kWave;
+  return pt::launch((const void*)&pt::s4_head_kernel, ((uint32_t)B + per - 1) / per,
+                    pt::kEndThreads, 0, stream, args);
+}
+
+int pt_s4_head_grad_workspace_bytes(int B, int H, int L, int outputs, size_t* bytes) {
+  if (!bytes) return PT_ERR_NULL;
+  const int st = pt::check_ends(B, H, L, outputs, pt::kHeadMaxOut);
+  const int n = B < pt::kEndRanges ? B : pt::kEndRanges;
+  if (st == PT_OK) *bytes = (size_t)n * (outputs * H + outputs) * 4;
+  return st;
+}
+
+int pt_s4_head_grad_f32(const float* x, const float* gy, const float* w, float* gx, float* dw,
+                        float* dbias, void* workspace, size_t workspace_bytes, int B, int H, int L,
+                        int outputs, void* stream) {
+  size_t need = 0;
+  int st = pt_s4_head_grad_workspace_bytes(B, H, L, outputs, &need);
+  if (st != PT_OK) return st;
+  if (!x || !gy || !w || !dw || !dbias) return PT_ERR_NULL;
+  if (!pt::aligned16(x) || (gx && !pt::aligned16(gx))) return PT_ERR_ALIGN;
+  if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
+  int per = (B + pt::kEndRanges - 1) / pt::kEndRanges;
+  const int grid = (B + per - 1) / per;
+  float* part = static_cast<float*>(workspace);
+  void* args[] = {&x, &gy, &w, &gx, &part, &B, &H, &L, &outputs, &per};
+  st = pt::launch((const void*)&pt::s4_head_grad_kernel, (uint32_t)grid, pt::kEndThreads, 0, stream,
+                  args);
+  if (st != PT_OK) return st;
+  return pt::reduce_launch(part, dw, dbias, outputs * H, outputs, grid, stream);
 }
 
 }  // extern "C"

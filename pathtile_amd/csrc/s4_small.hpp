@@ -321,4 +321,155 @@ __global__ __launch_bounds__(256) void s4_dw_reduce_kernel(const float* __restri
   }
 }
 
+
+// ---------------------------------------------------------------------------
+// The model's ends. Encoder: y[n][h] = sum_i x[n][i] w[h][i] + bias[h] over
+// NI <= 8 input features; bound by the write of y and, backward, by the read
+// of gy, which one pass turns into the gradients of w and bias. A thread keeps
+// four channels (their weights or sums in registers) and walks tokens.
+// ---------------------------------------------------------------------------
+constexpr int kEndThreads = 256;
+constexpr int kEncMaxIn = 8;
+constexpr int kHeadMaxOut = 4;
+
+template <int NI>
+__global__ __launch_bounds__(kEndThreads) void s4_encode_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ y, uint32_t ntok, int H) {
+  const int h4 = H / 4, c = threadIdx.x % h4, per = blockDim.x / h4;
+  float wr[4][NI];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) wr[r][i] = w[(4 * c + r) * NI + i];
+  const float4 b = reinterpret_cast<const float4*>(bias)[c];
+  const uint32_t step = gridDim.x * per;
+  for (uint32_t n = blockIdx.x * per + threadIdx.x / h4; n < ntok; n += step) {
+    float xi[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) xi[i] = x[(size_t)n * NI + i];
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int i = 0; i < NI; ++i) o[r] = fmaf(xi[i], wr[r][i], o[r]);
+    reinterpret_cast<float4*>(y)[(size_t)n * h4 + c] =
+        float4{o[0] + b.x, o[1] + b.y, o[2] + b.z, o[3] + b.w};
+  }
+}
+
+// Partials [block][H NI + H] for s4_dw_reduce_kernel.
+template <int NI>
+__global__ __launch_bounds__(kEndThreads) void s4_encode_grad_kernel(
+    const float* __restrict__ x, const float* __restrict__ gy, float* __restrict__ part,
+    uint32_t ntok, int H) {
+  __shared__ float red[kEndThreads][4 * (NI + 1) + 1];
+  const int h4 = H / 4, c = threadIdx.x % h4, row = threadIdx.x / h4, per = blockDim.x / h4;
+  float acc[4][NI + 1];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i <= NI; ++i) acc[r][i] = 0.0f;
+  const uint32_t step = gridDim.x * per;
+#pragma unroll 4
+  for (uint32_t n = blockIdx.x * per + row; n < ntok; n += step) {
+    const float4 g = reinterpret_cast<const float4*>(gy)[(size_t)n * h4 + c];
+    const float gv[4] = {g.x, g.y, g.z, g.w};
+    float xi[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) xi[i] = x[(size_t)n * NI + i];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i) acc[r][i] = fmaf(gv[r], xi[i], acc[r][i]);
+      acc[r][NI] += gv[r];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int i = 0; i <= NI; ++i) red[threadIdx.x][r * (NI + 1) + i] = acc[r][i];
+  __syncthreads();
+  float* const dst = part + (size_t)blockIdx.x * (H * NI + H);
+  for (int q = threadIdx.x; q < H * (NI + 1); q += blockDim.x) {
+    const int h = q / (NI + 1), i = q % (NI + 1);
+    float s = 0.0f;
+    for (int k = 0; k < per; ++k) s += red[k * h4 + h / 4][(h % 4) * (NI + 1) + i];
+    dst[i < NI ? h * NI + i : H * NI + h] = s;
+  }
+}
+
+// Head: out[b][o] = sum_h w[o][h] x[b][L-1][h] + bias[o], one wave per sample
+// (NO <= 4 outputs).
+__global__ __launch_bounds__(kEndThreads) void s4_head_kernel(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+    float* __restrict__ out, int B, int H, int L, int NO) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int b = blockIdx.x * (kEndThreads / kWave) + wave;
+  if (b >= B) return;
+  const float* row = x + ((size_t)b * L + L - 1) * H;
+  for (int o = 0; o < NO; ++o) {
+    float s = 0.0f;
+    for (int h = lane; h < H; h += kWave) s = fmaf(row[h], w[o * H + h], s);
+    s = wave_sum(s);
+    if (lane == 0) out[b * NO + o] = s + bias[o];
+  }
+}
+
+// Its gradients: gx is gy w in the last column and zero elsewhere (the write
+// of gx bounds it), with the partials [block][NO H + NO] of the weight and
+// bias gradients on the way.
+__global__ __launch_bounds__(kEndThreads) void s4_head_grad_kernel(
+    const float* __restrict__ x, const float* __restrict__ gy, const float* __restrict__ w,
+    float* __restrict__ gx, float* __restrict__ part, int B, int H, int L, int NO, int per) {
+  const int h4 = H / 4, n4 = L * h4;
+  const int b0 = blockIdx.x * per, b1 = b0 + per < B ? b0 + per : B;
+  const int c = threadIdx.x;  // channels 4 c .. of the weight gradient
+  float acc[kHeadMaxOut][4], accb[kHeadMaxOut];
+#pragma unroll
+  for (int o = 0; o < kHeadMaxOut; ++o) {
+    accb[o] = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[o][r] = 0.0f;
+  }
+  for (int b = b0; b < b1; ++b) {
+    float g[kHeadMaxOut];
+#pragma unroll
+    for (int o = 0; o < kHeadMaxOut; ++o) g[o] = o < NO ? gy[b * NO + o] : 0.0f;
+    if (gx) {
+      float4* dst = reinterpret_cast<float4*>(gx) + (size_t)b * n4;
+      for (int i = threadIdx.x; i < n4 - h4; i += kEndThreads) dst[i] = float4{0.f, 0.f, 0.f, 0.f};
+      if (c < h4) {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int o = 0; o < kHeadMaxOut; ++o)
+          if (o < NO)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = fmaf(g[o], w[o * H + 4 * c + r], v[r]);
+        dst[n4 - h4 + c] = float4{v[0], v[1], v[2], v[3]};
+      }
+    }
+    if (c < h4) {
+      const float4 xv = reinterpret_cast<const float4*>(x)[(size_t)b * n4 + n4 - h4 + c];
+#pragma unroll
+      for (int o = 0; o < kHeadMaxOut; ++o) {
+        acc[o][0] = fmaf(g[o], xv.x, acc[o][0]);
+        acc[o][1] = fmaf(g[o], xv.y, acc[o][1]);
+        acc[o][2] = fmaf(g[o], xv.z, acc[o][2]);
+        acc[o][3] = fmaf(g[o], xv.w, acc[o][3]);
+        accb[o] += g[o];
+      }
+    }
+  }
+  float* const dst = part + (size_t)blockIdx.x * (NO * H + NO);
+#pragma unroll
+  for (int o = 0; o < kHeadMaxOut; ++o)
+    if (o < NO) {
+      if (c < h4)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dst[o * H + 4 * c + r] = acc[o][r];
+      if (c == 0) dst[NO * H + o] = accb[o];
+    }
+}
+
 }  // namespace pt

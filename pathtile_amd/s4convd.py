@@ -154,6 +154,8 @@ class S4ConvKernel(nn.Module):
 # The whole block in fused HIP passes (pt_s4_block_*)
 # ---------------------------------------------------------------------------
 FUSED_MAX_H = 256  # H a multiple of 32 up to here
+# The model's ends: channels (a multiple of 4), input features, outputs
+ENDS_MAX_H, ENCODER_MAX_IN, HEAD_MAX_OUT = 1024, 8, 4
 
 
 def _size_query(fn: str, *args: int) -> int:
@@ -215,9 +217,7 @@ class S4BlockFused(torch.autograd.Function):
         runtime = get_runtime()
         runtime._check_open()
         B, L, H = x.shape
-        gy = gy.contiguous()
-        if gy.data_ptr() % 16:
-            gy = gy.clone()
+        gy = _aligned(gy.contiguous())
         gx = torch.empty_like(x) if need[0] else None
         taps = any(need[1:7])
         gp = [torch.empty_like(t) for t in (log_dt, c_re, c_im, log_a_re, a_im, skip)] \
@@ -279,6 +279,93 @@ def _tracing() -> bool:
                 or torch.is_autocast_enabled("cuda")
                 or torch.compiler.is_compiling() or torch.jit.is_tracing()
                 or nn.modules.module._has_any_global_hook())
+
+
+class EncoderFused(torch.autograd.Function):
+    """``nn.Linear`` over up to 8 input features: one pass over the output, and
+    one over its gradient for the weight and bias gradients."""
+
+    @staticmethod
+    def forward(ctx: Any, x, weight, bias):
+        B, L, n = x.shape
+        H = weight.shape[0]
+        y = torch.empty((B, L, H), device=x.device)
+        _call(_lib.load().pt_s4_encode_f32, x.device,
+              _ptr(x), _ptr(weight), _ptr(bias), _ptr(y), B, L, n, H)
+        ctx.save_for_backward(x, weight)
+        return y
+
+    @staticmethod
+    def backward(ctx: Any, gy: torch.Tensor):
+        x, weight = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if torch.is_grad_enabled():  # create_graph: differentiable operations
+            return (gy @ weight if need[0] else None,
+                    (gy.unsqueeze(-1) * x.unsqueeze(-2)).sum((0, 1)) if need[1] else None,
+                    gy.sum((0, 1)) if need[2] else None)
+        gx = gy @ weight if need[0] else None
+        gw = gb = None
+        if need[1] or need[2]:
+            B, L, n = x.shape
+            H = weight.shape[0]
+            gy = _aligned(gy.contiguous())
+            gw, gb = torch.empty_like(weight), torch.empty(H, device=x.device)
+            nbytes = _size_query("pt_s4_encode_grad_workspace_bytes", B, L, n, H)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            _call(_lib.load().pt_s4_encode_grad_f32, x.device,
+                  _ptr(x), _ptr(gy), _ptr(gw), _ptr(gb), _ptr(ws), nbytes, B, L, n, H)
+        return gx, gw if need[1] else None, gb if need[2] else None
+
+
+class HeadFused(torch.autograd.Function):
+    """The decoder at the last column, ``decoder(x)[:, -1, :]``: the columns
+    before it reach neither the output nor a gradient."""
+
+    @staticmethod
+    def forward(ctx: Any, x, weight, bias):
+        B, L, H = x.shape
+        n = weight.shape[0]
+        out = torch.empty((B, n), device=x.device)
+        _call(_lib.load().pt_s4_head_f32, x.device,
+              _ptr(x), _ptr(weight), _ptr(bias), _ptr(out), B, H, L, n)
+        ctx.save_for_backward(x, weight)
+        return out
+
+    @staticmethod
+    def backward(ctx: Any, gy: torch.Tensor):
+        x, weight = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        B, L, H = x.shape
+        if torch.is_grad_enabled():  # create_graph: differentiable operations
+            gx = nn.functional.pad((gy @ weight)[:, None, :], (0, 0, L - 1, 0)) if need[0] else None
+            return (gx, gy.t() @ x[:, -1, :] if need[1] else None,
+                    gy.sum(0) if need[2] else None)
+        n = weight.shape[0]
+        gy = gy.contiguous()
+        gx = torch.empty_like(x) if need[0] else None
+        gw, gb = torch.empty_like(weight), torch.empty(n, device=x.device)
+        nbytes = _size_query("pt_s4_head_grad_workspace_bytes", B, H, L, n)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        _call(_lib.load().pt_s4_head_grad_f32, x.device,
+              _ptr(x), _ptr(gy), _ptr(weight), None if gx is None else _ptr(gx), _ptr(gw),
+              _ptr(gb), _ptr(ws), nbytes, B, H, L, n)
+        return gx, gw if need[1] else None, gb if need[2] else None
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _plain_linear(m: nn.Module, x: torch.Tensor, width: int) -> bool:
+    """`m` is an ordinary FP32 ``nn.Linear`` with a bias for the contiguous
+    GPU tensor `x` [B, L, width], and nothing watches its call."""
+    return (type(m) is nn.Linear and type(x) is torch.Tensor and x.is_cuda and x.dim() == 3
+            and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and 0 < x.numel() < 2**31 and x.shape[2] == width == m.weight.shape[1]
+            and m.bias is not None and _no_hooks(m) and _backend() == "warp"
+            and all(type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32
+                    and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in (m.weight, m.bias)))
 
 
 class S4ConvBlock(nn.Module):
@@ -373,10 +460,21 @@ class Model(nn.Module):
         self.decoder = nn.Linear(hidden_dim, output_dim)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        x = self.encoder(x)
+        plain = not _tracing()
+        enc, dec = self.encoder, self.decoder
+        H = enc.out_features if type(enc) is nn.Linear else 0
+        if (plain and 4 <= H <= ENDS_MAX_H and H % 4 == 0 and x.dim() == 3
+                and 1 <= x.shape[2] <= ENCODER_MAX_IN and x.shape[0] * x.shape[1] * H < 2**31
+                and _plain_linear(enc, x, x.shape[2])):
+            x = EncoderFused.apply(x, enc.weight, enc.bias)
+        else:
+            x = enc(x)
         for block in self.blocks:
             x = block(x)
-        return self.decoder(x)[:, -1, :]
+        if (plain and x.dim() == 3 and 4 <= x.shape[2] <= ENDS_MAX_H and x.shape[2] % 4 == 0
+                and _plain_linear(dec, x, x.shape[2]) and dec.out_features <= HEAD_MAX_OUT):
+            return HeadFused.apply(x, dec.weight, dec.bias)
+        return dec(x)[:, -1, :]
 
 
 def rmsle(prediction: torch.Tensor, target: torch.Tensor) -> torch.Tensor:

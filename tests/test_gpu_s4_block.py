@@ -228,3 +228,48 @@ def test_fused_block_on_a_side_stream_under_graph_capture():
         torch.cuda.synchronize()
         ref = _grads(block, xs, gys)
         assert all(torch.equal(a, b) for a, b in zip(out, ref)), k
+
+
+@pytest.mark.parametrize("B,L,H,n_in,n_out", [(1, 1, 4, 1, 1), (3, 48, 128, 4, 1), (700, 5, 36, 8, 4),
+                                              (1500, 12, 1024, 3, 2), (33, 30, 260, 7, 3)])
+def test_model_ends_against_fp64(B, L, H, n_in, n_out):
+    """Encoder and last-column decoder, output and gradients, against FP64;
+    sums of up to B L products in FP32."""
+    from pathtile_amd import s4convd
+
+    print(f"[case] ends B={B} L={L} H={H} in={n_in} out={n_out}", flush=True)
+    torch.manual_seed(B + H)
+    enc, dec = torch.nn.Linear(n_in, H), torch.nn.Linear(H, n_out)
+    x, gy = torch.randn(B, L, n_in), torch.randn(B, n_out)
+    h, gh = torch.randn(B, L, H), torch.randn(B, L, H)
+
+    def grads(dev, dtype, encode, head):
+        e, d = copy.deepcopy(enc).to(dev, dtype), copy.deepcopy(dec).to(dev, dtype)
+        xi, hi = (t.to(dev, dtype).requires_grad_(True) for t in (x, h))
+        y, o = encode(e, xi), head(d, hi)
+        return [y, o, *torch.autograd.grad(y, (xi, e.weight, e.bias), gh.to(dev, dtype)),
+                *torch.autograd.grad(o, (hi, d.weight, d.bias), gy.to(dev, dtype))]
+
+    ref = grads("cpu", torch.float64, lambda m, t: m(t), lambda m, t: m(t)[:, -1, :])
+    got = grads("cuda", torch.float32,
+                lambda m, t: s4convd.EncoderFused.apply(t, m.weight, m.bias),
+                lambda m, t: s4convd.HeadFused.apply(t, m.weight, m.bias))
+    for a, b in zip(got, ref):
+        assert a.shape == b.shape and _rel(a, b) < 2e-6
+
+
+def test_model_ends_follow_hooks_and_devices():
+    """A hook on an end runs the module itself, with the same output."""
+    from pathtile_amd import s4convd
+
+    torch.manual_seed(3)
+    m = s4convd.Model(state_dim=8, hidden_dim=32, input_dim=4, output_dim=2, num_blocks=1,
+                      dropout=0.0).cuda()
+    x = torch.randn(5, 12, 4, device="cuda")
+    out, shapes = m(x), []
+    for end in (m.encoder, m.decoder):
+        end.register_forward_hook(lambda mod, i, o: shapes.append(tuple(o.shape)))
+    with torch.backends.cudnn.flags(enabled=False):
+        again = m(x)
+    assert shapes == [(5, 12, 32), (5, 12, 2)]
+    assert _rel(again, out) < 1e-6
