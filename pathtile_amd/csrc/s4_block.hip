@@ -13,13 +13,14 @@
 namespace pt {
 
 struct TailGeometry {
-  int nw, tok, dw_nw, dw_split;
-  size_t dw_lds;
+  int nw, tok, btok, dw_nw, dw_split;
+  size_t bwd_lds, dw_lds;
 };
 
 template <int CT>
 constexpr TailGeometry tail_geometry() {
-  return {TailGeo<CT>::NW, TailGeo<CT>::TOK, DwGeo<CT>::NW, DwGeo<CT>::SPLIT, DwGeo<CT>::lds};
+  return {TailGeo<CT>::NW,  TailGeo<CT>::TOK,   TailGeo<CT>::BTOK, DwGeo<CT>::NW,
+          DwGeo<CT>::SPLIT, tail_bwd_lds<CT>(), DwGeo<CT>::lds};
 }
 
 static constexpr TailGeometry kTail[kNumS4H] = {
@@ -50,22 +51,21 @@ static uint32_t dw_steps_per_range(uint32_t nsteps, int split) {
   return per < 4 ? 4 : per;
 }
 
-// Workspace of the backward, in floats: dP [2H][np] (later dX before its
-// transpose), du [B,H,L], the weight gradient's partials, dk [H][L], and the
+// Workspace of the backward, in floats: dP (blocks of 32 tokens; later dX
+// before its transpose), du [B,H,L], the weight gradient's partials, dk [H][L], and the
 // convolution's own partials.
 struct BwdLayout {
-  size_t np, du, part, dk, conv, conv_bytes, total;
+  size_t du, part, dk, conv, conv_bytes, total;
   uint32_t nsteps, per, ranges;
 };
 
 static int bwd_layout(int B, int H, int L, int threads, BwdLayout* o) {
   const TailGeometry& k = kTail[H / 32 - 1];
   const size_t ntok = (size_t)B * L;
-  o->np = round_up(ntok, 64);
   o->nsteps = (uint32_t)((ntok + kDwTok - 1) / kDwTok);
   o->per = dw_steps_per_range(o->nsteps, k.dw_split);
   o->ranges = (o->nsteps + o->per - 1) / o->per;
-  o->du = (size_t)2 * H * o->np;
+  o->du = (size_t)2 * H * round_up(ntok, 64);
   o->part = o->du + ntok * H;
   o->dk = o->part + round_up((size_t)o->ranges * (2 * H * H + 2 * H), 64);
   o->conv = o->dk + round_up((size_t)H * L, 64);
@@ -170,12 +170,13 @@ int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, 
 }
 
 int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
-                         const float* bias, float* y, int B, int H, int L, void* stream) {
+                         const float* bias, float* y, float* q, int B, int H, int L,
+                         void* stream) {
   const int st = pt::check_block(B, H, L, 1);
   if (st != PT_OK) return st;
   if (!v || !x || !prep || !w || !bias || !y) return PT_ERR_NULL;
   if (!pt::aligned16(v) || !pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(bias) ||
-      !pt::aligned16(y))
+      !pt::aligned16(y) || !pt::aligned16(q))
     return PT_ERR_ALIGN;
   const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
@@ -183,7 +184,7 @@ int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, cons
   uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
   const size_t lds = pt::tail_fwd_lds(H);
   const int block = k.nw * pt::kWave;
-  void* args[] = {&v, &x, &wf, &w, &bias, &y, &ntok, &uL, &magic, &ntiles};
+  void* args[] = {&v, &x, &wf, &w, &bias, &y, &q, &ntok, &uL, &magic, &ntiles};
   const void* fn = (const void*)pt::kTailFwd[H / 32 - 1];
   return pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
                     args);
@@ -199,8 +200,8 @@ int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block, 
   return st;
 }
 
-int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const unsigned char* mask,
-                        float scale, const float* prep, const float* w, const float* bias,
+int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const float* q,
+                        const unsigned char* mask, float scale, const float* prep, const float* w,
                         const float* log_dt, const float* c_re, const float* c_im,
                         const float* log_a_re, const float* a_im, float* gx, float* d_log_dt,
                         float* d_c_re, float* d_c_im, float* d_log_a_re, float* d_a_im,
@@ -209,14 +210,14 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
                         int dx_waves_per_block, int algo, int threads_per_block, void* stream) {
   int st = pt::check_block(B, H, L, states);
   if (st != PT_OK) return st;
-  if (!gy || !xt || !v || !prep || !w || !bias) return PT_ERR_NULL;
+  if (!gy || !xt || !v || !q || !prep || !w) return PT_ERR_NULL;
   const bool taps_grad = d_skip != nullptr;
   if (taps_grad && (!log_dt || !c_re || !c_im || !log_a_re || !a_im || !d_log_dt || !d_c_re ||
                     !d_c_im || !d_log_a_re || !d_a_im))
     return PT_ERR_NULL;
   if ((dw == nullptr) != (dbias == nullptr)) return PT_ERR_NULL;
   if (!pt::aligned16(gy) || !pt::aligned16(xt) || !pt::aligned16(v) || !pt::aligned16(prep) ||
-      !pt::aligned16(bias) || !pt::aligned16(workspace) || (gx && !pt::aligned16(gx)))
+      !pt::aligned16(q) || !pt::aligned16(workspace) || (gx && !pt::aligned16(gx)))
     return PT_ERR_ALIGN;
   pt::BwdLayout o;
   st = pt::bwd_layout(B, H, L, threads_per_block, &o);
@@ -227,13 +228,13 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
   float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk, *dxt = ws;
   const float* taps = prep;
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
-  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, np = (uint32_t)o.np;
+  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L;
   uint32_t magic = pt::token_magic(L);
   {
-    uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
-    const size_t lds = pt::tail_bwd_lds(H);
+    uint32_t ntiles = (ntok + k.btok - 1) / k.btok;
+    const size_t lds = k.bwd_lds;
     const int block = k.nw * pt::kWave;
-    void* args[] = {&gy, &v, &mask, &scale, &wf, &w, &bias, &du, &dp, &ntok, &uL, &magic, &ntiles, &np};
+    void* args[] = {&gy, &q, &v, &mask, &scale, &wf, &w, &du, &dp, &ntok, &uL, &magic, &ntiles};
     const void* fn = (const void*)pt::kTailBwd[H / 32 - 1];
     st = pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
                     args);
@@ -242,7 +243,7 @@ int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const 
   if (dw) {
     const void* fn = (const void*)pt::kDw[H / 32 - 1][L % 4 == 0];
     const float* cdp = dp;
-    void* args[] = {&cdp, &v, &part, &ntok, &uL, &magic, &o.nsteps, &o.per, &np};
+    void* args[] = {&cdp, &v, &part, &ntok, &uL, &magic, &o.nsteps, &o.per};
     st = pt::launch(fn, o.ranges * (uint32_t)k.dw_split, (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds,
                     stream, args);
     if (st != PT_OK) return st;

@@ -25,7 +25,7 @@
 namespace pt {
 
 constexpr int kS4MaxH = 256;     // largest H of the fused block (H % 32 == 0)
-constexpr int kDwTok = 32;       // tokens per step of the weight gradient
+constexpr int kDwTok = 32;       // tokens per step of the weight gradient, one block of dP
 
 // Waves of a tail workgroup for CT = H / 16 channel tiles: WPC waves side by
 // side on channels (MT tiles each, every tile with its gate tile H channels
@@ -43,16 +43,27 @@ struct TailGeo {
   static constexpr int GS = H + 8;       // BF16 values per token row of a g part
   static constexpr int PS = 2 * H + 8;   // the same for a dP part
   static constexpr int OS = H + 4;       // floats per token row of the output stage
-  // tokens per tile: the LDS holds the stages of 64 tokens up to H = 128
+  // tokens per forward tile: the LDS holds the stages of 64 tokens up to H = 128
   static constexpr int TOK = CT <= 8 ? 64 : 32;
+  // tokens per backward tile, and whether the LDS holds two dP stages of them
+  static constexpr int BTOK = 16 * WPT > 32 ? 16 * WPT : 32;
+  static constexpr bool TWO = CT <= 8;
 };
 
 __host__ __device__ constexpr int tail_tok(int H) { return H <= 128 ? 64 : 32; }
 __host__ __device__ constexpr size_t tail_fwd_lds(int H) {  // two g stages, the output stage
   return (size_t)tail_tok(H) * (2 * 3 * (H + 8) * 2 + (H + 4) * 4);
 }
-__host__ __device__ constexpr size_t tail_bwd_lds(int H) {  // g parts, dP parts
-  return (size_t)tail_tok(H) * 3 * ((H + 8) + (2 * H + 8)) * 2;
+// Byte offset of dP's (token, row) from the tile's first block of 32 tokens.
+constexpr int kDpTok = 32;
+template <int H>
+__device__ __forceinline__ uint32_t dp_offset(uint32_t tk, uint32_t row) {
+  return 4 * ((tk / kDpTok) * (2 * H * kDpTok) + row * kDpTok + tk % kDpTok);
+}
+
+template <int CT>
+constexpr size_t tail_bwd_lds() {  // dP parts
+  return (size_t)(TailGeo<CT>::TWO ? 2 : 1) * 3 * TailGeo<CT>::BTOK * TailGeo<CT>::PS * 2;
 }
 
 // Values of the split weights in the workspace: W as A operands of the
@@ -336,14 +347,15 @@ __device__ __forceinline__ void project_fix(f32x4& a, f32x4& b, const float* __r
 // here, 3.1 TB/s with the matrix cores 42% busy), so tile t + 1's gelu and split
 // run in the shadow of tile t's products, into the other of two stages. The
 // weight fragments stay in registers up to H = 128 (streamed from the L2 they
-// cost 511 us) and stream above. GLU results pass through an FP32 stage
+// cost 511 us) and stream above. For a later backward, q [2][tokens][H] gets
+// the values P[c] + bias and the gates' sigmoids. GLU results pass through an FP32 stage
 // to flat 16-byte rows with the residual.
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
     const float* __restrict__ v, const float* __restrict__ x, const __bf16* __restrict__ wf,
     const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y,
-    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t ntiles) {
+    float* __restrict__ q, uint32_t ntok, uint32_t L, uint32_t magic, uint32_t ntiles) {
   using G = TailGeo<CT>;
   constexpr int TOK = G::TOK, NT = TOK / 16 / G::WPT, SZ = 3 * TOK * G::GS, TH = G::NW * kWave;
   constexpr int R4 = TOK * G::H / 4 / TH;  // 16-byte pieces of a tile's rows per thread
@@ -389,12 +401,16 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
         if (__builtin_expect(!(finite4(a[0], a[1], a[2], a[3]) && finite4(b[0], b[1], b[2], b[3])), 0)) {
           if (n0 + tk < ntok) project_fix(a, b, v, w, token_base(n0 + tk, G::H, L, magic), c, G::H, L);
         }
-        float4 o;
-        o.x = (a[0] + ba.x) * sigmoid_f(b[0] + bb.x);
-        o.y = (a[1] + ba.y) * sigmoid_f(b[1] + bb.y);
-        o.z = (a[2] + ba.z) * sigmoid_f(b[2] + bb.z);
-        o.w = (a[3] + ba.w) * sigmoid_f(b[3] + bb.w);
-        *reinterpret_cast<float4*>(so + tk * G::OS + c) = o;
+        const float4 pa = {a[0] + ba.x, a[1] + ba.y, a[2] + ba.z, a[3] + ba.w};
+        const float4 ps = {sigmoid_f(b[0] + bb.x), sigmoid_f(b[1] + bb.y), sigmoid_f(b[2] + bb.z),
+                           sigmoid_f(b[3] + bb.w)};
+        *reinterpret_cast<float4*>(so + tk * G::OS + c) =
+            float4{pa.x * ps.x, pa.y * ps.y, pa.z * ps.z, pa.w * ps.w};
+        if (q) {
+          const uint32_t o = 4 * (tk * G::H + c);
+          buf_store4(pa, make_token_rows(q, n0, ntok, G::H), o);
+          buf_store4(ps, make_token_rows(q + (size_t)ntok * G::H, n0, ntok, G::H), o);
+        }
       }
     }
     __syncthreads();
@@ -409,54 +425,91 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Tail backward with respect to its input: from gy [B,L,H], du = dL/du
-// [B,H,L] (through GLU, projection, gelu and the dropout mask) and
-// dP [2 H][np] (token-contiguous rows, zero past the last token) for the
-// weight gradient. The pre-activations are recomputed. Per tile t: the
-// projection with tile t - 1's gelu gradient in its shadow, the GLU gradient
-// into the dP parts [part][token][PS], then W^T dP with tile t + 1's gelu in
-// its shadow; two barriers. B16384 L48 H128: 1421 us with the vector work in
-// phases of its own and erff, 1008 us now; what bounds it is the sum of matrix
-// (13 k cycles a tile) and vector work (16 k), which overlap in part.
+// Tail backward with respect to its input: from gy [B,L,H] and the forward's
+// q, du = dL/du [B,H,L] (through GLU, projection, gelu and the dropout mask)
+// and dP [blocks of 32 tokens][2 H][32] (zero past the last token) for the
+// weight gradient, whose loads it makes whole lines. A persistent workgroup walks tiles of 32 tokens (64 at
+// H = 32): tile t's product W^T dP from LDS, the weight fragments resident up
+// to H = 128, and in its shadow tile t + 1's GLU gradient into the other of
+// two dP stages and tile t - 1's gelu gradient; one barrier per tile. Above
+// H = 128 the LDS holds one stage, the GLU gradient comes before the product
+// and the fragments stream. Seven tensor passes of HBM bound it; recomputing
+// the pre-activations instead of reading q took 5 passes but 975 us at B16384
+// L48 H128 on the sum of its matrix and vector work, 698 us now (the forward,
+// which writes q, 388 -> 483).
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
-    const float* __restrict__ gy, const float* __restrict__ v, const uint8_t* __restrict__ mask,
-    float scale, const __bf16* __restrict__ wf, const float* __restrict__ w,
-    const float* __restrict__ bias, float* __restrict__ du, float* __restrict__ dp, uint32_t ntok,
-    uint32_t L, uint32_t magic, uint32_t ntiles, uint32_t np) {
+    const float* __restrict__ gy, const float* __restrict__ q, const float* __restrict__ v,
+    const uint8_t* __restrict__ mask, float scale, const __bf16* __restrict__ wf,
+    const float* __restrict__ w, float* __restrict__ du, float* __restrict__ dp, uint32_t ntok,
+    uint32_t L, uint32_t magic, uint32_t ntiles) {
   using G = TailGeo<CT>;
-  constexpr int TOK = G::TOK, NT = TOK / 16 / G::WPT;
+  constexpr int TOK = G::BTOK, NT = TOK / 16 / G::WPT, SZ = 3 * TOK * G::PS, KS = 2 * G::KS;
+  static_assert(NT >= 1, "every wave has tokens");
   typedef __bf16 bf16x4v __attribute__((ext_vector_type(4)));
   extern __shared__ __align__(16) char smem[];
-  __bf16* const sg = reinterpret_cast<__bf16*>(smem);
-  __bf16* const sp = sg + 3 * TOK * G::GS;
+  __bf16* const sp = reinterpret_cast<__bf16*>(smem);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ct0 = (wave % G::WPC) * G::MT, nt0 = (wave / G::WPC) * NT;
   const int tk0 = 16 * nt0 + (lane & 15);
   const int c0 = 16 * ct0 + 4 * (lane >> 4);
-  const __bf16* const w0 = wf + (size_t)ct0 * 2 * G::KS * 3 * 512 + lane * 8;
-  const __bf16* const wt0 = w0 + wfrag_values(G::H);
-  StreamedFrags<2 * G::MT, G::KS> frags(w0);
-  StreamedFrags<G::MT, 2 * G::KS> tfrags(wt0);
   const bool masked = mask != nullptr;
   const float keep = masked ? scale : 1.0f;
-  GeluStage<CT, TOK> stage;
-  stage.load(v, blockIdx.x * TOK, ntok, L, magic);
-  stage.template store<0, 1>(sg);
-  float4 g4[G::MT][NT];
-  auto load_gy = [&](uint32_t n0) {
-    const __amdgpu_buffer_rsrc_t gr = make_token_rows(gy, n0, ntok, G::H);
+  std::conditional_t<G::TWO, ResidentFrags<G::MT, KS>, StreamedFrags<G::MT, KS>> frags(
+      wf + wfrag_values(G::H) + (size_t)ct0 * KS * 3 * 512 + lane * 8);
+  constexpr int E = G::MT * NT * 4;  // du values per lane and tile: (m, nt, r)
+
+  // GLU gradient of the tile whose q and gy are loaded
+  float4 q1[G::MT][NT], q2[G::MT][NT], g4[G::MT][NT];
+  auto load_glu = [&](uint32_t n0) {
+    const __amdgpu_buffer_rsrc_t r1 = make_token_rows(q, n0, ntok, G::H);
+    const __amdgpu_buffer_rsrc_t r2 = make_token_rows(q + (size_t)ntok * G::H, n0, ntok, G::H);
+    const __amdgpu_buffer_rsrc_t rg = make_token_rows(gy, n0, ntok, G::H);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int m = 0; m < G::MT; ++m)
-        g4[m][nt] = buf_load4(gr, 4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m), 0);
+      for (int m = 0; m < G::MT; ++m) {
+        const uint32_t o = 4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m);
+        q1[m][nt] = buf_load4(r1, o, 0);
+        q2[m][nt] = buf_load4(r2, o, 0);
+        g4[m][nt] = buf_load4(rg, o, 0);
+      }
   };
-  load_gy(blockIdx.x * TOK);
-  frags.begin();
-  // the tile before: its W^T dP, inputs and mask, and where du goes (nowhere yet)
-  f32x4 dg[G::MT][NT];
+  float pa[8];  // four value and four gate gradients
+  auto glu = [&](auto slice, auto slices, uint32_t n0, __bf16* st) {
+    constexpr int I = decltype(slice)::value, N = decltype(slices)::value;
+    // past the last tile the stores are dropped
+    const __amdgpu_buffer_rsrc_t dr =
+        make_rsrc_n(dp + (size_t)n0 * (2 * G::H), n0 < ntok ? 2 * G::H * TOK * 4 : 0);
+#pragma unroll
+    for (int e = E * I / N; e < E * (I + 1) / N; ++e) {
+      const int r = e % 4, m = e / 4 % G::MT, nt = e / 4 / G::MT;
+      const int tk = tk0 + 16 * nt, c = c0 + 16 * m;
+      const bool in = n0 + tk < ntok;
+      const float a = (&q1[m][nt].x)[r], s = (&q2[m][nt].x)[r], g = (&g4[m][nt].x)[r];
+      pa[r] = in ? s * g : 0.0f;
+      pa[4 + r] = in ? (1.0f - s) * s * g * a : 0.0f;
+      buf_store1(pa[r], dr, dp_offset<G::H>(tk, c + r));
+      buf_store1(pa[4 + r], dr, dp_offset<G::H>(tk, G::H + c + r));
+      if (r == 3) {
+        bf16x8 parts[3];
+        split3_bf16x8(pa, parts[0], parts[1], parts[2]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+          __bf16* d = st + (p * TOK + tk) * G::PS + c;
+          *reinterpret_cast<bf16x4v*>(d) =
+              bf16x4v{parts[p][0], parts[p][1], parts[p][2], parts[p][3]};
+          *reinterpret_cast<bf16x4v*>(d + G::H) =
+              bf16x4v{parts[p][4], parts[p][5], parts[p][6], parts[p][7]};
+        }
+      }
+    }
+  };
+
+  // gelu gradient of a finished product: its values, mask and where du goes
+  // (nowhere before the first tile)
+  f32x4 dg[G::MT][NT], dgn[G::MT][NT];
   float vv[G::MT][NT][4];
   uint32_t mk[G::MT][NT][4], at[NT];
   Slab out = make_slab(du, ntok, ntok, G::H, L, magic);
@@ -473,106 +526,59 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
       }
     }
   }
-  constexpr int E = G::MT * NT;  // groups of four du values per lane and tile
-  auto finish = [&](auto slice, auto slices) {  // du of the tile before
+  auto finish = [&](auto slice, auto slices) {
     constexpr int I = decltype(slice)::value, N = decltype(slices)::value;
 #pragma unroll
     for (int e = E * I / N; e < E * (I + 1) / N; ++e) {
-      const int m = e % G::MT, nt = e / G::MT;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float o = dg[m][nt][r] * gelu_grad_f(vv[m][nt][r]);
-        o = o * (masked ? (float)mk[m][nt][r] : 1.0f) * keep;
-        buf_store1(o, out.r, 4 * (at[nt] + (uint32_t)(16 * m + r) * L));
-      }
+      const int r = e % 4, m = e / 4 % G::MT, nt = e / 4 / G::MT;
+      float o = dg[m][nt][r] * gelu_grad_f(vv[m][nt][r]);
+      o = o * (masked ? (float)mk[m][nt][r] : 1.0f) * keep;
+      buf_store1(o, out.r, 4 * (at[nt] + (uint32_t)(16 * m + r) * L));
     }
   };
-  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const uint32_t n0 = tile * TOK;
-    __syncthreads();  // tile t's g parts are written, tile t - 1's dP parts read
-    f32x4 acc[2 * G::MT][NT];
-    multiply<2 * G::MT, NT, G::KS, G::GS, TOK>(
-        acc, frags, sg + tk0 * G::GS + 8 * (lane >> 4),
-        [&](auto ks) { finish(ks, std::integral_constant<int, G::KS>{}); });
-    // Loads return in order, so the ones from HBM are issued where the next
-    // wait for a weight fragment is far off: behind the projection, with the
-    // GLU gradient and the next product's first step in between.
-    tfrags.begin();
-    out = make_slab(du, n0, ntok, G::H, L, magic);
-    stage.load(v, (tile + gridDim.x) * TOK, ntok, L, magic);
-    {
-      const Slab in = make_slab(v, n0, ntok, G::H, L, magic);
-      const __amdgpu_buffer_rsrc_t mr =
-          make_slab<1>(mask, masked ? n0 : ntok, ntok, G::H, L, magic).r;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        at[nt] = token_base(n0 + tk0 + 16 * nt, G::H, L, magic) - in.first + (uint32_t)c0 * L;
-#pragma unroll
-        for (int m = 0; m < G::MT; ++m)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t o = at[nt] + (uint32_t)(16 * m + r) * L;
-            vv[m][nt][r] = buf_load1(in.r, 4 * o, 0);
-            mk[m][nt][r] = __builtin_amdgcn_raw_buffer_load_b8(mr, o, 0, 0);
-          }
-      }
-    }
-#pragma unroll
-    for (int m = 0; m < G::MT; ++m) {
-      const int c = c0 + 16 * m;
-      const float4 ba = *reinterpret_cast<const float4*>(bias + c);
-      const float4 bb = *reinterpret_cast<const float4*>(bias + G::H + c);
-      const float vba[4] = {ba.x, ba.y, ba.z, ba.w}, vbb[4] = {bb.x, bb.y, bb.z, bb.w};
-      float* const da_row = dp + (size_t)c * np + n0 + tk0;
-      float* const db_row = da_row + (size_t)G::H * np;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int tk = tk0 + 16 * nt;
-        const bool in = n0 + tk < ntok;
-        f32x4 a = acc[2 * m][nt], b = acc[2 * m + 1][nt];
-        if (__builtin_expect(!(finite4(a[0], a[1], a[2], a[3]) && finite4(b[0], b[1], b[2], b[3])), 0)) {
-          if (in) project_fix(a, b, v, w, token_base(n0 + tk, G::H, L, magic), c, G::H, L);
-        }
-        const float g[4] = {g4[m][nt].x, g4[m][nt].y, g4[m][nt].z, g4[m][nt].w};
-        float pa[8];  // four value and four gate gradients
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float s = sigmoid_f(b[r] + vbb[r]);
-          const float da = s * g[r];
-          const float db = (1.0f - s) * s * g[r] * (a[r] + vba[r]);
-          pa[r] = in ? da : 0.0f;
-          pa[4 + r] = in ? db : 0.0f;
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          da_row[(size_t)r * np + 16 * nt] = pa[r];
-          db_row[(size_t)r * np + 16 * nt] = pa[4 + r];
-        }
-        bf16x8 parts[3];
-        split3_bf16x8(pa, parts[0], parts[1], parts[2]);
-#pragma unroll
-        for (int p = 0; p < 3; ++p) {
-          __bf16* d = sp + (p * TOK + tk) * G::PS + c;
-          *reinterpret_cast<bf16x4v*>(d) =
-              bf16x4v{parts[p][0], parts[p][1], parts[p][2], parts[p][3]};
-          *reinterpret_cast<bf16x4v*>(d + G::H) =
-              bf16x4v{parts[p][4], parts[p][5], parts[p][6], parts[p][7]};
-        }
-      }
+  using All = std::integral_constant<int, 1>;
+  using Steps = std::integral_constant<int, KS>;
+  using Zero = std::integral_constant<int, 0>;
+
+  load_glu(blockIdx.x * TOK);
+  if constexpr (G::TWO) {
+    glu(Zero{}, All{}, blockIdx.x * TOK, sp);
+    load_glu((blockIdx.x + gridDim.x) * TOK);
+  }
+  uint32_t cur = 0;
+  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, cur ^= G::TWO) {
+    const uint32_t n0 = tile * TOK, next = (tile + gridDim.x) * TOK;
+    if constexpr (!G::TWO) {
+      __syncthreads();  // the stage is read
+      glu(Zero{}, All{}, n0, sp);
+      load_glu(next);
     }
     __threadfence_block();
-    __syncthreads();  // the dP parts are written, the g parts read
-    load_gy((tile + gridDim.x) * TOK);
-    multiply<G::MT, NT, 2 * G::KS, G::PS, TOK>(
-        dg, tfrags, sp + tk0 * G::PS + 8 * (lane >> 4),
-        [&](auto ks) { stage.template store<decltype(ks)::value, 2 * G::KS>(sg); });
+    __syncthreads();  // tile t's dP parts are written
     frags.begin();
+    multiply<G::MT, NT, KS, G::PS, TOK>(
+        dgn, frags, sp + cur * SZ + tk0 * G::PS + 8 * (lane >> 4), [&](auto ks) {
+          finish(ks, Steps{});
+          if constexpr (G::TWO) glu(ks, Steps{}, next, sp + (cur ^ 1) * SZ);
+        });
+    if constexpr (G::TWO) load_glu(next + gridDim.x * TOK);
+    out = make_slab(du, n0, ntok, G::H, L, magic);
+    const Slab in = make_slab(v, n0, ntok, G::H, L, magic);
+    const __amdgpu_buffer_rsrc_t mr =
+        make_slab<1>(mask, masked ? n0 : ntok, ntok, G::H, L, magic).r;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < NT; ++nt) {
+      const uint32_t n = n0 + tk0 + 16 * nt;
+      at[nt] = token_base(n, G::H, L, magic) - in.first + (uint32_t)c0 * L;
 #pragma unroll
       for (int m = 0; m < G::MT; ++m) {
-        const uint32_t n = n0 + tk0 + 16 * nt;
-        f32x4& d = dg[m][nt];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t o = at[nt] + (uint32_t)(16 * m + r) * L;
+          vv[m][nt][r] = buf_load1(in.r, 4 * o, 0);
+          mk[m][nt][r] = __builtin_amdgcn_raw_buffer_load_b8(mr, o, 0, 0);
+        }
+        f32x4 d = dgn[m][nt];
         if (__builtin_expect(!finite4(d[0], d[1], d[2], d[3]), 0)) {
           if (n < ntok) {
 #pragma unroll 1
@@ -581,22 +587,25 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
               float s = 0.0f;
 #pragma unroll 1
               for (int o = 0; o < 2 * G::H; ++o)
-                s = fmaf(w[(size_t)o * G::H + c], dp[(size_t)o * np + n], s);
+                s = fmaf(w[(size_t)o * G::H + c],
+                         dp[(size_t)n0 * (2 * G::H) + dp_offset<G::H>(n - n0, o) / 4], s);
               set_elem(d, r, s);
             }
           }
         }
+        dg[m][nt] = d;
       }
+    }
   }
-  finish(std::integral_constant<int, 0>{}, std::integral_constant<int, 1>{});
+  finish(Zero{}, All{});
 }
 
 // ---------------------------------------------------------------------------
 // Weight gradient of the projection: dW[c][h] = sum_tok dP[c][tok] g[h][tok]
 // and dbias[c] = sum_tok dP[c][tok], split over the tokens. A workgroup takes
 // a contiguous run of 32-token steps and NB channels (columns); its waves own
-// rows of dP, read straight from memory in the A layout (each row's 32 tokens
-// are one 128-byte line) and split in registers; g is computed, split and
+// rows of dP, read straight from memory in the A layout (a step's block is
+// contiguous) and split in registers; g is computed, split and
 // shared through LDS [part][channel][40]. Partials [range][2 H H + 2 H] go to
 // the workspace for a fixed-order reduction. Step s + 1's gelu and splits run
 // in the shadow of step s's products: 381 us at B16384 L48 H128, 430 with them
@@ -616,7 +625,7 @@ struct DwGeo {
 template <int CT, bool VEC>
 __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     const float* __restrict__ dp, const float* __restrict__ v, float* __restrict__ part,
-    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t nsteps, uint32_t steps_per, uint32_t np) {
+    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t nsteps, uint32_t steps_per) {
   using D = DwGeo<CT>;
   constexpr int H = 16 * CT, NC = 16 * D::NB, TH = D::NW * kWave;
   constexpr int kUnits = NC * (kDwTok / 8);  // (channel, eight tokens)
@@ -637,7 +646,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     for (int n = 0; n < D::NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const float* const a0 =
-      dp + (size_t)(16 * wave * D::MT + (lane & 15)) * np + 8 * (lane >> 4);
+      dp + (16 * wave * D::MT + (lane & 15)) * kDpTok + 8 * (lane >> 4);
   float vr[U][8];
   float ar[D::MT][8];
   auto load_v = [&](uint32_t s) {
@@ -668,7 +677,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
   auto load_a = [&](uint32_t s) {
 #pragma unroll
     for (int m = 0; m < D::MT; ++m) {
-      const float* p = a0 + (size_t)16 * m * np + (size_t)s * kDwTok;
+      const float* p = a0 + 16 * m * kDpTok + (size_t)s * (2 * H * kDpTok);
       const float4 f0 = *reinterpret_cast<const float4*>(p);
       const float4 f1 = *reinterpret_cast<const float4*>(p + 4);
       ar[m][0] = f0.x;
@@ -776,7 +785,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
           const uint32_t e1 = s1 * kDwTok < ntok ? s1 * kDwTok : ntok;
 #pragma unroll 1
           for (uint32_t k = s0 * kDwTok; k < e1; ++k)
-            s = fmaf(dp[(size_t)c * np + k], gelu_f(v[token_base(k, H, L, magic) + (uint32_t)h * L]), s);
+            s = fmaf(dp[(size_t)(k / kDpTok) * (2 * H * kDpTok) + c * kDpTok + k % kDpTok], gelu_f(v[token_base(k, H, L, magic) + (uint32_t)h * L]), s);
         }
         dst[(size_t)c * H + h] = s;
       }

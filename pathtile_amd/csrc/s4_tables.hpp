@@ -10,12 +10,12 @@ namespace pt {
 constexpr int kNumS4H = 8;  // H = 32, 64, ..., 256
 
 using TailFwdFn = void (*)(const float*, const float*, const __bf16*, const float*, const float*,
-                           float*, uint32_t, uint32_t, uint32_t, uint32_t);
-using TailBwdFn = void (*)(const float*, const float*, const uint8_t*, float, const __bf16*,
-                           const float*, const float*, float*, float*, uint32_t, uint32_t, uint32_t,
-                           uint32_t, uint32_t);
+                           float*, float*, uint32_t, uint32_t, uint32_t, uint32_t);
+using TailBwdFn = void (*)(const float*, const float*, const float*, const uint8_t*, float,
+                           const __bf16*, const float*, float*, float*, uint32_t, uint32_t, uint32_t,
+                           uint32_t);
 using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t, uint32_t,
-                      uint32_t, uint32_t);
+                      uint32_t);
 
 extern const TailFwdFn kTailFwd[kNumS4H];
 extern const TailBwdFn kTailBwd[kNumS4H];

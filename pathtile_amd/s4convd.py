@@ -180,12 +180,14 @@ def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight
     return prep, xt, u
 
 
-def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias) -> torch.Tensor:
+def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias,
+                q: torch.Tensor | None = None) -> torch.Tensor:
     runtime = get_runtime()
     B, L, H = x.shape
     y = torch.empty_like(x)
     _call(runtime._lib.pt_s4_block_tail_f32, x.device,
-          _ptr(v), _ptr(x), _ptr(prep), _ptr(weight), _ptr(bias), _ptr(y), B, H, L)
+          _ptr(v), _ptr(x), _ptr(prep), _ptr(weight), _ptr(bias), _ptr(y),
+          None if q is None else _ptr(q), B, H, L)
     return y
 
 
@@ -201,16 +203,17 @@ class S4BlockFused(torch.autograd.Function):
         mask = None
         if p > 0.0:
             v, mask = torch.native_dropout(v, p, True)
-        y = _fused_tail(v, x, prep, weight, bias)
+        q = torch.empty((2, *x.shape), device=x.device)
+        y = _fused_tail(v, x, prep, weight, bias, q)
         ctx.save_for_backward(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-                              prep, xt, v, mask)
+                              prep, xt, v, q, mask)
         ctx.scale = 1.0 / (1.0 - p)
         return y
 
     @staticmethod
     def backward(ctx: Any, gy: torch.Tensor):
         (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-         prep, xt, v, mask) = ctx.saved_tensors
+         prep, xt, v, q, mask) = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():  # create_graph: differentiate the composition
             return _composed_grads(ctx, gy, mask)
@@ -231,8 +234,8 @@ class S4BlockFused(torch.autograd.Function):
             return None if t is None else _ptr(t)
 
         _call(runtime._lib.pt_s4_block_bwd_f32, x.device,
-              _ptr(gy), _ptr(xt), _ptr(v), opt(mask), ctx.scale, _ptr(prep), _ptr(weight),
-              _ptr(bias), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
+              _ptr(gy), _ptr(xt), _ptr(v), _ptr(q), opt(mask), ctx.scale, _ptr(prep),
+              _ptr(weight), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
               opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
               c_re.shape[1], runtime.dx_waves_per_block, runtime._rows_algo_id,
               runtime.bwdk_block)
