@@ -281,47 +281,42 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
  * diagonal state-space parameters log_dt [H], c_re, c_im, log_a_re, a_im
  * [H, states], skip [H], the projection w [2H, H] and bias [2H]:
  *   taps[h][t] = 2 Re sum_n C_eff[h,n] exp(dt A t) (+ skip[h] at t = L / 2)
- *   u = conv(x transposed to [B, H, L], taps)              (_mix)
- *   y = GLU(w gelu(v) + bias) + x, v = dropout(u) or u     (_tail)
- * and the gradients of y for gy [B, L, H] (_bwd). Served: H a multiple of 32
- * up to 256, 1 <= L <= 48, B >= 1, B H L < 2^31 (PT_ERR_SHAPE otherwise);
- * x, xt, u, v, q, y, gy, gx, prep, bias and workspace 16-byte aligned
- * (PT_ERR_ALIGN). The projection runs on the BF16 matrix cores with both
- * operands split three ways (FP32 accuracy; a sum that is not finite is
+ *   v = conv(x, taps) along L, or dropout of it            (_mix)
+ *   y = GLU(w gelu(v) + bias) + x                          (_tail)
+ * and the gradients of y for gy [B, L, H] (_bwd). All activations are [B, L,
+ * H]. Served: H a multiple of 32 up to 256, 1 <= L <= 48, B >= 1, B H L <
+ * 2^31 (PT_ERR_SHAPE otherwise); x, v, q, y, gy, gx, prep, bias and
+ * workspace 16-byte aligned (PT_ERR_ALIGN). The convolution is the
+ * reference's fmaf chain. The projection runs on the BF16 matrix cores with
+ * both operands split three ways (FP32 accuracy; a sum that is not finite is
  * recomputed by the FP32 chain).
  *
  * prep holds the taps and the split projection between the calls of one
  * block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
- * also lays out what _bwd needs. q [2, B L, H], written by _tail where not
- * NULL, holds the projection's values and the gates' sigmoids for _bwd. xt and
- * u are [B, H, L]; _bwd takes xt, the tail's input v, q, and dropout's byte
- * mask and scale (mask NULL: none). Its
+ * also lays out what _bwd needs. mask is dropout's byte mask in [B, H, L]
+ * order, 4-byte aligned (NULL: none): v = conv * mask * scale. q [2, B L, H], written by _tail where not NULL, holds the projection's values and the
+ * gates' sigmoids for _bwd, which takes x, v, q and the mask again. Its
  * outputs gx, {dw, dbias} and the six parameter gradients (all or none, by
- * d_skip) are each skipped where NULL. waves_per_block, algo,
- * dx_waves_per_block and threads_per_block are the convolution's
- * (pt_dwconv1d_fwd_f32_algo, pt_dwconv1d_dk_det_f32).
+ * d_skip) are each skipped where NULL.
  */
 int pt_s4_block_prep_values(int H, int L, size_t* floats);
 int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re,
                         const float* c_im, const float* log_a_re, const float* a_im,
-                        const float* skip, const float* w, float* prep, float* xt,
-                        float* u, int B, int H, int L, int states, int backward,
-                        int waves_per_block, int algo, void* stream);
-int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep,
-                         const float* w, const float* bias, float* y, float* q, int B,
-                         int H, int L, void* stream);
-int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block,
-                                    size_t* bytes);
-int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const float* q,
+                        const float* skip, const float* w, const unsigned char* mask,
+                        float scale, float* prep, float* v, int B, int H, int L, int states,
+                        int backward, void* stream);
+int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
+                         const float* bias, float* y, float* q, int B, int H, int L,
+                         void* stream);
+int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, size_t* bytes);
+int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const float* q,
                         const unsigned char* mask, float scale, const float* prep,
-                        const float* w, const float* log_dt,
-                        const float* c_re, const float* c_im, const float* log_a_re,
-                        const float* a_im, float* gx, float* d_log_dt, float* d_c_re,
-                        float* d_c_im, float* d_log_a_re, float* d_a_im,
-                        float* d_skip, float* dw, float* dbias, void* workspace,
-                        size_t workspace_bytes, int B, int H, int L, int states,
-                        int dx_waves_per_block, int algo, int threads_per_block,
-                        void* stream);
+                        const float* w, const float* log_dt, const float* c_re,
+                        const float* c_im, const float* log_a_re, const float* a_im,
+                        float* gx, float* d_log_dt, float* d_c_re, float* d_c_im,
+                        float* d_log_a_re, float* d_a_im, float* d_skip, float* dw,
+                        float* dbias, void* workspace, size_t workspace_bytes, int B,
+                        int H, int L, int states, void* stream);
 
 /*
  * The ends of the S4ConvD model (kernels/warp_tiled_ampere.py:1193-1215 in

@@ -42,6 +42,7 @@ SOURCES = [
     "inst_long_s3.hip",
     "inst_long_s3_vec.hip",
     "s4_block.hip",
+    "inst_s4_conv.hip",
     "inst_s4_tail_fwd.hip",
     "inst_s4_tail_bwd.hip",
     "inst_s4_dw.hip",

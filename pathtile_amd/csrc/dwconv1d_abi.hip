@@ -972,25 +972,43 @@ static int bf16_dk_launch(bool det, const void* gy, const void* x, float* dst,
 // of four at 48 columns), one resident pass of them over the GPU (the sample ranges are the resident workgroups per
 // channel group, rounded down so no workgroup waits for a second round),
 // at most one range per 4-sample step.
-static int dk_cl_launch(const float* x, const float* dy, float* dw, int B,
-                        int H, int L, int K, void* stream) {
+// Sample ranges of a channels-last DK call: one resident pass. Workgroups
+// that do not fit (LDS) give 0.
+int dk_cl_ranges(int B, int H, int L) {
   const DkClFn fn = kDkClTable[mfma_index(L)];
   const int nw = dk_cl_waves(16 * (mfma_index(L) + 1));
   const size_t lds = dk_cl_lds_bytes(16 * (mfma_index(L) + 1), L, nw);
-  if (lds > (size_t)max_lds_per_block()) return PT_ERR_CONFIG;
-  const int threads = nw * kWave;
+  if (lds > (size_t)max_lds_per_block()) return 0;
   const long long ngroups = (long long)H / kClChannels;
   const long long tsteps = ((long long)B + kCgStep - 1) / kCgStep;
-  const long long slots = (long long)num_cus() * blocks_per_cu((const void*)fn, threads, lds);
+  const long long slots =
+      (long long)num_cus() * blocks_per_cu((const void*)fn, nw * kWave, lds);
   long long nr = slots / ngroups;
   if (nr > tsteps) nr = tsteps;
-  if (nr < 1) nr = 1;
-  const long long nb = ngroups * nr;
+  return nr < 1 ? 1 : (int)nr;
+}
+
+static int dk_cl_launch(const float* x, const float* dy, float* dst, int B, int H, int L, int K,
+                        int nranges, int det, void* stream) {
+  const DkClFn fn = kDkClTable[mfma_index(L)];
+  const int nw = dk_cl_waves(16 * (mfma_index(L) + 1));
+  const size_t lds = dk_cl_lds_bytes(16 * (mfma_index(L) + 1), L, nw);
+  const long long nb = (long long)(H / kClChannels) * nranges;
+  if (nranges < 1) return PT_ERR_CONFIG;
   if (nb >= (1LL << 31)) return PT_ERR_SHAPE;
-  int nranges = (int)nr;
   uint32_t nblocks = (uint32_t)nb;
-  void* args[] = {&x, &dy, &dw, &B, &H, &L, &K, &nranges, &nblocks};
-  return launch((const void*)fn, nblocks, (uint32_t)threads, lds, stream, args);
+  void* args[] = {&x, &dy, &dst, &B, &H, &L, &K, &nranges, &nblocks, &det};
+  return launch((const void*)fn, nblocks, (uint32_t)(nw * kWave), lds, stream, args);
+}
+
+int dk_cl_det(const float* x, const float* dy, float* dk, float* partials, int B, int H, int L,
+              int K, int nranges, void* stream) {
+  const int st = dk_cl_launch(x, dy, partials, B, H, L, K, nranges, 1, stream);
+  if (st != PT_OK) return st;
+  int ncoef = H * K;
+  const float* cp = partials;
+  void* args[] = {&cp, &dk, &ncoef, &nranges};
+  return launch((const void*)&dk_reduce_kernel, (uint32_t)((ncoef + 3) / 4), 256, 0, stream, args);
 }
 
 // --- long rows: L up to kLongMaxL, K up to kLongMaxK -----------------------
@@ -1530,7 +1548,7 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
   if (pt::check_shape(B, H, L, K) != PT_OK) return PT_ERR_SHAPE;
   if (!pt::aligned(x, 16) || !pt::aligned(dy, 16) || !pt::aligned(dw, 4))
     return PT_ERR_SHAPE;
-  const int st = pt::dk_cl_launch(x, dy, dw, B, H, L, K, stream);
+  const int st = pt::dk_cl_launch(x, dy, dw, B, H, L, K, pt::dk_cl_ranges(B, H, L), 0, stream);
   return st == PT_ERR_HIP ? PT_ERR_HIP : (st == PT_OK ? PT_OK : PT_ERR_SHAPE);
 }
 

@@ -14,4 +14,11 @@ int num_cus();
 // Resident workgroups per CU for (kernel, block size, dynamic LDS), at least 1.
 int blocks_per_cu(const void* fn, int block, size_t lds);
 
+// Channels-last DK of dwconv1d_kernels.hpp: its sample ranges on the current
+// device (0: not served), and the deterministic form, dk [H, K] from
+// H * K * nranges floats of partials (B > 0, H % 32 == 0, 16-byte aligned).
+int dk_cl_ranges(int B, int H, int L);
+int dk_cl_det(const float* x, const float* dy, float* dk, float* partials, int B, int H, int L,
+              int K, int nranges, void* stream);
+
 }  // namespace pt

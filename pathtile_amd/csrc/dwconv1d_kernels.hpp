@@ -1969,7 +1969,8 @@ __global__ __launch_bounds__(512) void dwconv_dk_bf16mma_kernel(
 // of a tile hit 16 distinct banks, and the sample stride is padded to
 // 16 (mod 32) floats so the four 16-lane groups of a wave (four samples)
 // use disjoint banks. Steps are 4 samples (the FP32 MFMA K); the epilogue
-// is the shared one with the [K][H] output.
+// is the shared one with the [K][H] output, or with det != 0 one partial per
+// (h, j, range) for dk_reduce_kernel.
 // ---------------------------------------------------------------------------
 constexpr int kClChannels = 32;
 constexpr int kClWaves = kClChannels / kCgChannelsPerWave;  // 16
@@ -2003,7 +2004,7 @@ template <int LMAX, int CPW = kCgChannelsPerWave, int DEPTH = 1>
 __global__ __launch_bounds__(kClChannels / CPW * kWave) void dwconv_dk_cl_kernel(
     const float* __restrict__ x, const float* __restrict__ gy,
     float* __restrict__ dw, int B, int H, int L, int K, int nranges,
-    uint32_t nblocks) {
+    uint32_t nblocks, int det) {
   using G = CgGeo<LMAX>;
   constexpr int NT = G::nt;
   constexpr int NW = kClChannels / CPW;
@@ -2159,7 +2160,7 @@ __global__ __launch_bounds__(kClChannels / CPW * kWave) void dwconv_dk_cl_kernel
     }
   }
 
-  dk_cg_epilogue<LMAX, true, CPW>(acc, lds, dw, wave, NW, g, r, HC, L, K, nranges, 0, H);
+  dk_cg_epilogue<LMAX, true, CPW>(acc, lds, dw, wave, NW, g, r, HC, L, K, nranges, det, H);
 }
 
 // ---------------------------------------------------------------------------

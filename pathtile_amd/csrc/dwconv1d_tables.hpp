@@ -70,7 +70,7 @@ extern const RowsCgBf16Fn kRowsCgTableBf16[2][2][3];
 // 8-channel groups with plain input loads: [dx][row bucket]
 extern const RowsCgBf16Fn kRowsCgTableBf16PL[2][3];
 using DkClFn = void (*)(const float*, const float*, float*, int, int, int, int,
-                       int, uint32_t);
+                       int, uint32_t, int);
 extern const DkClFn kDkClTable[3];
 using RowsLongFn = void (*)(const float*, const float*, float*, int, int, int, int);
 using DkLongFn = void (*)(const float*, const float*, float*, int, int, int, int, int, int);

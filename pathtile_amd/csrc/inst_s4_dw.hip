@@ -3,13 +3,7 @@
 #include "s4_tables.hpp"
 
 namespace pt {
-const DwFn kDw[kNumS4H][2] = {
-    {&s4_dw_kernel<2, false>, &s4_dw_kernel<2, true>},
-    {&s4_dw_kernel<4, false>, &s4_dw_kernel<4, true>},
-    {&s4_dw_kernel<6, false>, &s4_dw_kernel<6, true>},
-    {&s4_dw_kernel<8, false>, &s4_dw_kernel<8, true>},
-    {&s4_dw_kernel<10, false>, &s4_dw_kernel<10, true>},
-    {&s4_dw_kernel<12, false>, &s4_dw_kernel<12, true>},
-    {&s4_dw_kernel<14, false>, &s4_dw_kernel<14, true>},
-    {&s4_dw_kernel<16, false>, &s4_dw_kernel<16, true>}};
+const DwFn kDw[kNumS4H] = {&s4_dw_kernel<2>,  &s4_dw_kernel<4>,  &s4_dw_kernel<6>,
+                           &s4_dw_kernel<8>,  &s4_dw_kernel<10>, &s4_dw_kernel<12>,
+                           &s4_dw_kernel<14>, &s4_dw_kernel<16>};
 }  // namespace pt

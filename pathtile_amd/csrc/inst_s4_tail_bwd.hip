@@ -3,8 +3,11 @@
 #include "s4_tables.hpp"
 
 namespace pt {
-const TailBwdFn kTailBwd[kNumS4H] = {
-    &s4_tail_bwd_kernel<2>,  &s4_tail_bwd_kernel<4>,  &s4_tail_bwd_kernel<6>,
-    &s4_tail_bwd_kernel<8>,  &s4_tail_bwd_kernel<10>, &s4_tail_bwd_kernel<12>,
-    &s4_tail_bwd_kernel<14>, &s4_tail_bwd_kernel<16>};
+const TailBwdFn kTailBwd[2][kNumS4H] = {
+    {&s4_tail_bwd_kernel<2, false>, &s4_tail_bwd_kernel<4, false>, &s4_tail_bwd_kernel<6, false>,
+     &s4_tail_bwd_kernel<8, false>, &s4_tail_bwd_kernel<10, false>, &s4_tail_bwd_kernel<12, false>,
+     &s4_tail_bwd_kernel<14, false>, &s4_tail_bwd_kernel<16, false>},
+    {&s4_tail_bwd_kernel<2, true>, &s4_tail_bwd_kernel<4, true>, &s4_tail_bwd_kernel<6, true>,
+     &s4_tail_bwd_kernel<8, true>, &s4_tail_bwd_kernel<10, true>, &s4_tail_bwd_kernel<12, true>,
+     &s4_tail_bwd_kernel<14, true>, &s4_tail_bwd_kernel<16, true>}};
 }  // namespace pt

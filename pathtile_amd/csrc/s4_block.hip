@@ -7,6 +7,7 @@
 
 #include "dwconv1d_host.hpp"
 #include "pathtile_hip.h"
+#include "s4_conv.hpp"
 #include "s4_small.hpp"
 #include "s4_tables.hpp"
 
@@ -35,7 +36,8 @@ static int check_block(int B, int H, int L, int states) {
   return PT_OK;
 }
 
-static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+static bool aligned(const void* p, uintptr_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
+static bool aligned16(const void* p) { return aligned(p, 16); }
 
 // token_base's multiplier for n / L.
 static uint32_t token_magic(int L) { return L == 1 ? 0u : (uint32_t)((1ULL << 32) / (unsigned)L) + 1u; }
@@ -51,27 +53,27 @@ static uint32_t dw_steps_per_range(uint32_t nsteps, int split) {
   return per < 4 ? 4 : per;
 }
 
-// Workspace of the backward, in floats: dP (blocks of 32 tokens; later dX
-// before its transpose), du [B,H,L], the weight gradient's partials, dk [H][L], and the
-// convolution's own partials.
+// Workspace of the backward, in floats: dP (blocks of 32 tokens), du, the
+// weight gradient's partials, dk [H][L] and its partials.
 struct BwdLayout {
-  size_t du, part, dk, conv, conv_bytes, total;
+  size_t du, part, dk, dkp, total;
   uint32_t nsteps, per, ranges;
+  int dk_ranges;
 };
 
-static int bwd_layout(int B, int H, int L, int threads, BwdLayout* o) {
+static int bwd_layout(int B, int H, int L, BwdLayout* o) {
   const TailGeometry& k = kTail[H / 32 - 1];
   const size_t ntok = (size_t)B * L;
   o->nsteps = (uint32_t)((ntok + kDwTok - 1) / kDwTok);
   o->per = dw_steps_per_range(o->nsteps, k.dw_split);
   o->ranges = (o->nsteps + o->per - 1) / o->per;
+  o->dk_ranges = dk_cl_ranges(B, H, L);
+  if (o->dk_ranges < 1) return PT_ERR_CONFIG;
   o->du = (size_t)2 * H * round_up(ntok, 64);
   o->part = o->du + ntok * H;
   o->dk = o->part + round_up((size_t)o->ranges * (2 * H * H + 2 * H), 64);
-  o->conv = o->dk + round_up((size_t)H * L, 64);
-  const int st = pt_dwconv1d_dk_det_workspace_bytes(B, H, L, L, threads, &o->conv_bytes);
-  if (st != PT_OK) return st;
-  o->total = o->conv * sizeof(float) + o->conv_bytes;
+  o->dkp = o->dk + round_up((size_t)H * L, 64);
+  o->total = (o->dkp + (size_t)H * L * o->dk_ranges) * sizeof(float);
   return PT_OK;
 }
 
@@ -80,22 +82,15 @@ static uint32_t resident_grid(const void* fn, int block, size_t lds, uint32_t wo
   return n < work ? n : work;
 }
 
-static int transpose_launch(const float* d, const float* add, float* out, int B, int H, int L,
-                            void* stream) {
-  const size_t lds = (size_t)L * (H + 1) * sizeof(float);
-  const bool vec = L % 4 == 0 && aligned16(d) && aligned16(out);
-  if (add) {
-    const void* fn = vec ? (const void*)&s4_transpose_add_kernel<true>
-                         : (const void*)&s4_transpose_add_kernel<false>;
-    void* args[] = {&d, &add, &out, &B, &H, &L};
-    return launch(fn, resident_grid(fn, kTransThreads, lds, (uint32_t)B), kTransThreads, lds,
-                  stream, args);
-  }
-  const void* fn =
-      vec ? (const void*)&s4_transpose_kernel<true> : (const void*)&s4_transpose_kernel<false>;
-  void* args[] = {&d, &out, &B, &H, &L};
-  return launch(fn, resident_grid(fn, kTransThreads, lds, (uint32_t)B), kTransThreads, lds, stream,
-                args);
+// add: the input gradient plus that tensor; else the forward, with a mask or not.
+static int conv_cl_launch(const float* x, const float* w, const float* add,
+                          const unsigned char* mask, float scale, float* y, int B, int H, int L,
+                          void* stream) {
+  const void* fn = (const void*)kConvCl[add ? 1 : mask ? 2 : 0][(L + 7) / 8 - 1];
+  const int block = conv_cl_threads(H), per = block / H;
+  void* args[] = {&x, &w, &add, &mask, &scale, &y, &B, &H, &L};
+  return launch(fn, resident_grid(fn, block, 0, (uint32_t)((B + per - 1) / per)), (uint32_t)block, 0,
+                stream, args);
 }
 
 // --- the model's ends ---------------------------------------------------------
@@ -145,28 +140,23 @@ int pt_s4_block_prep_values(int H, int L, size_t* floats) {
 
 int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, const float* c_im,
                         const float* log_a_re, const float* a_im, const float* skip,
-                        const float* w, float* prep, float* xt, float* u, int B, int H, int L,
-                        int states, int backward, int waves_per_block, int algo, void* stream) {
+                        const float* w, const unsigned char* mask, float scale, float* prep,
+                        float* v, int B, int H, int L, int states, int backward, void* stream) {
   int st = pt::check_block(B, H, L, states);
   if (st != PT_OK) return st;
-  if (!x || !log_dt || !c_re || !c_im || !log_a_re || !a_im || !skip || !w || !prep || !xt || !u)
+  if (!x || !log_dt || !c_re || !c_im || !log_a_re || !a_im || !skip || !w || !prep || !v)
     return PT_ERR_NULL;
-  if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(xt) || !pt::aligned16(u))
+  if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(v) || !pt::aligned(mask, 4))
     return PT_ERR_ALIGN;
   float* taps = prep;
   __bf16* wf = reinterpret_cast<__bf16*>(prep + pt::round_up((size_t)H * L, 64));
-  {
-    const int frags = 2 * H * H / 8 * (backward ? 2 : 1);
-    const uint32_t grid =
-        (uint32_t)(H + (frags + pt::kPrepThreads - 1) / pt::kPrepThreads);
-    void* args[] = {&log_dt, &c_re, &c_im, &log_a_re, &a_im, &skip, &w, &taps, &wf, &H, &L,
-                    &states, &backward};
-    st = pt::launch((const void*)&pt::s4_prep_kernel, grid, pt::kPrepThreads, 0, stream, args);
-    if (st != PT_OK) return st;
-  }
-  st = pt::transpose_launch(x, nullptr, xt, B, H, L, stream);
+  const int frags = 2 * H * H / 8 * (backward ? 2 : 1);
+  const uint32_t grid = (uint32_t)(H + (frags + pt::kPrepThreads - 1) / pt::kPrepThreads);
+  void* args[] = {&log_dt, &c_re, &c_im, &log_a_re, &a_im, &skip, &w, &taps, &wf, &H, &L,
+                  &states, &backward};
+  st = pt::launch((const void*)&pt::s4_prep_kernel, grid, pt::kPrepThreads, 0, stream, args);
   if (st != PT_OK) return st;
-  return pt_dwconv1d_fwd_f32_algo(xt, taps, u, B, H, L, L, waves_per_block, algo, stream);
+  return pt::conv_cl_launch(x, taps, nullptr, mask, scale, v, B, H, L, stream);
 }
 
 int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
@@ -180,85 +170,78 @@ int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, cons
     return PT_ERR_ALIGN;
   const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
-  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, magic = pt::token_magic(L);
+  uint32_t ntok = (uint32_t)B * (uint32_t)L;
   uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
   const size_t lds = pt::tail_fwd_lds(H);
   const int block = k.nw * pt::kWave;
-  void* args[] = {&v, &x, &wf, &w, &bias, &y, &q, &ntok, &uL, &magic, &ntiles};
+  void* args[] = {&v, &x, &wf, &w, &bias, &y, &q, &ntok, &ntiles};
   const void* fn = (const void*)pt::kTailFwd[H / 32 - 1];
   return pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
                     args);
 }
 
-int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, int threads_per_block, size_t* bytes) {
+int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, size_t* bytes) {
   if (!bytes) return PT_ERR_NULL;
   int st = pt::check_block(B, H, L, 1);
   if (st != PT_OK) return st;
   pt::BwdLayout o;
-  st = pt::bwd_layout(B, H, L, threads_per_block, &o);
+  st = pt::bwd_layout(B, H, L, &o);
   if (st == PT_OK) *bytes = o.total;
   return st;
 }
 
-int pt_s4_block_bwd_f32(const float* gy, const float* xt, const float* v, const float* q,
+int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const float* q,
                         const unsigned char* mask, float scale, const float* prep, const float* w,
                         const float* log_dt, const float* c_re, const float* c_im,
                         const float* log_a_re, const float* a_im, float* gx, float* d_log_dt,
                         float* d_c_re, float* d_c_im, float* d_log_a_re, float* d_a_im,
                         float* d_skip, float* dw, float* dbias, void* workspace,
-                        size_t workspace_bytes, int B, int H, int L, int states,
-                        int dx_waves_per_block, int algo, int threads_per_block, void* stream) {
+                        size_t workspace_bytes, int B, int H, int L, int states, void* stream) {
   int st = pt::check_block(B, H, L, states);
   if (st != PT_OK) return st;
-  if (!gy || !xt || !v || !q || !prep || !w) return PT_ERR_NULL;
+  if (!gy || !x || !v || !q || !prep || !w) return PT_ERR_NULL;
   const bool taps_grad = d_skip != nullptr;
   if (taps_grad && (!log_dt || !c_re || !c_im || !log_a_re || !a_im || !d_log_dt || !d_c_re ||
                     !d_c_im || !d_log_a_re || !d_a_im))
     return PT_ERR_NULL;
   if ((dw == nullptr) != (dbias == nullptr)) return PT_ERR_NULL;
-  if (!pt::aligned16(gy) || !pt::aligned16(xt) || !pt::aligned16(v) || !pt::aligned16(prep) ||
+  if (!pt::aligned16(gy) || !pt::aligned16(x) || !pt::aligned16(v) || !pt::aligned16(prep) ||
       !pt::aligned16(q) || !pt::aligned16(workspace) || (gx && !pt::aligned16(gx)))
     return PT_ERR_ALIGN;
   pt::BwdLayout o;
-  st = pt::bwd_layout(B, H, L, threads_per_block, &o);
+  st = pt::bwd_layout(B, H, L, &o);
   if (st != PT_OK) return st;
   if (!workspace || workspace_bytes < o.total) return PT_ERR_WORKSPACE;
   const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   float* const ws = static_cast<float*>(workspace);
-  float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk, *dxt = ws;
+  float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk;
   const float* taps = prep;
   const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
-  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L;
-  uint32_t magic = pt::token_magic(L);
+  uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, magic = pt::token_magic(L);
   {
     uint32_t ntiles = (ntok + k.btok - 1) / k.btok;
-    const size_t lds = k.bwd_lds;
     const int block = k.nw * pt::kWave;
     void* args[] = {&gy, &q, &v, &mask, &scale, &wf, &w, &du, &dp, &ntok, &uL, &magic, &ntiles};
-    const void* fn = (const void*)pt::kTailBwd[H / 32 - 1];
-    st = pt::launch(fn, pt::resident_grid(fn, block, lds, ntiles), (uint32_t)block, lds, stream,
-                    args);
+    const void* fn = (const void*)pt::kTailBwd[mask != nullptr][H / 32 - 1];
+    st = pt::launch(fn, pt::resident_grid(fn, block, k.bwd_lds, ntiles), (uint32_t)block,
+                    k.bwd_lds, stream, args);
     if (st != PT_OK) return st;
   }
   if (dw) {
-    const void* fn = (const void*)pt::kDw[H / 32 - 1][L % 4 == 0];
     const float* cdp = dp;
-    void* args[] = {&cdp, &v, &part, &ntok, &uL, &magic, &o.nsteps, &o.per};
-    st = pt::launch(fn, o.ranges * (uint32_t)k.dw_split, (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds,
-                    stream, args);
+    void* args[] = {&cdp, &v, &part, &ntok, &o.nsteps, &o.per};
+    st = pt::launch((const void*)pt::kDw[H / 32 - 1], o.ranges * (uint32_t)k.dw_split,
+                    (uint32_t)(k.dw_nw * pt::kWave), k.dw_lds, stream, args);
     if (st != PT_OK) return st;
     st = pt::reduce_launch(part, dw, dbias, 2 * H * H, 2 * H, (int)o.ranges, stream);
     if (st != PT_OK) return st;
   }
-  if (gx) {  // dX before its transpose takes dP's place, which is read by now
-    st = pt_dwconv1d_dx_f32_algo(du, taps, dxt, B, H, L, L, dx_waves_per_block, algo, stream);
-    if (st != PT_OK) return st;
-    st = pt::transpose_launch(dxt, gy, gx, B, H, L, stream);
+  if (gx) {
+    st = pt::conv_cl_launch(du, taps, gy, nullptr, 0.0f, gx, B, H, L, stream);
     if (st != PT_OK) return st;
   }
   if (!taps_grad) return PT_OK;
-  st = pt_dwconv1d_dk_det_f32(du, xt, dk, ws + o.conv, o.conv_bytes, B, H, L, L, threads_per_block,
-                              stream);
+  st = pt::dk_cl_det(x, du, dk, ws + o.dkp, B, H, L, L, o.dk_ranges, stream);
   if (st != PT_OK) return st;
   const float* cdk = dk;
   void* targs[] = {&cdk, &log_dt, &c_re, &c_im, &log_a_re, &a_im, &d_log_dt, &d_c_re, &d_c_im,

@@ -4,14 +4,15 @@
 //
 // One block computes, for x [B, L, H] and N2 complex states per channel,
 //   taps[h][t] = 2 Re sum_n C_eff[h,n] exp(dt[h] A[h,n] t)  (+ skip at L / 2)
-//   u [b,h,t]  = conv(x^T, taps),  v = dropout(u),  g = gelu(v)
-//   P [b,c,t]  = sum_h W[c][h] g[b,h,t] + bias[c],  c < 2 H
+//   u [b,t,h]  = conv(x, taps) over t,  v = dropout(u),  g = gelu(v)
+//   P [b,t,c]  = sum_h W[c][h] g[b,t,h] + bias[c],  c < 2 H
 //   y [b,t,c]  = P[c] sigmoid(P[H + c]) + x[b,t,c],  c < H
-// The convolution runs on the kernels of dwconv1d_kernels.hpp, the taps, their
-// gradient and the [B,L,H] <-> [B,H,L] transposes on those of s4_small.hpp.
-// Here is the tail (GELU, projection, GLU, residual) with its backward, each
-// one pass over its tensors. The tail treats the B L columns as one list of tokens
-// (token = b L + t), so its tiles do not depend on L.
+// in [B, L, H] throughout. The convolution and its input gradient are in
+// s4_conv.hpp, its weight gradient is the channels-last DK of
+// dwconv1d_kernels.hpp, taps, their gradient and the model's ends are in
+// s4_small.hpp. Here is the tail (GELU, projection, GLU, residual) with its
+// backward, each one pass over its tensors. The tail treats the B L columns as
+// one list of tokens (token = b L + t), so its tiles do not depend on L.
 //
 // The projection runs on the BF16 matrix cores with both operands split into
 // three BF16 parts (split3_bf16x8; six of the nine part products, dropped
@@ -179,27 +180,31 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_token_rows(const float* t
   return make_rsrc_n(t + (size_t)n0 * H, bytes);
 }
 
-// gelu(v) of TOK tokens, split into the three parts of the LDS stage
-// [part][token][GS]: a lane takes one token and eight channels, so a wave's
-// loads run along the tokens of one channel. store<I, N> does the I-th of N
-// slices of the work.
+// gelu of TOK tokens' values, split into the three parts of the LDS stage
+// [part][token][GS]: a lane takes eight channels of one token, 32 consecutive
+// bytes. store<I, N> does the I-th of N slices of the work.
 template <int CT, int TOK>
 struct GeluStage {
   using G = TailGeo<CT>;
-  static constexpr int TH = G::NW * kWave, kUnits = TOK * (G::H / 8);
+  static constexpr int TH = G::NW * kWave, kUnits = TOK * (G::H / 8), CPT = G::H / 8;
   static constexpr int U = (kUnits + TH - 1) / TH;
   float x[U][8];
 
-  __device__ __forceinline__ void load(const float* __restrict__ v, uint32_t n0, uint32_t ntok,
-                                       uint32_t L, uint32_t magic) {
-    const Slab s = make_slab(v, n0, ntok, G::H, L, magic);
+  __device__ __forceinline__ void load(const float* __restrict__ v, uint32_t n0, uint32_t ntok) {
+    const __amdgpu_buffer_rsrc_t r = make_token_rows(v, n0, ntok, G::H);
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const int u = threadIdx.x + i * TH;
-      const uint32_t at = token_base(n0 + u % TOK, G::H, L, magic) - s.first + 8 * (u / TOK) * L;
-#pragma unroll
-      for (int k = 0; k < 8; ++k)
-        x[i][k] = buf_load1(s.r, kUnits % TH == 0 || u < kUnits ? 4 * (at + k * L) : kOob, 0);
+      const uint32_t o = kUnits % TH == 0 || u < kUnits ? 32 * u : kOob;
+      const float4 a = buf_load4(r, o, 0), b = buf_load4(r, o + 16, 0);
+      x[i][0] = a.x;
+      x[i][1] = a.y;
+      x[i][2] = a.z;
+      x[i][3] = a.w;
+      x[i][4] = b.x;
+      x[i][5] = b.y;
+      x[i][6] = b.z;
+      x[i][7] = b.w;
     }
   }
 
@@ -207,14 +212,14 @@ struct GeluStage {
   __device__ __forceinline__ void store(__bf16* sg) {
 #pragma unroll
     for (int e = 8 * U * I / N; e < 8 * U * (I + 1) / N; ++e) {
-      const int i = e / 8;
+      const int i = e / 8, u = threadIdx.x + i * TH;
+      const bool on = kUnits % TH == 0 || u < kUnits;
       x[i][e % 8] = gelu_f(x[i][e % 8]);  // 0 past the last token
       if (e % 8 == 7) {
-        const int u = threadIdx.x + i * TH;
         bf16x8 hi, mid, lo;
         split3_bf16x8(x[i], hi, mid, lo);
         // units past the end write to a row padding that nothing reads
-        __bf16* d = sg + (u % TOK) * G::GS + (kUnits % TH == 0 || u < kUnits ? 8 * (u / TOK) : G::H);
+        __bf16* d = sg + (on ? (u / CPT) * G::GS + 8 * (u % CPT) : (u % TOK) * G::GS + G::H);
         *reinterpret_cast<bf16x8*>(d) = hi;
         *reinterpret_cast<bf16x8*>(d + TOK * G::GS) = mid;
         *reinterpret_cast<bf16x8*>(d + 2 * TOK * G::GS) = lo;
@@ -311,11 +316,11 @@ __device__ __forceinline__ void multiply(f32x4 (&acc)[M][NT], W& w, const __bf16
 
 // One pre-activation of one token by the FP32 chain, for values that the
 // split cannot carry (Inf, NaN, or rounding past BF16's largest value).
-__device__ __forceinline__ float project_one(const float* __restrict__ v, const float* __restrict__ w,
-                                             uint32_t base, int row, int H, int L) {
+__device__ __forceinline__ float project_one(const float* v, const float* __restrict__ w, int row,
+                                             int H) {
   float s = 0.0f;
 #pragma unroll 1
-  for (int h = 0; h < H; ++h) s = fmaf(w[(size_t)row * H + h], gelu_f(v[base + (uint32_t)(h * L)]), s);
+  for (int h = 0; h < H; ++h) s = fmaf(w[(size_t)row * H + h], gelu_f(v[h]), s);
   return s;
 }
 
@@ -326,19 +331,19 @@ __device__ __forceinline__ void set_elem(f32x4& a, int r, float v) {
   a[3] = r == 3 ? v : a[3];
 }
 
-// Recomputes a lane's four value and gate sums where one is not finite.
-__device__ __forceinline__ void project_fix(f32x4& a, f32x4& b, const float* __restrict__ v,
-                                            const float* __restrict__ w, uint32_t base, int c,
-                                            int H, uint32_t L) {
+// Recomputes a lane's four value and gate sums where one is not finite; v are
+// the token's values.
+__device__ __forceinline__ void project_fix(f32x4& a, f32x4& b, const float* v,
+                                            const float* __restrict__ w, int c, int H) {
 #pragma unroll 1
   for (int r = 0; r < 4; ++r) {
-    set_elem(a, r, project_one(v, w, base, c + r, H, L));
-    set_elem(b, r, project_one(v, w, base, H + c + r, H, L));
+    set_elem(a, r, project_one(v, w, c + r, H));
+    set_elem(b, r, project_one(v, w, H + c + r, H));
   }
 }
 
 // ---------------------------------------------------------------------------
-// Tail forward: y = GLU(W gelu(v) + bias) + x, v [B,H,L], x and y [B,L,H].
+// Tail forward: y = GLU(W gelu(v) + bias) + x, all [tokens][H].
 // A persistent workgroup, one per CU, walks tiles of 64 tokens (32 above
 // H = 128, what the LDS holds). gelu is as much vector work as the products
 // are matrix work, and both kinds from one wave overlap where they are
@@ -355,7 +360,7 @@ template <int CT>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
     const float* __restrict__ v, const float* __restrict__ x, const __bf16* __restrict__ wf,
     const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y,
-    float* __restrict__ q, uint32_t ntok, uint32_t L, uint32_t magic, uint32_t ntiles) {
+    float* __restrict__ q, uint32_t ntok, uint32_t ntiles) {
   using G = TailGeo<CT>;
   constexpr int TOK = G::TOK, NT = TOK / 16 / G::WPT, SZ = 3 * TOK * G::GS, TH = G::NW * kWave;
   constexpr int R4 = TOK * G::H / 4 / TH;  // 16-byte pieces of a tile's rows per thread
@@ -371,9 +376,9 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
   std::conditional_t<CT <= 8, ResidentFrags<2 * G::MT, G::KS>, StreamedFrags<2 * G::MT, G::KS>>
       frags(w0);
   GeluStage<CT, TOK> stage;
-  stage.load(v, blockIdx.x * TOK, ntok, L, magic);
+  stage.load(v, blockIdx.x * TOK, ntok);
   stage.template store<0, 1>(sg);
-  stage.load(v, (blockIdx.x + gridDim.x) * TOK, ntok, L, magic);
+  stage.load(v, (blockIdx.x + gridDim.x) * TOK, ntok);
   uint32_t cur = 0;
   for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, cur ^= 1) {
     const uint32_t n0 = tile * TOK;
@@ -388,7 +393,7 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
         acc, frags, sg + cur * SZ + tk0 * G::GS + 8 * (lane >> 4), [&](auto ks) {
           stage.template store<decltype(ks)::value, G::KS>(sg + (cur ^ 1) * SZ);
         });
-    stage.load(v, (tile + 2 * gridDim.x) * TOK, ntok, L, magic);
+    stage.load(v, (tile + 2 * gridDim.x) * TOK, ntok);
 #pragma unroll
     for (int m = 0; m < G::MT; ++m) {
       const int c = c0 + 16 * m;
@@ -399,7 +404,7 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
         const int tk = tk0 + 16 * nt;
         f32x4 a = acc[2 * m][nt], b = acc[2 * m + 1][nt];
         if (__builtin_expect(!(finite4(a[0], a[1], a[2], a[3]) && finite4(b[0], b[1], b[2], b[3])), 0)) {
-          if (n0 + tk < ntok) project_fix(a, b, v, w, token_base(n0 + tk, G::H, L, magic), c, G::H, L);
+          if (n0 + tk < ntok) project_fix(a, b, v + (size_t)(n0 + tk) * G::H, w, c, G::H);
         }
         const float4 pa = {a[0] + ba.x, a[1] + ba.y, a[2] + ba.z, a[3] + ba.w};
         const float4 ps = {sigmoid_f(b[0] + bb.x), sigmoid_f(b[1] + bb.y), sigmoid_f(b[2] + bb.z),
@@ -425,8 +430,8 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Tail backward with respect to its input: from gy [B,L,H] and the forward's
-// q, du = dL/du [B,H,L] (through GLU, projection, gelu and the dropout mask)
+// Tail backward with respect to its input: from gy [tokens][H] and the
+// forward's q and v, du = dL/du [tokens][H] (through GLU, projection, gelu and the dropout mask)
 // and dP [blocks of 32 tokens][2 H][32] (zero past the last token) for the
 // weight gradient, whose loads it makes whole lines. A persistent workgroup walks tiles of 32 tokens (64 at
 // H = 32): tile t's product W^T dP from LDS, the weight fragments resident up
@@ -435,10 +440,10 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
 // H = 128 the LDS holds one stage, the GLU gradient comes before the product
 // and the fragments stream. Seven tensor passes of HBM bound it; recomputing
 // the pre-activations instead of reading q took 5 passes but 975 us at B16384
-// L48 H128 on the sum of its matrix and vector work, 698 us now (the forward,
-// which writes q, 388 -> 483).
+// L48 H128 on the sum of its matrix and vector work, 605 us now (the forward,
+// which writes q, 388 -> 490).
 // ---------------------------------------------------------------------------
-template <int CT>
+template <int CT, bool MASK>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
     const float* __restrict__ gy, const float* __restrict__ q, const float* __restrict__ v,
     const uint8_t* __restrict__ mask, float scale, const __bf16* __restrict__ wf,
@@ -454,15 +459,16 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
   const int ct0 = (wave % G::WPC) * G::MT, nt0 = (wave / G::WPC) * NT;
   const int tk0 = 16 * nt0 + (lane & 15);
   const int c0 = 16 * ct0 + 4 * (lane >> 4);
-  const bool masked = mask != nullptr;
-  const float keep = masked ? scale : 1.0f;
   std::conditional_t<G::TWO, ResidentFrags<G::MT, KS>, StreamedFrags<G::MT, KS>> frags(
       wf + wfrag_values(G::H) + (size_t)ct0 * KS * 3 * 512 + lane * 8);
   constexpr int E = G::MT * NT * 4;  // du values per lane and tile: (m, nt, r)
 
   // GLU gradient of the tile whose q and gy are loaded
-  float4 q1[G::MT][NT], q2[G::MT][NT], g4[G::MT][NT];
-  auto load_glu = [&](uint32_t n0) {
+  struct Glu {
+    float4 q1[G::MT][NT], q2[G::MT][NT], g4[G::MT][NT];
+  };
+  Glu ga, gb;
+  auto load_glu = [&](Glu& s, uint32_t n0) {
     const __amdgpu_buffer_rsrc_t r1 = make_token_rows(q, n0, ntok, G::H);
     const __amdgpu_buffer_rsrc_t r2 = make_token_rows(q + (size_t)ntok * G::H, n0, ntok, G::H);
     const __amdgpu_buffer_rsrc_t rg = make_token_rows(gy, n0, ntok, G::H);
@@ -471,13 +477,13 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
 #pragma unroll
       for (int m = 0; m < G::MT; ++m) {
         const uint32_t o = 4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m);
-        q1[m][nt] = buf_load4(r1, o, 0);
-        q2[m][nt] = buf_load4(r2, o, 0);
-        g4[m][nt] = buf_load4(rg, o, 0);
+        s.q1[m][nt] = buf_load4(r1, o, 0);
+        s.q2[m][nt] = buf_load4(r2, o, 0);
+        s.g4[m][nt] = buf_load4(rg, o, 0);
       }
   };
   float pa[8];  // four value and four gate gradients
-  auto glu = [&](auto slice, auto slices, uint32_t n0, __bf16* st) {
+  auto glu = [&](const Glu& in_, auto slice, auto slices, uint32_t n0, __bf16* st) {
     constexpr int I = decltype(slice)::value, N = decltype(slices)::value;
     // past the last tile the stores are dropped
     const __amdgpu_buffer_rsrc_t dr =
@@ -487,7 +493,8 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
       const int r = e % 4, m = e / 4 % G::MT, nt = e / 4 / G::MT;
       const int tk = tk0 + 16 * nt, c = c0 + 16 * m;
       const bool in = n0 + tk < ntok;
-      const float a = (&q1[m][nt].x)[r], s = (&q2[m][nt].x)[r], g = (&g4[m][nt].x)[r];
+      const float a = (&in_.q1[m][nt].x)[r], s = (&in_.q2[m][nt].x)[r];
+      const float g = (&in_.g4[m][nt].x)[r];
       pa[r] = in ? s * g : 0.0f;
       pa[4 + r] = in ? (1.0f - s) * s * g * a : 0.0f;
       buf_store1(pa[r], dr, dp_offset<G::H>(tk, c + r));
@@ -509,75 +516,85 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
 
   // gelu gradient of a finished product: its values, mask and where du goes
   // (nowhere before the first tile)
-  f32x4 dg[G::MT][NT], dgn[G::MT][NT];
-  float vv[G::MT][NT][4];
-  uint32_t mk[G::MT][NT][4], at[NT];
-  Slab out = make_slab(du, ntok, ntok, G::H, L, magic);
+  f32x4 dg[G::MT][NT];
+  struct Vals {
+    float4 vv[G::MT][NT];
+    uint32_t mk[MASK ? G::MT : 1][MASK ? NT : 1][4];
+  };
+  Vals la, lb;
+  __amdgpu_buffer_rsrc_t out = make_token_rows(du, ntok, ntok, G::H);
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
-    at[nt] = 0;
 #pragma unroll
     for (int m = 0; m < G::MT; ++m) {
       dg[m][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      lb.vv[m][nt] = float4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (MASK) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        vv[m][nt][r] = 0.0f;
-        mk[m][nt][r] = 0;
+        for (int r = 0; r < 4; ++r) lb.mk[m][nt][r] = 0;
       }
     }
   }
-  auto finish = [&](auto slice, auto slices) {
+  float o4[4];
+  auto finish = [&](const Vals& l, auto slice, auto slices) {
     constexpr int I = decltype(slice)::value, N = decltype(slices)::value;
 #pragma unroll
     for (int e = E * I / N; e < E * (I + 1) / N; ++e) {
       const int r = e % 4, m = e / 4 % G::MT, nt = e / 4 / G::MT;
-      float o = dg[m][nt][r] * gelu_grad_f(vv[m][nt][r]);
-      o = o * (masked ? (float)mk[m][nt][r] : 1.0f) * keep;
-      buf_store1(o, out.r, 4 * (at[nt] + (uint32_t)(16 * m + r) * L));
+      o4[r] = dg[m][nt][r] * gelu_grad_f((&l.vv[m][nt].x)[r]);
+      if constexpr (MASK) o4[r] = o4[r] * (float)l.mk[m][nt][r] * scale;
+      if (r == 3)
+        buf_store4(float4{o4[0], o4[1], o4[2], o4[3]}, out,
+                   4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m));
     }
   };
   using All = std::integral_constant<int, 1>;
   using Steps = std::integral_constant<int, KS>;
   using Zero = std::integral_constant<int, 0>;
 
-  load_glu(blockIdx.x * TOK);
-  if constexpr (G::TWO) {
-    glu(Zero{}, All{}, blockIdx.x * TOK, sp);
-    load_glu((blockIdx.x + gridDim.x) * TOK);
-  }
   uint32_t cur = 0;
-  for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x, cur ^= G::TWO) {
+  // One tile. `now` holds the GLU inputs of the tile that this call's shadow
+  // (or, with one stage, its start) works on; `then` is loaded for the call
+  // after, a whole tile ahead of its use, as are `vals` for the tile's own
+  // gelu gradient, which runs in the next call's shadow.
+  auto body = [&](uint32_t tile, const Glu& now, Glu& then, Vals& vals, const Vals& before) {
     const uint32_t n0 = tile * TOK, next = (tile + gridDim.x) * TOK;
     if constexpr (!G::TWO) {
       __syncthreads();  // the stage is read
-      glu(Zero{}, All{}, n0, sp);
-      load_glu(next);
+      glu(now, Zero{}, All{}, n0, sp);
     }
     __threadfence_block();
     __syncthreads();  // tile t's dP parts are written
     frags.begin();
+    load_glu(then, G::TWO ? next + gridDim.x * TOK : next);
+    const __amdgpu_buffer_rsrc_t in = make_token_rows(v, n0, ntok, G::H);
+    const Slab ms = make_slab<1>(mask, n0, ntok, G::H, L, magic);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int m = 0; m < G::MT; ++m) {
+        vals.vv[m][nt] = buf_load4(in, 4 * ((tk0 + 16 * nt) * G::H + c0 + 16 * m), 0);
+        if constexpr (MASK) {
+          const uint32_t at = token_base(n0 + tk0 + 16 * nt, G::H, L, magic) - ms.first +
+                              (uint32_t)(c0 + 16 * m) * L;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            vals.mk[m][nt][r] = __builtin_amdgcn_raw_buffer_load_b8(ms.r, at + r * L, 0, 0);
+        }
+      }
+    f32x4 dgn[G::MT][NT];
     multiply<G::MT, NT, KS, G::PS, TOK>(
         dgn, frags, sp + cur * SZ + tk0 * G::PS + 8 * (lane >> 4), [&](auto ks) {
-          finish(ks, Steps{});
-          if constexpr (G::TWO) glu(ks, Steps{}, next, sp + (cur ^ 1) * SZ);
+          finish(before, ks, Steps{});
+          if constexpr (G::TWO) glu(now, ks, Steps{}, next, sp + (cur ^ 1) * SZ);
         });
-    if constexpr (G::TWO) load_glu(next + gridDim.x * TOK);
-    out = make_slab(du, n0, ntok, G::H, L, magic);
-    const Slab in = make_slab(v, n0, ntok, G::H, L, magic);
-    const __amdgpu_buffer_rsrc_t mr =
-        make_slab<1>(mask, masked ? n0 : ntok, ntok, G::H, L, magic).r;
+    out = make_token_rows(du, n0, ntok, G::H);
+    cur ^= G::TWO;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       const uint32_t n = n0 + tk0 + 16 * nt;
-      at[nt] = token_base(n, G::H, L, magic) - in.first + (uint32_t)c0 * L;
 #pragma unroll
       for (int m = 0; m < G::MT; ++m) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t o = at[nt] + (uint32_t)(16 * m + r) * L;
-          vv[m][nt][r] = buf_load1(in.r, 4 * o, 0);
-          mk[m][nt][r] = __builtin_amdgcn_raw_buffer_load_b8(mr, o, 0, 0);
-        }
         f32x4 d = dgn[m][nt];
         if (__builtin_expect(!finite4(d[0], d[1], d[2], d[3]), 0)) {
           if (n < ntok) {
@@ -596,8 +613,28 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
         dg[m][nt] = d;
       }
     }
+  };
+
+  load_glu(ga, blockIdx.x * TOK);
+  if constexpr (G::TWO) {
+    glu(ga, Zero{}, All{}, blockIdx.x * TOK, sp);
+    load_glu(ga, (blockIdx.x + gridDim.x) * TOK);
   }
-  finish(Zero{}, All{});
+  uint32_t tile = blockIdx.x;
+  while (true) {
+    if (tile >= ntiles) {
+      finish(lb, Zero{}, All{});
+      break;
+    }
+    body(tile, ga, gb, la, lb);
+    tile += gridDim.x;
+    if (tile >= ntiles) {
+      finish(la, Zero{}, All{});
+      break;
+    }
+    body(tile, gb, ga, lb, la);
+    tile += gridDim.x;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -608,7 +645,7 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
 // contiguous) and split in registers; g is computed, split and
 // shared through LDS [part][channel][40]. Partials [range][2 H H + 2 H] go to
 // the workspace for a fixed-order reduction. Step s + 1's gelu and splits run
-// in the shadow of step s's products: 381 us at B16384 L48 H128, 430 with them
+// in the shadow of step s's products: 354 us at B16384 L48 H128, 430 with them
 // ahead of the products.
 // ---------------------------------------------------------------------------
 template <int CT>
@@ -616,16 +653,19 @@ struct DwGeo {
   static constexpr int RT = 2 * CT;  // row tiles
   static constexpr int NW = RT % 8 == 0 ? 8 : RT == 4 ? 4 : RT == 12 ? 6 : RT / 4;
   static constexpr int MT = RT / NW;
-  static constexpr int NB = CT <= 8 ? CT : CT / 2;  // column tiles per workgroup
+  // column tiles per workgroup, so that the accumulators leave room for the loads
+  static constexpr int NB = CT <= 8 ? CT : CT % 4 == 0 ? CT / 4 : CT / 2;
+  static constexpr bool DEEP = CT <= 8 || CT == 12;     // two sets of loads in flight
+  static constexpr bool AHEAD = CT <= 8 || CT % 4 == 0;  // rows split a step ahead
   static constexpr int SPLIT = CT / NB;
   static constexpr int CS = kDwTok + 8;  // BF16 values per channel row of a part
   static constexpr size_t lds = (size_t)2 * 3 * NB * 16 * CS * 2;
 };
 
-template <int CT, bool VEC>
+template <int CT>
 __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     const float* __restrict__ dp, const float* __restrict__ v, float* __restrict__ part,
-    uint32_t ntok, uint32_t L, uint32_t magic, uint32_t nsteps, uint32_t steps_per) {
+    uint32_t ntok, uint32_t nsteps, uint32_t steps_per) {
   using D = DwGeo<CT>;
   constexpr int H = 16 * CT, NC = 16 * D::NB, TH = D::NW * kWave;
   constexpr int kUnits = NC * (kDwTok / 8);  // (channel, eight tokens)
@@ -634,7 +674,13 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
   extern __shared__ __align__(16) char smem[];
   __bf16* const sg = reinterpret_cast<__bf16*>(smem);  // two stages
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int range = blockIdx.x / D::SPLIT, nb = blockIdx.x % D::SPLIT;
+  // the workgroups of one range, which read the same rows, on one XCD
+  int range = blockIdx.x / D::SPLIT, nb = blockIdx.x % D::SPLIT;
+  if (D::SPLIT > 1 && gridDim.x % (kNumXcd * D::SPLIT) == 0) {
+    const int q = blockIdx.x / (kNumXcd * D::SPLIT), r = blockIdx.x % (kNumXcd * D::SPLIT);
+    range = q * kNumXcd + r % kNumXcd;
+    nb = r / kNumXcd;
+  }
   const uint32_t s0 = range * steps_per;
   const uint32_t s1 = s0 + steps_per < nsteps ? s0 + steps_per : nsteps;
   f32x4 acc[D::MT][D::NB];
@@ -647,34 +693,21 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
   }
   const float* const a0 =
       dp + (16 * wave * D::MT + (lane & 15)) * kDpTok + 8 * (lane >> 4);
-  float vr[U][8];
-  float ar[D::MT][8];
-  auto load_v = [&](uint32_t s) {
-    const Slab in = make_slab(v, s * kDwTok, ntok, H, L, magic);
+  // Two sets of a step's operands where the registers allow: the loads of step
+  // s + 3 are issued after step s and first used after step s + 1.
+  float va[U][8], vb[U][8], ra[D::MT][8], rb[D::MT][8];
+  auto load_v = [&](float (&vr)[U][8], uint32_t s) {  // a lane takes one channel: whole lines
+    const __amdgpu_buffer_rsrc_t in = make_token_rows(v, s * kDwTok, ntok, H);
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const int u = threadIdx.x + i * TH;
-      const uint32_t n = s * kDwTok + 8 * (u & 3);
-      const uint32_t c = (uint32_t)(nb * NC + (u >> 2)) * L - in.first;
-      const bool on = kUnits % TH == 0 || u < kUnits;
-      if constexpr (VEC) {  // L % 4 == 0: four tokens from a multiple of four lie in one row
+      const uint32_t o =
+          kUnits % TH == 0 || u < kUnits ? 4 * (8 * (u / NC) * H + nb * NC + u % NC) : kOob;
 #pragma unroll
-        for (int e = 0; e < 8; e += 4) {
-          const float4 f =
-              buf_load4(in.r, on ? 4 * (token_base(n + e, H, L, magic) + c) : kOob, 0);
-          vr[i][e] = f.x;
-          vr[i][e + 1] = f.y;
-          vr[i][e + 2] = f.z;
-          vr[i][e + 3] = f.w;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          vr[i][e] = buf_load1(in.r, on ? 4 * (token_base(n + e, H, L, magic) + c) : kOob, 0);
-      }
+      for (int e = 0; e < 8; ++e) vr[i][e] = buf_load1(in, o, 4 * e * H);
     }
   };
-  auto load_a = [&](uint32_t s) {
+  auto load_a = [&](float (&ar)[D::MT][8], uint32_t s) {
 #pragma unroll
     for (int m = 0; m < D::MT; ++m) {
       const float* p = a0 + 16 * m * kDpTok + (size_t)s * (2 * H * kDpTok);
@@ -690,8 +723,8 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
       ar[m][7] = f1.w;
     }
   };
-  // gelu and split of the values held in vr into a stage
-  auto store_v = [&](__bf16* st) {
+  // gelu and split of a set's values into a stage
+  auto store_v = [&](const float (&vr)[U][8], __bf16* st) {
 #pragma unroll
     for (int i = 0; i < U; ++i) {
       const int u = threadIdx.x + i * TH;
@@ -701,7 +734,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
       bf16x8 hi, mid, lo;
       split3_bf16x8(g, hi, mid, lo);
       if (kUnits % TH == 0 || u < kUnits) {
-        __bf16* d = st + (u >> 2) * D::CS + 8 * (u & 3);
+        __bf16* d = st + (u % NC) * D::CS + 8 * (u / NC);
         *reinterpret_cast<bf16x8*>(d) = hi;
         *reinterpret_cast<bf16x8*>(d + NC * D::CS) = mid;
         *reinterpret_cast<bf16x8*>(d + 2 * NC * D::CS) = lo;
@@ -709,7 +742,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     }
   };
   bf16x8 a[D::MT][3], an[D::MT][3];
-  auto split_a = [&](bf16x8 (&o)[D::MT][3]) {
+  auto split_a = [&](const float (&ar)[D::MT][8], bf16x8 (&o)[D::MT][3]) {
 #pragma unroll
     for (int m = 0; m < D::MT; ++m) {
 #pragma unroll
@@ -717,14 +750,19 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
       split3_bf16x8(ar[m], o[m][0], o[m][1], o[m][2]);
     }
   };
+  auto last = [&](uint32_t s) { return s < s1 ? s : s1 - 1; };
   if (s0 < s1) {
-    load_v(s0);
-    load_a(s0);
-    store_v(sg);
-    split_a(a);
-    if (s0 + 1 < s1) {
-      load_v(s0 + 1);
-      load_a(s0 + 1);
+    load_v(va, s0);
+    load_a(ra, s0);
+    store_v(va, sg);
+    load_v(va, last(s0 + 1));
+    if constexpr (D::AHEAD) {
+      split_a(ra, a);
+      load_a(ra, last(s0 + 1));
+    }
+    if constexpr (D::DEEP) {
+      load_v(vb, last(s0 + 2));
+      load_a(rb, last(s0 + 2));
     }
   }
   auto products = [&](const __bf16* st) {
@@ -749,24 +787,38 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     }
   };
   uint32_t s = s0;
-  for (; s + 1 < s1; ++s) {
+  auto step = [&](float (&vr)[U][8], float (&ar)[D::MT][8]) {
     __syncthreads();  // one per step: the stages alternate
+    if constexpr (!D::AHEAD) {
+      split_a(ar, a);
+      load_a(ar, s + 1);
+    }
     // step s's products, and in their shadow step s + 1's gelu and splits
     // (after them in program order: LDS writes cannot pass the products' reads)
     products(sg + ((s - s0) & 1) * SZ);
-    store_v(sg + ((s + 1 - s0) & 1) * SZ);
-    split_a(an);
+    store_v(vr, sg + ((s + 1 - s0) & 1) * SZ);
+    if constexpr (D::AHEAD) split_a(ar, an);
     __builtin_amdgcn_sched_barrier(0);
-    const uint32_t ahead = s + 2 < s1 ? s + 2 : s1 - 1;
-    load_v(ahead);
-    load_a(ahead);
+    load_v(vr, last(s + (D::DEEP ? 3 : 2)));
+    if constexpr (D::AHEAD) {
+      load_a(ar, last(s + (D::DEEP ? 3 : 2)));
 #pragma unroll
-    for (int m = 0; m < D::MT; ++m)
+      for (int m = 0; m < D::MT; ++m)
 #pragma unroll
-      for (int p = 0; p < 3; ++p) a[m][p] = an[m][p];
+        for (int p = 0; p < 3; ++p) a[m][p] = an[m][p];
+    }
+    ++s;
+  };
+  while (s + 1 < s1) {
+    step(va, ra);
+    if constexpr (D::DEEP) {
+      if (s + 1 >= s1) break;
+      step(vb, rb);
+    }
   }
   if (s < s1) {
     __syncthreads();
+    if constexpr (!D::AHEAD) split_a(ra, a);
     products(sg + ((s - s0) & 1) * SZ);
   }
   float* const dst = part + (size_t)range * (2 * H * H + 2 * H);
@@ -785,7 +837,8 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
           const uint32_t e1 = s1 * kDwTok < ntok ? s1 * kDwTok : ntok;
 #pragma unroll 1
           for (uint32_t k = s0 * kDwTok; k < e1; ++k)
-            s = fmaf(dp[(size_t)(k / kDpTok) * (2 * H * kDpTok) + c * kDpTok + k % kDpTok], gelu_f(v[token_base(k, H, L, magic) + (uint32_t)h * L]), s);
+            s = fmaf(dp[(size_t)(k / kDpTok) * (2 * H * kDpTok) + c * kDpTok + k % kDpTok],
+                     gelu_f(v[(size_t)k * H + h]), s);
         }
         dst[(size_t)c * H + h] = s;
       }

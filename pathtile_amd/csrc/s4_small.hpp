@@ -1,6 +1,6 @@
 // s4_small.hpp — the S4ConvD block's kernels besides the tail: taps and split
-// weights, the taps' gradient, transposes, and the reduction of the weight
-// gradient's partials. Included by s4_block.hip alone.
+// weights, the taps' gradient, the reduction of the weight gradient's partials,
+// and the model's ends. Included by s4_block.hip alone.
 
 #pragma once
 
@@ -213,87 +213,6 @@ __global__ __launch_bounds__(kPrepThreads) void s4_taps_grad_kernel(
   if (tid == 0) {
     d_log_dt[h] = ddt_sum;
     d_skip[h] = sdk[L / 2];
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Transposes of whole samples, [L][H] <-> [H][L]; both sides move 16-byte
-// pieces (dwords where L % 4 != 0) through one LDS tile per workgroup with an
-// odd row stride. ADD: the [L][H] result also gets `add` (the residual
-// gradient). Bound by HBM: one read and one write of the tensor.
-// ---------------------------------------------------------------------------
-constexpr int kTransThreads = 256;
-
-template <bool VEC>
-__global__ __launch_bounds__(kTransThreads) void s4_transpose_kernel(
-    const float* __restrict__ x, float* __restrict__ out, int B, int H, int L) {
-  extern __shared__ float tile[];  // [L][S]
-  const int S = H + 1, n4 = L * H / 4, h4 = H / 4;
-  for (int b = blockIdx.x; b < B; b += gridDim.x) {
-    const float* src = x + (size_t)b * L * H;
-    float* dst = out + (size_t)b * L * H;
-    for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-      const float4 v = reinterpret_cast<const float4*>(src)[i];
-      const int t = i / h4, c = 4 * (i - t * h4);
-      float* p = tile + t * S + c;
-      p[0] = v.x;
-      p[1] = v.y;
-      p[2] = v.z;
-      p[3] = v.w;
-    }
-    __syncthreads();
-    if constexpr (VEC) {
-      const int l4 = L / 4;
-      for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-        const int c = i / l4, t = 4 * (i - c * l4);
-        const float* p = tile + t * S + c;
-        reinterpret_cast<float4*>(dst)[i] = float4{p[0], p[S], p[2 * S], p[3 * S]};
-      }
-    } else {
-      for (int i = threadIdx.x; i < L * H; i += kTransThreads) {
-        const int c = i / L, t = i - c * L;
-        dst[i] = tile[t * S + c];
-      }
-    }
-    __syncthreads();
-  }
-}
-
-template <bool VEC>
-__global__ __launch_bounds__(kTransThreads) void s4_transpose_add_kernel(
-    const float* __restrict__ d, const float* __restrict__ add, float* __restrict__ out, int B,
-    int H, int L) {
-  extern __shared__ float tile[];
-  const int S = H + 1, n4 = L * H / 4, h4 = H / 4;
-  for (int b = blockIdx.x; b < B; b += gridDim.x) {
-    const float* src = d + (size_t)b * L * H;
-    if constexpr (VEC) {
-      const int l4 = L / 4;
-      for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-        const float4 v = reinterpret_cast<const float4*>(src)[i];
-        const int c = i / l4, t = 4 * (i - c * l4);
-        float* p = tile + t * S + c;
-        p[0] = v.x;
-        p[S] = v.y;
-        p[2 * S] = v.z;
-        p[3 * S] = v.w;
-      }
-    } else {
-      for (int i = threadIdx.x; i < L * H; i += kTransThreads) {
-        const int c = i / L, t = i - c * L;
-        tile[t * S + c] = src[i];
-      }
-    }
-    __syncthreads();
-    const float4* a4 = reinterpret_cast<const float4*>(add + (size_t)b * L * H);
-    float4* o4 = reinterpret_cast<float4*>(out + (size_t)b * L * H);
-    for (int i = threadIdx.x; i < n4; i += kTransThreads) {
-      const int t = i / h4, c = 4 * (i - t * h4);
-      const float* p = tile + t * S + c;
-      const float4 a = a4[i];
-      o4[i] = float4{p[0] + a.x, p[1] + a.y, p[2] + a.z, p[3] + a.w};
-    }
-    __syncthreads();
   }
 }
 

@@ -9,16 +9,18 @@ namespace pt {
 
 constexpr int kNumS4H = 8;  // H = 32, 64, ..., 256
 
+using ConvClFn = void (*)(const float*, const float*, const float*, const uint8_t*, float, float*,
+                          int, int, int);
 using TailFwdFn = void (*)(const float*, const float*, const __bf16*, const float*, const float*,
-                           float*, float*, uint32_t, uint32_t, uint32_t, uint32_t);
+                           float*, float*, uint32_t, uint32_t);
 using TailBwdFn = void (*)(const float*, const float*, const float*, const uint8_t*, float,
                            const __bf16*, const float*, float*, float*, uint32_t, uint32_t, uint32_t,
                            uint32_t);
-using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t, uint32_t,
-                      uint32_t);
+using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t);
 
+extern const ConvClFn kConvCl[3][6];  // [forward, dx, forward with mask][row bucket 8, ..., 48]
 extern const TailFwdFn kTailFwd[kNumS4H];
-extern const TailBwdFn kTailBwd[kNumS4H];
-extern const DwFn kDw[kNumS4H][2];  // [16-byte loads]
+extern const TailBwdFn kTailBwd[2][kNumS4H];  // [dropout mask]
+extern const DwFn kDw[kNumS4H];
 
 }  // namespace pt

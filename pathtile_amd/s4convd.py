@@ -164,20 +164,30 @@ def _size_query(fn: str, *args: int) -> int:
     return int(out.value)
 
 
-def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight,
-               backward: bool):
-    """Taps, split projection, transposed input and the convolution's output:
-    (prep, xt, u), xt and u [B, H, L]."""
+def _dropout_mask(x: torch.Tensor, p: float) -> torch.Tensor | None:
+    """The mask that the dropout module draws for the convolution's output in
+    its [B, H, L] shape: PyTorch's own draw for a tensor of that shape, whose
+    values (here the input's) it does not depend on."""
+    if p == 0.0:
+        return None
+    B, L, H = x.shape
+    return torch.native_dropout(x.detach().view(B, H, L), p, True)[1]
+
+
+def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask,
+               scale: float, backward: bool):
+    """Taps and split projection (prep) and the convolution's output after
+    dropout, v [B, L, H]."""
     runtime = get_runtime()
     runtime._check_open()
     B, L, H = x.shape
     prep = torch.empty(_size_query("pt_s4_block_prep_values", H, L), device=x.device)
-    xt, u = torch.empty((2, B, H, L), device=x.device).unbind(0)
+    v = torch.empty_like(x)
     _call(runtime._lib.pt_s4_block_mix_f32, x.device,
           _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
-          _ptr(skip), _ptr(weight), _ptr(prep), _ptr(xt), _ptr(u), B, H, L, c_re.shape[1],
-          int(backward), runtime.waves_per_block, runtime._rows_algo_id)
-    return prep, xt, u
+          _ptr(skip), _ptr(weight), None if mask is None else _ptr(mask), scale, _ptr(prep),
+          _ptr(v), B, H, L, c_re.shape[1], int(backward))
+    return prep, v
 
 
 def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias,
@@ -193,27 +203,25 @@ def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias,
 
 class S4BlockFused(torch.autograd.Function):
     """``S4ConvBlock.forward`` as one function of the input and the block's
-    parameters: transposes, taps, convolution with the skip term, dropout,
-    GELU, projection, GLU and residual. Dropout's mask is PyTorch's own draw
-    for a tensor of the convolution's shape, as the separate module draws it."""
+    parameters: taps, convolution with the skip term, dropout, GELU,
+    projection, GLU and residual, all in [B, L, H]."""
 
     @staticmethod
     def forward(ctx: Any, x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, p: float):
-        prep, xt, v = _fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, True)
-        mask = None
-        if p > 0.0:
-            v, mask = torch.native_dropout(v, p, True)
+        mask = _dropout_mask(x, p)
+        ctx.scale = 1.0 / (1.0 - p)
+        prep, v = _fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask,
+                             ctx.scale, True)
         q = torch.empty((2, *x.shape), device=x.device)
         y = _fused_tail(v, x, prep, weight, bias, q)
         ctx.save_for_backward(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-                              prep, xt, v, q, mask)
-        ctx.scale = 1.0 / (1.0 - p)
+                              prep, v, q, mask)
         return y
 
     @staticmethod
     def backward(ctx: Any, gy: torch.Tensor):
         (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-         prep, xt, v, q, mask) = ctx.saved_tensors
+         prep, v, q, mask) = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():  # create_graph: differentiate the composition
             return _composed_grads(ctx, gy, mask)
@@ -227,18 +235,17 @@ class S4BlockFused(torch.autograd.Function):
             if taps else [None] * 6
         proj = need[7] or need[8]
         gw, gb = (torch.empty_like(weight), torch.empty_like(bias)) if proj else (None, None)
-        nbytes = _size_query("pt_s4_block_bwd_workspace_bytes", B, H, L, runtime.bwdk_block)
+        nbytes = _size_query("pt_s4_block_bwd_workspace_bytes", B, H, L)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
 
         def opt(t):
             return None if t is None else _ptr(t)
 
         _call(runtime._lib.pt_s4_block_bwd_f32, x.device,
-              _ptr(gy), _ptr(xt), _ptr(v), _ptr(q), opt(mask), ctx.scale, _ptr(prep),
+              _ptr(gy), _ptr(x), _ptr(v), _ptr(q), opt(mask), ctx.scale, _ptr(prep),
               _ptr(weight), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
               opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
-              c_re.shape[1], runtime.dx_waves_per_block, runtime._rows_algo_id,
-              runtime.bwdk_block)
+              c_re.shape[1])
         grads = [gx, gp[5], *gp[:5], gw, gb]
         return (*(g if n else None for g, n in zip(grads, need)), None)
 
@@ -431,9 +438,8 @@ class S4ConvBlock(nn.Module):
                                             or any(t.requires_grad for t in params)):
                 return S4BlockFused.apply(x, *params, p)
             skip, *kernel, weight, bias = params
-            prep, _, v = _fused_mix(x, skip, *kernel, weight, False)
-            if p > 0.0:
-                v = torch.native_dropout(v, p, True)[0]
+            mask = _dropout_mask(x, p)
+            prep, v = _fused_mix(x, skip, *kernel, weight, mask, 1.0 / (1.0 - p), False)
             return _fused_tail(v, x, prep, weight, bias)
         x_hl = x.transpose(1, 2).contiguous()
         y = self.kernel_layer(x_hl, self.skip)

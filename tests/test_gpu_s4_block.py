@@ -100,10 +100,12 @@ def test_fused_block_many_tiles_per_workgroup():
     _check(got, ref, names)
 
 
-def test_fused_block_dropout_draws_the_modules_mask():
+@pytest.mark.parametrize("B,H,L", [(33, 96, 29), (17, 32, 48), (5, 256, 36), (9, 160, 3)])
+def test_fused_block_dropout_draws_the_modules_mask(B, H, L):
     """Training with dropout: the mask of the separate module under the same
-    seed, in the output and the gradients."""
-    block, x, gy = _make(33, 96, 29, 16, p=0.3)
+    seed, in the output and the gradients (whole dwords of mask bytes and
+    single ones)."""
+    block, x, gy = _make(B, H, L, 16, p=0.3)
     block.cuda().train()
     torch.manual_seed(5)
     got = _grads(block, x.cuda(), gy.cuda())
