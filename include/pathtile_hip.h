@@ -183,6 +183,23 @@ int pt_dwconv1d_dk_det_f32(const float* dy, const float* x, float* dk,
                            void* stream);
 
 /*
+ * Both gradients: pt_dwconv1d_dx_f32_algo and pt_dwconv1d_dk_det_f32, or one
+ * kernel that reads dy once for both (the FP32 matrix cores' sums; dk
+ * deterministic as there, in its own order). one_pass: PT_BWD_AUTO takes the
+ * one kernel where it is faster, with H % 8 == 0, 16-byte aligned tensors,
+ * algo not PT_ROWS_VALU and no PATHTILE_* kernel choice set; PT_BWD_SEPARATE
+ * never. The workspace serves either.
+ */
+#define PT_BWD_AUTO 0
+#define PT_BWD_SEPARATE 1
+int pt_dwconv1d_bwd_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
+                                    size_t* bytes);
+int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* dx,
+                        float* dk, void* workspace, size_t workspace_bytes, int B, int H,
+                        int L, int K, int waves_per_block, int algo,
+                        int threads_per_block, int one_pass, void* stream);
+
+/*
  * Deterministic weight gradient that allocates nothing and takes no
  * workspace. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving

@@ -32,6 +32,10 @@ PT_ROWS_AUTO = 0
 PT_ROWS_VALU = 1
 PT_ROWS_MATRIX = 2
 
+# pt_dwconv1d_bwd_f32's one_pass
+PT_BWD_AUTO = 0
+PT_BWD_SEPARATE = 1
+
 PT_KERNEL_FWD = 0
 PT_KERNEL_DX = 1
 PT_KERNEL_DK = 2
@@ -63,6 +67,10 @@ SIGNATURES = {
         _i, [_vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _vp]
     ),
     "pt_dwconv1d_dk_det_f32_noalloc": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "pt_dwconv1d_bwd_workspace_bytes": (_i, [_i, _i, _i, _i, _i, _szp]),
+    "pt_dwconv1d_bwd_f32": (
+        _i, [_vp] * 6 + [ctypes.c_size_t] + [_i] * 8 + [_vp]
+    ),
     "pt_dwconv1d_fwd_bf16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "pt_dwconv1d_dx_bf16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "pt_dwconv1d_dk_atomic_bf16": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp]),

@@ -13,6 +13,7 @@
 #include <atomic>
 #include <mutex>
 
+#include "dwconv1d_bwd.hpp"
 #include "dwconv1d_host.hpp"
 #include "dwconv1d_kernels.hpp"
 #include "dwconv1d_tables.hpp"
@@ -1150,6 +1151,61 @@ static int dk_det_launch(const float* dy, const float* x, float* dk,
   return launch((const void*)&dk_reduce_kernel, grid, 256, 0, stream, args);
 }
 
+// --- one-pass backward -------------------------------------------------------
+// dX and dK from one read of dY (dwconv_bwd_cg_kernel), one 8-channel
+// workgroup per CU. Served wherever the channel-group dX is: H % 8 == 0 and
+// 16-byte aligned tensors, any L. One pass / separate with inputs rotated past
+// the MALL: B16384 H128 L48 K48 0.85, B32768 H256 L48 K4 0.83, B16384 H128 L4
+// K4 0.74, L16 K16 0.80, L32 K32 0.81, B60000 H8 L24 K24 0.56, B1000 H96 L37
+// K48 0.85, B64 H16 L48 K48 0.96; bwd_cg_wins has the exception.
+static bool bwd_cg_ok(int H, int L, const void* gy, const void* x, const void* gx) {
+  return rows_cg_ok(H, L, gy, gx) && aligned(x, 16) &&
+         bwd_cg_lds_bytes(L, 16 * (mfma_index(L) + 1)) <= (size_t)max_lds_per_block();
+}
+
+// Ranges: two workgroups per CU where they fit (rows of up to 16 columns by
+// registers: 128 a lane at 32 columns spilled, 280 against 142 us at B16384
+// H128 L32 K32) and get at least kRowsCgMinSteps steps each.
+static int bwd_cg_ranges(int B, int H, int L) {
+  const int lmax = 16 * (mfma_index(L) + 1);
+  const long long ngroups = H / kRowsCgWaves;
+  const long long tsteps = ((long long)B + kRowsCgStep - 1) / kRowsCgStep;
+  const int fit = blocks_per_cu((const void*)kBwdCg[0][L % 4 == 0][mfma_index(L)],
+                                kRowsCgWaves * kWave, bwd_cg_lds_bytes(L, lmax));
+  int per_cu = fit < 2 ? 1 : 2;
+  if (per_cu == 2 && tsteps < (long long)kRowsCgMinSteps * (num_cus() * 2 / ngroups)) per_cu = 1;
+  long long nr = (long long)num_cus() * per_cu / ngroups;
+  if (nr > tsteps) nr = tsteps;
+  return nr < 1 ? 1 : (int)nr;
+}
+
+// Few taps leave the separate dX without the band's padding; with rows of the
+// 48-column bucket (one workgroup per CU by LDS) and fewer than four steps a
+// range, where prologue and epilogue count, that was worth up to 10% (one pass
+// / separate at K = 4: B300 H264 L40 1.11, B800 H64 L40 1.05, B100 H512 L48 1.02;
+// from five steps on 0.87-0.95, at K = L 0.80-0.92 with any number).
+static bool bwd_cg_wins(int B, int H, int L, int K) {
+  return K >= 8 || L <= 32 ||
+         (long long)B >= 4LL * kRowsCgStep * bwd_cg_ranges(B, H, L);
+}
+
+static int bwd_cg_launch(const float* gy, const float* x, const float* w, float* gx, float* gk,
+                         float* partials, int B, int H, int L, int K, void* stream) {
+  const BwdCgFn fn = kBwdCg[!rows_plain_loads(B, H, L)][L % 4 == 0][mfma_index(L)];
+  int nranges = bwd_cg_ranges(B, H, L);
+  const long long nb = (long long)(H / kRowsCgWaves) * nranges;
+  if (nb >= (1LL << 31)) return PT_ERR_SHAPE;
+  uint32_t nblocks = (uint32_t)nb;
+  void* args[] = {&gy, &x, &w, &gx, &partials, &B, &H, &L, &K, &nranges, &nblocks};
+  const int st = launch((const void*)fn, nblocks, kRowsCgWaves * kWave,
+                        bwd_cg_lds_bytes(L, 16 * (mfma_index(L) + 1)), stream, args);
+  if (st != PT_OK) return st;
+  int ncoef = H * K;
+  const float* cp = partials;
+  void* rargs[] = {&cp, &gk, &ncoef, &nranges};
+  return launch((const void*)&dk_reduce_kernel, (uint32_t)((ncoef + 3) / 4), 256, 0, stream, rargs);
+}
+
 static const void* kernel_for(int kernel_id, int L, int K) {
   if (L < 1 || L > kMaxL || K < 1 || K > kMaxK) return nullptr;
   const int li = lbucket_index(L), ki = kbucket_index(K);
@@ -1296,6 +1352,41 @@ int pt_dwconv1d_dk_det_f32(const float* dy, const float* x, float* dk,
   if (!pt::aligned(workspace, 4)) return PT_ERR_ALIGN;
   return pt::dk_det_launch(dy, x, dk, (float*)workspace, B, H, L, K,
                            threads_per_block, g, stream);
+}
+
+int pt_dwconv1d_bwd_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
+                                    size_t* bytes) {
+  const int st = pt_dwconv1d_dk_det_workspace_bytes(B, H, L, K, threads_per_block, bytes);
+  if (st != PT_OK || B == 0 || H < pt::kRowsCgWaves || H % pt::kRowsCgWaves != 0) return st;
+  const size_t one = (size_t)H * K * pt::bwd_cg_ranges(B, H, L) * sizeof(float);
+  if (*bytes < one) *bytes = one;
+  return PT_OK;
+}
+
+int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* dx, float* dk,
+                        void* workspace, size_t workspace_bytes, int B, int H, int L, int K,
+                        int waves_per_block, int algo, int threads_per_block, int one_pass,
+                        void* stream) {
+  if (one_pass < PT_BWD_AUTO || one_pass > PT_BWD_SEPARATE) return PT_ERR_CONFIG;
+  int st = pt::check_shape(B, H, L, K);
+  if (st != PT_OK) return st;
+  // A caller who asked for the reference's chain, or for one kernel family
+  // through the environment, gets the separate launches.
+  if (one_pass != PT_BWD_SEPARATE && B > 0 && H > 0 && pt::valid_wpb(waves_per_block) &&
+      pt::valid_dk_threads(threads_per_block) && algo != PT_ROWS_VALU &&
+      (algo == PT_ROWS_AUTO || algo == PT_ROWS_MATRIX) && !getenv("PATHTILE_ROWS_ALGO") &&
+      !getenv("PATHTILE_ROWS_CHANNELS") && !getenv("PATHTILE_DK_ALGO") && dy && x && w && dx && dk &&
+      pt::aligned(w, 4) && pt::aligned(dk, 4) && pt::bwd_cg_ok(H, L, dy, x, dx) &&
+      pt::bwd_cg_wins(B, H, L, K)) {
+    const size_t need = (size_t)H * K * pt::bwd_cg_ranges(B, H, L) * sizeof(float);
+    if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
+    if (!pt::aligned(workspace, 4)) return PT_ERR_ALIGN;
+    return pt::bwd_cg_launch(dy, x, w, dx, dk, (float*)workspace, B, H, L, K, stream);
+  }
+  st = pt_dwconv1d_dx_f32_algo(dy, w, dx, B, H, L, K, waves_per_block, algo, stream);
+  if (st != PT_OK) return st;
+  return pt_dwconv1d_dk_det_f32(dy, x, dk, workspace, workspace_bytes, B, H, L, K,
+                                threads_per_block, stream);
 }
 
 int pt_dwconv1d_dk_det_f32_noalloc(const float* dy, const float* x, float* dk,

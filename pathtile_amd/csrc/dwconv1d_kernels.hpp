@@ -1532,7 +1532,7 @@ __host__ __device__ constexpr size_t cg_lds_bytes(int lmax, int wpb, int L,
 // Epilogue shared by the channel-group DK kernels. Per wave: D_c through
 // the wave's own LDS tile (the stages are free after the kernel's last
 // barrier), then lane j < K sums D_c[t][t + j - p] over t in [t0, t1) in
-// four fixed-order partial sums, all reads issued at once (the t loop is
+// NS fixed-order partial sums, all reads issued at once (the t loop is
 // unrolled over the bucket, out-of-range terms masked). The workgroup's
 // channels are consecutive, so its hc x K tap sums are one contiguous block
 // of dk: they are collected in LDS and added with one coalesced atomic per
@@ -1540,7 +1540,7 @@ __host__ __device__ constexpr size_t cg_lds_bytes(int lmax, int wpb, int L,
 // and channel, which contended badly at small K). det: write the sums as
 // partials [h][j][nranges] instead. CL: dk is [K][H] (the channels-last
 // layout's dw), whose hc channels of one tap are contiguous; atomics only.
-template <int LMAX, bool CL = false, int CPW = kCgChannelsPerWave>
+template <int LMAX, bool CL = false, int CPW = kCgChannelsPerWave, int NS = 4>
 __device__ __forceinline__ void dk_cg_epilogue(
     const f32x4 (&acc)[CPW][LMAX / 16][LMAX / 16], float* lds,
     float* __restrict__ dst, int wave, int wpb, int g, int r, int hc, int L,
@@ -1569,7 +1569,9 @@ __device__ __forceinline__ void dk_cg_epilogue(
       const int m = j - (K >> 1);
       const int t0 = max(0, -m);
       const int t1 = min(L, L - m);
-      float v4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      float vs[NS];
+#pragma unroll
+      for (int n = 0; n < NS; ++n) vs[n] = 0.0f;
 #pragma unroll
       for (int t = 0; t < G::dim; ++t) {
         // D_c[t][t + m] = dt[m + t * (dstride + 1)]; masked terms read a
@@ -1577,9 +1579,13 @@ __device__ __forceinline__ void dk_cg_epilogue(
         int idx = m + t * (G::dstride + 1);
         idx = idx < 0 ? 0 : (idx < G::dim * G::dstride ? idx : G::dim * G::dstride - 1);
         const float d = dt[idx];
-        v4[t & 3] += (t >= t0 && t < t1) ? d : 0.0f;
+        vs[t % NS] += (t >= t0 && t < t1) ? d : 0.0f;
       }
-      const float v = (v4[0] + v4[1]) + (v4[2] + v4[3]);
+#pragma unroll
+      for (int n = 1; n < NS; n *= 2)
+#pragma unroll
+        for (int e = 0; e < NS; e += 2 * n) vs[e] += vs[e + n];
+      const float v = vs[0];
       if (det) {
         dst[((size_t)(g * hc + hl) * K + j) * (size_t)nranges + r] = v;
       } else {

@@ -69,6 +69,10 @@ using DkBf16Fn = void (*)(const uint16_t*, const uint16_t*, float*, int, int,
 extern const RowsCgBf16Fn kRowsCgTableBf16[2][2][3];
 // 8-channel groups with plain input loads: [dx][row bucket]
 extern const RowsCgBf16Fn kRowsCgTableBf16PL[2][3];
+// one-pass dX + dK: [non-temporal loads][L % 4 == 0][row bucket 16, 32, 48]
+using BwdCgFn = void (*)(const float*, const float*, const float*, float*, float*, int, int, int,
+                         int, int, uint32_t);
+extern const BwdCgFn kBwdCg[2][2][3];
 using DkClFn = void (*)(const float*, const float*, float*, int, int, int, int,
                        int, uint32_t, int);
 extern const DkClFn kDkClTable[3];

@@ -602,6 +602,30 @@ class HipWarpRuntime:
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_det", launch, {"B": B, "H": H, "L": L, "K": K})
 
+    def launch_backward(self, gy: torch.Tensor, x: torch.Tensor, k: torch.Tensor,
+                        gx: torch.Tensor, gk: torch.Tensor) -> None:
+        """dX and the deterministic dK in one call of the library, which reads
+        gy once for both where its one-pass kernel serves (pt_dwconv1d_bwd_f32);
+        with KERNEL_EVENTS recording, the two launches that it names."""
+        self._check_open()
+        B, H, L, K = self._check_shapes(gy, k)
+        if KERNEL_EVENTS.enabled:
+            self.launch_bwd_input(gy, k, gx)
+            self.launch_bwd_weight_deterministic(gy, x, gk, K)
+            return
+        if gx.shape != gy.shape or gx.dtype != torch.float32 or gx.device != gy.device:
+            raise ValueError("gx must be a float32 tensor shaped like gy on gy's device")
+        self._check_bwd_weight(gy, x, gk, K)
+        self._require_contiguous(k, gx)
+        out = ctypes.c_size_t(0)
+        st = self._lib.pt_dwconv1d_bwd_workspace_bytes(B, H, L, K, self.bwdk_block,
+                                                       ctypes.byref(out))
+        _lib.check(st, "pt_dwconv1d_bwd_workspace_bytes")
+        ws = self._get_workspace(out.value, x.device)
+        _call(self._lib.pt_dwconv1d_bwd_f32, x.device,
+              _ptr(gy), _ptr(x), _ptr(k), _ptr(gx), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K,
+              self.dx_waves_per_block, self._rows_algo_id, self.bwdk_block, _lib.PT_BWD_AUTO)
+
     # ------------------------------------------------------------- BF16 I/O
     # No counterpart in the reference (FP32 only): bfloat16 activations and
     # gradients, FP32 taps and dK, FP32 accumulation on the matrix cores.
@@ -928,13 +952,16 @@ class DepthConvAmpere(torch.autograd.Function):
         if tuple(gy_c.shape) != (B, H, L):
             raise ValueError("Unexpected gradient shape")
         gx = torch.empty_like(x_c)
-        runtime.launch_bwd_input(gy_c, k_c, gx)
         # The reference zero-fills gk and adds into it with atomics
-        # (:890-893). The two-pass dK overwrites gk instead: no memset, a
+        # (:890-893). The deterministic dK overwrites gk instead: no memset, a
         # fixed summation order (reproducible gradients), and on MI355X the
         # same time as zero-fill + atomics.
         gk = torch.empty_like(k_c)
-        runtime.launch_bwd_weight_deterministic(gy_c, x_c, gk, K)
+        if type(runtime) is HipWarpRuntime:
+            runtime.launch_backward(gy_c, x_c, k_c, gx, gk)
+        else:  # a runtime of the caller's own may replace either launch
+            runtime.launch_bwd_input(gy_c, k_c, gx)
+            runtime.launch_bwd_weight_deterministic(gy_c, x_c, gk, K)
         return gx, gk
 
 

@@ -35,7 +35,7 @@ from torch import nn
 
 from . import _lib
 from .runtime import (
-    KERNEL_EVENTS, MAX_L, _call, _ptr, get_runtime, reference_depthwise_conv,
+    KERNEL_EVENTS, MAX_L, HipWarpRuntime, _call, _ptr, get_runtime, reference_depthwise_conv,
 )
 
 
@@ -76,6 +76,12 @@ class DepthConvSkipAmpere(torch.autograd.Function):
         B, H, L, K = ctx.params
         gy_c = gy.contiguous()
         gx = gk = gskip = None
+        if (type(runtime) is HipWarpRuntime and ctx.needs_input_grad[0]
+                and (ctx.needs_input_grad[1] or ctx.needs_input_grad[2])):
+            gx, dk = torch.empty_like(x_c), torch.empty_like(k_eff)
+            runtime.launch_backward(gy_c, x_c, k_eff, gx, dk)
+            return (gx, dk if ctx.needs_input_grad[1] else None,
+                    dk[:, K // 2].contiguous() if ctx.needs_input_grad[2] else None)
         if ctx.needs_input_grad[0]:
             gx = torch.empty_like(x_c)
             runtime.launch_bwd_input(gy_c, k_eff, gx)

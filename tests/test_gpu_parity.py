@@ -754,3 +754,53 @@ def test_runtime_rows_algo_overrides_the_environment(env, monkeypatch):
     assert oracle.normalized_max_abs(dx, oracle.dx_f64(dy, w)) < FWD_TOL
     r_valu.close()
     r_mfma.close()
+
+
+@pytest.mark.parametrize("B,H,L,K", [(1, 8, 9, 3), (16, 8, 16, 16), (17, 24, 17, 48), (250, 16, 31, 8),
+                                     (33, 40, 32, 32), (100, 8, 33, 8), (100, 8, 33, 7), (129, 104, 48, 48),
+                                     (1500, 96, 37, 48), (1400, 104, 47, 1),
+                                     (9000, 16, 20, 11), (300, 8, 4, 4), (70, 16, 2, 3), (40000, 8, 1, 1)])
+def test_one_pass_backward(rt, B, H, L, K):
+    """pt_dwconv1d_bwd_f32's one kernel against FP64 (the bars of dX and dK),
+    a repeat bit for bit, and the separate launches where they are asked for;
+    one range and many, ragged steps, every row bucket, and the rule on few taps."""
+    import ctypes
+
+    from pathtile_amd import _lib
+
+    lib = _lib.load()
+    print(f"[case] one-pass backward B={B} H={H} L={L} K={K}", flush=True)
+    x, w, dy = _inputs(B, H, L, K, seed=B + L)
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    need = ctypes.c_size_t(0)
+    assert lib.pt_dwconv1d_bwd_workspace_bytes(B, H, L, K, 128, ctypes.byref(need)) == 0
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(one_pass):
+        dx = torch.full_like(xd, float("nan"))
+        dk = torch.full((H, K), float("nan"), device="cuda")
+        ws = torch.full((need.value // 4 + 1,), float("nan"), device="cuda")
+        st = lib.pt_dwconv1d_bwd_f32(dyd.data_ptr(), xd.data_ptr(), wd.data_ptr(), dx.data_ptr(),
+                                     dk.data_ptr(), ws.data_ptr(), need.value, B, H, L, K, 4, 0,
+                                     128, one_pass, stream)
+        assert st == 0
+        return dx, dk
+
+    dx, dk = run(_lib.PT_BWD_AUTO)
+    dx2, dk2 = run(_lib.PT_BWD_AUTO)
+    assert torch.equal(dx, dx2) and torch.equal(dk, dk2)
+    assert oracle.normalized_max_abs(dx.cpu().numpy(), oracle.dx_f64(dy, w)) < FWD_TOL
+    assert oracle.normalized_max_abs(dk.cpu().numpy(), oracle.dk_f64(dy, x, K)) < DK_TOL
+    sx, sk = torch.empty_like(dx), torch.empty_like(dk)
+    rt.launch_bwd_input(dyd, wd, sx)
+    rt.launch_bwd_weight_deterministic(dyd, xd, sk, K)
+    if rt.bwdk_block == 128 and rt.dx_waves_per_block == 4:
+        px, pk = run(_lib.PT_BWD_SEPARATE)
+        assert torch.equal(px, sx) and torch.equal(pk, sk)
+        if K == 7:  # few taps, few steps: the separate launches
+            assert torch.equal(dx, sx) and torch.equal(dk, sk)
+    # an infinite dY reaches the outputs that the reference's chain gives it to
+    dyd[0, 1, L // 2] = float("inf")
+    dx, _ = run(_lib.PT_BWD_AUTO)
+    rt.launch_bwd_input(dyd, wd, sx)
+    assert torch.equal(torch.isfinite(dx), torch.isfinite(sx))
