@@ -970,13 +970,12 @@ static int bf16_dk_launch(bool det, const void* gy, const void* x, float* dst,
 }
 
 // Channels-last DK: 32-channel workgroups (16 waves of two channels, or 8
-// of four at 48 columns), one resident pass of them over the GPU (the sample ranges are the resident workgroups per
-// channel group, rounded down so no workgroup waits for a second round),
-// at most one range per 4-sample step.
-// Sample ranges of a channels-last DK call: one resident pass. Workgroups
-// that do not fit (LDS) give 0.
+// of four at 48 columns), one resident pass of them over the GPU (the sample
+// ranges are the resident workgroups per channel group, rounded down so no
+// workgroup waits for a second round), at most one range per 4-sample step; 0
+// where a workgroup does not fit (LDS).
 int dk_cl_ranges(int B, int H, int L) {
-  const DkClFn fn = kDkClTable[mfma_index(L)];
+  const DkClFn fn = kDkClTable[0][mfma_index(L)];
   const int nw = dk_cl_waves(16 * (mfma_index(L) + 1));
   const size_t lds = dk_cl_lds_bytes(16 * (mfma_index(L) + 1), L, nw);
   if (lds > (size_t)max_lds_per_block()) return 0;
@@ -991,14 +990,14 @@ int dk_cl_ranges(int B, int H, int L) {
 
 static int dk_cl_launch(const float* x, const float* dy, float* dst, int B, int H, int L, int K,
                         int nranges, int det, void* stream) {
-  const DkClFn fn = kDkClTable[mfma_index(L)];
+  const DkClFn fn = kDkClTable[det][mfma_index(L)];
   const int nw = dk_cl_waves(16 * (mfma_index(L) + 1));
   const size_t lds = dk_cl_lds_bytes(16 * (mfma_index(L) + 1), L, nw);
   const long long nb = (long long)(H / kClChannels) * nranges;
   if (nranges < 1) return PT_ERR_CONFIG;
   if (nb >= (1LL << 31)) return PT_ERR_SHAPE;
   uint32_t nblocks = (uint32_t)nb;
-  void* args[] = {&x, &dy, &dst, &B, &H, &L, &K, &nranges, &nblocks, &det};
+  void* args[] = {&x, &dy, &dst, &B, &H, &L, &K, &nranges, &nblocks};
   return launch((const void*)fn, nblocks, (uint32_t)(nw * kWave), lds, stream, args);
 }
 

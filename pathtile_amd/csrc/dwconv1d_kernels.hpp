@@ -1975,7 +1975,7 @@ __global__ __launch_bounds__(512) void dwconv_dk_bf16mma_kernel(
 // of a tile hit 16 distinct banks, and the sample stride is padded to
 // 16 (mod 32) floats so the four 16-lane groups of a wave (four samples)
 // use disjoint banks. Steps are 4 samples (the FP32 MFMA K); the epilogue
-// is the shared one with the [K][H] output, or with det != 0 one partial per
+// is the shared one with the [K][H] output, or with DET one partial per
 // (h, j, range) for dk_reduce_kernel.
 // ---------------------------------------------------------------------------
 constexpr int kClChannels = 32;
@@ -2006,11 +2006,11 @@ __host__ __device__ constexpr size_t dk_cl_lds_bytes(int lmax, int L, int waves 
   return stages > dtile ? stages : dtile;
 }
 
-template <int LMAX, int CPW = kCgChannelsPerWave, int DEPTH = 1>
+template <int LMAX, int CPW, int DEPTH, bool DET>
 __global__ __launch_bounds__(kClChannels / CPW * kWave) void dwconv_dk_cl_kernel(
     const float* __restrict__ x, const float* __restrict__ gy,
     float* __restrict__ dw, int B, int H, int L, int K, int nranges,
-    uint32_t nblocks, int det) {
+    uint32_t nblocks) {
   using G = CgGeo<LMAX>;
   constexpr int NT = G::nt;
   constexpr int NW = kClChannels / CPW;
@@ -2166,7 +2166,7 @@ __global__ __launch_bounds__(kClChannels / CPW * kWave) void dwconv_dk_cl_kernel
     }
   }
 
-  dk_cg_epilogue<LMAX, true, CPW>(acc, lds, dw, wave, NW, g, r, HC, L, K, nranges, det, H);
+  dk_cg_epilogue<LMAX, true, CPW>(acc, lds, dw, wave, NW, g, r, HC, L, K, nranges, DET, H);
 }
 
 // ---------------------------------------------------------------------------

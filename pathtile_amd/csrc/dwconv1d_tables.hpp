@@ -74,8 +74,9 @@ using BwdCgFn = void (*)(const float*, const float*, const float*, float*, float
                          int, int, uint32_t);
 extern const BwdCgFn kBwdCg[2][2][3];
 using DkClFn = void (*)(const float*, const float*, float*, int, int, int, int,
-                       int, uint32_t, int);
-extern const DkClFn kDkClTable[3];
+                       int, uint32_t);
+// [deterministic partials][row bucket]
+extern const DkClFn kDkClTable[2][3];
 using RowsLongFn = void (*)(const float*, const float*, float*, int, int, int, int);
 using DkLongFn = void (*)(const float*, const float*, float*, int, int, int, int, int, int);
 constexpr int kNumLongLB = 5;  // long-row buckets 64, 96, 128, 160, 192
