@@ -13,8 +13,8 @@ __host__ __device__ constexpr size_t bwd_cg_lds_bytes(int L, int lmax) {
   return stages > dtile ? stages : dtile;
 }
 
-// The separate kernels move five tensor passes (dX: dY in, dX out; dK: dY and
-// x in) where four suffice; this one reads dY once. It is
+// The separate kernels move four tensor passes (dX: dY in, dX out; dK: dY and
+// x in) where three suffice; this one reads dY once. It is
 // dwconv_rows_cg_kernel's dX (8 channels, one per wave, 16-sample steps, band
 // matrix of the taps in registers, outputs through LDS) with x staged beside
 // dY and the step's dK contraction D += dY^T x after the dX products: MFMA i of
