@@ -23,9 +23,16 @@ struct Cf { float re, im; };
 __device__ __forceinline__ Cf cmul(Cf a, Cf b) {
   return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
 }
+// b scaled by a power of two to about 1 first: |b|^2 would leave FP32's range
+// where b itself is an ordinary value (below 1e-19 or above 1e19).
 __device__ __forceinline__ Cf cdiv(Cf a, Cf b) {
+  const float m = fmaxf(fabsf(b.re), fabsf(b.im));
+  int e = 0;
+  frexpf(m, &e);
+  e = m > 0.0f && m < INFINITY ? -e : 0;
+  b = {ldexpf(b.re, e), ldexpf(b.im, e)};
   const float d = 1.0f / (b.re * b.re + b.im * b.im);
-  return {(a.re * b.re + a.im * b.im) * d, (a.im * b.re - a.re * b.im) * d};
+  return {ldexpf((a.re * b.re + a.im * b.im) * d, e), ldexpf((a.im * b.re - a.re * b.im) * d, e)};
 }
 __device__ __forceinline__ Cf cexpm1(Cf a) {
   float s, c;

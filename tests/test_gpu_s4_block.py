@@ -177,6 +177,22 @@ def test_fused_block_non_finite_values_stay_in_their_windows():
         assert bool((torch.isfinite(a) == torch.isfinite(b)).all())
 
 
+@pytest.mark.parametrize("log_a_re", [-50.0, -60.0])
+def test_fused_block_poles_near_zero(log_a_re):
+    """|A|^2 below FP32's range: the taps reach their limit 2 Re sum C dt, as
+    they do to |dt A| L <= 3e-5 of it at A = -exp(-12)."""
+    block, x, _ = _make(3, 32, 48, 16)
+    block.cuda()
+    out = []
+    for a in (log_a_re, -12.0):
+        with torch.no_grad():
+            block.kernel_layer.log_A_re.fill_(a)
+            block.kernel_layer.A_im.zero_()
+            assert block._fused_inputs(x.cuda()) is not None
+            out.append(block(x.cuda()))
+    assert _rel(*out) < 1e-4
+
+
 @pytest.mark.parametrize("how", ["hook", "collector", "strided", "autocast", "channels", "gelu"])
 def test_separate_operations_still_serve(how):
     """Each condition that rules the fused passes out runs the separate
