@@ -249,6 +249,14 @@ int pt_dwconv1d_dk_det_bf16(const void* dy, const void* x, float* dk,
                             int H, int L, int K, int threads_per_block,
                             void* stream);
 
+/* Both gradients of BF16 tensors, as pt_dwconv1d_bwd_f32: one kernel that
+ * reads dy once (dx the bits of pt_dwconv1d_dx_bf16), or the two calls. */
+int pt_dwconv1d_bwd_bf16_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
+                                         size_t* bytes);
+int pt_dwconv1d_bwd_bf16(const void* dy, const void* x, const float* w, void* dx,
+                         float* dk, void* workspace, size_t workspace_bytes, int B, int H,
+                         int L, int K, int threads_per_block, int one_pass, void* stream);
+
 /*
  * Long rows: L up to 192 and K up to 256 (taps past the row add nothing),
  * the regime of the

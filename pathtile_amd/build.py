@@ -34,6 +34,7 @@ SOURCES = [
     "inst_dk_mfma.hip",
     "inst_dk_cg1.hip",
     "inst_bwd_cg.hip",
+    "inst_bwd_bf16.hip",
     "inst_rows_mfma.hip",
     "inst_rows_mfma_u.hip",
     "inst_bf16.hip",

@@ -1205,6 +1205,42 @@ static int bwd_cg_launch(const float* gy, const float* x, const float* w, float*
   return launch((const void*)&dk_reduce_kernel, (uint32_t)((ncoef + 3) / 4), 256, 0, stream, rargs);
 }
 
+// The same for BF16 tensors, two workgroups per CU: served wherever the two
+// kernels are, since it was faster at every size measured (one pass / separate:
+// B16384 H128 L48 K48 0.86, K4 0.88, B32768 H256 L48 0.92, B16384 H128 L32 0.78,
+// L16 0.73, L4 0.69, B1000 H96 L36 K48 0.77, B300 H264 L40 K4 0.78, B64 H16 L48
+// 0.76).
+static int bwd_bf16_ranges(int B, int H, int L) {
+  const int lmax = 16 * (mfma_index(L) + 1);
+  const long long ngroups = H / kRowsCgWaves;
+  const long long tsteps = ((long long)B + kRowsCgStep - 1) / kRowsCgStep;
+  const int fit = blocks_per_cu((const void*)kBwdBf16[0][mfma_index(L)], kRowsCgWaves * kWave,
+                                bwd_bf16_lds_bytes(L, lmax));
+  int per_cu = fit < 2 ? 1 : 2;
+  if (per_cu == 2 && tsteps < (long long)kRowsCgMinSteps * (num_cus() * 2 / ngroups)) per_cu = 1;
+  long long nr = (long long)num_cus() * per_cu / ngroups;
+  if (nr > tsteps) nr = tsteps;
+  return nr < 1 ? 1 : (int)nr;
+}
+
+static int bwd_bf16_launch(const uint16_t* gy, const uint16_t* x, const float* w, uint16_t* gx,
+                           float* gk, float* partials, int B, int H, int L, int K, void* stream) {
+  const BwdBf16Fn fn =
+      kBwdBf16[2.0 * (double)B * (double)H * (double)L > kRowsPlainLoadBytes][mfma_index(L)];
+  int nranges = bwd_bf16_ranges(B, H, L);
+  const long long nb = (long long)(H / kRowsCgWaves) * nranges;
+  if (nb >= (1LL << 31)) return PT_ERR_SHAPE;
+  uint32_t nblocks = (uint32_t)nb;
+  void* args[] = {&gy, &x, &w, &gx, &partials, &B, &H, &L, &K, &nranges, &nblocks};
+  const int st = launch((const void*)fn, nblocks, kRowsCgWaves * kWave,
+                        bwd_bf16_lds_bytes(L, 16 * (mfma_index(L) + 1)), stream, args);
+  if (st != PT_OK) return st;
+  int ncoef = H * K;
+  const float* cp = partials;
+  void* rargs[] = {&cp, &gk, &ncoef, &nranges};
+  return launch((const void*)&dk_reduce_kernel, (uint32_t)((ncoef + 3) / 4), 256, 0, stream, rargs);
+}
+
 static const void* kernel_for(int kernel_id, int L, int K) {
   if (L < 1 || L > kMaxL || K < 1 || K > kMaxK) return nullptr;
   const int li = lbucket_index(L), ki = kbucket_index(K);
@@ -1556,6 +1592,37 @@ int pt_dwconv1d_dk_det_bf16(const void* dy, const void* x, float* dk,
   const uint32_t grid = (uint32_t)((ncoef + 3) / 4);
   return pt::launch((const void*)&pt::dk_reduce_kernel, grid, 256, 0, stream,
                     args);
+}
+
+int pt_dwconv1d_bwd_bf16_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
+                                         size_t* bytes) {
+  const int st = pt_dwconv1d_dk_det_bf16_workspace_bytes(B, H, L, K, threads_per_block, bytes);
+  if (st != PT_OK || B == 0 || H == 0 || H % pt::kRowsCgWaves != 0) return st;
+  const size_t one = (size_t)H * K * pt::bwd_bf16_ranges(B, H, L) * sizeof(float);
+  if (*bytes < one) *bytes = one;
+  return PT_OK;
+}
+
+int pt_dwconv1d_bwd_bf16(const void* dy, const void* x, const float* w, void* dx, float* dk,
+                         void* workspace, size_t workspace_bytes, int B, int H, int L, int K,
+                         int threads_per_block, int one_pass, void* stream) {
+  if (one_pass < PT_BWD_AUTO || one_pass > PT_BWD_SEPARATE) return PT_ERR_CONFIG;
+  int st = pt::bf16_dk_check(B, H, L, K, threads_per_block);
+  if (st != PT_OK) return st;
+  if (one_pass == PT_BWD_AUTO && B > 0 && H > 0 && L % 4 == 0 && H % pt::kRowsCgWaves == 0 && dy &&
+      x && w && dx && dk && pt::aligned(dy, 16) && pt::aligned(x, 16) && pt::aligned(dx, 16) &&
+      pt::aligned(w, 4) && pt::aligned(dk, 4) &&
+      pt::bwd_bf16_lds_bytes(L, 16 * (pt::mfma_index(L) + 1)) <= (size_t)pt::max_lds_per_block()) {
+    const size_t need = (size_t)H * K * pt::bwd_bf16_ranges(B, H, L) * sizeof(float);
+    if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
+    if (!pt::aligned(workspace, 4)) return PT_ERR_ALIGN;
+    return pt::bwd_bf16_launch((const uint16_t*)dy, (const uint16_t*)x, w, (uint16_t*)dx, dk,
+                               (float*)workspace, B, H, L, K, stream);
+  }
+  st = pt_dwconv1d_dx_bf16(dy, w, dx, B, H, L, K, stream);
+  if (st != PT_OK) return st;
+  return pt_dwconv1d_dk_det_bf16(dy, x, dk, workspace, workspace_bytes, B, H, L, K,
+                                 threads_per_block, stream);
 }
 
 int pt_dwconv1d_fwd_long_f32(const float* x, const float* w, float* y, int B,

@@ -73,6 +73,10 @@ extern const RowsCgBf16Fn kRowsCgTableBf16PL[2][3];
 using BwdCgFn = void (*)(const float*, const float*, const float*, float*, float*, int, int, int,
                          int, int, uint32_t);
 extern const BwdCgFn kBwdCg[2][2][3];
+// the same for BF16 tensors: [non-temporal loads][row bucket]
+using BwdBf16Fn = void (*)(const uint16_t*, const uint16_t*, const float*, uint16_t*, float*, int,
+                           int, int, int, int, uint32_t);
+extern const BwdBf16Fn kBwdBf16[2][3];
 using DkClFn = void (*)(const float*, const float*, float*, int, int, int, int,
                        int, uint32_t);
 // [deterministic partials][row bucket]

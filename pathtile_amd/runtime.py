@@ -721,6 +721,28 @@ class HipWarpRuntime:
 
         (collector or KERNEL_EVENTS).launch("bwd_weight_det_bf16", launch, {"B": B, "H": H, "L": L, "K": K})
 
+    def launch_backward_bf16(self, gy: torch.Tensor, x: torch.Tensor, k: torch.Tensor,
+                             gx: torch.Tensor, gk: torch.Tensor) -> None:
+        """launch_backward for bfloat16 gy, x and gx (pt_dwconv1d_bwd_bf16)."""
+        self._check_open()
+        B, H, L, K = self._check_bf16(gy, k, "gy")
+        if KERNEL_EVENTS.enabled:
+            self.launch_bwd_input_bf16(gy, k, gx)
+            self.launch_bwd_weight_deterministic_bf16(gy, x, gk, K)
+            return
+        if gx.dtype != torch.bfloat16 or gx.shape != gy.shape or gx.device != gy.device:
+            raise ValueError("gx must be a bfloat16 tensor shaped like gy on gy's device")
+        self._check_bf16_dk(gy, x, gk, K)
+        self._require_contiguous(k, gx)
+        out = ctypes.c_size_t(0)
+        st = self._lib.pt_dwconv1d_bwd_bf16_workspace_bytes(B, H, L, K, self.bwdk_block,
+                                                            ctypes.byref(out))
+        _lib.check(st, "pt_dwconv1d_bwd_bf16_workspace_bytes")
+        ws = self._get_workspace(out.value, x.device)
+        _call(self._lib.pt_dwconv1d_bwd_bf16, x.device,
+              _ptr(gy), _ptr(x), _ptr(k), _ptr(gx), _ptr(gk), _ptr(ws), ws.numel(), B, H, L, K,
+              self.bwdk_block, _lib.PT_BWD_AUTO)
+
     def launch_bwd_weight_channels_last(self, x: torch.Tensor, gy: torch.Tensor,
                                         dw: torch.Tensor, gz: int = 1,
                                         collector: KernelEventCollector | None = None,
@@ -993,6 +1015,10 @@ class DepthConvBf16(torch.autograd.Function):
         B, H, L, K = ctx.params
         gy_c = gy.to(torch.bfloat16).contiguous()
         gx = gk = None
+        if type(runtime) is HipWarpRuntime and all(ctx.needs_input_grad):
+            gx, gk = torch.empty_like(x_c), torch.empty_like(k_c)
+            runtime.launch_backward_bf16(gy_c, x_c, k_c, gx, gk)
+            return gx, gk
         if ctx.needs_input_grad[0]:
             gx = torch.empty_like(x_c)
             runtime.launch_bwd_input_bf16(gy_c, k_c, gx)

@@ -136,6 +136,50 @@ def test_bf16_large_shape_sampled_rows(rt, shape):
     assert oracle.normalized_max_abs(g.cpu().numpy(), oracle.dk_f64(dy.float(), x.float(), K)) < DK_TOL
 
 
+@pytest.mark.parametrize("shape", [
+    (1, 8, 4, 3), (15, 8, 16, 16), (17, 24, 12, 48), (250, 16, 20, 8), (33, 40, 32, 32),
+    (100, 8, 36, 7), (129, 104, 48, 48), (1500, 96, 44, 1), (9000, 16, 28, 11), (40000, 8, 8, 9),
+    (22016, 128, 48, 40)], ids=lambda s: "B{}H{}L{}K{}".format(*s))
+def test_bf16_one_pass_backward(rt, shape):
+    """pt_dwconv1d_bwd_bf16's one kernel, from a workspace of NaN: dX the bits
+    of the separate kernel, dK at its bar and repeatable; the separate launches where
+    they are asked for; an infinite dY in the same outputs."""
+    import ctypes
+
+    from pathtile_amd import _lib
+
+    lib = _lib.load()
+    B, H, L, K = shape
+    x, w, dy = _inputs(B, H, L, K, seed=13 + B + L)
+    xd, wd, dyd = x.cuda(), w.cuda(), dy.cuda()
+    threads = 64 if H % 16 else 128
+    need = ctypes.c_size_t(0)
+    assert lib.pt_dwconv1d_bwd_bf16_workspace_bytes(B, H, L, K, 64, ctypes.byref(need)) == 0
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(one_pass):
+        dx = torch.full_like(xd, float("nan"))
+        dk = torch.full((H, K), float("nan"), device="cuda")
+        ws = torch.full((need.value // 4 + 1,), float("nan"), device="cuda")
+        assert lib.pt_dwconv1d_bwd_bf16(dyd.data_ptr(), xd.data_ptr(), wd.data_ptr(),
+                                        dx.data_ptr(), dk.data_ptr(), ws.data_ptr(), need.value,
+                                        B, H, L, K, threads, one_pass, stream) == 0
+        return dx, dk
+
+    dx, dk = run(_lib.PT_BWD_AUTO)
+    dx2, dk2 = run(_lib.PT_BWD_AUTO)
+    assert torch.equal(dx, dx2) and torch.equal(dk, dk2)
+    sx, sk = run(_lib.PT_BWD_SEPARATE)
+    assert torch.equal(dx, sx)
+    ref = torch.from_numpy(oracle.dk_f64(dy.float(), x.float(), K))
+    assert oracle.normalized_max_abs(dk.cpu().numpy(), ref.numpy()) < DK_TOL
+    err, sep = (float((t.cpu().double() - ref).norm() / ref.norm()) for t in (dk, sk))
+    print(f"[dk] one pass {err:.2e} separate {sep:.2e}", flush=True)
+    dyd[0, 1, L // 2] = float("inf")
+    dx, sx = run(_lib.PT_BWD_AUTO)[0], run(_lib.PT_BWD_SEPARATE)[0]
+    assert torch.equal(torch.isfinite(dx), torch.isfinite(sx))
+
+
 def test_bf16_layout_and_dtype_errors(rt):
     x = torch.zeros(4, 8, 18, device="cuda", dtype=torch.bfloat16)
     w = torch.zeros(8, 5, device="cuda")
