@@ -220,17 +220,19 @@ class S4BlockFused(torch.autograd.Function):
                              ctx.scale, True)
         q = torch.empty((2, *x.shape), device=x.device)
         y = _fused_tail(v, x, prep, weight, bias, q)
-        ctx.save_for_backward(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-                              prep, v, q, mask)
+        saved = (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, prep, v, q, mask)
+        ctx.forms = [_form(t) for t in saved]
+        ctx.save_for_backward(*saved)
         return y
 
     @staticmethod
     def backward(ctx: Any, gy: torch.Tensor):
-        (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-         prep, v, q, mask) = ctx.saved_tensors
+        saved = ctx.saved_tensors
         need = ctx.needs_input_grad
         if torch.is_grad_enabled():  # create_graph: differentiate the composition
-            return _composed_grads(ctx, gy, mask)
+            return _composed_grads(ctx, gy, saved[-1])
+        (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
+         prep, v, q, mask) = map(_unpacked, saved, ctx.forms)
         runtime = get_runtime()
         runtime._check_open()
         B, L, H = x.shape
@@ -308,6 +310,7 @@ class EncoderFused(torch.autograd.Function):
         y = torch.empty((B, L, H), device=x.device)
         _call(_lib.load().pt_s4_encode_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(y), B, L, n, H)
+        ctx.forms = _form(x), _form(weight)
         ctx.save_for_backward(x, weight)
         return y
 
@@ -322,6 +325,7 @@ class EncoderFused(torch.autograd.Function):
         gx = gy @ weight if need[0] else None
         gw = gb = None
         if need[1] or need[2]:
+            x, weight = map(_unpacked, (x, weight), ctx.forms)
             B, L, n = x.shape
             H = weight.shape[0]
             gy = _aligned(gy.contiguous())
@@ -344,6 +348,7 @@ class HeadFused(torch.autograd.Function):
         out = torch.empty((B, n), device=x.device)
         _call(_lib.load().pt_s4_head_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(out), B, H, L, n)
+        ctx.forms = _form(x), _form(weight)
         ctx.save_for_backward(x, weight)
         return out
 
@@ -356,6 +361,7 @@ class HeadFused(torch.autograd.Function):
             gx = nn.functional.pad((gy @ weight)[:, None, :], (0, 0, L - 1, 0)) if need[0] else None
             return (gx, gy.t() @ x[:, -1, :] if need[1] else None,
                     gy.sum(0) if need[2] else None)
+        x, weight = map(_unpacked, (x, weight), ctx.forms)
         n = weight.shape[0]
         gy = gy.contiguous()
         gx = torch.empty_like(x) if need[0] else None
@@ -370,6 +376,19 @@ class HeadFused(torch.autograd.Function):
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
     return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _form(t: torch.Tensor | None):
+    return None if t is None else (t.shape, t.dtype, t.device)
+
+
+def _unpacked(t: torch.Tensor | None, form):
+    """A saved tensor for a kernel that takes its address: a saved-tensor hook
+    may give back other strides or another alignment (copied), or another
+    shape, type or device than the `_form` it was saved in (refused)."""
+    if _form(t) != form:
+        raise RuntimeError(f"saved tensor {form} was unpacked as {_form(t)}")
+    return None if t is None else _aligned(t.contiguous())
 
 
 def _plain_linear(m: nn.Module, x: torch.Tensor, width: int) -> bool:

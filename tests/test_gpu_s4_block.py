@@ -291,3 +291,44 @@ def test_model_ends_follow_hooks_and_devices():
         again = m(x)
     assert shapes == [(5, 12, 32), (5, 12, 2)]
     assert _rel(again, out) < 1e-6
+
+
+@pytest.mark.parametrize("part", ["model", "block", "encoder"])
+@pytest.mark.parametrize("how", ["strided", "half", "host"])
+def test_saved_tensor_hooks_of_the_fused_functions(how, part):
+    """What a hook unpacks reaches the kernels whole: strided copies give the
+    same gradients, another type or device is refused."""
+    from pathtile_amd import s4convd
+
+    torch.manual_seed(5)
+    model = s4convd.Model(state_dim=16, hidden_dim=64, num_blocks=1, dropout=0.1).cuda()
+    x = torch.randn(33, 20, 64 if part == "block" else 4, device="cuda")
+    if part == "block":
+        part, model = model.blocks[0], model.blocks[0]
+    elif part == "encoder":
+        model = model.encoder
+        part = lambda x: s4convd.EncoderFused.apply(x, model.weight, model.bias)  # noqa: E731
+    else:
+        part = model
+
+    def unpack(t):
+        if how == "strided":  # every second value of a buffer
+            wide = torch.empty((*t.shape, 2), dtype=t.dtype, device=t.device)
+            wide[..., 0] = t
+            return wide[..., 0]
+        return t.to(torch.float16) if how == "half" else t.cpu()
+
+    def step(hooked):
+        torch.manual_seed(6)
+        if hooked:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t.detach().clone(), unpack):
+                out = part(x)
+        else:
+            out = part(x)
+        return torch.autograd.grad(out, tuple(model.parameters()), torch.ones_like(out))
+
+    if how == "strided":  # the same kernels on the same values: the same bits
+        assert all(torch.equal(a, b) for a, b in zip(step(True), step(False)))
+    else:
+        with pytest.raises(RuntimeError, match="was unpacked as"):
+            step(True)
