@@ -187,7 +187,7 @@ def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight
     runtime = get_runtime()
     runtime._check_open()
     B, L, H = x.shape
-    prep = torch.empty(_size_query("pt_s4_block_prep_values", H, L), device=x.device)
+    prep = x.new_empty(_size_query("pt_s4_block_prep_values", H, L))
     v = torch.empty_like(x)
     _call(runtime._lib.pt_s4_block_mix_f32, x.device,
           _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
@@ -218,7 +218,7 @@ class S4BlockFused(torch.autograd.Function):
         ctx.scale = 1.0 / (1.0 - p)
         prep, v = _fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask,
                              ctx.scale, True)
-        q = torch.empty((2, *x.shape), device=x.device)
+        q = x.new_empty((2, *x.shape))
         y = _fused_tail(v, x, prep, weight, bias, q)
         saved = (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, prep, v, q, mask)
         ctx.forms = [_form(t) for t in saved]
@@ -307,7 +307,7 @@ class EncoderFused(torch.autograd.Function):
     def forward(ctx: Any, x, weight, bias):
         B, L, n = x.shape
         H = weight.shape[0]
-        y = torch.empty((B, L, H), device=x.device)
+        y = x.new_empty((B, L, H))
         _call(_lib.load().pt_s4_encode_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(y), B, L, n, H)
         ctx.forms = _form(x), _form(weight)
@@ -329,7 +329,7 @@ class EncoderFused(torch.autograd.Function):
             B, L, n = x.shape
             H = weight.shape[0]
             gy = _aligned(gy.contiguous())
-            gw, gb = torch.empty_like(weight), torch.empty(H, device=x.device)
+            gw, gb = torch.empty_like(weight), weight.new_empty(H)
             nbytes = _size_query("pt_s4_encode_grad_workspace_bytes", B, L, n, H)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             _call(_lib.load().pt_s4_encode_grad_f32, x.device,
@@ -345,7 +345,7 @@ class HeadFused(torch.autograd.Function):
     def forward(ctx: Any, x, weight, bias):
         B, L, H = x.shape
         n = weight.shape[0]
-        out = torch.empty((B, n), device=x.device)
+        out = x.new_empty((B, n))
         _call(_lib.load().pt_s4_head_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(out), B, H, L, n)
         ctx.forms = _form(x), _form(weight)
@@ -365,7 +365,7 @@ class HeadFused(torch.autograd.Function):
         n = weight.shape[0]
         gy = gy.contiguous()
         gx = torch.empty_like(x) if need[0] else None
-        gw, gb = torch.empty_like(weight), torch.empty(n, device=x.device)
+        gw, gb = torch.empty_like(weight), weight.new_empty(n)
         nbytes = _size_query("pt_s4_head_grad_workspace_bytes", B, H, L, n)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
         _call(_lib.load().pt_s4_head_grad_f32, x.device,

@@ -332,3 +332,30 @@ def test_saved_tensor_hooks_of_the_fused_functions(how, part):
     else:
         with pytest.raises(RuntimeError, match="was unpacked as"):
             step(True)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float64])
+def test_fused_model_under_another_default_dtype(dtype):
+    """An FP32 model's step does not depend on torch's default dtype: the
+    same bits."""
+    from pathtile_amd import s4convd
+
+    torch.manual_seed(8)
+    model = s4convd.Model(state_dim=8, hidden_dim=64, output_dim=2, num_blocks=2,
+                          dropout=0.1).cuda()
+    x = torch.randn(17, 20, 4, device="cuda")
+
+    def step():
+        torch.manual_seed(9)
+        out = model(x)
+        return [out, *torch.autograd.grad(out, tuple(model.parameters()), torch.ones_like(out))]
+
+    ref = step()
+    old = torch.get_default_dtype()
+    torch.set_default_dtype(dtype)
+    try:
+        got = step()
+    finally:
+        torch.set_default_dtype(old)
+    for a, b in zip(got, ref):
+        assert a.dtype == torch.float32 and torch.equal(a, b)
