@@ -261,8 +261,11 @@ class S4BlockFused(torch.autograd.Function):
 def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
     """The block's gradients through differentiable operations on the saved
     inputs, for a backward that is itself differentiated (the convolution's
-    own backward stays first order, as its autograd function is)."""
-    inputs = ctx.saved_tensors[:9]
+    own backward stays first order, as its autograd function is). They are
+    taken at aliases: where x was computed from the same parameters, as in a
+    block applied twice, a gradient with respect to the tensors themselves
+    would follow that path too, which the engine adds by itself."""
+    inputs = [t.view_as(t) for t in ctx.saved_tensors[:9]]
     x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
     k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
     v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)

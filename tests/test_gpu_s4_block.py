@@ -359,3 +359,22 @@ def test_fused_model_under_another_default_dtype(dtype):
         torch.set_default_dtype(old)
     for a, b in zip(got, ref):
         assert a.dtype == torch.float32 and torch.equal(a, b)
+
+
+def test_fused_block_applied_twice_under_create_graph():
+    """Gradients of a block that is applied to its own output, taken with
+    create_graph: those of the separate operations."""
+    block, x, gy = _make(3, 32, 20, 8)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+    inputs = (x.requires_grad_(True), *block.parameters())
+
+    def grads():
+        return torch.autograd.grad(block(block(x)), inputs, gy, create_graph=True)
+
+    with torch.backends.cudnn.flags(enabled=False):
+        got = grads()
+        block.activation.register_forward_hook(lambda *a: None)
+        ref = grads()
+    for a, b in zip(got, ref):
+        assert _rel(a, b) < PAR_TOL

@@ -61,3 +61,52 @@ def test_buffers_are_fp32_under_any_default_dtype(calls, default_dtype, dtype):
     assert {n for n, _ in calls} == {
         "pt_s4_block_mix_f32", "pt_s4_block_tail_f32", "pt_s4_block_bwd_f32", "pt_s4_encode_f32",
         "pt_s4_encode_grad_f32", "pt_s4_head_f32", "pt_s4_head_grad_f32"}
+
+
+@pytest.fixture
+def composed(monkeypatch):
+    """Native forward passes of the block replaced by the operations they
+    fuse, and the convolution by a differentiable one."""
+    def conv(x, k, skip):
+        return s4convd.reference_depthwise_conv(x, k) + x * skip.unsqueeze(-1)
+
+    def mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask, scale, backward):
+        k = s4convd._taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
+        v = conv(x.transpose(1, 2), k, skip)
+        if mask is not None:
+            v = v * mask * scale
+        return x.new_empty(0), v.transpose(1, 2).contiguous()
+
+    def tail(v, x, prep, weight, bias, q=None):
+        z = torch.nn.functional.conv1d(torch.nn.functional.gelu(v.transpose(1, 2)), weight, bias)
+        return torch.nn.functional.glu(z, dim=1).transpose(1, 2) + x
+
+    monkeypatch.setattr(s4convd, "depthwise_conv_skip_ampere", conv)
+    monkeypatch.setattr(s4convd, "_fused_mix", mix)
+    monkeypatch.setattr(s4convd, "_fused_tail", tail)
+
+
+@pytest.mark.parametrize("applications", [1, 2, 3])
+def test_weight_tied_blocks_keep_their_gradients_under_create_graph(calls, composed, applications):
+    """One block applied several times: gradients with create_graph equal
+    those of the separate operations (FP64), and so do second derivatives."""
+    torch.manual_seed(applications)
+    B, L, H, half = 3, 7, 32, 4
+    inputs = [t.double().requires_grad_(True) for t in _block_inputs(B, L, H, half)]
+
+    def grads(block):
+        y = inputs[0]
+        for _ in range(applications):
+            y = block(y, *inputs[1:])
+        gs = torch.autograd.grad(y.square().sum(), inputs, create_graph=True)
+        # create_graph again, so that no native backward runs
+        second = torch.autograd.grad(sum(g.square().sum() for g in gs), inputs, create_graph=True)
+        return [g.detach() for g in (*gs, *second)]
+
+    def separate(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias):
+        _, v = s4convd._fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, None, 1.0,
+                                  True)
+        return s4convd._fused_tail(v, x, None, weight, bias)
+
+    for a, b in zip(grads(lambda *t: s4convd.S4BlockFused.apply(*t, 0.0)), grads(separate)):
+        assert float((a - b).norm() / b.norm()) < 1e-10
