@@ -394,16 +394,31 @@ def _unpacked(t: torch.Tensor | None, form):
     return None if t is None else _aligned(t.contiguous())
 
 
-def _plain_linear(m: nn.Module, x: torch.Tensor, width: int) -> bool:
-    """`m` is an ordinary FP32 ``nn.Linear`` with a bias for the contiguous
-    GPU tensor `x` [B, L, width], and nothing watches its call."""
-    return (type(m) is nn.Linear and type(x) is torch.Tensor and x.is_cuda and x.dim() == 3
-            and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
-            and 0 < x.numel() < 2**31 and x.shape[2] == width == m.weight.shape[1]
-            and m.bias is not None and _no_hooks(m) and _backend() == "warp"
+def _whole_linear(m: nn.Module) -> bool:
+    """`m` is an ordinary FP32 ``nn.Linear`` whose call nothing watches, with
+    one bias value per row of its weight, as the kernels read them
+    (``F.linear`` broadcasts fewer). The sizes are the tensors' own:
+    ``out_features`` does not follow a replaced weight."""
+    return (type(m) is nn.Linear and m.bias is not None and _no_hooks(m)
+            and m.weight.dim() == 2 and m.bias.shape == m.weight.shape[:1]
             and all(type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32
-                    and t.device == x.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    and t.is_contiguous() and t.data_ptr() % 16 == 0
                     for t in (m.weight, m.bias)))
+
+
+def _plain_linear(m: nn.Module, x: torch.Tensor) -> bool:
+    """`m` is a `_whole_linear` for the contiguous GPU tensor `x` [B, L, width]."""
+    return (type(x) is torch.Tensor and x.is_cuda and x.dim() == 3
+            and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
+            and 0 < x.numel() < 2**31 and _backend() == "warp" and _whole_linear(m)
+            and x.shape[2] == m.weight.shape[1]
+            and m.weight.device == x.device and m.bias.device == x.device)
+
+
+def _end_served(x: torch.Tensor, channels: int) -> bool:
+    """The ends' kernels serve `channels` channels at the columns of `x`."""
+    return (4 <= channels <= ENDS_MAX_H and channels % 4 == 0
+            and x.shape[0] * x.shape[1] * channels < 2**31)
 
 
 class S4ConvBlock(nn.Module):
@@ -499,17 +514,15 @@ class Model(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         plain = not _tracing()
         enc, dec = self.encoder, self.decoder
-        H = enc.out_features if type(enc) is nn.Linear else 0
-        if (plain and 4 <= H <= ENDS_MAX_H and H % 4 == 0 and x.dim() == 3
-                and 1 <= x.shape[2] <= ENCODER_MAX_IN and x.shape[0] * x.shape[1] * H < 2**31
-                and _plain_linear(enc, x, x.shape[2])):
+        if plain and _plain_linear(enc, x) and x.shape[2] <= ENCODER_MAX_IN and _end_served(
+                x, enc.weight.shape[0]):
             x = EncoderFused.apply(x, enc.weight, enc.bias)
         else:
             x = enc(x)
         for block in self.blocks:
             x = block(x)
-        if (plain and x.dim() == 3 and 4 <= x.shape[2] <= ENDS_MAX_H and x.shape[2] % 4 == 0
-                and _plain_linear(dec, x, x.shape[2]) and dec.out_features <= HEAD_MAX_OUT):
+        if plain and _plain_linear(dec, x) and dec.weight.shape[0] <= HEAD_MAX_OUT and _end_served(
+                x, x.shape[2]):
             return HeadFused.apply(x, dec.weight, dec.bias)
         return dec(x)[:, -1, :]
 

@@ -110,3 +110,45 @@ def test_weight_tied_blocks_keep_their_gradients_under_create_graph(calls, compo
 
     for a, b in zip(grads(lambda *t: s4convd.S4BlockFused.apply(*t, 0.0)), grads(separate)):
         assert float((a - b).norm() / b.norm()) < 1e-10
+
+
+def _linear(how):
+    m = torch.nn.Linear(8, 12)
+    if how == "one bias":  # F.linear broadcasts it
+        m.bias = torch.nn.Parameter(torch.randn(1))
+    elif how == "short bias":
+        m.bias = torch.nn.Parameter(torch.randn(4))
+    elif how == "vector":
+        m.weight = torch.nn.Parameter(torch.randn(8))
+    elif how == "no bias":
+        m.bias = None
+    elif how == "double":
+        m.double()
+    elif how == "transposed":
+        m.weight = torch.nn.Parameter(torch.randn(8, 12).t())
+    elif how == "misaligned":
+        m.bias = torch.nn.Parameter(torch.randn(13)[1:])
+    elif how == "hook":
+        m.register_forward_hook(lambda *a: None)
+    elif how == "replaced":  # whole, with other sizes than out_features says
+        m.weight = torch.nn.Parameter(torch.randn(20, 8))
+        m.bias = torch.nn.Parameter(torch.randn(20))
+    return m
+
+
+@pytest.mark.parametrize("how", ["one bias", "short bias", "vector", "no bias", "double",
+                                 "transposed", "misaligned", "hook"])
+def test_linear_modules_that_the_kernels_cannot_read(how):
+    """Modules that run as themselves: their weight and bias are not what the
+    ends' kernels read, one value per output among them."""
+    assert not s4convd._whole_linear(_linear(how))
+
+
+def test_linear_modules_are_taken_by_their_tensors():
+    assert s4convd._whole_linear(_linear("as made"))
+    assert s4convd._whole_linear(_linear("replaced"))
+    x = torch.empty(3, 5, 4, device="meta")
+    assert s4convd._end_served(x, 1024) and s4convd._end_served(x, 4)
+    for channels in (0, 2, 6, 1028):
+        assert not s4convd._end_served(x, channels)
+    assert not s4convd._end_served(torch.empty(2**20, 2, 1, device="meta"), 1024)
