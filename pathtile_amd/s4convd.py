@@ -288,6 +288,8 @@ def _tracing() -> bool:
     """True where something watches or rewrites the block's single operations:
     compilers and tracers, functorch transforms, forward-mode AD, dispatch and
     function modes (but the default-device one), autocast, module hooks."""
+    if torch.compiler.is_compiling():  # first: a compiler cannot trace the rest
+        return True
     if torch._C._len_torch_function_stack():
         from torch.overrides import _get_current_function_mode_stack
         from torch.utils._device import DeviceContext
@@ -298,7 +300,7 @@ def _tracing() -> bool:
                 or torch.autograd.forward_ad._current_level >= 0
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.is_autocast_enabled("cuda")
-                or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch.jit.is_tracing()
                 or nn.modules.module._has_any_global_hook())
 
 
@@ -442,6 +444,8 @@ class S4ConvBlock(nn.Module):
         a shape the fused passes do not serve, modules that were replaced,
         subclassed or hooked, kernel timing through KERNEL_EVENTS (its phases
         are the separate launches), or tracing of any kind."""
+        if _tracing():  # before the rest, which a tracer cannot follow
+            return None
         kl, act, drop, out = self.kernel_layer, self.activation, self.dropout, self.output_linear
         if not (type(x) is torch.Tensor and x.dim() == 3 and x.is_cuda
                 and type(kl) is S4ConvKernel and type(act) is nn.GELU
@@ -467,7 +471,7 @@ class S4ConvBlock(nn.Module):
             if not (type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32
                     and t.device == x.device and t.shape == shape and t.is_contiguous()):
                 return None
-        if conv.bias.data_ptr() % 16 or _tracing():
+        if conv.bias.data_ptr() % 16:
             return None
         if not all(_no_hooks(m) for m in (kl, act, drop, out, conv, out[1])):
             return None

@@ -408,3 +408,21 @@ def test_model_ends_with_replaced_parameters(end, how):
     with torch.backends.cudnn.flags(enabled=False):
         ref = m.decoder(m.blocks[0](m.encoder(x)))[:, -1, :]
     assert out.shape == ref.shape and _rel(out, ref) < 1e-6
+
+
+def test_model_compiles_to_one_graph_on_the_gpu():
+    """The "pytorch" backend's composition as one graph of the compiler: the
+    gate asks nothing of a GPU tensor that a compiler cannot trace."""
+    from pathtile_amd import s4convd
+    from pathtile_amd.kernels import warp_tiled_ampere as wta
+
+    torch.manual_seed(6)
+    m = s4convd.Model(state_dim=8, hidden_dim=32, num_blocks=2, dropout=0.0).cuda()
+    x = torch.randn(3, 20, 4, device="cuda")
+    old, wta.TRAIN_CONV_BACKEND = wta.TRAIN_CONV_BACKEND, "pytorch"
+    try:
+        with torch.backends.cudnn.flags(enabled=False), torch.no_grad():
+            torch._dynamo.reset()
+            assert _rel(torch.compile(m, fullgraph=True, backend="eager")(x), m(x)) < 1e-6
+    finally:
+        wta.TRAIN_CONV_BACKEND = old

@@ -152,3 +152,38 @@ def test_linear_modules_are_taken_by_their_tensors():
     for channels in (0, 2, 6, 1028):
         assert not s4convd._end_served(x, channels)
     assert not s4convd._end_served(torch.empty(2**20, 2, 1, device="meta"), 1024)
+
+
+@pytest.fixture
+def pytorch_model(monkeypatch):
+    from pathtile_amd.kernels import warp_tiled_ampere as wta
+
+    monkeypatch.setattr(wta, "TRAIN_CONV_BACKEND", "pytorch")
+    torch.manual_seed(2)
+    return s4convd.Model(state_dim=8, hidden_dim=32, num_blocks=2, dropout=0.0)
+
+
+@pytest.mark.parametrize("how", ["compile", "export", "fx", "jit", "vmap"])
+def test_model_can_be_traced(pytorch_model, how):
+    """The choice of the fused functions leaves the model to tracers: one
+    whole graph for the compiler, and module graphs with the blocks as
+    leaves."""
+    m, x = pytorch_model.eval(), torch.randn(3, 20, 4)
+    with torch.no_grad():
+        ref = m(x)
+        if how == "compile":
+            torch._dynamo.reset()
+            got = torch.compile(m, fullgraph=True, backend="eager")(x)
+        elif how == "export":
+            got = torch.export.export(m, (x,), strict=True).module()(x)
+        elif how == "fx":
+            class Blocks(torch.fx.Tracer):
+                def is_leaf_module(self, mod, name):
+                    return isinstance(mod, s4convd.S4ConvBlock) or super().is_leaf_module(mod, name)
+
+            got = torch.fx.GraphModule(m, Blocks().trace(m))(x)
+        elif how == "jit":
+            got = torch.jit.trace(m, x)(x)
+        else:
+            got = torch.vmap(m)(x[None])[0]
+    assert torch.allclose(got, ref, rtol=1e-6, atol=1e-6)
