@@ -443,7 +443,8 @@ class S4ConvBlock(nn.Module):
         runs as separate operations: another backend, layout, type or device,
         a shape the fused passes do not serve, modules that were replaced,
         subclassed or hooked, kernel timing through KERNEL_EVENTS (its phases
-        are the separate launches), or tracing of any kind."""
+        are the separate launches), a runtime of the caller's own (it may
+        replace any launch), or tracing of any kind."""
         if _tracing():  # before the rest, which a tracer cannot follow
             return None
         kl, act, drop, out = self.kernel_layer, self.activation, self.dropout, self.output_linear
@@ -465,7 +466,7 @@ class S4ConvBlock(nn.Module):
                 and half >= 1 and B >= 1 and x.numel() < 2**31
                 and conv.groups == 1 and conv.stride == (1,) and conv.padding == (0,)
                 and conv.bias is not None and _backend() == "warp"
-                and not KERNEL_EVENTS.enabled):
+                and not KERNEL_EVENTS.enabled and type(get_runtime()) is HipWarpRuntime):
             return None
         for t, shape in zip(params, shapes):
             if not (type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32

@@ -426,3 +426,33 @@ def test_model_compiles_to_one_graph_on_the_gpu():
             assert _rel(torch.compile(m, fullgraph=True, backend="eager")(x), m(x)) < 1e-6
     finally:
         wta.TRAIN_CONV_BACKEND = old
+
+
+def test_separate_launches_of_a_callers_runtime(monkeypatch):
+    """A runtime that replaces the launches gets them from the block."""
+    from pathtile_amd import runtime
+
+    seen = []
+
+    class Recording(runtime.HipWarpRuntime):
+        def launch_fwd(self, *args, **kw):
+            seen.append("fwd")
+            super().launch_fwd(*args, **kw)
+
+        def launch_bwd_input(self, *args, **kw):
+            seen.append("dx")
+            super().launch_bwd_input(*args, **kw)
+
+        def launch_bwd_weight_deterministic(self, *args, **kw):
+            seen.append("dk")
+            super().launch_bwd_weight_deterministic(*args, **kw)
+
+    block, x, gy = _make(5, 64, 16, 8)
+    ref = _fp64(block, x, gy)
+    block.cuda()
+    monkeypatch.setattr(runtime, "_RUNTIME", Recording())
+    with torch.backends.cudnn.flags(enabled=False):
+        got = _grads(block, x.cuda(), gy.cuda())
+    assert seen == ["fwd", "dx", "dk"]
+    for a, b in zip(got, ref):
+        assert _rel(a, b) < PAR_TOL
