@@ -183,6 +183,13 @@ int pt_dwconv1d_dk_det_f32(const float* dy, const float* x, float* dk,
                            void* stream);
 
 /*
+ * 1 where PATHTILE_ROWS_ALGO, PATHTILE_ROWS_CHANNELS or PATHTILE_DK_ALGO is
+ * set (read on every call): the one-pass backward and the S4ConvD block's
+ * fused passes then leave the convolution to the launches that follow them.
+ */
+int pt_kernel_choice_forced(void);
+
+/*
  * Both gradients: pt_dwconv1d_dx_f32_algo and pt_dwconv1d_dk_det_f32, or one
  * kernel that reads dy once for both (the FP32 matrix cores' sums; dk
  * deterministic as there, in its own order). one_pass: PT_BWD_AUTO takes the

@@ -67,6 +67,7 @@ SIGNATURES = {
         _i, [_vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _i, _vp]
     ),
     "pt_dwconv1d_dk_det_f32_noalloc": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "pt_kernel_choice_forced": (_i, []),
     "pt_dwconv1d_bwd_workspace_bytes": (_i, [_i, _i, _i, _i, _i, _szp]),
     "pt_dwconv1d_bwd_f32": (
         _i, [_vp] * 6 + [ctypes.c_size_t] + [_i] * 8 + [_vp]

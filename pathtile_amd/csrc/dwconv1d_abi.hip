@@ -1150,6 +1150,14 @@ static int dk_det_launch(const float* dy, const float* x, float* dk,
   return launch((const void*)&dk_reduce_kernel, grid, 256, 0, stream, args);
 }
 
+// The environment names a kernel of the short rows (rows_algo,
+// rows_cg_channels_env, dk_algo): fused forms leave the call to the launches
+// that read it.
+static bool kernel_choice_forced() {
+  return getenv("PATHTILE_ROWS_ALGO") || getenv("PATHTILE_ROWS_CHANNELS") ||
+         getenv("PATHTILE_DK_ALGO");
+}
+
 // --- one-pass backward -------------------------------------------------------
 // dX and dK from one read of dY (dwconv_bwd_cg_kernel), one 8-channel
 // workgroup per CU. Served wherever the channel-group dX is: H % 8 == 0 and
@@ -1389,6 +1397,8 @@ int pt_dwconv1d_dk_det_f32(const float* dy, const float* x, float* dk,
                            threads_per_block, g, stream);
 }
 
+int pt_kernel_choice_forced(void) { return pt::kernel_choice_forced() ? 1 : 0; }
+
 int pt_dwconv1d_bwd_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
                                     size_t* bytes) {
   const int st = pt_dwconv1d_dk_det_workspace_bytes(B, H, L, K, threads_per_block, bytes);
@@ -1409,8 +1419,8 @@ int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* 
   // through the environment, gets the separate launches.
   if (one_pass != PT_BWD_SEPARATE && B > 0 && H > 0 && pt::valid_wpb(waves_per_block) &&
       pt::valid_dk_threads(threads_per_block) && algo != PT_ROWS_VALU &&
-      (algo == PT_ROWS_AUTO || algo == PT_ROWS_MATRIX) && !getenv("PATHTILE_ROWS_ALGO") &&
-      !getenv("PATHTILE_ROWS_CHANNELS") && !getenv("PATHTILE_DK_ALGO") && dy && x && w && dx && dk &&
+      (algo == PT_ROWS_AUTO || algo == PT_ROWS_MATRIX) && !pt::kernel_choice_forced() && dy && x &&
+      w && dx && dk &&
       pt::aligned(w, 4) && pt::aligned(dk, 4) && pt::bwd_cg_ok(H, L, dy, x, dx) &&
       pt::bwd_cg_wins(B, H, L, K)) {
     const size_t need = (size_t)H * K * pt::bwd_cg_ranges(B, H, L) * sizeof(float);

@@ -279,6 +279,14 @@ def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
     return (*(next(got) if n else None for n in need), None)
 
 
+def _free_choice(runtime: Any) -> bool:
+    """Nobody has a say in the convolution's launches: the runtime is the
+    framework's own class (another may replace any launch) and neither it nor
+    the environment names a kernel."""
+    return (type(runtime) is HipWarpRuntime and runtime.rows_algo == "auto"
+            and not runtime._lib.pt_kernel_choice_forced())
+
+
 def _no_hooks(m: nn.Module) -> bool:
     return not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                 or m._backward_pre_hooks or "forward" in m.__dict__)
@@ -443,8 +451,8 @@ class S4ConvBlock(nn.Module):
         runs as separate operations: another backend, layout, type or device,
         a shape the fused passes do not serve, modules that were replaced,
         subclassed or hooked, kernel timing through KERNEL_EVENTS (its phases
-        are the separate launches), a runtime of the caller's own (it may
-        replace any launch), or tracing of any kind."""
+        are the separate launches), a runtime of the caller's own or a kernel
+        choice (`_free_choice`), or tracing of any kind."""
         if _tracing():  # before the rest, which a tracer cannot follow
             return None
         kl, act, drop, out = self.kernel_layer, self.activation, self.dropout, self.output_linear
@@ -466,7 +474,7 @@ class S4ConvBlock(nn.Module):
                 and half >= 1 and B >= 1 and x.numel() < 2**31
                 and conv.groups == 1 and conv.stride == (1,) and conv.padding == (0,)
                 and conv.bias is not None and _backend() == "warp"
-                and not KERNEL_EVENTS.enabled and type(get_runtime()) is HipWarpRuntime):
+                and not KERNEL_EVENTS.enabled and _free_choice(get_runtime())):
             return None
         for t, shape in zip(params, shapes):
             if not (type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32

@@ -456,3 +456,27 @@ def test_separate_launches_of_a_callers_runtime(monkeypatch):
     assert seen == ["fwd", "dx", "dk"]
     for a, b in zip(got, ref):
         assert _rel(a, b) < PAR_TOL
+
+
+@pytest.mark.parametrize("how", ["PATHTILE_ROWS_ALGO", "PATHTILE_DK_ALGO", "rows_algo"])
+def test_forced_kernel_choices_reach_the_blocks_launches(monkeypatch, how):
+    """With a kernel named by the environment or the runtime the block runs
+    the launches that follow it: the bits of the convolution's own function."""
+    from pathtile_amd import runtime, s4convd
+
+    block, x, gy = _make(40, 64, 48, 8)
+    block.cuda()
+    x = x.cuda()
+    assert block._fused_inputs(x) is not None
+    if how == "rows_algo":
+        monkeypatch.setattr(runtime, "_RUNTIME", runtime.HipWarpRuntime(rows_algo="mfma"))
+    else:
+        monkeypatch.setenv(how, "valu")
+    assert block._fused_inputs(x) is None
+    seen = []
+    block.dropout.register_forward_pre_hook(lambda m, i: seen.append(i[0]))
+    with torch.backends.cudnn.flags(enabled=False):
+        _grads(block, x, gy.cuda())
+    k = block.kernel_layer.build_kernel(48, x.device)
+    own = s4convd.depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, block.skip)
+    assert torch.equal(seen[0], own)

@@ -187,3 +187,25 @@ def test_model_can_be_traced(pytorch_model, how):
         else:
             got = torch.vmap(m)(x[None])[0]
     assert torch.allclose(got, ref, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("name,value", [("PATHTILE_ROWS_ALGO", "valu"),
+                                        ("PATHTILE_ROWS_CHANNELS", "8"),
+                                        ("PATHTILE_DK_ALGO", "valu")])
+def test_a_kernel_choice_reaches_the_launches(monkeypatch, name, value):
+    """A choice of the environment or of the runtime, and a runtime of the
+    caller's own, rule the fused block out."""
+    class Own(runtime.HipWarpRuntime):
+        pass
+
+    for n in ("PATHTILE_ROWS_ALGO", "PATHTILE_ROWS_CHANNELS", "PATHTILE_DK_ALGO"):
+        monkeypatch.delenv(n, raising=False)
+    rt = runtime.HipWarpRuntime()
+    assert s4convd._free_choice(rt)
+    assert not s4convd._free_choice(Own()) and not s4convd._free_choice(object())
+    for algo in ("valu", "mfma"):
+        assert not s4convd._free_choice(runtime.HipWarpRuntime(rows_algo=algo))
+    monkeypatch.setenv(name, value)
+    assert not s4convd._free_choice(rt)
+    monkeypatch.delenv(name)
+    assert s4convd._free_choice(rt)
