@@ -229,7 +229,7 @@ class S4BlockFused(torch.autograd.Function):
     def backward(ctx: Any, gy: torch.Tensor):
         saved = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():  # create_graph: differentiate the composition
+        if _as_operations(gy):
             return _composed_grads(ctx, gy, saved[-1])
         (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
          prep, v, q, mask) = map(_unpacked, saved, ctx.forms)
@@ -258,24 +258,34 @@ class S4BlockFused(torch.autograd.Function):
         return (*(g if n else None for g, n in zip(grads, need)), None)
 
 
+def _as_operations(gy: torch.Tensor) -> bool:
+    """The backward runs as torch's operations instead of the kernels: it is
+    itself differentiated (create_graph), or `gy` is a batch of gradients
+    (is_grads_batched, vmap over the backward), which has no address."""
+    return (torch.is_grad_enabled() or torch._C._functorch.is_legacy_batchedtensor(gy)
+            or torch._C._functorch.is_functorch_wrapped_tensor(gy))
+
+
 def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
-    """The block's gradients through differentiable operations on the saved
-    inputs, for a backward that is itself differentiated (the convolution's
-    own backward stays first order, as its autograd function is). They are
-    taken at aliases: where x was computed from the same parameters, as in a
-    block applied twice, a gradient with respect to the tensors themselves
-    would follow that path too, which the engine adds by itself."""
-    inputs = [t.view_as(t) for t in ctx.saved_tensors[:9]]
-    x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
-    k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
-    v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)
-    if mask is not None:
-        v = v * mask * ctx.scale
-    z = nn.functional.conv1d(nn.functional.gelu(v), weight, bias)
-    y = nn.functional.glu(z, dim=1).transpose(1, 2) + x
+    """The block's gradients through torch's operations on the saved inputs
+    (the convolution's own backward stays first order and takes one gradient,
+    as its autograd function is). They are taken at aliases: where x was
+    computed from the same parameters, as in a block applied twice, a gradient
+    with respect to the tensors themselves would follow that path too, which
+    the engine adds by itself."""
+    create_graph = torch.is_grad_enabled()
     need = ctx.needs_input_grad[:9]
-    got = iter(torch.autograd.grad(y, [t for t, n in zip(inputs, need) if n], gy,
-                                   create_graph=True))
+    with torch.enable_grad():
+        inputs = [t.view_as(t) if n else t.detach() for t, n in zip(ctx.saved_tensors, need)]
+        x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
+        k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
+        v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)
+        if mask is not None:
+            v = v * mask * ctx.scale
+        z = nn.functional.conv1d(nn.functional.gelu(v), weight, bias)
+        y = nn.functional.glu(z, dim=1).transpose(1, 2) + x
+        got = iter(torch.autograd.grad(y, [t for t, n in zip(inputs, need) if n], gy,
+                                       create_graph=create_graph))
     return (*(next(got) if n else None for n in need), None)
 
 
@@ -331,7 +341,7 @@ class EncoderFused(torch.autograd.Function):
     def backward(ctx: Any, gy: torch.Tensor):
         x, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if torch.is_grad_enabled():  # create_graph: differentiable operations
+        if _as_operations(gy):
             return (gy @ weight if need[0] else None,
                     (gy.unsqueeze(-1) * x.unsqueeze(-2)).sum((0, 1)) if need[1] else None,
                     gy.sum((0, 1)) if need[2] else None)
@@ -370,7 +380,7 @@ class HeadFused(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
         B, L, H = x.shape
-        if torch.is_grad_enabled():  # create_graph: differentiable operations
+        if _as_operations(gy):
             gx = nn.functional.pad((gy @ weight)[:, None, :], (0, 0, L - 1, 0)) if need[0] else None
             return (gx, gy.t() @ x[:, -1, :] if need[1] else None,
                     gy.sum(0) if need[2] else None)

@@ -480,3 +480,21 @@ def test_forced_kernel_choices_reach_the_blocks_launches(monkeypatch, how):
     k = block.kernel_layer.build_kernel(48, x.device)
     own = s4convd.depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, block.skip)
     assert torch.equal(seen[0], own)
+
+
+def test_batches_of_gradients_of_the_projection():
+    """is_grads_batched where the separate operations take it: with the
+    convolution's side frozen, against one gradient at a time."""
+    block, x, gy = _make(3, 32, 20, 8)
+    block.cuda()
+    x, conv = x.cuda(), block.output_linear[0]
+    for q in block.parameters():
+        q.requires_grad_(q is conv.weight or q is conv.bias)
+    y = block(x)
+    gys = torch.stack([gy.cuda(), 2 - gy.cuda()])
+    wrt = (conv.weight, conv.bias)
+    with torch.backends.cudnn.flags(enabled=False):
+        batch = torch.autograd.grad(y, wrt, gys, is_grads_batched=True, retain_graph=True)
+    for i in range(2):
+        for a, b in zip(batch, torch.autograd.grad(y, wrt, gys[i], retain_graph=True)):
+            assert _rel(a[i], b) < PAR_TOL

@@ -209,3 +209,29 @@ def test_a_kernel_choice_reaches_the_launches(monkeypatch, name, value):
     assert not s4convd._free_choice(rt)
     monkeypatch.delenv(name)
     assert s4convd._free_choice(rt)
+
+
+@pytest.mark.parametrize("how", ["is_grads_batched", "vmap"])
+def test_batches_of_gradients(calls, composed, how):
+    """Each gradient of the batch by itself, for the block and the model's
+    ends."""
+    torch.manual_seed(11)
+    B, L, H, n = 2, 6, 32, 3
+    inputs = [t.double().requires_grad_(True) for t in _block_inputs(B, L, H, 4)]
+    y = s4convd.S4BlockFused.apply(*inputs, 0.0)
+    x, w, b = (t.double().requires_grad_(True) for t in (_f32(B, L, 4), _f32(H, 4), _f32(H)))
+    e = s4convd.EncoderFused.apply(x, w, b)
+    h, dw, db = (t.double().requires_grad_(True) for t in (_f32(B, L, H), _f32(2, H), _f32(2)))
+    o = s4convd.HeadFused.apply(h, dw, db)
+    for out, wrt in ((y, inputs), (e, (x, w, b)), (o, (h, dw, db))):
+        gys = torch.randn(n, *out.shape, dtype=out.dtype)
+        before = len(calls)
+        if how == "vmap":
+            batch = torch.vmap(lambda g: torch.autograd.grad(out, wrt, g, retain_graph=True))(gys)
+        else:
+            batch = torch.autograd.grad(out, wrt, gys, is_grads_batched=True, retain_graph=True)
+        assert len(calls) == before  # no kernel saw the batch
+        for i in range(n):
+            ones = torch.autograd.grad(out, wrt, gys[i], create_graph=True)
+            for a, g in zip(batch, ones):
+                assert torch.allclose(a[i], g, rtol=1e-10, atol=1e-12)
