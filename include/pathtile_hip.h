@@ -325,7 +325,8 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
  *
  * prep holds the taps and the split projection between the calls of one
  * block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
- * also lays out what _bwd needs. mask is dropout's byte mask in [B, H, L]
+ * also lays out what _bwd needs. x_copy (NULL: none) gets x, for a _bwd that
+ * must not depend on what becomes of x. mask is dropout's byte mask in [B, H, L]
  * order, 4-byte aligned (NULL: none): v = conv * mask * scale. q [2, B L, H], written by _tail where not NULL, holds the projection's values and the
  * gates' sigmoids for _bwd, which takes x, v, q and the mask again. Its
  * outputs gx, {dw, dbias} and the six parameter gradients (all or none, by
@@ -335,8 +336,8 @@ int pt_s4_block_prep_values(int H, int L, size_t* floats);
 int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re,
                         const float* c_im, const float* log_a_re, const float* a_im,
                         const float* skip, const float* w, const unsigned char* mask,
-                        float scale, float* prep, float* v, int B, int H, int L, int states,
-                        int backward, void* stream);
+                        float scale, float* prep, float* v, float* x_copy, int B, int H, int L,
+                        int states, int backward, void* stream);
 int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
                          const float* bias, float* y, float* q, int B, int H, int L,
                          void* stream);

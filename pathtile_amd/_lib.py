@@ -90,7 +90,7 @@ SIGNATURES = {
     ),
     "pt_s4_block_prep_values": (_i, [_i, _i, _szp]),
     "pt_s4_block_mix_f32": (
-        _i, [_vp] * 9 + [ctypes.c_float] + [_vp] * 2 + [_i] * 5 + [_vp]
+        _i, [_vp] * 9 + [ctypes.c_float] + [_vp] * 3 + [_i] * 5 + [_vp]
     ),
     "pt_s4_block_tail_f32": (_i, [_vp] * 7 + [_i] * 3 + [_vp]),
     "pt_s4_block_bwd_workspace_bytes": (_i, [_i, _i, _i, _szp]),

@@ -82,13 +82,15 @@ static uint32_t resident_grid(const void* fn, int block, size_t lds, uint32_t wo
   return n < work ? n : work;
 }
 
-// add: the input gradient plus that tensor; else the forward, with a mask or not.
+// add: the input gradient plus that tensor; else the forward, with or without
+// a mask and a copy of x.
 static int conv_cl_launch(const float* x, const float* w, const float* add,
-                          const unsigned char* mask, float scale, float* y, int B, int H, int L,
-                          void* stream) {
-  const void* fn = (const void*)kConvCl[add ? 1 : mask ? 2 : 0][(L + 7) / 8 - 1];
+                          const unsigned char* mask, float scale, float* y, float* xcopy, int B,
+                          int H, int L, void* stream) {
+  const int form = add ? 1 : xcopy ? (mask ? 4 : 3) : mask ? 2 : 0;
+  const void* fn = (const void*)kConvCl[form][(L + 7) / 8 - 1];
   const int block = conv_cl_threads(H), per = block / H;
-  void* args[] = {&x, &w, &add, &mask, &scale, &y, &B, &H, &L};
+  void* args[] = {&x, &w, &add, &mask, &scale, &y, &xcopy, &B, &H, &L};
   return launch(fn, resident_grid(fn, block, 0, (uint32_t)((B + per - 1) / per)), (uint32_t)block, 0,
                 stream, args);
 }
@@ -141,12 +143,14 @@ int pt_s4_block_prep_values(int H, int L, size_t* floats) {
 int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, const float* c_im,
                         const float* log_a_re, const float* a_im, const float* skip,
                         const float* w, const unsigned char* mask, float scale, float* prep,
-                        float* v, int B, int H, int L, int states, int backward, void* stream) {
+                        float* v, float* x_copy, int B, int H, int L, int states, int backward,
+                        void* stream) {
   int st = pt::check_block(B, H, L, states);
   if (st != PT_OK) return st;
   if (!x || !log_dt || !c_re || !c_im || !log_a_re || !a_im || !skip || !w || !prep || !v)
     return PT_ERR_NULL;
-  if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(v) || !pt::aligned(mask, 4))
+  if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(v) ||
+      !pt::aligned16(x_copy) || !pt::aligned(mask, 4))
     return PT_ERR_ALIGN;
   float* taps = prep;
   __bf16* wf = reinterpret_cast<__bf16*>(prep + pt::round_up((size_t)H * L, 64));
@@ -156,7 +160,7 @@ int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, 
                   &states, &backward};
   st = pt::launch((const void*)&pt::s4_prep_kernel, grid, pt::kPrepThreads, 0, stream, args);
   if (st != PT_OK) return st;
-  return pt::conv_cl_launch(x, taps, nullptr, mask, scale, v, B, H, L, stream);
+  return pt::conv_cl_launch(x, taps, nullptr, mask, scale, v, x_copy, B, H, L, stream);
 }
 
 int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, const float* w,
@@ -237,7 +241,7 @@ int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const f
     if (st != PT_OK) return st;
   }
   if (gx) {
-    st = pt::conv_cl_launch(du, taps, gy, nullptr, 0.0f, gx, B, H, L, stream);
+    st = pt::conv_cl_launch(du, taps, gy, nullptr, 0.0f, gx, nullptr, B, H, L, stream);
     if (st != PT_OK) return st;
   }
   if (!taps_grad) return PT_OK;

@@ -25,14 +25,16 @@ __host__ __device__ constexpr int conv_cl_threads(int H) {
 // The unrolled window of LMAX columns has zero taps beyond the call's K;
 // where such a tap meets a value that is not finite the chain is repeated
 // without them. MASK: the output times a dropout mask [B, H, L], whose row a
-// lane reads as whole dwords, and scale. Bound by the FMA issue at 48 taps (36 per output on average, 92 us of
+// lane reads as whole dwords, and scale. COPY: x as it was read, for a
+// backward that must not depend on what becomes of x. Bound by the FMA issue at 48 taps (36 per output on average, 92 us of
 // it at B16384 L48 H128): FWD 200 us, DX 246 us there, against 305 and 366 with
 // the transposes.
-template <int LMAX, bool DX, bool MASK>
+template <int LMAX, bool DX, bool MASK, bool COPY>
 __global__ __launch_bounds__(kConvClThreads, LMAX > 40 ? 3 : 4) void s4_conv_cl_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ add,
-    const uint8_t* __restrict__ mask, float scale, float* __restrict__ y, int B, int H, int L) {
-  static_assert(!(DX && MASK), "the mask belongs to the forward's output");
+    const uint8_t* __restrict__ mask, float scale, float* __restrict__ y,
+    float* __restrict__ xcopy, int B, int H, int L) {
+  static_assert(!(DX && (MASK || COPY)), "mask and copy belong to the forward");
   constexpr int LO = DX ? -(LMAX / 2 - 1) : -(LMAX / 2);  // smallest column offset s - t
   const int h = threadIdx.x % H, sub = threadIdx.x / H, per = blockDim.x / H, p = L / 2;
   float tap[LMAX];  // of offset LO + i
@@ -59,6 +61,7 @@ __global__ __launch_bounds__(kConvClThreads, LMAX > 40 ? 3 : 4) void s4_conv_cl_
     const __amdgpu_buffer_rsrc_t rx = make_rsrc_n(x + base, bytes);
     const __amdgpu_buffer_rsrc_t ry = make_rsrc_n(y + base, bytes);
     const __amdgpu_buffer_rsrc_t ra = make_rsrc_n(DX ? add + base : x, DX ? bytes : 0);
+    const __amdgpu_buffer_rsrc_t rc = make_rsrc_n(COPY ? xcopy + base : y, COPY ? bytes : 0);
     float v[LMAX];
     const uint32_t lane = copy(lane_off);
 #pragma unroll
@@ -122,6 +125,7 @@ __global__ __launch_bounds__(kConvClThreads, LMAX > 40 ? 3 : 4) void s4_conv_cl_
           if constexpr (DX) o[r] += e[r];
           if constexpr (MASK) o[r] = o[r] * (float)((keep[t0 / 4] >> (8 * r)) & 0xffu) * scale;
           buf_store1(o[r], ry, off(at, t0 + r));
+          if constexpr (COPY) buf_store1(v[t0 + r], rc, off(at, t0 + r));
         }
       }
     });

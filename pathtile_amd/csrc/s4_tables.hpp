@@ -10,7 +10,7 @@ namespace pt {
 constexpr int kNumS4H = 8;  // H = 32, 64, ..., 256
 
 using ConvClFn = void (*)(const float*, const float*, const float*, const uint8_t*, float, float*,
-                          int, int, int);
+                          float*, int, int, int);
 using TailFwdFn = void (*)(const float*, const float*, const __bf16*, const float*, const float*,
                            float*, float*, uint32_t, uint32_t);
 using TailBwdFn = void (*)(const float*, const float*, const float*, const uint8_t*, float,
@@ -18,7 +18,8 @@ using TailBwdFn = void (*)(const float*, const float*, const float*, const uint8
                            uint32_t);
 using DwFn = void (*)(const float*, const float*, float*, uint32_t, uint32_t, uint32_t);
 
-extern const ConvClFn kConvCl[3][6];  // [forward, dx, forward with mask][row bucket 8, ..., 48]
+// [forward, dx, forward with mask, with copy, with both][row bucket 8, ..., 48]
+extern const ConvClFn kConvCl[5][6];
 extern const TailFwdFn kTailFwd[kNumS4H];
 extern const TailBwdFn kTailBwd[2][kNumS4H];  // [dropout mask]
 extern const DwFn kDw[kNumS4H];

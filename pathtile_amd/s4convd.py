@@ -181,9 +181,9 @@ def _dropout_mask(x: torch.Tensor, p: float) -> torch.Tensor | None:
 
 
 def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask,
-               scale: float, backward: bool):
+               scale: float, backward: bool, x_copy: torch.Tensor | None = None):
     """Taps and split projection (prep) and the convolution's output after
-    dropout, v [B, L, H]."""
+    dropout, v [B, L, H]; x into x_copy."""
     runtime = get_runtime()
     runtime._check_open()
     B, L, H = x.shape
@@ -192,7 +192,8 @@ def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight
     _call(runtime._lib.pt_s4_block_mix_f32, x.device,
           _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
           _ptr(skip), _ptr(weight), None if mask is None else _ptr(mask), scale, _ptr(prep),
-          _ptr(v), B, H, L, c_re.shape[1], int(backward))
+          _ptr(v), None if x_copy is None else _ptr(x_copy), B, H, L, c_re.shape[1],
+          int(backward))
     return prep, v
 
 
@@ -210,25 +211,42 @@ def _fused_tail(v: torch.Tensor, x: torch.Tensor, prep, weight, bias,
 class S4BlockFused(torch.autograd.Function):
     """``S4ConvBlock.forward`` as one function of the input and the block's
     parameters: taps, convolution with the skip term, dropout, GELU,
-    projection, GLU and residual, all in [B, L, H]."""
+    projection, GLU and residual, all in [B, L, H]. The backward reads x. With
+    ``copy`` it reads a copy that the convolution writes on its way, so that
+    x may change in between (``x += block(x)``; the separate operations save
+    the copy that their transpose makes). The copy is a second output: that
+    ties it to x for a backward that is differentiated."""
 
     @staticmethod
-    def forward(ctx: Any, x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, p: float):
+    def forward(ctx: Any, x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, p: float,
+                copy: bool = False):
         mask = _dropout_mask(x, p)
         ctx.scale = 1.0 / (1.0 - p)
+        ctx.set_materialize_grads(False)
+        x_copy = torch.empty_like(x) if copy else None
         prep, v = _fused_mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask,
-                             ctx.scale, True)
+                             ctx.scale, True, x_copy)
         q = x.new_empty((2, *x.shape))
         y = _fused_tail(v, x, prep, weight, bias, q)
-        saved = (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, prep, v, q, mask)
+        saved = (x_copy if copy else x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
+                 prep, v, q, mask)
         ctx.forms = [_form(t) for t in saved]
         ctx.save_for_backward(*saved)
-        return y
+        return (y, x_copy) if copy else y
 
     @staticmethod
-    def backward(ctx: Any, gy: torch.Tensor):
+    def backward(ctx: Any, gy: torch.Tensor | None, g_copy: torch.Tensor | None = None):
+        grads = [None] * len(ctx.needs_input_grad)
+        if gy is not None:
+            grads[:9] = S4BlockFused._backward(ctx, gy)
+        if g_copy is not None and ctx.needs_input_grad[0]:
+            grads[0] = g_copy if grads[0] is None else grads[0] + g_copy
+        return tuple(grads)
+
+    @staticmethod
+    def _backward(ctx: Any, gy: torch.Tensor):
         saved = ctx.saved_tensors
-        need = ctx.needs_input_grad
+        need = ctx.needs_input_grad[:9]
         if _as_operations(gy):
             return _composed_grads(ctx, gy, saved[-1])
         (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
@@ -255,7 +273,7 @@ class S4BlockFused(torch.autograd.Function):
               opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
               c_re.shape[1])
         grads = [gx, gp[5], *gp[:5], gw, gb]
-        return (*(g if n else None for g, n in zip(grads, need)), None)
+        return [g if n else None for g, n in zip(grads, need)]
 
 
 def _as_operations(gy: torch.Tensor) -> bool:
@@ -286,7 +304,7 @@ def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
         y = nn.functional.glu(z, dim=1).transpose(1, 2) + x
         got = iter(torch.autograd.grad(y, [t for t, n in zip(inputs, need) if n], gy,
                                        create_graph=create_graph))
-    return (*(next(got) if n else None for n in need), None)
+    return [next(got) if n else None for n in need]
 
 
 def _free_choice(runtime: Any) -> bool:
@@ -419,20 +437,22 @@ def _whole_linear(m: nn.Module) -> bool:
     one bias value per row of its weight, as the kernels read them
     (``F.linear`` broadcasts fewer). The sizes are the tensors' own:
     ``out_features`` does not follow a replaced weight."""
-    return (type(m) is nn.Linear and m.bias is not None and _no_hooks(m)
-            and m.weight.dim() == 2 and m.bias.shape == m.weight.shape[:1]
+    if not (type(m) is nn.Linear and _no_hooks(m)):
+        return False
+    w, b = m.weight, m.bias
+    return (b is not None and w.dim() == 2 and b.shape == w.shape[:1]
             and all(type(t) in (nn.Parameter, torch.Tensor) and t.dtype == torch.float32
-                    and t.is_contiguous() and t.data_ptr() % 16 == 0
-                    for t in (m.weight, m.bias)))
+                    and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (w, b)))
 
 
 def _plain_linear(m: nn.Module, x: torch.Tensor) -> bool:
     """`m` is a `_whole_linear` for the contiguous GPU tensor `x` [B, L, width]."""
-    return (type(x) is torch.Tensor and x.is_cuda and x.dim() == 3
+    if not (type(x) is torch.Tensor and x.is_cuda and x.dim() == 3
             and x.dtype == torch.float32 and x.is_contiguous() and x.data_ptr() % 16 == 0
-            and 0 < x.numel() < 2**31 and _backend() == "warp" and _whole_linear(m)
-            and x.shape[2] == m.weight.shape[1]
-            and m.weight.device == x.device and m.bias.device == x.device)
+            and 0 < x.numel() < 2**31 and _backend() == "warp" and _whole_linear(m)):
+        return False
+    w = m.weight
+    return x.shape[2] == w.shape[1] and w.device == x.device and m.bias.device == x.device
 
 
 def _end_served(x: torch.Tensor, channels: int) -> bool:
@@ -502,7 +522,9 @@ class S4ConvBlock(nn.Module):
             p = float(self.dropout.p) if self.dropout.training else 0.0
             if torch.is_grad_enabled() and (x.requires_grad
                                             or any(t.requires_grad for t in params)):
-                return S4BlockFused.apply(x, *params, p)
+                if getattr(x, "_held_by_model_alone", False):
+                    return S4BlockFused.apply(x, *params, p)
+                return S4BlockFused.apply(x, *params, p, True)[0]
             skip, *kernel, weight, bias = params
             mask = _dropout_mask(x, p)
             prep, v = _fused_mix(x, skip, *kernel, weight, mask, 1.0 / (1.0 - p), False)
@@ -536,14 +558,21 @@ class Model(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         plain = not _tracing()
+        saving = plain and torch.is_grad_enabled()
         enc, dec = self.encoder, self.decoder
         if plain and _plain_linear(enc, x) and x.shape[2] <= ENCODER_MAX_IN and _end_served(
                 x, enc.weight.shape[0]):
             x = EncoderFused.apply(x, enc.weight, enc.bias)
+            held = saving  # x is a new tensor that nothing else has seen
         else:
             x = enc(x)
+            held = saving and type(enc) is nn.Linear and _no_hooks(enc)
         for block in self.blocks:
+            unseen = saving and type(block) is S4ConvBlock and _no_hooks(block)
+            if held and unseen:
+                x._held_by_model_alone = True
             x = block(x)
+            held = unseen
         if plain and _plain_linear(dec, x) and dec.weight.shape[0] <= HEAD_MAX_OUT and _end_served(
                 x, x.shape[2]):
             return HeadFused.apply(x, dec.weight, dec.bias)

@@ -498,3 +498,18 @@ def test_batches_of_gradients_of_the_projection():
     for i in range(2):
         for a, b in zip(batch, torch.autograd.grad(y, wrt, gys[i], retain_graph=True)):
             assert _rel(a[i], b) < PAR_TOL
+
+
+def test_fused_blocks_input_may_change_before_its_backward():
+    block, x, gy = _make(4, 64, 24, 8)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+
+    def grads(change):
+        h = x.clone()
+        y = block(h)
+        if change:
+            h += y.detach()
+        return torch.autograd.grad(y, tuple(block.parameters()), gy)
+
+    assert all(torch.equal(a, b) for a, b in zip(grads(True), grads(False)))

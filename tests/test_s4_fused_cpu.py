@@ -70,7 +70,10 @@ def composed(monkeypatch):
     def conv(x, k, skip):
         return s4convd.reference_depthwise_conv(x, k) + x * skip.unsqueeze(-1)
 
-    def mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask, scale, backward):
+    def mix(x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, mask, scale, backward,
+            x_copy=None):
+        if x_copy is not None:
+            x_copy.copy_(x)
         k = s4convd._taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
         v = conv(x.transpose(1, 2), k, skip)
         if mask is not None:
@@ -86,8 +89,10 @@ def composed(monkeypatch):
     monkeypatch.setattr(s4convd, "_fused_tail", tail)
 
 
+@pytest.mark.parametrize("copy", [False, True])
 @pytest.mark.parametrize("applications", [1, 2, 3])
-def test_weight_tied_blocks_keep_their_gradients_under_create_graph(calls, composed, applications):
+def test_weight_tied_blocks_keep_their_gradients_under_create_graph(calls, composed, applications,
+                                                                    copy):
     """One block applied several times: gradients with create_graph equal
     those of the separate operations (FP64), and so do second derivatives."""
     torch.manual_seed(applications)
@@ -108,7 +113,11 @@ def test_weight_tied_blocks_keep_their_gradients_under_create_graph(calls, compo
                                   True)
         return s4convd._fused_tail(v, x, None, weight, bias)
 
-    for a, b in zip(grads(lambda *t: s4convd.S4BlockFused.apply(*t, 0.0)), grads(separate)):
+    def fused_block(*t):
+        y = s4convd.S4BlockFused.apply(*t, 0.0, copy)
+        return y[0] if copy else y
+
+    for a, b in zip(grads(fused_block), grads(separate)):
         assert float((a - b).norm() / b.norm()) < 1e-10
 
 
@@ -235,3 +244,60 @@ def test_batches_of_gradients(calls, composed, how):
             ones = torch.autograd.grad(out, wrt, gys[i], create_graph=True)
             for a, g in zip(batch, ones):
                 assert torch.allclose(a[i], g, rtol=1e-10, atol=1e-12)
+
+
+@pytest.fixture
+def fused(calls, composed, monkeypatch):
+    """Blocks and ends take their fused functions on the CPU."""
+    def params(block, x):
+        kl, conv = block.kernel_layer, block.output_linear[0]
+        return (block.skip, kl.log_dt, kl.C_re, kl.C_im, kl.log_A_re, kl.A_im, conv.weight,
+                conv.bias)
+
+    monkeypatch.setattr(s4convd.S4ConvBlock, "_fused_inputs", params)
+    monkeypatch.setattr(s4convd, "_plain_linear", lambda m, x: s4convd._whole_linear(m))
+
+
+def test_a_blocks_input_may_change_before_its_backward(fused):
+    """``x += block(x)``: the block's gradients are those at the values that
+    it saw."""
+    torch.manual_seed(12)
+    block = s4convd.S4ConvBlock(32, 8, 0.0)
+    x = torch.randn(3, 6, 32)
+
+    def grads(change):
+        h = x.clone()
+        y = block(h)
+        if change:
+            h += y.detach()
+        return torch.autograd.grad(y.sum(), tuple(block.parameters()), create_graph=True)
+
+    for a, b in zip(grads(True), grads(False)):
+        assert torch.equal(a, b)
+
+
+def _copies(out):
+    seen, todo = set(), [out.grad_fn]
+    while todo:
+        f = todo.pop()
+        if f is not None and f not in seen:
+            seen.add(f)
+            todo += [g for g, _ in f.next_functions]
+    return sum(len(f.needs_input_grad) == 11 for f in seen if f.name() == "S4BlockFusedBackward")
+
+
+@pytest.mark.parametrize("how,copies", [("plain", 0), ("encoder hook", 1), ("block hook", 2),
+                                        ("identity encoder", 1)])
+def test_the_models_own_activations_are_not_copied(fused, how, copies):
+    """Between the modules of a model only it holds an activation, unless a
+    module is hooked (its input and output are then seen) or replaced."""
+    m = s4convd.Model(state_dim=8, hidden_dim=32, input_dim=8, num_blocks=3, dropout=0.0)
+    if how == "encoder hook":
+        m.encoder.register_forward_hook(lambda *a: None)
+    elif how == "block hook":
+        m.blocks[1].register_forward_hook(lambda *a: None)
+    elif how == "identity encoder":
+        m.encoder = torch.nn.Identity()
+    x = torch.randn(2, 6, 32 if how == "identity encoder" else 8)
+    x.requires_grad_(how == "identity encoder")
+    assert _copies(m(x)) == copies
