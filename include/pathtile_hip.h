@@ -358,7 +358,7 @@ int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const f
  * outputs] = x[:, L-1, :] w^T + bias, w [outputs, H], outputs <= 4: the
  * decoder at the one column that the model returns. The *_grad calls give the
  * gradients of w and bias by a fixed-order reduction, and the head's gx [B,
- * L, H] (NULL: skipped), zero before the last column. bias, y, gy of the
+ * L, H] (NULL: skipped, and w may be too), zero before the last column. bias, y, gy of the
  * encoder and x, gx of the head are 16-byte aligned.
  */
 int pt_s4_encode_f32(const float* x, const float* w, const float* bias, float* y, int B,

@@ -319,7 +319,7 @@ int pt_s4_head_grad_f32(const float* x, const float* gy, const float* w, float* 
   size_t need = 0;
   int st = pt_s4_head_grad_workspace_bytes(B, H, L, outputs, &need);
   if (st != PT_OK) return st;
-  if (!x || !gy || !w || !dw || !dbias) return PT_ERR_NULL;
+  if (!x || !gy || (gx && !w) || !dw || !dbias) return PT_ERR_NULL;
   if (!pt::aligned16(x) || (gx && !pt::aligned16(gx))) return PT_ERR_ALIGN;
   if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
   int per = (B + pt::kEndRanges - 1) / pt::kEndRanges;

@@ -342,7 +342,9 @@ def _tracing() -> bool:
 
 class EncoderFused(torch.autograd.Function):
     """``nn.Linear`` over up to 8 input features: one pass over the output, and
-    one over its gradient for the weight and bias gradients."""
+    one over its gradient for the weight and bias gradients. Like the module
+    it saves x for the weight's gradient and the weight for x's, and neither
+    where nobody asks."""
 
     @staticmethod
     def forward(ctx: Any, x, weight, bias):
@@ -351,36 +353,36 @@ class EncoderFused(torch.autograd.Function):
         y = x.new_empty((B, L, H))
         _call(_lib.load().pt_s4_encode_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(y), B, L, n, H)
-        ctx.forms = _form(x), _form(weight)
-        ctx.save_for_backward(x, weight)
+        need = ctx.needs_input_grad
+        saved = (x if need[1] else None, weight if need[0] else None)
+        ctx.forms = [_form(t) for t in saved]
+        ctx.save_for_backward(*saved)
         return y
 
     @staticmethod
     def backward(ctx: Any, gy: torch.Tensor):
         x, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
-        if _as_operations(gy):
-            return (gy @ weight if need[0] else None,
-                    (gy.unsqueeze(-1) * x.unsqueeze(-2)).sum((0, 1)) if need[1] else None,
-                    gy.sum((0, 1)) if need[2] else None)
         gx = gy @ weight if need[0] else None
-        gw = gb = None
-        if need[1] or need[2]:
-            x, weight = map(_unpacked, (x, weight), ctx.forms)
-            B, L, n = x.shape
-            H = weight.shape[0]
-            gy = _aligned(gy.contiguous())
-            gw, gb = torch.empty_like(weight), weight.new_empty(H)
-            nbytes = _size_query("pt_s4_encode_grad_workspace_bytes", B, L, n, H)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
-            _call(_lib.load().pt_s4_encode_grad_f32, x.device,
-                  _ptr(x), _ptr(gy), _ptr(gw), _ptr(gb), _ptr(ws), nbytes, B, L, n, H)
-        return gx, gw if need[1] else None, gb if need[2] else None
+        if not need[1] or _as_operations(gy):
+            return (gx, (gy.unsqueeze(-1) * x.unsqueeze(-2)).sum((0, 1)) if need[1] else None,
+                    gy.sum((0, 1)) if need[2] else None)
+        x = _unpacked(x, ctx.forms[0])
+        B, L, n = x.shape
+        H = gy.shape[2]
+        gy = _aligned(gy.contiguous())
+        gw, gb = gy.new_empty((H, n)), gy.new_empty(H)
+        nbytes = _size_query("pt_s4_encode_grad_workspace_bytes", B, L, n, H)
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+        _call(_lib.load().pt_s4_encode_grad_f32, x.device,
+              _ptr(x), _ptr(gy), _ptr(gw), _ptr(gb), _ptr(ws), nbytes, B, L, n, H)
+        return gx, gw, gb if need[2] else None
 
 
 class HeadFused(torch.autograd.Function):
     """The decoder at the last column, ``decoder(x)[:, -1, :]``: the columns
-    before it reach neither the output nor a gradient."""
+    before it reach neither the output nor a gradient. Saves what the module
+    does (EncoderFused)."""
 
     @staticmethod
     def forward(ctx: Any, x, weight, bias):
@@ -389,30 +391,33 @@ class HeadFused(torch.autograd.Function):
         out = x.new_empty((B, n))
         _call(_lib.load().pt_s4_head_f32, x.device,
               _ptr(x), _ptr(weight), _ptr(bias), _ptr(out), B, H, L, n)
-        ctx.forms = _form(x), _form(weight)
-        ctx.save_for_backward(x, weight)
+        need = ctx.needs_input_grad
+        saved = (x if need[1] else None, weight if need[0] else None)
+        ctx.shape = x.shape
+        ctx.forms = [_form(t) for t in saved]
+        ctx.save_for_backward(*saved)
         return out
 
     @staticmethod
     def backward(ctx: Any, gy: torch.Tensor):
         x, weight = ctx.saved_tensors
         need = ctx.needs_input_grad
-        B, L, H = x.shape
-        if _as_operations(gy):
+        B, L, H = ctx.shape
+        if not need[1] or _as_operations(gy):
             gx = nn.functional.pad((gy @ weight)[:, None, :], (0, 0, L - 1, 0)) if need[0] else None
             return (gx, gy.t() @ x[:, -1, :] if need[1] else None,
                     gy.sum(0) if need[2] else None)
         x, weight = map(_unpacked, (x, weight), ctx.forms)
-        n = weight.shape[0]
+        n = gy.shape[1]
         gy = gy.contiguous()
         gx = torch.empty_like(x) if need[0] else None
-        gw, gb = torch.empty_like(weight), weight.new_empty(n)
+        gw, gb = gy.new_empty((n, H)), gy.new_empty(n)
         nbytes = _size_query("pt_s4_head_grad_workspace_bytes", B, H, L, n)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
         _call(_lib.load().pt_s4_head_grad_f32, x.device,
-              _ptr(x), _ptr(gy), _ptr(weight), None if gx is None else _ptr(gx), _ptr(gw),
-              _ptr(gb), _ptr(ws), nbytes, B, H, L, n)
-        return gx, gw if need[1] else None, gb if need[2] else None
+              _ptr(x), _ptr(gy), None if weight is None else _ptr(weight),
+              None if gx is None else _ptr(gx), _ptr(gw), _ptr(gb), _ptr(ws), nbytes, B, H, L, n)
+        return gx, gw, gb if need[2] else None
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:

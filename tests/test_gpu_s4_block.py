@@ -513,3 +513,21 @@ def test_fused_blocks_input_may_change_before_its_backward():
         return torch.autograd.grad(y, tuple(block.parameters()), gy)
 
     assert all(torch.equal(a, b) for a, b in zip(grads(True), grads(False)))
+
+
+def test_model_ends_partial_gradients():
+    """Every choice of the gradients that are asked for gives the same values."""
+    from pathtile_amd import s4convd
+
+    torch.manual_seed(14)
+    for fn, rows in ((s4convd.EncoderFused, 12), (s4convd.HeadFused, 3)):
+        x, w, b = (torch.randn(*shape, device="cuda") for shape in ((9, 7, 8), (rows, 8), (rows,)))
+        full = None
+        for needs in range(7, 0, -1):
+            ts = [t.clone().requires_grad_(bool(needs >> i & 1)) for i, t in enumerate((x, w, b))]
+            out = fn.apply(*ts)
+            g = iter(torch.autograd.grad(out, [t for t in ts if t.requires_grad], out.detach()))
+            got = [next(g) if t.requires_grad else None for t in ts]
+            full = full or got
+            for a, c in zip(got, full):
+                assert a is None or _rel(a, c) < 1e-6

@@ -301,3 +301,27 @@ def test_the_models_own_activations_are_not_copied(fused, how, copies):
     x = torch.randn(2, 6, 32 if how == "identity encoder" else 8)
     x.requires_grad_(how == "identity encoder")
     assert _copies(m(x)) == copies
+
+
+@pytest.mark.parametrize("end", ["EncoderFused", "HeadFused"])
+def test_the_ends_save_what_their_gradients_read(calls, end):
+    """As nn.Linear: x for the weight's gradient, the weight for x's. What no
+    gradient reads may change before the backward."""
+    fn, n = getattr(s4convd, end), 8 if end == "EncoderFused" else 2
+    for needs in range(8):
+        x, w, b = _f32(3, 5, 4), _f32(n, 4), _f32(n)
+        for i, t in enumerate((x, w, b)):
+            t.requires_grad_(bool(needs >> i & 1))
+        out = fn.apply(x, w, b)
+        if not needs:
+            assert out.grad_fn is None
+            continue
+        with torch.no_grad():
+            if not w.requires_grad:
+                x += 1
+            if not x.requires_grad:
+                w += 1
+            b += 1
+        wrt = [t for t in (x, w, b) if t.requires_grad]
+        for g, t in zip(torch.autograd.grad(out, wrt, torch.ones_like(out)), wrt):
+            assert g.shape == t.shape and g.dtype == torch.float32
