@@ -201,6 +201,10 @@ int pt_kernel_choice_forced(void);
 #define PT_BWD_SEPARATE 1
 int pt_dwconv1d_bwd_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
                                     size_t* bytes);
+/* Whether pt_dwconv1d_bwd_f32 with PT_BWD_AUTO takes the one kernel for this
+ * shape and alignment on the current device (the dispatch itself answers). */
+int pt_dwconv1d_bwd_one_pass(int B, int H, int L, int K, int waves_per_block, int algo,
+                             int threads_per_block, int aligned16, int* one_pass);
 int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* dx,
                         float* dk, void* workspace, size_t workspace_bytes, int B, int H,
                         int L, int K, int waves_per_block, int algo,
@@ -260,6 +264,8 @@ int pt_dwconv1d_dk_det_bf16(const void* dy, const void* x, float* dk,
  * reads dy once (dx the bits of pt_dwconv1d_dx_bf16), or the two calls. */
 int pt_dwconv1d_bwd_bf16_workspace_bytes(int B, int H, int L, int K, int threads_per_block,
                                          size_t* bytes);
+int pt_dwconv1d_bwd_bf16_one_pass(int B, int H, int L, int K, int threads_per_block,
+                                  int aligned16, int* one_pass);
 int pt_dwconv1d_bwd_bf16(const void* dy, const void* x, const float* w, void* dx,
                          float* dk, void* workspace, size_t workspace_bytes, int B, int H,
                          int L, int K, int threads_per_block, int one_pass, void* stream);

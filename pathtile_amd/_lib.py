@@ -69,6 +69,7 @@ SIGNATURES = {
     "pt_dwconv1d_dk_det_f32_noalloc": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "pt_kernel_choice_forced": (_i, []),
     "pt_dwconv1d_bwd_workspace_bytes": (_i, [_i, _i, _i, _i, _i, _szp]),
+    "pt_dwconv1d_bwd_one_pass": (_i, [_i] * 8 + [_ip]),
     "pt_dwconv1d_bwd_f32": (
         _i, [_vp] * 6 + [ctypes.c_size_t] + [_i] * 8 + [_vp]
     ),
@@ -81,6 +82,7 @@ SIGNATURES = {
     ),
     "flash_dk_fp32": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "pt_dwconv1d_bwd_bf16_workspace_bytes": (_i, [_i, _i, _i, _i, _i, _szp]),
+    "pt_dwconv1d_bwd_bf16_one_pass": (_i, [_i] * 6 + [_ip]),
     "pt_dwconv1d_bwd_bf16": (_i, [_vp] * 6 + [ctypes.c_size_t] + [_i] * 6 + [_vp]),
     "pt_dwconv1d_fwd_long_f32": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),
     "pt_dwconv1d_dx_long_f32": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp]),

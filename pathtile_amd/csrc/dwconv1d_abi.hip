@@ -1196,6 +1196,18 @@ static bool bwd_cg_wins(int B, int H, int L, int K) {
          (long long)B >= 4LL * kRowsCgStep * bwd_cg_ranges(B, H, L);
 }
 
+// The one-pass kernel serves this call and is taken. A caller who asked for the
+// reference's chain, or for one kernel family through the environment, gets
+// the separate launches.
+static bool bwd_cg_taken(int B, int H, int L, int K, int waves_per_block, int algo,
+                         int threads_per_block, int one_pass, const void* gy, const void* x,
+                         const void* gx) {
+  return one_pass == PT_BWD_AUTO && B > 0 && H > 0 && valid_wpb(waves_per_block) &&
+         valid_dk_threads(threads_per_block) &&
+         (algo == PT_ROWS_AUTO || algo == PT_ROWS_MATRIX) && !kernel_choice_forced() &&
+         bwd_cg_ok(H, L, gy, x, gx) && bwd_cg_wins(B, H, L, K);
+}
+
 static int bwd_cg_launch(const float* gy, const float* x, const float* w, float* gx, float* gk,
                          float* partials, int B, int H, int L, int K, void* stream) {
   const BwdCgFn fn = kBwdCg[!rows_plain_loads(B, H, L)][L % 4 == 0][mfma_index(L)];
@@ -1229,6 +1241,13 @@ static int bwd_bf16_ranges(int B, int H, int L) {
   long long nr = (long long)num_cus() * per_cu / ngroups;
   if (nr > tsteps) nr = tsteps;
   return nr < 1 ? 1 : (int)nr;
+}
+
+static bool bwd_bf16_taken(int B, int H, int L, int one_pass, const void* gy, const void* x,
+                           const void* gx) {
+  return one_pass == PT_BWD_AUTO && B > 0 && H > 0 && L % 4 == 0 && H % kRowsCgWaves == 0 &&
+         aligned(gy, 16) && aligned(x, 16) && aligned(gx, 16) &&
+         bwd_bf16_lds_bytes(L, 16 * (mfma_index(L) + 1)) <= (size_t)max_lds_per_block();
 }
 
 static int bwd_bf16_launch(const uint16_t* gy, const uint16_t* x, const float* w, uint16_t* gx,
@@ -1408,6 +1427,18 @@ int pt_dwconv1d_bwd_workspace_bytes(int B, int H, int L, int K, int threads_per_
   return PT_OK;
 }
 
+int pt_dwconv1d_bwd_one_pass(int B, int H, int L, int K, int waves_per_block, int algo,
+                             int threads_per_block, int aligned16, int* one_pass) {
+  if (!one_pass) return PT_ERR_NULL;
+  *one_pass = 0;
+  const int st = pt::check_shape(B, H, L, K);
+  if (st != PT_OK) return st;
+  const void* p = reinterpret_cast<const void*>((uintptr_t)(aligned16 ? 256 : 260));
+  *one_pass = pt::bwd_cg_taken(B, H, L, K, waves_per_block, algo, threads_per_block, PT_BWD_AUTO,
+                               p, p, p);
+  return PT_OK;
+}
+
 int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* dx, float* dk,
                         void* workspace, size_t workspace_bytes, int B, int H, int L, int K,
                         int waves_per_block, int algo, int threads_per_block, int one_pass,
@@ -1415,14 +1446,8 @@ int pt_dwconv1d_bwd_f32(const float* dy, const float* x, const float* w, float* 
   if (one_pass < PT_BWD_AUTO || one_pass > PT_BWD_SEPARATE) return PT_ERR_CONFIG;
   int st = pt::check_shape(B, H, L, K);
   if (st != PT_OK) return st;
-  // A caller who asked for the reference's chain, or for one kernel family
-  // through the environment, gets the separate launches.
-  if (one_pass != PT_BWD_SEPARATE && B > 0 && H > 0 && pt::valid_wpb(waves_per_block) &&
-      pt::valid_dk_threads(threads_per_block) && algo != PT_ROWS_VALU &&
-      (algo == PT_ROWS_AUTO || algo == PT_ROWS_MATRIX) && !pt::kernel_choice_forced() && dy && x &&
-      w && dx && dk &&
-      pt::aligned(w, 4) && pt::aligned(dk, 4) && pt::bwd_cg_ok(H, L, dy, x, dx) &&
-      pt::bwd_cg_wins(B, H, L, K)) {
+  if (dy && x && w && dx && dk && pt::aligned(w, 4) && pt::aligned(dk, 4) &&
+      pt::bwd_cg_taken(B, H, L, K, waves_per_block, algo, threads_per_block, one_pass, dy, x, dx)) {
     const size_t need = (size_t)H * K * pt::bwd_cg_ranges(B, H, L) * sizeof(float);
     if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
     if (!pt::aligned(workspace, 4)) return PT_ERR_ALIGN;
@@ -1613,16 +1638,25 @@ int pt_dwconv1d_bwd_bf16_workspace_bytes(int B, int H, int L, int K, int threads
   return PT_OK;
 }
 
+int pt_dwconv1d_bwd_bf16_one_pass(int B, int H, int L, int K, int threads_per_block,
+                                  int aligned16, int* one_pass) {
+  if (!one_pass) return PT_ERR_NULL;
+  *one_pass = 0;
+  const int st = pt::bf16_dk_check(B, H, L, K, threads_per_block);
+  if (st != PT_OK) return st;
+  const void* p = reinterpret_cast<const void*>((uintptr_t)(aligned16 ? 256 : 260));
+  *one_pass = pt::bwd_bf16_taken(B, H, L, PT_BWD_AUTO, p, p, p);
+  return PT_OK;
+}
+
 int pt_dwconv1d_bwd_bf16(const void* dy, const void* x, const float* w, void* dx, float* dk,
                          void* workspace, size_t workspace_bytes, int B, int H, int L, int K,
                          int threads_per_block, int one_pass, void* stream) {
   if (one_pass < PT_BWD_AUTO || one_pass > PT_BWD_SEPARATE) return PT_ERR_CONFIG;
   int st = pt::bf16_dk_check(B, H, L, K, threads_per_block);
   if (st != PT_OK) return st;
-  if (one_pass == PT_BWD_AUTO && B > 0 && H > 0 && L % 4 == 0 && H % pt::kRowsCgWaves == 0 && dy &&
-      x && w && dx && dk && pt::aligned(dy, 16) && pt::aligned(x, 16) && pt::aligned(dx, 16) &&
-      pt::aligned(w, 4) && pt::aligned(dk, 4) &&
-      pt::bwd_bf16_lds_bytes(L, 16 * (pt::mfma_index(L) + 1)) <= (size_t)pt::max_lds_per_block()) {
+  if (dy && x && w && dx && dk && pt::aligned(w, 4) && pt::aligned(dk, 4) &&
+      pt::bwd_bf16_taken(B, H, L, one_pass, dy, x, dx)) {
     const size_t need = (size_t)H * K * pt::bwd_bf16_ranges(B, H, L) * sizeof(float);
     if (!workspace || workspace_bytes < need) return PT_ERR_WORKSPACE;
     if (!pt::aligned(workspace, 4)) return PT_ERR_ALIGN;

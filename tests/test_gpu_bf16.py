@@ -247,3 +247,31 @@ def test_bf16_random_shapes(rt, shape):
     assert oracle.normalized_max_abs(ga.cpu().numpy(), ref) < DK_TOL
     assert oracle.normalized_max_abs(g1.cpu().numpy(), ref) < DK_TOL
     assert torch.equal(g1, g2)
+
+
+@pytest.mark.parametrize("B,H,L,K", [
+    (1, 8, 4, 3), (15, 8, 16, 16), (17, 24, 12, 48), (250, 16, 20, 8), (33, 40, 32, 32),
+    (100, 8, 36, 7), (129, 104, 48, 48), (1500, 96, 44, 1), (9000, 16, 28, 11), (40000, 8, 8, 9),
+    (22016, 128, 48, 40)])
+def test_bf16_one_pass_backward_is_taken(B, H, L, K):
+    """The dispatch takes the one kernel at every shape of
+    test_bf16_one_pass_backward, and not for tensors off a 16-byte boundary;
+    the launch follows (its dK, in its own order, has other bits than the
+    separate launches' wherever the sums are long)."""
+    import ctypes
+
+    from pathtile_amd import _lib, runtime
+
+    lib = _lib.load()
+    rt = runtime.HipWarpRuntime(bwdk_block=64)  # any H that is a multiple of 8
+    for aligned in (1, 0):
+        out = ctypes.c_int(-1)
+        assert lib.pt_dwconv1d_bwd_bf16_one_pass(B, H, L, K, 64, aligned, ctypes.byref(out)) == 0
+        assert out.value == aligned
+    if B * L < 1000:
+        return
+    x, w, dy = (t.cuda() for t in _inputs(B, H, L, K, seed=13 + B + L))
+    dx, dk, sk = torch.empty_like(x), torch.empty_like(w), torch.empty_like(w)
+    rt.launch_backward_bf16(dy, x, w, dx, dk)
+    rt.launch_bwd_weight_deterministic_bf16(dy, x, sk, K)
+    assert not torch.equal(dk, sk)

@@ -804,3 +804,42 @@ def test_one_pass_backward(rt, B, H, L, K):
     dx, _ = run(_lib.PT_BWD_AUTO)
     rt.launch_bwd_input(dyd, wd, sx)
     assert torch.equal(torch.isfinite(dx), torch.isfinite(sx))
+
+
+@pytest.mark.parametrize("B,H,L,K,taken", [
+    # every shape of test_one_pass_backward, and both sides of each rule
+    (1, 8, 9, 3, 1), (16, 8, 16, 16, 1), (17, 24, 17, 48, 1), (250, 16, 31, 8, 1),
+    (33, 40, 32, 32, 1), (100, 8, 33, 8, 1), (100, 8, 33, 7, 0), (129, 104, 48, 48, 1),
+    (1500, 96, 37, 48, 1), (1400, 104, 47, 1, 1), (1200, 104, 47, 1, 0), (9000, 16, 20, 11, 1),
+    (300, 8, 4, 4, 1), (70, 16, 2, 3, 1), (40000, 8, 1, 1, 1), (100, 8, 32, 7, 1),
+    (100, 12, 48, 48, 0), (0, 8, 48, 48, 0)])
+def test_one_pass_backward_is_taken(rt, monkeypatch, B, H, L, K, taken):
+    """The dispatch takes the one kernel where the tests above mean it to,
+    and the launch follows: its dK, in its own order, has other bits than the
+    separate launches' wherever the sums are long."""
+    import ctypes
+
+    from pathtile_amd import _lib
+
+    lib = _lib.load()
+
+    def ask(algo=_lib.PT_ROWS_AUTO, aligned=1):
+        out = ctypes.c_int(-1)
+        assert lib.pt_dwconv1d_bwd_one_pass(B, H, L, K, 4, algo, 128, aligned,
+                                            ctypes.byref(out)) == 0
+        return out.value
+
+    assert ask() == ask(_lib.PT_ROWS_MATRIX) == taken
+    assert ask(_lib.PT_ROWS_VALU) == ask(aligned=0) == 0
+    for name in ("PATHTILE_ROWS_ALGO", "PATHTILE_ROWS_CHANNELS", "PATHTILE_DK_ALGO"):
+        with monkeypatch.context() as m:
+            m.setenv(name, "valu")
+            assert ask() == 0
+    if B * L < 1000:
+        return
+    x, w, dy = (t.cuda() for t in _inputs(B, H, L, K, seed=B + L))
+    dx, sx, dk, sk = (torch.empty_like(t) for t in (x, x, w, w))
+    rt.launch_backward(dy, x, w, dx, dk)
+    rt.launch_bwd_input(dy, w, sx)
+    rt.launch_bwd_weight_deterministic(dy, x, sk, K)
+    assert torch.equal(dk, sk) == (not taken)
