@@ -26,7 +26,7 @@
 namespace pt {
 
 constexpr int kS4MaxH = 256;     // largest H of the fused block (H % 32 == 0)
-constexpr int kDwTok = 32;       // tokens per step of the weight gradient, one block of dP
+constexpr int kDwTok = 32;       // tokens per block of dP and step of the weight gradient
 
 // Waves of a tail workgroup for CT = H / 16 channel tiles: WPC waves side by
 // side on channels (MT tiles each, every tile with its gate tile H channels
@@ -56,10 +56,9 @@ __host__ __device__ constexpr size_t tail_fwd_lds(int H) {  // two g stages, the
   return (size_t)tail_tok(H) * (2 * 3 * (H + 8) * 2 + (H + 4) * 4);
 }
 // Byte offset of dP's (token, row) from the tile's first block of 32 tokens.
-constexpr int kDpTok = 32;
 template <int H>
 __device__ __forceinline__ uint32_t dp_offset(uint32_t tk, uint32_t row) {
-  return 4 * ((tk / kDpTok) * (2 * H * kDpTok) + row * kDpTok + tk % kDpTok);
+  return 4 * ((tk / kDwTok) * (2 * H * kDwTok) + row * kDwTok + tk % kDwTok);
 }
 
 template <int CT>
@@ -692,7 +691,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
     for (int n = 0; n < D::NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const float* const a0 =
-      dp + (16 * wave * D::MT + (lane & 15)) * kDpTok + 8 * (lane >> 4);
+      dp + (16 * wave * D::MT + (lane & 15)) * kDwTok + 8 * (lane >> 4);
   // Two sets of a step's operands where the registers allow: the loads of step
   // s + 3 are issued after step s and first used after step s + 1.
   float va[U][8], vb[U][8], ra[D::MT][8], rb[D::MT][8];
@@ -710,7 +709,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
   auto load_a = [&](float (&ar)[D::MT][8], uint32_t s) {
 #pragma unroll
     for (int m = 0; m < D::MT; ++m) {
-      const float* p = a0 + 16 * m * kDpTok + (size_t)s * (2 * H * kDpTok);
+      const float* p = a0 + 16 * m * kDwTok + (size_t)s * (2 * H * kDwTok);
       const float4 f0 = *reinterpret_cast<const float4*>(p);
       const float4 f1 = *reinterpret_cast<const float4*>(p + 4);
       ar[m][0] = f0.x;
@@ -837,7 +836,7 @@ __global__ __launch_bounds__(DwGeo<CT>::NW* kWave, 2) void s4_dw_kernel(
           const uint32_t e1 = s1 * kDwTok < ntok ? s1 * kDwTok : ntok;
 #pragma unroll 1
           for (uint32_t k = s0 * kDwTok; k < e1; ++k)
-            s = fmaf(dp[(size_t)(k / kDpTok) * (2 * H * kDpTok) + c * kDpTok + k % kDpTok],
+            s = fmaf(dp[(size_t)(k / kDwTok) * (2 * H * kDwTok) + c * kDwTok + k % kDwTok],
                      gelu_f(v[(size_t)k * H + h]), s);
         }
         dst[(size_t)c * H + h] = s;
