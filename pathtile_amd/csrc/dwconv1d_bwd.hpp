@@ -274,7 +274,6 @@ __global__ __launch_bounds__(kRowsCgWaves* kWave, 4) void dwconv_bwd_bf16_kernel
   constexpr int NUB = LMAX / 4;   // input columns per K group of a lane
   constexpr int NG = NUB / 4;     // MFMAs (16 input columns) per dX tile
   constexpr int TH = HC * kWave;
-  constexpr int kDepth = 1;   // steps in flight in registers
   constexpr int kNpt = (HC * LMAX * kRowsCgStep / 8 + TH - 1) / TH;
   extern __shared__ float lds[];
 
@@ -307,7 +306,7 @@ __global__ __launch_bounds__(kRowsCgWaves* kWave, 4) void dwconv_bwd_bf16_kernel
     eoff[i] = (uint32_t)k * row_bytes + grp_bytes + 16u * (uint32_t)q;
     elds[i] = (uint32_t)(k * sk + 8 * q);
   }
-  u32x4 stg[kDepth][2][kNpt];  // [step][dY, x]
+  u32x4 stg[2][kNpt];  // dY, x of the step in flight
   auto load_step = [&](int s, u32x4 (&st)[2][kNpt]) {
     const int bs = (r + s * nranges) * kRowsCgStep;
     const size_t at = (size_t)bs * (size_t)H * (size_t)L;
@@ -417,26 +416,18 @@ __global__ __launch_bounds__(kRowsCgWaves* kWave, 4) void dwconv_bwd_bf16_kernel
   };
 
   if (nsteps > 0) {
-#pragma unroll
-    for (int d = 0; d < kDepth; ++d)
-      if (d < nsteps) load_step(d, stg[d]);
-    store_stage(0, stg[0]);
-    if (kDepth < nsteps) load_step(kDepth, stg[0]);
+    load_step(0, stg);
+    store_stage(0, stg);
+    if (1 < nsteps) load_step(1, stg);
     __syncthreads();
-    for (int s0 = 0; s0 < nsteps; s0 += kDepth) {
-#pragma unroll
-      for (int d = 0; d < kDepth; ++d) {
-        const int s = s0 + d;
-        if (s < nsteps) {
-          if (s + 1 < nsteps) {
-            store_stage((s + 1) & 1, stg[(d + 1) % kDepth]);
-            if (s + 1 + kDepth < nsteps) load_step(s + 1 + kDepth, stg[(d + 1) % kDepth]);
-          }
-          mfma_step(s);
-          __syncthreads();
-          flush_out(s);
-        }
+    for (int s = 0; s < nsteps; ++s) {
+      if (s + 1 < nsteps) {
+        store_stage((s + 1) & 1, stg);
+        if (s + 2 < nsteps) load_step(s + 2, stg);
       }
+      mfma_step(s);
+      __syncthreads();
+      flush_out(s);
     }
     __syncthreads();  // the epilogue's tiles take the stages' place
   }
