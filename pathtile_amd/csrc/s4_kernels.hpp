@@ -72,9 +72,12 @@ __host__ __device__ constexpr size_t wfrag_values(int H) { return (size_t)3 * 2 
 
 // The normal distribution function without branches: for a = |x|,
 // Q(a) = 1 - cdf(a) = exp(-a^2 / 2) R(a) with R(a) = erfcx(a / sqrt 2) / 2 as
-// an 8-term polynomial in t = 1 / (1 + 9/32 a), fitted (weighted minimax, the
-// coefficients rounded to FP32 one after the other) to 4e-10 of gelu; 20
-// instructions where erff takes about 75 on both of its branches. The
+// t times a polynomial of degree 7 in t = 1 / (1 + 9/32 a); 20 instructions
+// where erff takes about 75 on both of its branches. The fit minimises the
+// largest max(1, a) |error of Q| over 0 <= a <= 8 (Lawson's weighted least
+// squares), its coefficients rounded to FP32 from the constant up with the
+// others fitted again: 3.9e-10 of the cdf and of gelu, of which 2.1e-10 before
+// the rounding (the CPU tests fit it anew). The
 // exponential also gives the density. a is cut at 20, where Q underflows, so
 // that infinities keep the formula's values (gelu(-inf) = NaN).
 struct NormalCdf {

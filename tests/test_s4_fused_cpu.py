@@ -325,3 +325,48 @@ def test_the_ends_save_what_their_gradients_read(calls, end):
         wrt = [t for t in (x, w, b) if t.requires_grad]
         for g, t in zip(torch.autograd.grad(out, wrt, torch.ones_like(out)), wrt):
             assert g.shape == t.shape and g.dtype == torch.float32
+
+
+def test_gelu_polynomial_against_a_new_fit():
+    """The coefficients in s4_kernels.hpp: their error in FP64, and that of a
+    fit by the method that the comment there names (Lawson's iteration for
+    the weighted minimax, one coefficient rounded at a time)."""
+    import re
+    from pathlib import Path
+
+    import numpy as np
+    from scipy.special import erfcx
+
+    text = (Path(s4convd.__file__).parent / "csrc" / "s4_kernels.hpp").read_text()
+    body = text[text.index("NormalCdf normal_cdf"):text.index("float gelu_f")]
+    have = [float(c) for c in re.findall(r"(?:r = |t, )(-?[\d.]+)f[;)]", body)
+            if abs(float(c)) < 1.0][::-1]
+    assert len(have) == 8
+
+    def parts(a):
+        t = 1 / (1 + 9 / 32 * a)
+        return t, np.maximum(1, a) * np.exp(-a * a / 2), erfcx(a / np.sqrt(2)) / 2
+
+    def worst(c):
+        t, w, r = parts(np.linspace(0, 20, 100001))
+        return np.abs(w * (t * np.polynomial.polynomial.polyval(t, c) - r)).max()
+
+    def fit(fixed):
+        t, w, r = parts(np.linspace(0, 8, 2001))
+        n = len(fixed)
+        A = np.stack([w * t * t**k for k in range(n, 8)], 1)
+        b = w * (r - t * np.polynomial.polynomial.polyval(t, fixed or [0.0]))
+        p, best = np.ones(len(t)), (np.inf, None)
+        for _ in range(300):
+            c = np.linalg.lstsq(A * np.sqrt(p)[:, None], b * np.sqrt(p), rcond=None)[0]
+            e = np.abs(A @ c - b)
+            best = min(best, (e.max(), list(c)), key=lambda q: q[0])
+            p = p * e / (p * e).sum()
+        return best
+
+    fixed = []
+    for _ in range(8):
+        fixed.append(float(np.float32(fit(fixed)[1][0])))
+    assert fit([])[0] < 2.2e-10
+    assert worst(have) < 4e-10 and worst(have) < 1.2 * worst(fixed)
+    np.testing.assert_allclose(have, fixed, rtol=1e-4)
