@@ -195,7 +195,10 @@ int pt_kernel_choice_forced(void);
  * deterministic as there, in its own order). one_pass: PT_BWD_AUTO takes the
  * one kernel where it is faster, with H % 8 == 0, 16-byte aligned tensors,
  * algo not PT_ROWS_VALU and no PATHTILE_* kernel choice set; PT_BWD_SEPARATE
- * never. The workspace serves either.
+ * never. The workspace serves either. The one kernel sums dx on the matrix
+ * cores also where pt_dwconv1d_dx_f32's rule takes a VALU kernel for few taps
+ * (the reference's chain bit for bit: PT_ROWS_VALU keeps it), and does not use
+ * waves_per_block and threads_per_block.
  */
 #define PT_BWD_AUTO 0
 #define PT_BWD_SEPARATE 1

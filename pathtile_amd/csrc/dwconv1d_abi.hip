@@ -1160,7 +1160,7 @@ static bool kernel_choice_forced() {
 
 // --- one-pass backward -------------------------------------------------------
 // dX and dK from one read of dY (dwconv_bwd_cg_kernel), one 8-channel
-// workgroup per CU. Served wherever the channel-group dX is: H % 8 == 0 and
+// workgroup per CU or two (bwd_cg_ranges). Served wherever the channel-group dX is: H % 8 == 0 and
 // 16-byte aligned tensors, any L. One pass / separate with inputs rotated past
 // the MALL: B16384 H128 L48 K48 0.85, B32768 H256 L48 K4 0.83, B16384 H128 L4
 // K4 0.74, L16 K16 0.80, L32 K32 0.81, B60000 H8 L24 K24 0.56, B1000 H96 L37

@@ -44,9 +44,10 @@ static uint32_t token_magic(int L) { return L == 1 ? 0u : (uint32_t)((1ULL << 32
 
 static size_t round_up(size_t n, size_t q) { return (n + q - 1) / q * q; }
 
-// Token ranges of the weight gradient: one workgroup per CU (its accumulators
-// and fragments take half of the registers), at least four 32-token steps
-// each. A function of the shape alone, so that the workspace is too.
+// Token ranges of the weight gradient: one workgroup on each of 256 CUs (its
+// accumulators and fragments take half of the registers), at least four
+// 32-token steps each. The count depends on the shape alone, so that dW's bits
+// do; the whole workspace also on the device, through dk_cl_ranges.
 static uint32_t dw_steps_per_range(uint32_t nsteps, int split) {
   const uint32_t ranges = 256u / (uint32_t)split;
   const uint32_t per = (nsteps + ranges - 1) / ranges;

@@ -26,9 +26,13 @@ __host__ __device__ constexpr int conv_cl_threads(int H) {
 // where such a tap meets a value that is not finite the chain is repeated
 // without them. MASK: the output times a dropout mask [B, H, L], whose row a
 // lane reads as whole dwords, and scale. COPY: x as it was read, for a
-// backward that must not depend on what becomes of x. Bound by the FMA issue at 48 taps (36 per output on average, 92 us of
-// it at B16384 L48 H128): FWD 200 us, DX 246 us there, against 305 and 366 with
-// the transposes.
+// backward that must not depend on what becomes of x, stored with the outputs
+// (one block's forward and backward at B2048 L48 H128 368 -> 377 us; stored
+// before the products, where the loads then have to be waited for at once, 389;
+// a separate copy 379). 36 FMAs per output on average at 48 taps are 92 us of
+// issue at B16384 L48 H128, beside two tensor passes (128 us at the rate of a
+// large copy): FWD 176 us (4.6 TB/s), 231 with the mask, DX, three passes, 241
+// (5.0 TB/s), VALU 45 to 47% busy, against 305 and 366 with the transposes.
 template <int LMAX, bool DX, bool MASK, bool COPY>
 __global__ __launch_bounds__(kConvClThreads, LMAX > 40 ? 3 : 4) void s4_conv_cl_kernel(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ add,

@@ -350,13 +350,14 @@ __device__ __forceinline__ void project_fix(f32x4& a, f32x4& b, const float* v,
 // H = 128, what the LDS holds). gelu is as much vector work as the products
 // are matrix work, and both kinds from one wave overlap where they are
 // interleaved in one stretch of code (two workgroups that share a CU fall
-// into step instead and add the two up: 452 us at B16384 L48 H128, 388
-// here, 3.1 TB/s with the matrix cores 42% busy), so tile t + 1's gelu and split
-// run in the shadow of tile t's products, into the other of two stages. The
-// weight fragments stay in registers up to H = 128 (streamed from the L2 they
-// cost 511 us) and stream above. For a later backward, q [2][tokens][H] gets
-// the values P[c] + bias and the gates' sigmoids. GLU results pass through an FP32 stage
-// to flat 16-byte rows with the residual.
+// into step instead and add the two up: 452 us at B16384 L48 H128 against 388),
+// so tile t + 1's gelu and split run in the shadow of tile t's products, into
+// the other of two stages. The weight fragments stay in registers up to H = 128
+// (streamed from the L2 they cost 511 us) and stream above. For a later backward, q [2][tokens][H] gets
+// the values P[c] + bias and the gates' sigmoids. GLU results pass through an
+// FP32 stage to flat 16-byte rows with the residual. Averages of a trace at
+// B16384 L48 H128: 442 us, 459 with q (4.4 TB/s, matrix cores 32% and VALU 45%
+// busy).
 // ---------------------------------------------------------------------------
 template <int CT>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
@@ -442,8 +443,9 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_fwd_kernel(
 // H = 128 the LDS holds one stage, the GLU gradient comes before the product
 // and the fragments stream. Seven tensor passes of HBM bound it; recomputing
 // the pre-activations instead of reading q took 5 passes but 975 us at B16384
-// L48 H128 on the sum of its matrix and vector work, 605 us now (the forward,
-// which writes q, 388 -> 490).
+// L48 H128 on the sum of its matrix and vector work, 698 with q read (the
+// forward, which writes it, 388 -> 483 then). Now 632 us in a trace (4.5 TB/s,
+// matrix cores 22% and VALU 33% busy).
 // ---------------------------------------------------------------------------
 template <int CT, bool MASK>
 __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
@@ -648,7 +650,11 @@ __global__ __launch_bounds__(TailGeo<CT>::NW* kWave, 2) void s4_tail_bwd_kernel(
 // shared through LDS [part][channel][40]. Partials [range][2 H H + 2 H] go to
 // the workspace for a fixed-order reduction. Step s + 1's gelu and splits run
 // in the shadow of step s's products: 354 us at B16384 L48 H128, 430 with them
-// ahead of the products.
+// ahead of the products; with two sets of loads in flight 315 (matrix cores 47%
+// and VALU 55% busy). The matrix instruction's rounding towards minus infinity
+// (step_negated) is not cancelled here: it moves dW by -2.8e-6 of its mean
+// magnitude there, of an error against FP64 of 2.3e-6 (7.4e-6 as a library FP32
+// product; B2048 L48 H128 4.3e-7 against 3.5e-6).
 // ---------------------------------------------------------------------------
 template <int CT>
 struct DwGeo {

@@ -368,7 +368,9 @@ class HipWarpRuntime:
 
     waves_per_block     FWD wavefronts per workgroup (1, 2, 4, 8, 16)
     dx_waves_per_block  dX wavefronts per workgroup (default: waves_per_block)
-    bwdk_block          dK threads per workgroup (multiple of 64, <= 768)
+    bwdk_block          dK threads per workgroup (multiple of 64, <= 768); this
+                        and dx_waves_per_block configure the separate launches
+                        (the one-pass backward has a geometry of its own)
     bwdk_btile          samples per dK wave chunk; fixed at 64 (one per lane)
     fast_math           accepted for signature compatibility; the kernels are
                         FMA-only, so it changes nothing
@@ -606,7 +608,10 @@ class HipWarpRuntime:
                         gx: torch.Tensor, gk: torch.Tensor) -> None:
         """dX and the deterministic dK in one call of the library, which reads
         gy once for both where its one-pass kernel serves (pt_dwconv1d_bwd_f32);
-        with KERNEL_EVENTS recording, the two launches that it names."""
+        with KERNEL_EVENTS recording, the two launches that it names. The one
+        pass sums dX on the matrix cores also where launch_bwd_input's rule
+        takes a VALU kernel (few taps): rows_algo="valu" keeps the reference's
+        chain bit for bit here too."""
         self._check_open()
         B, H, L, K = self._check_shapes(gy, k)
         if KERNEL_EVENTS.enabled:
