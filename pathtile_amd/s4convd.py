@@ -248,7 +248,7 @@ class S4BlockFused(torch.autograd.Function):
         saved = ctx.saved_tensors
         need = ctx.needs_input_grad[:9]
         if _as_operations(gy):
-            return _composed_grads(ctx, gy, saved[-1])
+            return _composed_grads(ctx, gy, saved[10], saved[-1])
         (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
          prep, v, q, mask) = map(_unpacked, saved, ctx.forms)
         runtime = get_runtime()
@@ -284,7 +284,7 @@ def _as_operations(gy: torch.Tensor) -> bool:
             or torch._C._functorch.is_functorch_wrapped_tensor(gy))
 
 
-def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
+def _composed_grads(ctx: Any, gy: torch.Tensor, v, mask):
     """The block's gradients through torch's operations on the saved inputs
     (the convolution's own backward stays first order and takes one gradient,
     as its autograd function is). They are taken at aliases: where x was
@@ -296,10 +296,13 @@ def _composed_grads(ctx: Any, gy: torch.Tensor, mask):
     with torch.enable_grad():
         inputs = [t.view_as(t) if n else t.detach() for t, n in zip(ctx.saved_tensors, need)]
         x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
-        k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
-        v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)
-        if mask is not None:
-            v = v * mask * ctx.scale
+        if any(need[:7]):
+            k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])
+            v = depthwise_conv_skip_ampere(x.transpose(1, 2).contiguous(), k, skip)
+            if mask is not None:
+                v = v * mask * ctx.scale
+        else:  # the forward's, without a convolution that vmap cannot enter
+            v = v.detach().transpose(1, 2)
         z = nn.functional.conv1d(nn.functional.gelu(v), weight, bias)
         y = nn.functional.glu(z, dim=1).transpose(1, 2) + x
         got = iter(torch.autograd.grad(y, [t for t, n in zip(inputs, need) if n], gy,

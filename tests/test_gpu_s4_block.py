@@ -482,8 +482,9 @@ def test_forced_kernel_choices_reach_the_blocks_launches(monkeypatch, how):
     assert torch.equal(seen[0], own)
 
 
-def test_batches_of_gradients_of_the_projection():
-    """is_grads_batched where the separate operations take it: with the
+@pytest.mark.parametrize("how", ["is_grads_batched", "vmap"])
+def test_batches_of_gradients_of_the_projection(how):
+    """Batches of gradients where the separate operations take them: with the
     convolution's side frozen, against one gradient at a time."""
     block, x, gy = _make(3, 32, 20, 8)
     block.cuda()
@@ -494,7 +495,10 @@ def test_batches_of_gradients_of_the_projection():
     gys = torch.stack([gy.cuda(), 2 - gy.cuda()])
     wrt = (conv.weight, conv.bias)
     with torch.backends.cudnn.flags(enabled=False):
-        batch = torch.autograd.grad(y, wrt, gys, is_grads_batched=True, retain_graph=True)
+        if how == "vmap":
+            batch = torch.vmap(lambda g: torch.autograd.grad(y, wrt, g, retain_graph=True))(gys)
+        else:
+            batch = torch.autograd.grad(y, wrt, gys, is_grads_batched=True, retain_graph=True)
     for i in range(2):
         for a, b in zip(batch, torch.autograd.grad(y, wrt, gys[i], retain_graph=True)):
             assert _rel(a[i], b) < PAR_TOL

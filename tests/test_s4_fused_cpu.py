@@ -370,3 +370,23 @@ def test_gelu_polynomial_against_a_new_fit():
     assert fit([])[0] < 2.2e-10
     assert worst(have) < 4e-10 and worst(have) < 1.2 * worst(fixed)
     np.testing.assert_allclose(have, fixed, rtol=1e-4)
+
+
+def test_projections_gradients_need_no_second_convolution(calls, composed, monkeypatch):
+    """Batched gradients of the projection alone come from the forward's
+    values: vmap cannot enter the convolution's autograd function."""
+    torch.manual_seed(13)
+    inputs = [t.double() for t in _block_inputs(2, 6, 32, 4)]
+    wrt = [t.requires_grad_(True) for t in inputs[7:]]
+    y = s4convd.S4BlockFused.apply(*inputs, 0.5)
+
+    def refuse(*args):
+        raise AssertionError("a convolution ran")
+
+    monkeypatch.setattr(s4convd, "depthwise_conv_skip_ampere", refuse)
+    gys = torch.randn(3, *y.shape, dtype=y.dtype)
+    batch = torch.vmap(lambda g: torch.autograd.grad(y, wrt, g, retain_graph=True))(gys)
+    for i in range(3):
+        ones = torch.autograd.grad(y, wrt, gys[i], create_graph=True)
+        for a, g in zip(batch, ones):
+            assert torch.allclose(a[i], g, rtol=1e-10, atol=1e-12)
