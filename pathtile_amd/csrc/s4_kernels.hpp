@@ -109,13 +109,14 @@ __device__ __forceinline__ float gelu_grad_f(float x) {
   return fmaf(x, n.e * 0.39894228040143268f, n.cdf);
 }
 
-// 1 / (1 + exp(-x)), NaN kept; past 87 the result is 1 or below FP32's range.
+// 1 / (1 + exp(-x)), NaN kept; above 87 the result is 1, and 0 where exp(-x)
+// is past FP32's range (an infinite value times such a gate is NaN).
 __device__ __forceinline__ float sigmoid_f(float x) {
   const float c = x > 87.0f ? 87.0f : x < -87.0f ? -87.0f : x;
   const float d =
       1.0f + __builtin_amdgcn_exp2f(-fmaf(c, 1.44269502162933349609375f, c * 1.92596303e-08f));
   const float t = __builtin_amdgcn_rcpf(d);
-  return fmaf(t, fmaf(-d, t, 1.0f), t);
+  return x < -88.7228394f ? 0.0f : fmaf(t, fmaf(-d, t, 1.0f), t);
 }
 
 __device__ __forceinline__ bool finite4(float a, float b, float c, float d) {

@@ -535,3 +535,20 @@ def test_model_ends_partial_gradients():
             full = full or got
             for a, c in zip(got, full):
                 assert a is None or _rel(a, c) < 1e-6
+
+
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+def test_fused_block_kinds_of_non_finite_outputs(value):
+    """An infinite skip term makes whole rows of values and gates infinite:
+    every output is finite, an infinity of a sign, or NaN as it is for the
+    separate operations."""
+    block, x, _ = _make(4, 64, 24, 16)
+    block.cuda()
+    x = x.cuda()
+    with torch.no_grad(), torch.backends.cudnn.flags(enabled=False):
+        block.skip[5] = value
+        got = block(x)
+        block.activation.register_forward_hook(lambda *a: None)
+        ref = block(x)
+    for kind in (torch.isfinite, torch.isposinf, torch.isneginf, torch.isnan):
+        assert torch.equal(kind(got), kind(ref)), kind.__name__
