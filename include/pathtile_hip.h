@@ -332,8 +332,8 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
  * both operands split three ways (FP32 accuracy; a sum that is not finite is
  * recomputed by the FP32 chain).
  *
- * prep holds the taps and the split projection between the calls of one
- * block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
+ * prep holds the taps, the split projection, dt and Re A between the calls of
+ * one block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
  * also lays out what _bwd needs. x_copy (NULL: none) gets x, for a _bwd that
  * must not depend on what becomes of x. mask is dropout's byte mask in [B, H, L]
  * order, 4-byte aligned (NULL: none): v = conv * mask * scale. q [2, B L, H], written by _tail where not NULL, holds the projection's values and the
@@ -341,7 +341,7 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
  * outputs gx, {dw, dbias} and the six parameter gradients (all or none, by
  * d_skip) are each skipped where NULL.
  */
-int pt_s4_block_prep_values(int H, int L, size_t* floats);
+int pt_s4_block_prep_values(int H, int L, int states, size_t* floats);
 int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re,
                         const float* c_im, const float* log_a_re, const float* a_im,
                         const float* skip, const float* w, const unsigned char* mask,
@@ -353,9 +353,8 @@ int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, cons
 int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, size_t* bytes);
 int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const float* q,
                         const unsigned char* mask, float scale, const float* prep,
-                        const float* w, const float* log_dt, const float* c_re,
-                        const float* c_im, const float* log_a_re, const float* a_im,
-                        float* gx, float* d_log_dt, float* d_c_re, float* d_c_im,
+                        const float* w, const float* c_re, const float* c_im,
+                        const float* a_im, float* gx, float* d_log_dt, float* d_c_re, float* d_c_im,
                         float* d_log_a_re, float* d_a_im, float* d_skip, float* dw,
                         float* dbias, void* workspace, size_t workspace_bytes, int B,
                         int H, int L, int states, void* stream);

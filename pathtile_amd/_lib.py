@@ -90,14 +90,14 @@ SIGNATURES = {
     "pt_dwconv1d_dk_long_f32": (
         _i, [_vp, _vp, _vp, _vp, ctypes.c_size_t, _i, _i, _i, _i, _vp]
     ),
-    "pt_s4_block_prep_values": (_i, [_i, _i, _szp]),
+    "pt_s4_block_prep_values": (_i, [_i] * 3 + [_szp]),
     "pt_s4_block_mix_f32": (
         _i, [_vp] * 9 + [ctypes.c_float] + [_vp] * 3 + [_i] * 5 + [_vp]
     ),
     "pt_s4_block_tail_f32": (_i, [_vp] * 7 + [_i] * 3 + [_vp]),
     "pt_s4_block_bwd_workspace_bytes": (_i, [_i, _i, _i, _szp]),
     "pt_s4_block_bwd_f32": (
-        _i, [_vp] * 5 + [ctypes.c_float] + [_vp] * 17 + [ctypes.c_size_t] + [_i] * 4 + [_vp]
+        _i, [_vp] * 5 + [ctypes.c_float] + [_vp] * 15 + [ctypes.c_size_t] + [_i] * 4 + [_vp]
     ),
     "pt_s4_encode_f32": (_i, [_vp] * 4 + [_i] * 4 + [_vp]),
     "pt_s4_encode_grad_workspace_bytes": (_i, [_i] * 4 + [_szp]),

@@ -44,6 +44,10 @@ static uint32_t token_magic(int L) { return L == 1 ? 0u : (uint32_t)((1ULL << 32
 
 static size_t round_up(size_t n, size_t q) { return (n + q - 1) / q * q; }
 
+// prep, in floats: taps, the split weights, the poles.
+static size_t prep_weights(int H, int L) { return round_up((size_t)H * L, 64); }
+static size_t prep_poles(int H, int L) { return prep_weights(H, L) + wfrag_values(H); }
+
 // Token ranges of the weight gradient: one workgroup on each of 256 CUs (its
 // accumulators and fragments take half of the registers), at least four
 // 32-token steps each. The count depends on the shape alone, so that dW's bits
@@ -133,11 +137,11 @@ static int reduce_launch(const float* part, float* dw, float* db, int nw, int nb
 
 extern "C" {
 
-int pt_s4_block_prep_values(int H, int L, size_t* floats) {
+int pt_s4_block_prep_values(int H, int L, int states, size_t* floats) {
   if (!floats) return PT_ERR_NULL;
-  const int st = pt::check_block(1, H, L, 1);
+  const int st = pt::check_block(1, H, L, states);
   if (st != PT_OK) return st;
-  *floats = pt::round_up((size_t)H * L, 64) + pt::wfrag_values(H);
+  *floats = pt::prep_poles(H, L) + (size_t)H * (1 + (size_t)states);
   return PT_OK;
 }
 
@@ -153,12 +157,12 @@ int pt_s4_block_mix_f32(const float* x, const float* log_dt, const float* c_re, 
   if (!pt::aligned16(x) || !pt::aligned16(prep) || !pt::aligned16(v) ||
       !pt::aligned16(x_copy) || !pt::aligned(mask, 4))
     return PT_ERR_ALIGN;
-  float* taps = prep;
-  __bf16* wf = reinterpret_cast<__bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  float *taps = prep, *poles = prep + pt::prep_poles(H, L);
+  __bf16* wf = reinterpret_cast<__bf16*>(prep + pt::prep_weights(H, L));
   const int frags = 2 * H * H / 8 * (backward ? 2 : 1);
   const uint32_t grid = (uint32_t)(H + (frags + pt::kPrepThreads - 1) / pt::kPrepThreads);
-  void* args[] = {&log_dt, &c_re, &c_im, &log_a_re, &a_im, &skip, &w, &taps, &wf, &H, &L,
-                  &states, &backward};
+  void* args[] = {&log_dt, &c_re, &c_im, &log_a_re, &a_im, &skip, &w, &taps, &wf,
+                  &poles, &H, &L, &states, &backward};
   st = pt::launch((const void*)&pt::s4_prep_kernel, grid, pt::kPrepThreads, 0, stream, args);
   if (st != PT_OK) return st;
   return pt::conv_cl_launch(x, taps, nullptr, mask, scale, v, x_copy, B, H, L, stream);
@@ -174,7 +178,7 @@ int pt_s4_block_tail_f32(const float* v, const float* x, const float* prep, cons
       !pt::aligned16(y) || !pt::aligned16(q))
     return PT_ERR_ALIGN;
   const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
-  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::prep_weights(H, L));
   uint32_t ntok = (uint32_t)B * (uint32_t)L;
   uint32_t ntiles = (ntok + k.tok - 1) / k.tok;
   const size_t lds = pt::tail_fwd_lds(H);
@@ -197,17 +201,16 @@ int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, size_t* bytes) {
 
 int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const float* q,
                         const unsigned char* mask, float scale, const float* prep, const float* w,
-                        const float* log_dt, const float* c_re, const float* c_im,
-                        const float* log_a_re, const float* a_im, float* gx, float* d_log_dt,
-                        float* d_c_re, float* d_c_im, float* d_log_a_re, float* d_a_im,
-                        float* d_skip, float* dw, float* dbias, void* workspace,
+                        const float* c_re, const float* c_im, const float* a_im, float* gx,
+                        float* d_log_dt, float* d_c_re, float* d_c_im, float* d_log_a_re,
+                        float* d_a_im, float* d_skip, float* dw, float* dbias, void* workspace,
                         size_t workspace_bytes, int B, int H, int L, int states, void* stream) {
   int st = pt::check_block(B, H, L, states);
   if (st != PT_OK) return st;
   if (!gy || !x || !v || !q || !prep || !w) return PT_ERR_NULL;
   const bool taps_grad = d_skip != nullptr;
-  if (taps_grad && (!log_dt || !c_re || !c_im || !log_a_re || !a_im || !d_log_dt || !d_c_re ||
-                    !d_c_im || !d_log_a_re || !d_a_im))
+  if (taps_grad && (!c_re || !c_im || !a_im || !d_log_dt || !d_c_re || !d_c_im || !d_log_a_re ||
+                    !d_a_im))
     return PT_ERR_NULL;
   if ((dw == nullptr) != (dbias == nullptr)) return PT_ERR_NULL;
   if (!pt::aligned16(gy) || !pt::aligned16(x) || !pt::aligned16(v) || !pt::aligned16(prep) ||
@@ -220,8 +223,8 @@ int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const f
   const pt::TailGeometry& k = pt::kTail[H / 32 - 1];
   float* const ws = static_cast<float*>(workspace);
   float *dp = ws, *du = ws + o.du, *part = ws + o.part, *dk = ws + o.dk;
-  const float* taps = prep;
-  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::round_up((size_t)H * L, 64));
+  const float *taps = prep, *poles = prep + pt::prep_poles(H, L);
+  const __bf16* wf = reinterpret_cast<const __bf16*>(prep + pt::prep_weights(H, L));
   uint32_t ntok = (uint32_t)B * (uint32_t)L, uL = (uint32_t)L, magic = pt::token_magic(L);
   {
     uint32_t ntiles = (ntok + k.btok - 1) / k.btok;
@@ -249,8 +252,8 @@ int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const f
   st = pt::dk_cl_det(x, du, dk, ws + o.dkp, B, H, L, L, o.dk_ranges, stream);
   if (st != PT_OK) return st;
   const float* cdk = dk;
-  void* targs[] = {&cdk, &log_dt, &c_re, &c_im, &log_a_re, &a_im, &d_log_dt, &d_c_re, &d_c_im,
-                   &d_log_a_re, &d_a_im, &d_skip, &L, &states};
+  void* targs[] = {&cdk, &poles, &c_re, &c_im, &a_im, &d_log_dt, &d_c_re, &d_c_im, &d_log_a_re,
+                   &d_a_im, &d_skip, &L, &states};
   return pt::launch((const void*)&pt::s4_taps_grad_kernel, (uint32_t)H, pt::kPrepThreads, 0, stream,
                     targs);
 }

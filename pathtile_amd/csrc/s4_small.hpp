@@ -15,7 +15,8 @@ namespace pt {
 // l % 16, contraction values 8 (l / 16) .. + 7), three parts each:
 //   wf[((ct * 2 + half) * KS + ks) * 3 + part][lane][8]   rows of W
 //   wt[(ct * 2 KS + ks) * 3 + part][lane][8]              rows of W^T
-// so that a wave's fragment is one contiguous 1 KiB read.
+// so that a wave's fragment is one contiguous 1 KiB read. poles: dt [H], then
+// Re A [H][N2], which the taps' gradient reads.
 // The taps are the reference's formula in FP32 with exp(dt A) - 1 from
 // expm1 and sin^2 (no cancellation at small dt A).
 // ---------------------------------------------------------------------------
@@ -55,19 +56,21 @@ __global__ __launch_bounds__(kPrepThreads) void s4_prep_kernel(
     const float* __restrict__ c_im, const float* __restrict__ log_a_re,
     const float* __restrict__ a_im, const float* __restrict__ skip,
     const float* __restrict__ w, float* __restrict__ taps, __bf16* __restrict__ wf,
-    int H, int L, int N2, int transposed) {
+    float* __restrict__ poles, int H, int L, int N2, int transposed) {
   const int tid = threadIdx.x;
   if ((int)blockIdx.x < H) {
     const int h = blockIdx.x;
     __shared__ float ce[2][kPrepStates], da[2][kPrepStates];
     __shared__ float part[kMaxL][kPrepStates + 1];
     const float dt = expf(log_dt[h]);
+    if (tid == 0) poles[h] = dt;
     float acc = 0.0f;  // thread t < L: taps[h][t]
     for (int n0 = 0; n0 < N2; n0 += kPrepStates) {
       const int nn = N2 - n0 < kPrepStates ? N2 - n0 : kPrepStates;
       if (tid < nn) {
         const int i = h * N2 + n0 + tid;
         const Cf A = {-expf(log_a_re[i]), a_im[i]};
+        poles[H + i] = A.re;
         const Cf dA = {A.re * dt, A.im * dt};
         const Cf e = cdiv(cmul(Cf{c_re[i], c_im[i]}, cexpm1(dA)), A);
         ce[0][tid] = e.re;
@@ -126,7 +129,8 @@ __global__ __launch_bounds__(kPrepThreads) void s4_prep_kernel(
 
 // ---------------------------------------------------------------------------
 // Gradient of the taps with respect to the kernel's parameters, from
-// dk [H][L]: with z = exp(dt A), E = z - 1, S0 = sum_t dk[t] z^t,
+// dk [H][L] and the preparation's poles: with z = exp(dt A), E = z - 1,
+// S0 = sum_t dk[t] z^t,
 // S1 = sum_t t dk[t] z^t per state,
 //   dL = 2 Re sum_n ( S0 E / A dC + R dA + (S0 C z + C_eff A S1) ddt ),
 //   R  = S0 C / A^2 (z dt A - E) + dt C_eff S1,
@@ -134,9 +138,8 @@ __global__ __launch_bounds__(kPrepThreads) void s4_prep_kernel(
 // that factor and E are computed in FP64 (a handful of operations per state).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kPrepThreads) void s4_taps_grad_kernel(
-    const float* __restrict__ dk, const float* __restrict__ log_dt,
-    const float* __restrict__ c_re, const float* __restrict__ c_im,
-    const float* __restrict__ log_a_re, const float* __restrict__ a_im,
+    const float* __restrict__ dk, const float* __restrict__ poles,
+    const float* __restrict__ c_re, const float* __restrict__ c_im, const float* __restrict__ a_im,
     float* __restrict__ d_log_dt, float* __restrict__ d_c_re, float* __restrict__ d_c_im,
     float* __restrict__ d_log_a_re, float* __restrict__ d_a_im, float* __restrict__ d_skip,
     int L, int N2) {
@@ -146,16 +149,17 @@ __global__ __launch_bounds__(kPrepThreads) void s4_taps_grad_kernel(
   __shared__ float s1r[kPrepStates][kChunks], s1i[kPrepStates][kChunks];
   __shared__ float ddt[kPrepStates];
   const int h = blockIdx.x, tid = threadIdx.x;
+  const float* const a_re = poles + gridDim.x;  // after dt, one per channel
   if (tid < L) sdk[tid] = dk[h * L + tid];
   __syncthreads();
-  const float dt = expf(log_dt[h]);
+  const float dt = poles[h];
   float ddt_sum = 0.0f;  // thread 0
   for (int n0 = 0; n0 < N2; n0 += kPrepStates) {
     const int nn = N2 - n0 < kPrepStates ? N2 - n0 : kPrepStates;
     const int n = tid / kChunks, q = tid % kChunks;
     if (n < nn) {
       const int i = h * N2 + n0 + n;
-      const Cf dA = {-expf(log_a_re[i]) * dt, a_im[i] * dt};
+      const Cf dA = {a_re[i] * dt, a_im[i] * dt};
       Cf s0 = {0.f, 0.f}, s1 = {0.f, 0.f};
       for (int t = q; t < L; t += kChunks) {
         const Cf z = cexp_at(dA, (float)t);
@@ -180,7 +184,7 @@ __global__ __launch_bounds__(kPrepThreads) void s4_taps_grad_kernel(
         S1r += s1r[tid][k];
         S1i += s1i[tid][k];
       }
-      const double ar = -(double)expf(log_a_re[i]), ai = a_im[i], d = dt;
+      const double ar = a_re[i], ai = a_im[i], d = dt;
       const double cr = c_re[i], ci = c_im[i];
       const double xr = ar * d, xi = ai * d;
       double sn, cs;

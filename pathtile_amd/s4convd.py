@@ -187,7 +187,7 @@ def _fused_mix(x: torch.Tensor, skip, log_dt, c_re, c_im, log_a_re, a_im, weight
     runtime = get_runtime()
     runtime._check_open()
     B, L, H = x.shape
-    prep = x.new_empty(_size_query("pt_s4_block_prep_values", H, L))
+    prep = x.new_empty(_size_query("pt_s4_block_prep_values", H, L, c_re.shape[1]))
     v = torch.empty_like(x)
     _call(runtime._lib.pt_s4_block_mix_f32, x.device,
           _ptr(x), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
@@ -215,7 +215,10 @@ class S4BlockFused(torch.autograd.Function):
     ``copy`` it reads a copy that the convolution writes on its way, so that
     x may change in between (``x += block(x)``; the separate operations save
     the copy that their transpose makes). The copy is a second output: that
-    ties it to x for a backward that is differentiated."""
+    ties it to x for a backward that is differentiated. Of the parameters it
+    saves those that the separate operations save as they are, so that the
+    others may change as well: their values are in prep, and only a backward
+    as torch's operations reads them again."""
 
     @staticmethod
     def forward(ctx: Any, x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias, p: float,
@@ -228,10 +231,11 @@ class S4BlockFused(torch.autograd.Function):
                              ctx.scale, True, x_copy)
         q = x.new_empty((2, *x.shape))
         y = _fused_tail(v, x, prep, weight, bias, q)
-        saved = (x_copy if copy else x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-                 prep, v, q, mask)
+        saved = (x_copy if copy else x, c_re, c_im, a_im, weight, prep, v, q, mask)
         ctx.forms = [_form(t) for t in saved]
         ctx.save_for_backward(*saved)
+        ctx.unsaved = skip, log_dt, log_a_re, bias
+        ctx.versions = _versions(ctx.unsaved)
         return (y, x_copy) if copy else y
 
     @staticmethod
@@ -248,9 +252,9 @@ class S4BlockFused(torch.autograd.Function):
         saved = ctx.saved_tensors
         need = ctx.needs_input_grad[:9]
         if _as_operations(gy):
-            return _composed_grads(ctx, gy, saved[10], saved[-1])
-        (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias,
-         prep, v, q, mask) = map(_unpacked, saved, ctx.forms)
+            return _composed_grads(ctx, gy)
+        x, c_re, c_im, a_im, weight, prep, v, q, mask = map(_unpacked, saved, ctx.forms)
+        skip, log_dt, log_a_re, bias = ctx.unsaved
         runtime = get_runtime()
         runtime._check_open()
         B, L, H = x.shape
@@ -269,11 +273,14 @@ class S4BlockFused(torch.autograd.Function):
 
         _call(runtime._lib.pt_s4_block_bwd_f32, x.device,
               _ptr(gy), _ptr(x), _ptr(v), _ptr(q), opt(mask), ctx.scale, _ptr(prep),
-              _ptr(weight), _ptr(log_dt), _ptr(c_re), _ptr(c_im), _ptr(log_a_re), _ptr(a_im),
-              opt(gx), *(opt(t) for t in gp), opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L,
-              c_re.shape[1])
+              _ptr(weight), _ptr(c_re), _ptr(c_im), _ptr(a_im), opt(gx), *(opt(t) for t in gp),
+              opt(gw), opt(gb), _ptr(ws), nbytes, B, H, L, c_re.shape[1])
         grads = [gx, gp[5], *gp[:5], gw, gb]
         return [g if n else None for g, n in zip(grads, need)]
+
+
+def _versions(tensors) -> list:
+    return [None if t.is_inference() else t._version for t in tensors]
 
 
 def _as_operations(gy: torch.Tensor) -> bool:
@@ -284,7 +291,7 @@ def _as_operations(gy: torch.Tensor) -> bool:
             or torch._C._functorch.is_functorch_wrapped_tensor(gy))
 
 
-def _composed_grads(ctx: Any, gy: torch.Tensor, v, mask):
+def _composed_grads(ctx: Any, gy: torch.Tensor):
     """The block's gradients through torch's operations on the saved inputs
     (the convolution's own backward stays first order and takes one gradient,
     as its autograd function is). They are taken at aliases: where x was
@@ -293,8 +300,14 @@ def _composed_grads(ctx: Any, gy: torch.Tensor, v, mask):
     the engine adds by itself."""
     create_graph = torch.is_grad_enabled()
     need = ctx.needs_input_grad[:9]
+    x, c_re, c_im, a_im, weight, _, v, _, mask = ctx.saved_tensors
+    skip, log_dt, log_a_re, bias = ctx.unsaved
+    if _versions(ctx.unsaved) != ctx.versions:
+        raise RuntimeError("a parameter of the block was modified by an inplace operation "
+                           "before a backward that is differentiated")
     with torch.enable_grad():
-        inputs = [t.view_as(t) if n else t.detach() for t, n in zip(ctx.saved_tensors, need)]
+        inputs = [t.view_as(t) if n else t.detach() for t, n in zip(
+            (x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias), need)]
         x, skip, log_dt, c_re, c_im, log_a_re, a_im, weight, bias = inputs
         if any(need[:7]):
             k = _taps(log_dt, c_re, c_im, log_a_re, a_im, x.shape[1])

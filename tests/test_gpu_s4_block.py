@@ -552,3 +552,18 @@ def test_fused_block_kinds_of_non_finite_outputs(value):
         ref = block(x)
     for kind in (torch.isfinite, torch.isposinf, torch.isneginf, torch.isnan):
         assert torch.equal(kind(got), kind(ref)), kind.__name__
+
+
+@pytest.mark.parametrize("name", ["skip", "kernel_layer.log_dt", "kernel_layer.log_A_re",
+                                  "output_linear.0.bias"])
+def test_fused_blocks_parameters_that_may_change_before_its_backward(name):
+    """The gradients are those at the values that the forward saw."""
+    block, x, gy = _make(4, 64, 24, 16)
+    block.cuda()
+    x, gy = x.cuda(), gy.cuda()
+    ref = _grads(block, x, gy)[1:]
+    y = block(x.requires_grad_(True))
+    with torch.no_grad():
+        block.get_parameter(name).add_(0.5)
+    got = torch.autograd.grad(y, (x, *block.parameters()), gy)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))

@@ -46,7 +46,7 @@ def test_buffers_are_fp32_under_any_default_dtype(calls, default_dtype, dtype):
     B, L, H, half = 3, 5, 32, 4
     inputs = tuple(t.requires_grad_(True) for t in _block_inputs(B, L, H, half))
     y = s4convd.S4BlockFused.apply(*inputs, 0.0)
-    prep, v, q = y.grad_fn.saved_tensors[9:12]
+    prep, v, q = y.grad_fn.saved_tensors[5:8]
     for t in (y, prep, v, q, *torch.autograd.grad(y, inputs, torch.ones_like(y))):
         assert t.dtype == torch.float32
     assert q.shape == (2, B, L, H)
@@ -390,3 +390,27 @@ def test_projections_gradients_need_no_second_convolution(calls, composed, monke
         ones = torch.autograd.grad(y, wrt, gys[i], create_graph=True)
         for a, g in zip(batch, ones):
             assert torch.allclose(a[i], g, rtol=1e-10, atol=1e-12)
+
+
+PARAMETERS = ("skip", "log_dt", "c_re", "c_im", "log_a_re", "a_im", "weight", "bias")
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+@pytest.mark.parametrize("changed", range(8), ids=lambda i: PARAMETERS[i])
+def test_parameters_that_change_before_the_backward(calls, composed, changed, create_graph):
+    """As with the separate operations: those that they save as they are
+    raise, the others do not; a backward that is differentiated reads all of
+    them and raises for each."""
+    inputs = [t.requires_grad_(True) for t in _block_inputs(2, 6, 32, 4)]
+    y = s4convd.S4BlockFused.apply(*inputs, 0.0)
+    with torch.no_grad():
+        inputs[1 + changed].add_(1.0)
+
+    def backward():
+        return torch.autograd.grad(y.sum(), inputs, create_graph=create_graph)
+
+    if create_graph or PARAMETERS[changed] in ("c_re", "c_im", "a_im", "weight"):
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            backward()
+    else:
+        assert [g.shape for g in backward()] == [t.shape for t in inputs]
