@@ -335,9 +335,11 @@ int flash_dk_fp32(const float* x, const float* dy, float* dw, int B, int H,
  * prep holds the taps, the split projection, dt and Re A between the calls of
  * one block: pt_s4_block_prep_values floats, filled by _mix; backward != 0 there
  * also lays out what _bwd needs. x_copy (NULL: none) gets x, for a _bwd that
- * must not depend on what becomes of x. mask is dropout's byte mask in [B, H, L]
- * order, 4-byte aligned (NULL: none): v = conv * mask * scale. q [2, B L, H], written by _tail where not NULL, holds the projection's values and the
- * gates' sigmoids for _bwd, which takes x, v, q and the mask again. Its
+ * must not depend on what becomes of x. mask is dropout's byte mask in
+ * [B, H, L] order, 4-byte aligned (NULL: none): v = conv * mask * scale.
+ * q [2, B L, H], written by _tail where not NULL, holds the projection's
+ * values and the gates' sigmoids for _bwd, which takes x (or its copy), v, q,
+ * the mask and prep again, and c_re, c_im, a_im and w as _mix had them. Its
  * outputs gx, {dw, dbias} and the six parameter gradients (all or none, by
  * d_skip) are each skipped where NULL.
  */
@@ -354,8 +356,8 @@ int pt_s4_block_bwd_workspace_bytes(int B, int H, int L, size_t* bytes);
 int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const float* q,
                         const unsigned char* mask, float scale, const float* prep,
                         const float* w, const float* c_re, const float* c_im,
-                        const float* a_im, float* gx, float* d_log_dt, float* d_c_re, float* d_c_im,
-                        float* d_log_a_re, float* d_a_im, float* d_skip, float* dw,
+                        const float* a_im, float* gx, float* d_log_dt, float* d_c_re,
+                        float* d_c_im, float* d_log_a_re, float* d_a_im, float* d_skip, float* dw,
                         float* dbias, void* workspace, size_t workspace_bytes, int B,
                         int H, int L, int states, void* stream);
 
@@ -366,8 +368,8 @@ int pt_s4_block_bwd_f32(const float* gy, const float* x, const float* v, const f
  * outputs] = x[:, L-1, :] w^T + bias, w [outputs, H], outputs <= 4: the
  * decoder at the one column that the model returns. The *_grad calls give the
  * gradients of w and bias by a fixed-order reduction, and the head's gx [B,
- * L, H] (NULL: skipped, and w may be too), zero before the last column. bias, y, gy of the
- * encoder and x, gx of the head are 16-byte aligned.
+ * L, H] (NULL: skipped, and w may be NULL too), zero before the last column.
+ * bias, y, gy of the encoder and x, gx of the head are 16-byte aligned.
  */
 int pt_s4_encode_f32(const float* x, const float* w, const float* bias, float* y, int B,
                      int L, int inputs, int H, void* stream);
